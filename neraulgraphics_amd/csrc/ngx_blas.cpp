@@ -232,10 +232,8 @@ void build_meshes(const MeshInput &in, BuiltMeshes &out) {
         WideNode &w = out.wide[wide_index[i]];
         const BlasNode &l = out.nodes[n.a], &r = out.nodes[n.a + 1];
         for (int k = 0; k < 3; ++k) {
-            w.l_lo[k] = l.lo[k];
-            w.l_hi[k] = l.hi[k];
-            w.r_lo[k] = r.lo[k];
-            w.r_hi[k] = r.hi[k];
+            w.set_left(k, l.lo[k], l.hi[k]);
+            w.set_right(k, r.lo[k], r.hi[k]);
         }
         child_ref(l, n.a, w.left, w.left_count);
         child_ref(r, n.a + 1, w.right, w.right_count);

@@ -41,10 +41,17 @@ static_assert(sizeof(TlasNode) == 32 && sizeof(BlasNode) == 32, "32-byte nodes")
 // of the same array; < 0 a leaf, ~ref being an instance (top level) or the first triangle of a run of
 // `count` (bottom level).
 struct alignas(64) WideNode {
-    float l_lo[3], l_hi[3];
-    float r_lo[3], r_hi[3];
+    float plane[3][4];  // per axis: left lo, right lo, left hi, right hi
     int32_t left, right;
     int32_t left_count, right_count;
+    __host__ __device__ void set_left(const int axis, const float lo, const float hi) {
+        plane[axis][0] = lo;
+        plane[axis][2] = hi;
+    }
+    __host__ __device__ void set_right(const int axis, const float lo, const float hi) {
+        plane[axis][1] = lo;
+        plane[axis][3] = hi;
+    }
 };
 static_assert(sizeof(WideNode) == 64, "64-byte wide node");
 
@@ -106,9 +113,21 @@ __device__ __forceinline__ float rcp_rn(const float x) {
 
 __device__ __forceinline__ float3 normalize3(const float3 v) { return mul3(v, rcp_rn(sqrtf(dot3(v, v)))); }
 
-// 1/x that never gives infinity (mesh_dev.h:58-61).
-__device__ __forceinline__ float safe_rcp(const float x) { return rcp_rn(fabsf(x) < 1e-12f ? copysignf(1e-12f, x) : x); }
-__device__ __forceinline__ float3 safe_inverse(const float3 d) { return mk3(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z)); }
+// rcp_rn within its range, without the check.
+__device__ __forceinline__ float rcp_in_range(const float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+
+// 1/x that never gives infinity (mesh_dev.h:58-61), per component. The smallest magnitude inverted is 1e-12, so only
+// the upper end of rcp_rn's range is checked, once for the three (a NaN gives a NaN either way).
+__device__ __forceinline__ float safe_nonzero(const float x) { return fabsf(x) < 1e-12f ? copysignf(1e-12f, x) : x; }
+__device__ __forceinline__ float3 safe_inverse(const float3 d) {
+    const float3 s = mk3(safe_nonzero(d.x), safe_nonzero(d.y), safe_nonzero(d.z));
+    float3 r = mk3(rcp_in_range(s.x), rcp_in_range(s.y), rcp_in_range(s.z));
+    if (__builtin_expect(fmaxf(fmaxf(fabsf(s.x), fabsf(s.y)), fabsf(s.z)) >= 0x1p126f, 0)) r = mk3(1.0f / s.x, 1.0f / s.y, 1.0f / s.z);
+    return r;
+}
 
 // Slab test (mesh_dev.h:66-74): entry distance, or NO_HIT when missed or beyond tmax.
 __device__ __forceinline__ float box_entry(const float lx, const float ly, const float lz, const float hx, const float hy,
@@ -128,13 +147,20 @@ __device__ __forceinline__ float box_entry(const float lx, const float ly, const
 // terms, 0 and tmax, are numbers). Computing lim once per node keeps the per-box work to the slab test.
 constexpr float BELOW_NO_HIT = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, NO_HIT) - 1u);
 __device__ __forceinline__ float box_limit(const float tmax) { return fminf(tmax, BELOW_NO_HIT); }
+// fminf of two values known not to be signalling NaNs. The compiler, which cannot know that of a value read from LDS or
+// another lane, would first multiply each operand out (one instruction more per use).
+__device__ __forceinline__ float min_quiet(const float a, const float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
 __device__ __forceinline__ bool box_hit(const float lx, const float ly, const float lz, const float hx, const float hy,
                                         const float hz, const float3 o, const float3 inv_d, const float lim, float &tn) {
     const float tx0 = (lx - o.x) * inv_d.x, tx1 = (hx - o.x) * inv_d.x;
     const float ty0 = (ly - o.y) * inv_d.y, ty1 = (hy - o.y) * inv_d.y;
     const float tz0 = (lz - o.z) * inv_d.z, tz1 = (hz - o.z) * inv_d.z;
     tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), 0.0f));
-    const float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fminf(fmaxf(tz0, tz1), lim));
+    const float tf = min_quiet(fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fmaxf(tz0, tz1)), lim);
     return tn <= tf;
 }
 
@@ -147,22 +173,22 @@ __device__ __forceinline__ void load_tri(const float *tris, const size_t j, floa
 }
 
 // Two-sided Moller-Trumbore (mesh_dev.h:80-99), triangle given as v0, e1, e2.
+// Every condition is worked out and the lot taken together: an early way out for some of a wave's lanes saves the others
+// nothing and costs a change of the execution mask. A lane that fails the first condition may hold any values after it.
 __device__ __forceinline__ bool triangle_hit(const float3 v0, const float3 e1, const float3 e2, const float3 o, const float3 d,
                                              const float tmax, float &t, float &bu, float &bv) {
     const float3 p = cross3(d, e2);
     const float det = dot3(e1, p);
-    if (fabsf(det) < 1e-14f) return false;
-    const float inv_det = rcp_rn(det);
+    float inv_det = rcp_in_range(det);
+    if (__builtin_expect(!(fabsf(det) < 0x1p126f), 0)) inv_det = 1.0f / det;
     const float3 s = sub3(o, v0);
     const float u = dot3(s, p) * inv_det;
-    if (u < 0.0f || u > 1.0f) return false;
     const float3 q = cross3(s, e1);
     const float v = dot3(d, q) * inv_det;
-    if (v < 0.0f || u + v > 1.0f) return false;
     t = dot3(e2, q) * inv_det;
     bu = u;
     bv = v;
-    return t > 0.0f && t < tmax;
+    return !(fabsf(det) < 1e-14f) & !(u < 0.0f) & !(u > 1.0f) & !(v < 0.0f) & !(u + v > 1.0f) & (t > 0.0f) & (t < tmax);
 }
 
 // ------------------------------------------------------------------ wave primitives --

@@ -78,10 +78,8 @@ __global__ __launch_bounds__(256) void refit_layout_kernel(const MeshRefitArgs A
         const SkipNode &l = A.skip[n.a], &r = A.skip[n.a + 1];
         WideNode &o = A.wide[w];
         for (int ax = 0; ax < 3; ++ax) {
-            o.l_lo[ax] = l.lo[ax];
-            o.l_hi[ax] = l.hi[ax];
-            o.r_lo[ax] = r.lo[ax];
-            o.r_hi[ax] = r.hi[ax];
+            o.set_left(ax, l.lo[ax], l.hi[ax]);
+            o.set_right(ax, r.lo[ax], r.hi[ax]);
         }
     }
     if (node == A.root) {

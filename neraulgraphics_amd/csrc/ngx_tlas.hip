@@ -241,8 +241,8 @@ __device__ __forceinline__ void write_interior(const TlasBuildArgs &A, const int
     A.nodes[gi] = node;
     WideNode wn;
     for (int ax = 0; ax < 3; ++ax) {
-        wn.l_lo[ax] = llo[ax]; wn.l_hi[ax] = lhi[ax];
-        wn.r_lo[ax] = rlo[ax]; wn.r_hi[ax] = rhi[ax];
+        wn.set_left(ax, llo[ax], lhi[ax]);
+        wn.set_right(ax, rlo[ax], rhi[ax]);
     }
     wn.left = l >= n - 1 ? ~(a + id(l - (n - 1))) : a + l;
     wn.right = r >= n - 1 ? ~(a + id(r - (n - 1))) : a + r;

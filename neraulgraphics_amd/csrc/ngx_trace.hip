@@ -12,6 +12,13 @@
 // ray enters before its current closest distance, and keeps a hit only when strictly closer
 // (mesh_dev.h:98), so the result equals the per-ray walk's except where two surfaces meet the ray at the
 // same distance.
+//
+// What bounds these kernels is instruction issue, of vector, scalar and branch instructions together (the 4096-world
+// 128x128 render: 5.66 G vector, 3.36 G scalar and 0.83 G branch instructions; its time follows their sum), so the
+// walks are written for few instructions a visit: arguments read where they are used, wave-uniform stacks in vector
+// registers, a triangle test without early ways out, one range check for three reciprocals, selects where both sides
+// are cheap. Together 8.44 -> 7.69 ms there, 13.7 -> 13.2 ms for 67 M LiDAR rays.
+#include <cstddef>
 #include <mutex>
 #include "ngx_kernels.h"
 
@@ -28,6 +35,56 @@ struct LaneHit {
     float u, v;
 };
 
+// The kernel's arguments, read from their segment again wherever this is called: the empty asm statement keeps the
+// compiler from seeing that it is the same address, so it loads a field where the field is used (through the scalar
+// cache) rather than once at the start. A traversal kernel has more arguments than scalar registers to hold them across
+// its walk, and one held all the same is kept in a lane of a vector register, which costs a vector instruction a read.
+template <class T>
+using KernelArgs = __attribute__((address_space(4))) const T;
+template <class T>
+__device__ __forceinline__ KernelArgs<T> &kernel_args() {
+    auto *p = (KernelArgs<T> *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *p;
+}
+// A pointer to global memory, which the compiler cannot tell of one read from the arguments this way.
+template <class T>
+__device__ __forceinline__ T *in_global(T *p) { return (T *)(__attribute__((address_space(1))) T *)p; }
+
+// The scene of the running kernel, whose arguments begin with a TraceScene.
+struct Scene {
+#define NGX_SCENE_POINTER(type, name) \
+    __device__ __forceinline__ type *name() const { return in_global(kernel_args<TraceScene>().name); }
+#define NGX_SCENE_VALUE(type, name) \
+    __device__ __forceinline__ type name() const { return kernel_args<TraceScene>().name; }
+    NGX_SCENE_POINTER(const WideNode, tlas_wide)
+    NGX_SCENE_POINTER(const int, tlas_parent)
+    NGX_SCENE_POINTER(const int, blas_parent)
+    NGX_SCENE_POINTER(const int, blas_wide_node)
+    NGX_SCENE_POINTER(const int, roots)
+    NGX_SCENE_POINTER(const InstanceRec, inst)
+    NGX_SCENE_POINTER(const MeshRoot, mesh_roots)
+    NGX_SCENE_POINTER(const WideNode, blas_wide)
+    NGX_SCENE_POINTER(const float, tris)
+    NGX_SCENE_POINTER(const float4, attrs)
+    NGX_SCENE_POINTER(const float4, spheres)
+    NGX_SCENE_POINTER(const SkipNode, skip)
+    NGX_SCENE_POINTER(int, overflow)
+    NGX_SCENE_VALUE(int, total)
+    NGX_SCENE_VALUE(int, sphere_count)
+    NGX_SCENE_VALUE(float, floor_y)
+    NGX_SCENE_VALUE(float, floor_hx)
+    NGX_SCENE_VALUE(float, floor_zmin)
+    NGX_SCENE_VALUE(float, floor_zmax)
+    NGX_SCENE_VALUE(int, pair_limit)
+    NGX_SCENE_VALUE(int, lane_min_tris)
+    NGX_SCENE_VALUE(int, share_cap)
+#undef NGX_SCENE_POINTER
+#undef NGX_SCENE_VALUE
+};
+static_assert(offsetof(RenderArgs, s) == 0 && offsetof(RgbArgs, r) == 0 && offsetof(RayArgs, s) == 0 &&
+              offsetof(DepthBackwardArgs, s) == 0 && offsetof(RangeBackwardArgs, s) == 0, "every kernel's arguments begin with the scene");
+
 // Traversal counters of one wavefront, wave-uniform. NoStats compiles them away; WaveStats is only used by the
 // instrumented kernel built with NGX_TRACE_STATS.
 enum StatIndex { ST_TLAS_NODES, ST_TLAS_LANES, ST_INSTANCES, ST_INSTANCE_LANES, ST_INSTANCE_ROOT_LANES, ST_BLAS_NODES,
@@ -41,26 +98,32 @@ enum StatIndex { ST_TLAS_NODES, ST_TLAS_LANES, ST_INSTANCES, ST_INSTANCE_LANES, 
 // skip layout, which needs fewer registers (the RGB kernel, whose spills the other raises: body_worlds RGB 34.7 ->
 // 44.4 ms, where the depth kernel gains 10.1 -> 9.3 ms and the LiDAR query 21.1 -> 16.4 ms).
 struct NoStats {
-    static constexpr bool kAnyHit = false, kHandoff = true, kTwoChild = true;
+    static constexpr bool kAnyHit = false, kHandoff = true, kTwoChild = true, kOneOrigin = false;
+    __device__ __forceinline__ void add(int, int) {}
+};
+// Camera rays: every ray of the wave starts at the camera, so what an instance makes of the origin is one point for the
+// wave, held in scalar registers.
+struct CameraRays {
+    static constexpr bool kAnyHit = false, kHandoff = true, kTwoChild = true, kOneOrigin = true;
     __device__ __forceinline__ void add(int, int) {}
 };
 struct ShadeRays {
-    static constexpr bool kAnyHit = false, kHandoff = false, kTwoChild = false;
+    static constexpr bool kAnyHit = false, kHandoff = false, kTwoChild = false, kOneOrigin = false;
     __device__ __forceinline__ void add(int, int) {}
 };
 struct Occlusion {
-    static constexpr bool kAnyHit = true, kHandoff = false, kTwoChild = false;
+    static constexpr bool kAnyHit = true, kHandoff = false, kTwoChild = false, kOneOrigin = false;
     __device__ __forceinline__ void add(int, int) {}
 };
 // Shadow rays of the two-pass picture, whose second pass holds no primary walk: the depth kernel's walk, stopping
 // each ray at its first hit (body_worlds RGB + depth + ID 26.9 ms a step with the one-box-a-step walk here, 26.1 so).
 struct OcclusionTwoChild {
-    static constexpr bool kAnyHit = true, kHandoff = true, kTwoChild = true;
+    static constexpr bool kAnyHit = true, kHandoff = true, kTwoChild = true, kOneOrigin = false;
     __device__ __forceinline__ void add(int, int) {}
 };
 #ifdef NGX_TRACE_STATS
 struct WaveStats {
-    static constexpr bool kAnyHit = false, kHandoff = true, kTwoChild = true;
+    static constexpr bool kAnyHit = false, kHandoff = true, kTwoChild = true, kOneOrigin = true;
     int c[ST_COUNT];
     __device__ __forceinline__ void add(const int k, const int v) { c[k] += v; }
 };
@@ -76,9 +139,9 @@ __device__ __forceinline__ Wide load_wide(const WideNode *nodes, const int index
     const float4 f0 = sload4(p), f1 = sload4(p + 1), f2 = sload4(p + 2);
     const int4 f3 = sload4i(reinterpret_cast<const int4 *>(p + 3));
     Wide w;
-    w.l_lo[0] = f0.x; w.l_lo[1] = f0.y; w.l_lo[2] = f0.z; w.l_hi[0] = f0.w;
-    w.l_hi[1] = f1.x; w.l_hi[2] = f1.y; w.r_lo[0] = f1.z; w.r_lo[1] = f1.w;
-    w.r_lo[2] = f2.x; w.r_hi[0] = f2.y; w.r_hi[1] = f2.z; w.r_hi[2] = f2.w;
+    w.l_lo[0] = f0.x; w.r_lo[0] = f0.y; w.l_hi[0] = f0.z; w.r_hi[0] = f0.w;
+    w.l_lo[1] = f1.x; w.r_lo[1] = f1.y; w.l_hi[1] = f1.z; w.r_hi[1] = f1.w;
+    w.l_lo[2] = f2.x; w.r_lo[2] = f2.y; w.l_hi[2] = f2.z; w.r_hi[2] = f2.w;
     w.left = f3.x; w.right = f3.y; w.lcount = f3.z; w.rcount = f3.w;
     return w;
 }
@@ -94,20 +157,21 @@ __device__ __forceinline__ Wide load_wide(const WideNode *nodes, const int index
 // order as the floats do). That is what testing the triangles one by one with a strict "closer than"
 // keeps (mesh_dev.h:98, :186-199). A ray's limit is not lowered until its batch is tested, so a few
 // more boxes may be entered; that costs time, not correctness.
+// 3,328 bytes a wavefront.
 struct PairLds {
     int pair[64];                  // ray lane | triangle << 6
     unsigned long long best[64];   // per ray lane: distance bits << 32 | pair number
-    float2 uv[64];                 // per pair: barycentrics of its hit
-    float2 hit_uv[64];             // per ray lane: barycentrics of its closest hit so far
-    int hit_inst[64], hit_tri[64]; // per ray lane: instance and triangle of its closest hit so far (-1: none)
+    int4 hit[64];                  // per ray lane: instance (-1: none), triangle and barycentrics of its closest hit so far
     // the per-lane bottom-level walk's shared work: subtrees given away (ray lane | node << 6), and a ring of
     // leaves waiting for their triangle tests (first triangle; ray lane | count << 6)
     int share[128];
-    int leaf_first[128], leaf_ray_count[128];
-    // the packet walk's two wave-uniform stacks (top level, bottom level): node reference and lane mask
-    int st_ref[2][WALK_STACK];
-    uint32_t st_lo[2][WALK_STACK], st_hi[2][WALK_STACK];
+    int2 leaf[128];
 };
+
+// v of the lane whose number is in bits 2 to 7 of four_times_lane.
+__device__ __forceinline__ float lane_read(const float v, const int four_times_lane) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(four_times_lane, __float_as_int(v)));
+}
 
 // Orders a wavefront's LDS accesses: a wavefront's LDS operations are performed in order, so a
 // compiler barrier is all that is needed between one lane's write and another lane's read.
@@ -121,41 +185,40 @@ __device__ __forceinline__ int rank_in(const uint64_t mask) {
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// A wave-uniform stack of (node reference, lane mask) in the wavefront's LDS: one lane writes a push, every
-// lane reads a pop (the same address for all, so it is broadcast) and the value is taken as uniform.
-struct LdsStack {
-    int *ref;
-    uint32_t *lo, *hi;
-    int *overflow;
+// old with lane `lane`'s value replaced by v (both wave-uniform); clang has no builtin of this instruction's name.
+extern "C" __device__ __attribute__((const)) int ngx_write_lane(int v, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+__device__ __forceinline__ int write_lane(const int v, const int lane, const int old) { return ngx_write_lane(v, lane, old); }
+
+// A wave-uniform stack of (node reference, lane mask) in three vector registers, entry k in lane k: a push or a pop is
+// three instructions and waits for nothing.
+struct WaveStack {
+    int ref, lo, hi;
     int sp;
-    __device__ __forceinline__ LdsStack(PairLds *L, const int level, int *flag)
-        : ref(L->st_ref[level]), lo(L->st_lo[level]), hi(L->st_hi[level]), overflow(flag), sp(0) {}
+    __device__ __forceinline__ WaveStack() : ref(0), lo(0), hi(0), sp(0) {}
     // Depth bounds keep sp below WALK_STACK (a top-level tree has fewer than 64 levels below a world's root, and the
     // host refuses bottom-level trees deeper than 60). A tree that breaks them anyway loses the entry that does not
     // fit, and the walk reports it through the scene's overflow flag, which the host turns into an error.
     __device__ __forceinline__ void push(const int r, const uint64_t m) {
-        if (sp >= WALK_STACK) {
-            if (lane_id() == 0) *overflow = 1;
+        if (__builtin_expect(sp >= WALK_STACK, 0)) {
+            if (lane_id() == 0) *Scene().overflow() = 1;
             return;
         }
-        if (lane_id() == 0) {
-            ref[sp] = r;
-            lo[sp] = (uint32_t)m;
-            hi[sp] = (uint32_t)(m >> 32);
-        }
+        ref = write_lane(r, sp, ref);
+        lo = write_lane((int)(uint32_t)m, sp, lo);
+        hi = write_lane((int)(uint32_t)(m >> 32), sp, hi);
         ++sp;
     }
     __device__ __forceinline__ void pop(int &r, uint64_t &m) {
         --sp;
-        wave_lds_order();
-        r = uniform(ref[sp]);
-        m = ((uint64_t)uniform_u(hi[sp]) << 32) | uniform_u(lo[sp]);
+        r = __builtin_amdgcn_readlane(ref, sp);
+        m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, sp) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, sp);
     }
 };
+static_assert(WALK_STACK <= 64, "an entry a lane");
 
 // Tests the queued pairs of instance inst, whose mesh-space ray is (lo, ld) in each ray's lane.
 template <class Stats>
-__device__ __forceinline__ void flush_pairs(const TraceScene &S, PairLds *L, int &pairs, const int inst, const float3 lo,
+__device__ __forceinline__ void flush_pairs(const Scene S, PairLds *L, int &pairs, const int inst, const float3 lo,
                                             const float3 ld, float &tmax, Stats &stats) {
     if (pairs == 0) return;
     stats.add(ST_TRIANGLES, 1);
@@ -164,38 +227,35 @@ __device__ __forceinline__ void flush_pairs(const TraceScene &S, PairLds *L, int
     L->best[lane] = ((unsigned long long)__float_as_uint(tmax) << 32) | 0xffffffffull;
     wave_lds_order();
     const bool act = lane < pairs;
-    const int e = act ? L->pair[lane] : 0;
+    const int e = L->pair[lane];
     const int r = e & 63;
-    const float3 po = mk3(__shfl(lo.x, r, 64), __shfl(lo.y, r, 64), __shfl(lo.z, r, 64));
+    float3 po = lo;
+    if (!Stats::kOneOrigin) po = mk3(__shfl(lo.x, r, 64), __shfl(lo.y, r, 64), __shfl(lo.z, r, 64));
     const float3 pd = mk3(__shfl(ld.x, r, 64), __shfl(ld.y, r, 64), __shfl(ld.z, r, 64));
     const float pt = __shfl(tmax, r, 64);
+    pairs = 0;
+    float t = 0.0f, bu = 0.0f, bv = 0.0f;
+    bool found = false;
     if (act) {
         float3 v0, e1, e2;
-        load_tri(S.tris, (size_t)(e >> 6), v0, e1, e2);
-        float t, bu, bv;
-        if (triangle_hit(v0, e1, e2, po, pd, pt, t, bu, bv)) {
-            atomicMin(&L->best[r], ((unsigned long long)__float_as_uint(t) << 32) | (unsigned)lane);
-            L->uv[lane] = make_float2(bu, bv);
-        }
+        load_tri(S.tris(), (uint32_t)e >> 6, v0, e1, e2);
+        found = triangle_hit(v0, e1, e2, po, pd, pt, t, bu, bv);
     }
+    if (ballot(found) == 0) return;
+    const unsigned long long mine = ((unsigned long long)__float_as_uint(t) << 32) | (unsigned)lane;
+    if (found) atomicMin(&L->best[r], mine);
     wave_lds_order();
+    // the pair that won writes its ray's hit; it is kept in LDS, not registers, until the walk is over
+    if (found && L->best[r] == mine) L->hit[r] = make_int4(inst, (int)((uint32_t)e >> 6), __float_as_int(bu), __float_as_int(bv));
     const unsigned long long b = L->best[lane];
-    const unsigned p = (unsigned)b;
-    if (p != 0xffffffffu) {
-        tmax = Stats::kAnyHit ? -1.0f : __uint_as_float((unsigned)(b >> 32));
-        // the hit is kept in LDS, not registers, until the walk is over
-        L->hit_inst[lane] = inst;
-        L->hit_tri[lane] = L->pair[p] >> 6;
-        L->hit_uv[lane] = L->uv[p];
-    }
+    tmax = !Stats::kAnyHit ? __uint_as_float((unsigned)(b >> 32)) : (unsigned)b != 0xffffffffu ? -1.0f : tmax;
     wave_lds_order();
-    pairs = 0;
 }
 
 // Queues the triangles first .. first+count-1 for the rays in mask, testing the queue first whenever it
 // would overflow.
 template <class Stats>
-__device__ __forceinline__ void add_leaf(const TraceScene &S, PairLds *L, int &pairs, const int first, const int count,
+__device__ __forceinline__ void add_leaf(const Scene S, PairLds *L, int &pairs, const int first, const int count,
                                          const uint64_t mask, const int inst, const float3 lo, const float3 ld, float &tmax,
                                          LaneHit &h, Stats &stats) {
     const int m = popc64(mask);
@@ -205,7 +265,7 @@ __device__ __forceinline__ void add_leaf(const TraceScene &S, PairLds *L, int &p
     const int fit = 64 / m;
     for (int done = 0; done < count;) {
         const int c = min(count - done, fit);
-        if (pairs + m * c > S.pair_limit) flush_pairs(S, L, pairs, inst, lo, ld, tmax, stats);
+        if (pairs + m * c > S.pair_limit()) flush_pairs(S, L, pairs, inst, lo, ld, tmax, stats);
         if (in) {
             const int base = pairs + rank * c;
             for (int k = 0; k < c; ++k) L->pair[base + k] = lane | ((first + done + k) << 6);
@@ -240,7 +300,7 @@ constexpr int SHARE_CAP = SHARE_STACK, LEAF_RING = 128;
 #endif
 
 template <bool FORCE, class Stats>
-__device__ __forceinline__ void test_queued_leaves(const TraceScene &S, PairLds *L, int &head, int &count, const int g,
+__device__ __forceinline__ void test_queued_leaves(const Scene S, PairLds *L, int &head, int &count, const int g,
                                                    const float3 lo, const float3 ld, float &tmax, Stats &stats) {
     const int lane = lane_id();
     while (count > 0) {
@@ -248,8 +308,9 @@ __device__ __forceinline__ void test_queued_leaves(const TraceScene &S, PairLds 
         const int avail = min(count, 64);
         const bool mine = lane < avail;
         const int slot = (head + lane) & (LEAF_RING - 1);
-        const int rc = mine ? L->leaf_ray_count[slot] : 0;
-        const int first = mine ? L->leaf_first[slot] : 0;
+        const int2 queued_leaf = L->leaf[slot];
+        const int rc = mine ? queued_leaf.y : 0;
+        const int first = queued_leaf.x;
         const int c = rc >> 6;
         const int c0 = __builtin_amdgcn_readlane(c, 0);
         if (c0 > 64) {
@@ -259,8 +320,7 @@ __device__ __forceinline__ void test_queued_leaves(const TraceScene &S, PairLds 
             wave_lds_order();
             L->pair[lane] = ray0 | ((first0 + lane) << 6);
             if (lane == 0) {
-                L->leaf_first[head] = first0 + 64;
-                L->leaf_ray_count[head] = ray0 | ((c0 - 64) << 6);
+                L->leaf[head] = make_int2(first0 + 64, ray0 | ((c0 - 64) << 6));
             }
             int pairs = 64;
             flush_pairs(S, L, pairs, g, lo, ld, tmax, stats);
@@ -290,11 +350,12 @@ __device__ __forceinline__ void share_subtree(PairLds *L, int &top, const uint64
 
 // Walks the `top` subtrees on the shared stack (rays of instance g, whose mesh-space rays are in their own lanes).
 template <class Stats>
-__device__ void walk_shared(const TraceScene &S, PairLds *L, const int g, int top, const float3 lo, const float3 ld,
+__device__ void walk_shared(const Scene S, PairLds *L, const int g, int top, const float3 lo, const float3 ld,
                             const float3 inv_ld, float &tmax, Stats &stats) {
     const int lane = lane_id();
     int head = 0, queued = 0;
     int ray = -1, cur = -1, end = -1, oct = 0;
+    const SkipNode *const skip = S.skip();
     float3 wlo = lo, wld = ld, winv = inv_ld;
     float wlim = tmax;
     while (true) {
@@ -320,7 +381,7 @@ __device__ void walk_shared(const TraceScene &S, PairLds *L, const int g, int to
             if (take) {
                 oct = (wld.x >= 0.0f ? 1 : 0) | (wld.y >= 0.0f ? 2 : 0) | (wld.z >= 0.0f ? 4 : 0);
                 cur = start;
-                end = S.skip[start].escape[oct];
+                end = skip[start].escape[oct];
             }
         }
         const uint64_t busy = ballot(ray >= 0);
@@ -334,7 +395,7 @@ __device__ void walk_shared(const TraceScene &S, PairLds *L, const int g, int to
         int esc = unknown_i();
         if (in_mask(busy)) {
             // a 32-bit byte offset from the array's base (node indices stay below 2^25)
-            const char *np = reinterpret_cast<const char *>(S.skip) + (uint32_t)cur * (uint32_t)sizeof(SkipNode);
+            const char *np = reinterpret_cast<const char *>(skip) + (uint32_t)cur * (uint32_t)sizeof(SkipNode);
             f0 = reinterpret_cast<const float4 *>(np)[0];
             f1 = reinterpret_cast<const float4 *>(np)[1];
             esc = reinterpret_cast<const SkipNode *>(np)->escape[oct];
@@ -361,8 +422,7 @@ __device__ void walk_shared(const TraceScene &S, PairLds *L, const int g, int to
         if (lm != 0) {
             if (in_mask(lm)) {
                 const int slot = (head + queued + rank_in(lm)) & (LEAF_RING - 1);
-                L->leaf_first[slot] = a;
-                L->leaf_ray_count[slot] = ray | (meta << 6);
+                L->leaf[slot] = make_int2(a, ray | (meta << 6));
             }
             queued += popc64(lm);
         }
@@ -384,37 +444,35 @@ __device__ void walk_shared(const TraceScene &S, PairLds *L, const int g, int to
 // one path down a tree, one a level at most, and the host refuses bottom-level trees of WALK_STACK levels or more, so
 // WALK_STACK entries hold them. Leaves are queued and tested in batches as in the walk above.
 template <class Stats>
-__device__ void walk_shared_two_child(const TraceScene &S, PairLds *L, const int g, int top, const float3 lo,
+__device__ void walk_shared_two_child(const Scene S, PairLds *L, const int g, int top, const float3 lo,
                                       const float3 ld, const float3 inv_ld, float &tmax, Stats &stats) {
-    const int lane = lane_id();
     int head = 0, queued = 0;
-    int ray = -1, cur = -1;
+    // A lane's work as the stacks hold it, ray lane | node << 6 (so its upper bits are the node's byte offset), or
+    // negative: idle. Lane reads take the low bits of 4 x a lane number, so work << 2 reads the ray's lane.
+    int work = -1;
     float3 wlo = lo, winv = inv_ld;
-    float wlim = tmax;
+    float wlim = box_limit(tmax);
     int own[WALK_STACK];
     int own_n = 0;
+    const char *const nodes = reinterpret_cast<const char *>(S.blas_wide());
+    const int share_cap = S.share_cap();
     while (true) {
-        const uint64_t idle = ballot(ray < 0);
-        const uint64_t resume = idle & ballot(own_n > 0);
-        if (idle != 0 && (top > 0 || resume != 0)) {
-            const uint64_t takers = idle & ~resume;
+        uint64_t busy = ballot(work >= 0);
+        const uint64_t resume = ~busy & ballot(own_n > 0);
+        if (~busy != 0 && (top | (int)(resume != 0)) != 0) {
+            const uint64_t takers = ~(busy | resume);
             const int n = min(popc64(takers), top);
             const int rk = rank_in(takers);
             wave_lds_order();
-            int e = -1;
-            if (in_mask(takers) && rk < n) e = L->share[top - 1 - rk];
-            if (in_mask(resume)) e = own[--own_n];
+            if (in_mask(takers) && rk < n) work = L->share[top - 1 - rk];
+            if (in_mask(resume)) work = own[--own_n];
             top -= n;
-            if (e >= 0) {
-                ray = e & 63;
-                cur = e >> 6;
-            }
-            const int src = ray >= 0 ? ray : lane;
-            wlo = mk3(__shfl(lo.x, src, 64), __shfl(lo.y, src, 64), __shfl(lo.z, src, 64));
-            winv = mk3(__shfl(inv_ld.x, src, 64), __shfl(inv_ld.y, src, 64), __shfl(inv_ld.z, src, 64));
-            wlim = __shfl(tmax, src, 64);
+            const int src = work << 2;
+            if (!Stats::kOneOrigin) wlo = mk3(lane_read(lo.x, src), lane_read(lo.y, src), lane_read(lo.z, src));
+            winv = mk3(lane_read(inv_ld.x, src), lane_read(inv_ld.y, src), lane_read(inv_ld.z, src));
+            wlim = min_quiet(lane_read(tmax, src), BELOW_NO_HIT);
+            busy = ballot(work >= 0);
         }
-        const uint64_t busy = ballot(ray >= 0);
         if (busy == 0) break;
         stats.add(ST_BLAS_NODES, 1);
         stats.add(ST_BLAS_LANES, popc64(busy));
@@ -425,123 +483,83 @@ __device__ void walk_shared_two_child(const TraceScene &S, PairLds *L, const int
         int4 f3 = make_int4(unknown_i(), unknown_i(), unknown_i(), unknown_i());
         if (in_mask(busy)) {
             // a 32-bit byte offset from the array's base (node indices stay below 2^25)
-            const float4 *np = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(S.blas_wide) +
-                                                                (uint32_t)cur * (uint32_t)sizeof(WideNode));
+            const float4 *np = reinterpret_cast<const float4 *>(nodes + ((uint32_t)work & ~63u));
             f0 = np[0];
             f1 = np[1];
             f2 = np[2];
             f3 = *reinterpret_cast<const int4 *>(np + 3);
         }
-        const float lim = box_limit(wlim);
         float dl, dr;
-        const uint64_t hl = busy & ballot(box_hit(f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, wlo, winv, lim, dl));
-        const uint64_t hr = busy & ballot(box_hit(f1.z, f1.w, f2.x, f2.y, f2.z, f2.w, wlo, winv, lim, dr));
+        const uint64_t hl = busy & ballot(box_hit(f0.x, f1.x, f2.x, f0.z, f1.z, f2.z, wlo, winv, wlim, dl));
+        const uint64_t hr = busy & ballot(box_hit(f0.y, f1.y, f2.y, f0.w, f1.w, f2.w, wlo, winv, wlim, dr));
         const uint64_t lleaf = ballot(f3.x < 0), rleaf = ballot(f3.y < 0);
         const uint64_t ll = hl & lleaf, rl = hr & rleaf;    // leaves entered
         const uint64_t li = hl & ~lleaf, ri = hr & ~rleaf;  // interior children entered
-        const int nl = popc64(ll), nr = popc64(rl);
-        if (nl + nr != 0) {
+        if ((ll | rl) != 0) {
+            const int nl = popc64(ll), nr = popc64(rl);
             // a step queues at most 128 leaves, so the ring holds them once what waits is tested
-            if (queued + nl + nr > LEAF_RING) {
+            if (__builtin_expect(queued + nl + nr > LEAF_RING, 0)) {
                 test_queued_leaves<true>(S, L, head, queued, g, lo, ld, tmax, stats);
-                wlim = __shfl(tmax, ray >= 0 ? ray : lane, 64);
+                wlim = min_quiet(lane_read(tmax, work << 2), BELOW_NO_HIT);
             }
-            if (in_mask(ll)) {
-                const int slot = (head + queued + rank_in(ll)) & (LEAF_RING - 1);
-                L->leaf_first[slot] = ~f3.x;
-                L->leaf_ray_count[slot] = ray | (f3.z << 6);
-            }
-            if (in_mask(rl)) {
-                const int slot = (head + queued + nl + rank_in(rl)) & (LEAF_RING - 1);
-                L->leaf_first[slot] = ~f3.y;
-                L->leaf_ray_count[slot] = ray | (f3.w << 6);
-            }
+            const int ray = work & 63;
+            if (in_mask(ll)) L->leaf[(head + queued + rank_in(ll)) & (LEAF_RING - 1)] = make_int2(~f3.x, ray | (f3.z << 6));
+            if (in_mask(rl)) L->leaf[(head + queued + nl + rank_in(rl)) & (LEAF_RING - 1)] = make_int2(~f3.y, ray | (f3.w << 6));
             queued += nl + nr;
         }
+        // on to the nearer of the interior children entered (the left one when they are as near)
+        const uint64_t go_left = li & (~ri | ballot(dl <= dr));
         const uint64_t both = li & ri;
-        const bool left_near = dl <= dr;
-        const int near = in_mask(both) ? (left_near ? f3.x : f3.y) : in_mask(li) ? f3.x : in_mask(ri) ? f3.y : -1;
+        const int ray = work & 63;
+        const int near = in_mask(go_left) ? f3.x : f3.y;
         if (both != 0) {
-            const int far = left_near ? f3.y : f3.x;
+            const int far = ray | ((in_mask(go_left) ? f3.y : f3.x) << 6);
             // the lowest-ranked lanes fill the shared stack's room; the others keep their far child
-            const uint64_t given = both & ballot(rank_in(both) < S.share_cap - top);
-            if (in_mask(given)) L->share[top + rank_in(given)] = ray | (far << 6);
-            top += popc64(given);
-            if (in_mask(both & ~given)) {
-                if (own_n < WALK_STACK) own[own_n++] = ray | (far << 6);
-                else *S.overflow = 1;
+            const int room = share_cap - top, rk = rank_in(both), n = popc64(both);
+            if (n <= room) {
+                if (in_mask(both)) L->share[top + rk] = far;
+                top += n;
+            } else {
+                const uint64_t given = both & ballot(rk < room);
+                if (in_mask(given)) L->share[top + rk] = far;
+                top += popc64(given);
+                if (in_mask(both & ~given)) {
+                    if (own_n < WALK_STACK) own[own_n++] = far;
+                    else *S.overflow() = 1;
+                }
             }
         }
-        if (in_mask(busy)) {
-            cur = near;
-            if (near < 0) ray = -1;
-        }
+        work = in_mask(li | ri) ? ray | (near << 6) : -1;
         if (queued >= NGX_LEAF_BATCH) {
             test_queued_leaves<false>(S, L, head, queued, g, lo, ld, tmax, stats);
-            wlim = __shfl(tmax, ray >= 0 ? ray : lane, 64);
+            wlim = min_quiet(lane_read(tmax, work << 2), BELOW_NO_HIT);
         }
     }
     test_queued_leaves<true>(S, L, head, queued, g, lo, ld, tmax, stats);
 }
 
-// One instance for the lanes in mask: the ray moved into mesh space (mesh_dev.h:164-171, direction not
-// renormalized so t is shared), then the mesh's own tree.
-// BLAS: how bottom levels are walked: 0 as a packet; 1 lane by lane for meshes of lane_min_tris triangles or more,
-// as a packet otherwise; 2 lane by lane for every mesh (the packet code is then not built, which frees registers; a
-// mesh of a single leaf is still tested as one batch).
-template <int BLAS, class Stats>
-__device__ void visit_instance(const TraceScene &S, PairLds *L, const int g, const uint64_t mask, const float3 o,
-                               const float3 d, float &tmax, LaneHit &h, Stats &stats) {
-    stats.add(ST_INSTANCES, 1);
-    stats.add(ST_INSTANCE_LANES, popc64(mask));
-    const float4 *rp = reinterpret_cast<const float4 *>(S.inst + g);
-    const float4 r0 = sload4(rp), r1 = sload4(rp + 1), r2 = sload4(rp + 2);
-    const int4 meta = sload4i(reinterpret_cast<const int4 *>(rp + 3));
-    const float3 lo = mk3(dot3(xyz(r0), o) + r0.w, dot3(xyz(r1), o) + r1.w, dot3(xyz(r2), o) + r2.w);
-    const float3 ld = mk3(dot3(xyz(r0), d), dot3(xyz(r1), d), dot3(xyz(r2), d));
-    const float3 inv_d = safe_inverse(ld);
-    const float4 *mp = reinterpret_cast<const float4 *>(S.mesh_roots + meta.x);
-    const float4 m0 = sload4(mp), m1 = sload4(mp + 1);
-    float root_t;
-    const uint64_t root_mask = mask & ballot(box_hit(m0.x, m0.y, m0.z, m1.x, m1.y, m1.z, lo, inv_d, box_limit(tmax), root_t));
-    if (root_mask == 0) return;
-    stats.add(ST_INSTANCE_ROOT_LANES, popc64(root_mask));
-    int shared = 0;  // subtrees given to the shared per-lane walk
-    constexpr bool LANES = BLAS != 0;
-    const int root_ref = __float_as_int(m0.w);
-    if (BLAS == 2 || (BLAS == 1 && meta.z >= S.lane_min_tris)) {
-        if constexpr (Stats::kTwoChild) {
-            // the two-child layout starts below the root's box; a mesh of one leaf is tested as a batch below
-            if (root_ref >= 0) {
-                share_subtree(L, shared, root_mask, root_ref);
-                walk_shared_two_child(S, L, g, shared, lo, ld, inv_d, tmax, stats);
-                return;
-            }
-        } else {
-            share_subtree(L, shared, root_mask, meta.w);
-            walk_shared(S, L, g, shared, lo, ld, inv_d, tmax, stats);
-            return;
-        }
-    }
+// The bottom level of one instance walked as a packet from its root node for the rays in root_mask. With LANES, subtrees
+// entered by few rays are left on the shared stack (shared counts them).
+template <bool LANES, class Stats>
+__device__ __forceinline__ void walk_packet(const Scene S, PairLds *L, const int g, const int root_ref, const uint64_t root_mask,
+                                            const float3 lo, const float3 ld, const float3 inv_d, float &tmax, LaneHit &h,
+                                            int &shared, Stats &stats) {
     int pairs = 0;
-    if (root_ref < 0) {
-        add_leaf(S, L, pairs, ~root_ref, __float_as_int(m1.w), root_mask, g, lo, ld, tmax, h, stats);
-        flush_pairs(S, L, pairs, g, lo, ld, tmax, stats);
-        return;
-    }
-    LdsStack st(L, 1, S.overflow);
+    WaveStack st;
+    const WideNode *const nodes = S.blas_wide();
+    const float3 lov = Stats::kOneOrigin ? in_vgpr3(lo) : lo;  // the nodes' planes are scalars too
     int cur = root_ref;
     uint64_t cm = root_mask;
     while (true) {
-        const Wide w = load_wide(S.blas_wide, cur);
+        const Wide w = load_wide(nodes, cur);
         stats.add(ST_BLAS_NODES, 1);
         stats.add(ST_BLAS_LANES, popc64(cm));
         // every lane runs the tests (a vector instruction costs the same for 1 lane or 64); the masks keep
         // the lanes of this node
         const float lim = box_limit(tmax);
         float dl, dr;
-        const uint64_t ml = cm & ballot(box_hit(w.l_lo[0], w.l_lo[1], w.l_lo[2], w.l_hi[0], w.l_hi[1], w.l_hi[2], lo, inv_d, lim, dl));
-        const uint64_t mr = cm & ballot(box_hit(w.r_lo[0], w.r_lo[1], w.r_lo[2], w.r_hi[0], w.r_hi[1], w.r_hi[2], lo, inv_d, lim, dr));
+        const uint64_t ml = cm & ballot(box_hit(w.l_lo[0], w.l_lo[1], w.l_lo[2], w.l_hi[0], w.l_hi[1], w.l_hi[2], lov, inv_d, lim, dl));
+        const uint64_t mr = cm & ballot(box_hit(w.r_lo[0], w.r_lo[1], w.r_lo[2], w.r_hi[0], w.r_hi[1], w.r_hi[2], lov, inv_d, lim, dr));
         int next_ref, next_count;
         uint64_t next_mask;
         if (ml != 0 && mr != 0) {
@@ -570,7 +588,7 @@ __device__ void visit_instance(const TraceScene &S, PairLds *L, const int g, con
             if (next_mask != 0 && next_ref >= 0) {
                 const int n = popc64(next_mask);
                 if (!LANES || !Stats::kHandoff || n > NGX_HANDOFF_LANES || shared + n > SHARE_CAP) break;
-                share_subtree(L, shared, next_mask, Stats::kTwoChild ? next_ref : S.blas_wide_node[next_ref]);
+                share_subtree(L, shared, next_mask, Stats::kTwoChild ? next_ref : S.blas_wide_node()[next_ref]);
             } else if (next_mask != 0) {
                 add_leaf(S, L, pairs, ~next_ref, next_count, next_mask, g, lo, ld, tmax, h, stats);
             }
@@ -584,7 +602,7 @@ __device__ void visit_instance(const TraceScene &S, PairLds *L, const int g, con
                 next_ref = r;
             } else {
                 const int parent = (~r) >> 1, side = (~r) & 1;
-                const Wide pw = load_wide(S.blas_wide, parent);
+                const Wide pw = load_wide(nodes, parent);
                 next_ref = side ? pw.right : pw.left;
                 next_count = side ? pw.rcount : pw.lcount;
             }
@@ -594,6 +612,52 @@ __device__ void visit_instance(const TraceScene &S, PairLds *L, const int g, con
         cm = next_mask;
     }
     flush_pairs(S, L, pairs, g, lo, ld, tmax, stats);
+}
+
+// One instance for the lanes in mask: the ray moved into mesh space (mesh_dev.h:164-171, direction not
+// renormalized so t is shared), then the mesh's own tree.
+// BLAS: how bottom levels are walked: 0 as a packet; 1 lane by lane for meshes of lane_min_tris triangles or more,
+// as a packet otherwise; 2 lane by lane for every mesh (the packet code is then not built, which frees registers; a
+// mesh of a single leaf is still tested as one batch).
+template <int BLAS, class Stats>
+__device__ void visit_instance(const Scene S, PairLds *L, const int g, const uint64_t mask, const float3 o,
+                               const float3 d, float &tmax, LaneHit &h, Stats &stats) {
+    stats.add(ST_INSTANCES, 1);
+    stats.add(ST_INSTANCE_LANES, popc64(mask));
+    const float4 *rp = reinterpret_cast<const float4 *>(S.inst() + g);
+    const float4 r0 = sload4(rp), r1 = sload4(rp + 1), r2 = sload4(rp + 2);
+    const int4 meta = sload4i(reinterpret_cast<const int4 *>(rp + 3));
+    float3 lo = mk3(dot3(xyz(r0), o) + r0.w, dot3(xyz(r1), o) + r1.w, dot3(xyz(r2), o) + r2.w);
+    if (Stats::kOneOrigin) lo = mk3(uniform_f(lo.x), uniform_f(lo.y), uniform_f(lo.z));
+    const float3 ld = mk3(dot3(xyz(r0), d), dot3(xyz(r1), d), dot3(xyz(r2), d));
+    const float3 inv_d = safe_inverse(ld);
+    const float4 *mp = reinterpret_cast<const float4 *>(S.mesh_roots() + meta.x);
+    const float4 m0 = sload4(mp), m1 = sload4(mp + 1);
+    float root_t;
+    const uint64_t root_mask = mask & ballot(box_hit(m0.x, m0.y, m0.z, m1.x, m1.y, m1.z, lo, inv_d, box_limit(tmax), root_t));
+    if (root_mask == 0) return;
+    stats.add(ST_INSTANCE_ROOT_LANES, popc64(root_mask));
+    int shared = 0;  // subtrees given to the shared per-lane walk
+    constexpr bool LANES = BLAS != 0;
+    const int root_ref = __float_as_int(m0.w);
+    const bool lanes = BLAS == 2 || (BLAS == 1 && meta.z >= S.lane_min_tris());
+    if constexpr (!Stats::kTwoChild) {
+        if (lanes) {
+            share_subtree(L, shared, root_mask, meta.w);
+            walk_shared(S, L, g, shared, lo, ld, inv_d, tmax, stats);
+            return;
+        }
+    }
+    if (root_ref < 0) {
+        // a mesh of one leaf, tested as a batch
+        int pairs = 0;
+        add_leaf(S, L, pairs, ~root_ref, __float_as_int(m1.w), root_mask, g, lo, ld, tmax, h, stats);
+        flush_pairs(S, L, pairs, g, lo, ld, tmax, stats);
+        return;
+    }
+    // the two-child layout starts below the root's box
+    if (lanes) share_subtree(L, shared, root_mask, root_ref);
+    else if (BLAS != 2) walk_packet<LANES>(S, L, g, root_ref, root_mask, lo, ld, inv_d, tmax, h, shared, stats);
     if (LANES && shared > 0) {
         if constexpr (Stats::kTwoChild) walk_shared_two_child(S, L, g, shared, lo, ld, inv_d, tmax, stats);
         else walk_shared(S, L, g, shared, lo, ld, inv_d, tmax, stats);
@@ -603,58 +667,49 @@ __device__ void visit_instance(const TraceScene &S, PairLds *L, const int g, con
 // The closest instance hit in one world for the lanes in live (mesh_dev.h:177-205). tmax is each lane's
 // distance to beat on entry and its closest distance on return.
 template <int BLAS, class Stats>
-__device__ void trace_world(const TraceScene &S, PairLds *L, const int world, const float3 o, const float3 d,
+__device__ void trace_world(const Scene S, PairLds *L, const int world, const float3 o, const float3 d,
                             const uint64_t live, float &tmax, LaneHit &h, Stats &stats) {
     if (live == 0) return;
-    const int root = uniform(S.roots[world]);
+    const int root = uniform(S.roots()[world]);
     if (root < 0) return;
     // the origin in vector registers: for camera rays it is the same in every lane
     const float3 ov = in_vgpr3(o);
-    if (root >= S.total - 1) {
-        visit_instance<BLAS>(S, L, root - (S.total - 1), live, ov, d, tmax, h, stats);
-        return;
-    }
     const float3 inv_d = safe_inverse(d);
+    float lim = box_limit(tmax);
     // One entry is pushed per level at most. Below a world's root every level fixes at least one more bit
     // of a Morton code (30 bits) or, among equal codes, of the leaves' positions (at most ceil(log2 n) + 1
     // bits over n consecutive positions): fewer than 64 levels for any n < 2^31, so 64 entries do.
-    LdsStack st(L, 0, S.overflow);
-    int cur = root;
-    uint64_t cm = live;
+    WaveStack st;
+    const WideNode *const nodes = S.tlas_wide();
+    const int first_leaf = S.total() - 1;
+    // what to visit next: a node, or below zero an instance (a one-instance world's root is one)
+    int next_ref = root >= first_leaf ? ~(root - first_leaf) : root;
+    uint64_t next_mask = live;
     while (true) {
-        const Wide w = load_wide(S.tlas_wide, cur);
-        stats.add(ST_TLAS_NODES, 1);
-        stats.add(ST_TLAS_LANES, popc64(cm));
-        const float lim = box_limit(tmax);
-        float dl, dr;
-        const uint64_t ml = cm & ballot(box_hit(w.l_lo[0], w.l_lo[1], w.l_lo[2], w.l_hi[0], w.l_hi[1], w.l_hi[2], ov, inv_d, lim, dl));
-        const uint64_t mr = cm & ballot(box_hit(w.r_lo[0], w.r_lo[1], w.r_lo[2], w.r_hi[0], w.r_hi[1], w.r_hi[2], ov, inv_d, lim, dr));
-        int next_ref;
-        uint64_t next_mask;
-        if (ml != 0 && mr != 0) {
-            const uint64_t near_left = ml & (~mr | ballot(dl <= dr));
-            const bool left_first = 2 * popc64(near_left) >= popc64(ml | mr);
-            if (left_first) {
-                st.push(w.right, mr);
-                next_ref = w.left; next_mask = ml;
-            } else {
-                st.push(w.left, ml);
-                next_ref = w.right; next_mask = mr;
-            }
-        } else if (ml != 0) {
-            next_ref = w.left; next_mask = ml;
-        } else if (mr != 0) {
-            next_ref = w.right; next_mask = mr;
-        } else {
-            next_ref = 0; next_mask = 0;
-        }
         while (next_mask == 0 || next_ref < 0) {
-            if (next_mask != 0) visit_instance<BLAS>(S, L, ~next_ref, next_mask, ov, d, tmax, h, stats);
+            if (next_mask != 0) {
+                visit_instance<BLAS>(S, L, ~next_ref, next_mask, ov, d, tmax, h, stats);
+                lim = min_quiet(tmax, BELOW_NO_HIT);
+            }
             if (st.sp == 0) return;
             st.pop(next_ref, next_mask);
         }
-        cur = next_ref;
-        cm = next_mask;
+        const Wide w = load_wide(nodes, next_ref);
+        stats.add(ST_TLAS_NODES, 1);
+        stats.add(ST_TLAS_LANES, popc64(next_mask));
+        float dl, dr;
+        const uint64_t ml = next_mask & ballot(box_hit(w.l_lo[0], w.l_lo[1], w.l_lo[2], w.l_hi[0], w.l_hi[1], w.l_hi[2], ov, inv_d, lim, dl));
+        const uint64_t mr = next_mask & ballot(box_hit(w.r_lo[0], w.r_lo[1], w.r_lo[2], w.r_hi[0], w.r_hi[1], w.r_hi[2], ov, inv_d, lim, dr));
+        next_ref = ml != 0 ? w.left : w.right;
+        next_mask = ml != 0 ? ml : mr;
+        if (ml != 0 && mr != 0) {
+            // a lane is nearer the left child when it enters only the left, or the left no later than the right
+            const uint64_t near_left = ml & (~mr | ballot(dl <= dr));
+            const bool left_first = 2 * popc64(near_left) >= popc64(ml | mr);
+            next_ref = left_first ? w.left : w.right;
+            next_mask = left_first ? ml : mr;
+            st.push(left_first ? w.right : w.left, left_first ? mr : ml);
+        }
     }
 }
 
@@ -669,7 +724,7 @@ __device__ void trace_world(const TraceScene &S, PairLds *L, const int world, co
 // postponed until every lane of the wave has one, then instance entries and triangle runs are done
 // together (the "while-while" organisation of Aila and Laine, 2009).
 template <class Stats>
-__device__ void trace_world_lanes(const TraceScene &S, const int world, const float3 o, const float3 d, const bool live,
+__device__ void trace_world_lanes(const Scene S, const int world, const float3 o, const float3 d, const bool live,
                                   float &tmax, LaneHit &h, Stats &stats) {
     constexpr int NODE = 0, LEAF = 1, BACK = 2, DONE = 3;
     const float3 inv_d = safe_inverse(d);
@@ -681,12 +736,12 @@ __device__ void trace_world_lanes(const TraceScene &S, const int world, const fl
     float3 lo = o, ld = d, inv_ld = inv_d;
     if (live) {
         // an empty world's root is -1; test that first, since with no instances at all total - 1 is -1 too
-        const int root = S.roots[world];
+        const int root = S.roots()[world];
         if (root < 0) {
             state = DONE;
-        } else if (root >= S.total - 1) {
+        } else if (root >= S.total() - 1) {
             state = LEAF;
-            leaf_ref = ~(root - (S.total - 1));
+            leaf_ref = ~(root - (S.total() - 1));
         } else {
             state = NODE;
             cur_t = root;
@@ -708,12 +763,12 @@ __device__ void trace_world_lanes(const TraceScene &S, const int world, const fl
                 int depth = bottom ? depth_b : depth_t;
                 const bool pending = on_back && (bits & 1ull);
                 if (on_node || pending) {
-                    const float4 *np = reinterpret_cast<const float4 *>((bottom ? S.blas_wide : S.tlas_wide) + cur);
+                    const float4 *np = reinterpret_cast<const float4 *>((bottom ? S.blas_wide() : S.tlas_wide()) + cur);
                     const float4 f0 = np[0], f1 = np[1], f2 = np[2];
                     const int4 f3 = *reinterpret_cast<const int4 *>(np + 3);
                     const float3 ro = bottom ? lo : o, ri = bottom ? inv_ld : inv_d;
-                    const float dl = box_entry(f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, ro, ri, tmax);
-                    const float dr = box_entry(f1.z, f1.w, f2.x, f2.y, f2.z, f2.w, ro, ri, tmax);
+                    const float dl = box_entry(f0.x, f1.x, f2.x, f0.z, f1.z, f2.z, ro, ri, tmax);
+                    const float dr = box_entry(f0.y, f1.y, f2.y, f0.w, f1.w, f2.w, ro, ri, tmax);
                     const bool hl = dl < NO_HIT, hr = dr < NO_HIT;
                     int child = 0, child_count = 0;
                     bool go = false;
@@ -747,7 +802,7 @@ __device__ void trace_world_lanes(const TraceScene &S, const int world, const fl
                             bits <<= 1;
                             side <<= 1;
                             // a 65th level would push the root's bit out of the trail
-                            if (++depth >= 64) *S.overflow = 1;
+                            if (++depth >= 64) *S.overflow() = 1;
                             state = NODE;
                         } else {
                             state = LEAF;
@@ -757,7 +812,7 @@ __device__ void trace_world_lanes(const TraceScene &S, const int world, const fl
                     }
                 } else {
                     // climb one level; a level whose root is finished hands back to the level above
-                    const int parent = cur < 0 ? -1 : (bottom ? S.blas_parent : S.tlas_parent)[cur];
+                    const int parent = cur < 0 ? -1 : (bottom ? S.blas_parent() : S.tlas_parent())[cur];
                     if (parent < 0) {
                         if (bottom) level = 0;  // the instance is done: resume the top level where it left off
                         else state = DONE;
@@ -788,13 +843,13 @@ __device__ void trace_world_lanes(const TraceScene &S, const int world, const fl
             stats.add(ST_INSTANCE_LANES, popc64(ballot(enter)));
             if (enter) {
                 g = ~leaf_ref;
-                const float4 *rp = reinterpret_cast<const float4 *>(S.inst + g);
+                const float4 *rp = reinterpret_cast<const float4 *>(S.inst() + g);
                 const float4 r0 = rp[0], r1 = rp[1], r2 = rp[2];
                 const int mesh = reinterpret_cast<const int4 *>(rp + 3)->x;
                 lo = mk3(dot3(xyz(r0), o) + r0.w, dot3(xyz(r1), o) + r1.w, dot3(xyz(r2), o) + r2.w);
                 ld = mk3(dot3(xyz(r0), d), dot3(xyz(r1), d), dot3(xyz(r2), d));
                 inv_ld = safe_inverse(ld);
-                const float4 *mp = reinterpret_cast<const float4 *>(S.mesh_roots + mesh);
+                const float4 *mp = reinterpret_cast<const float4 *>(S.mesh_roots() + mesh);
                 const float4 m0 = mp[0], m1 = mp[1];
                 if (box_entry(m0.x, m0.y, m0.z, m1.x, m1.y, m1.z, lo, inv_ld, tmax) < NO_HIT) {
                     level = 1;
@@ -823,7 +878,7 @@ __device__ void trace_world_lanes(const TraceScene &S, const int world, const fl
                 const int first = ~leaf_ref;
                 for (int j = first; j < first + leaf_count; ++j) {
                     float3 v0, e1, e2;
-                    load_tri(S.tris, (size_t)j, v0, e1, e2);
+                    load_tri(S.tris(), (size_t)j, v0, e1, e2);
                     float t, bu, bv;
                     if (triangle_hit(v0, e1, e2, lo, ld, tmax, t, bu, bv)) {
                         tmax = Stats::kAnyHit ? -1.0f : t;
@@ -851,12 +906,12 @@ template <int WALK>
 constexpr int blas_mode() { return WALK == WALK_SHARED ? 2 : WALK == WALK_HYBRID ? 1 : 0; }
 
 template <int WALK, class Stats>
-__device__ __forceinline__ int scene_hit(const TraceScene &S, PairLds *L, const int world, const float3 o, const float3 d,
+__device__ __forceinline__ int scene_hit(const Scene S, PairLds *L, const int world, const float3 o, const float3 d,
                                          const uint64_t live, float &best, LaneHit &h, Stats &stats, const float start = 1e30f) {
     best = start;
     int best_sphere = -1;
-    for (int i = 0; i < S.sphere_count; ++i) {
-        const float4 sp = sload4(S.spheres + i);
+    for (int i = 0; i < S.sphere_count(); ++i) {
+        const float4 sp = sload4(S.spheres() + i);
         const float3 L = sub3(xyz(sp), o);
         const float tca = dot3(L, d);
         const float r2 = sp.w * sp.w;
@@ -872,10 +927,10 @@ __device__ __forceinline__ int scene_hit(const TraceScene &S, PairLds *L, const 
     }
     bool hit_floor = false;
     if (fabsf(d.y) > 1e-3f) {
-        const float dist = (S.floor_y - o.y) / d.y;
+        const float dist = (S.floor_y() - o.y) / d.y;
         if (dist > 0.0f && dist < best) {
             const float3 pt = add3(o, mul3(d, dist));
-            if (fabsf(pt.x) < S.floor_hx && pt.z > S.floor_zmin && pt.z < S.floor_zmax) {
+            if (fabsf(pt.x) < S.floor_hx() && pt.z > S.floor_zmin() && pt.z < S.floor_zmax()) {
                 best = dist;
                 hit_floor = true;
             }
@@ -885,16 +940,16 @@ __device__ __forceinline__ int scene_hit(const TraceScene &S, PairLds *L, const 
     h.tri = -1;
     if (WALK != WALK_LANES) {
         const int lane = lane_id();
-        L->hit_inst[lane] = -1;
+        L->hit[lane].x = -1;
         wave_lds_order();
         trace_world<blas_mode<WALK>()>(S, L, world, o, d, live, best, h, stats);
         wave_lds_order();
-        h.inst = L->hit_inst[lane];
+        const int4 k = L->hit[lane];
+        h.inst = k.x;
         if (h.inst >= 0) {
-            h.tri = L->hit_tri[lane];
-            const float2 uv = L->hit_uv[lane];
-            h.u = uv.x;
-            h.v = uv.y;
+            h.tri = k.y;
+            h.u = __int_as_float(k.z);
+            h.v = __int_as_float(k.w);
         }
     } else trace_world_lanes(S, world, o, d, ((live >> lane_id()) & 1ull) != 0, best, h, stats);
     if (h.inst >= 0) return OBJECT_INSTANCE;
@@ -904,19 +959,19 @@ __device__ __forceinline__ int scene_hit(const TraceScene &S, PairLds *L, const 
 }
 
 // Normal and object ID of a hit (render_core.h:119-141, mesh_dev.h:238-262).
-__device__ __forceinline__ void surface(const TraceScene &S, const int kind, const float3 o, const float3 d, const float t,
+__device__ __forceinline__ void surface(const Scene S, const int kind, const float3 o, const float3 d, const float t,
                                         const LaneHit &h, float3 &normal, int &object) {
     if (kind == OBJECT_INSTANCE) {
-        const InstanceRec &rec = S.inst[h.inst];
+        const InstanceRec &rec = S.inst()[h.inst];
         const float3 r0 = xyz(rec.inv[0]), r1 = xyz(rec.inv[1]), r2 = xyz(rec.inv[2]);
         float3 v0, e1, e2;
-        load_tri(S.tris, (size_t)h.tri, v0, e1, e2);
+        load_tri(S.tris(), (size_t)h.tri, v0, e1, e2);
         const float3 nl = cross3(e1, e2);
         float3 geometric = normalize3(add3(add3(mul3(r0, nl.x), mul3(r1, nl.y)), mul3(r2, nl.z)));
         if (dot3(geometric, d) > 0.0f) geometric = neg3(geometric);
         normal = geometric;
-        if (S.attrs != nullptr) {
-            const float4 *ap = S.attrs + 4 * (size_t)h.tri;
+        if (S.attrs() != nullptr) {
+            const float4 *ap = S.attrs() + 4 * (size_t)h.tri;
             const float4 a0 = ap[0], a1 = ap[1], a2 = ap[2], a3 = ap[3];
             if (__float_as_int(a3.w) & 1) {
                 const float w0 = 1.0f - h.u - h.v;
@@ -932,15 +987,15 @@ __device__ __forceinline__ void surface(const TraceScene &S, const int kind, con
         normal = mk3(0.0f, 1.0f, 0.0f);
         object = OBJECT_FLOOR;
     } else {
-        const float4 sp = S.spheres[kind - OBJECT_SPHERE];
+        const float4 sp = S.spheres()[kind - OBJECT_SPHERE];
         normal = normalize3(sub3(add3(o, mul3(d, t)), xyz(sp)));
         object = kind;
     }
 }
 
 // The object ID surface() gives, without the normal: what a frame of depth and IDs alone needs.
-__device__ __forceinline__ int object_of(const TraceScene &S, const int kind, const LaneHit &h) {
-    return kind == OBJECT_INSTANCE ? OBJECT_INSTANCE + S.inst[h.inst].tmpl : kind;
+__device__ __forceinline__ int object_of(const Scene S, const int kind, const LaneHit &h) {
+    return kind == OBJECT_INSTANCE ? OBJECT_INSTANCE + S.inst()[h.inst].tmpl : kind;
 }
 
 struct Cam {
@@ -988,35 +1043,45 @@ __device__ __forceinline__ long long wave_tile(const int xcd_remap, const long l
 
 // One 64-pixel tile of one view: camera ray per lane, closest hit, depth / normal / object ID.
 template <int WALK>
-__device__ __forceinline__ void render_tile(const RenderArgs &A, PairLds *L, const long long tile) {
+__device__ __forceinline__ void render_tile(PairLds *L, const long long tile) {
     const int lane = lane_id();
-    const int view = (int)(tile / A.tiles_per_view);
-    const int t = (int)(tile % A.tiles_per_view);
-    const int tx = t % A.tiles_x, ty = t / A.tiles_x;
-    const int x = tx * A.tile_w + lane % A.tile_w;
-    const int y = ty * A.tile_h + lane / A.tile_w;
-    const bool valid = x < A.width && y < A.height;
-    const int world = view / A.cameras_per_world;
-    const Cam cam = load_camera(A.cams + 12 * (size_t)view);
-    const float3 d = pixel_ray(cam, A.fov_scale, A.aspect, x, y, A.width, A.height);
+    float3 d;
+    Cam cam;
+    int view, x, y, world;
+    bool valid;
+    {
+        const auto &A = kernel_args<RenderArgs>();
+        view = (int)(tile / A.tiles_per_view);
+        const int t = (int)(tile % A.tiles_per_view);
+        const int tx = t % A.tiles_x, ty = t / A.tiles_x;
+        x = tx * A.tile_w + lane % A.tile_w;
+        y = ty * A.tile_h + lane / A.tile_w;
+        valid = x < A.width && y < A.height;
+        world = view / A.cameras_per_world;
+        cam = load_camera(A.cams + 12 * (size_t)view);
+        d = pixel_ray(cam, A.fov_scale, A.aspect, x, y, A.width, A.height);
+    }
     float best;
     LaneHit h;
-    NoStats stats;
-    const int kind = scene_hit<WALK>(A.s, L, world, cam.pos, d, ballot(valid), best, h, stats);
+    CameraRays stats;
+    const int kind = scene_hit<WALK>(Scene(), L, world, cam.pos, d, ballot(valid), best, h, stats);
     if (!valid) return;
+    const auto &A = kernel_args<RenderArgs>();
     const size_t idx = ((size_t)view * A.height + y) * A.width + x;
     const bool found = kind != OBJECT_NONE;
-    if (A.depth) A.depth[idx] = found ? best * dot3(d, cam.fwd) : __int_as_float(0x7f800000);
-    if (A.normal) {
+    float *const depth = in_global(A.depth), *const normals = in_global(A.normal);
+    int32_t *const object_id = in_global(A.object_id);
+    if (depth) depth[idx] = found ? best * dot3(d, cam.fwd) : __int_as_float(0x7f800000);
+    if (normals) {
         float3 normal = mk3(0.0f, 0.0f, 0.0f);
         int object = OBJECT_NONE;
-        if (found) surface(A.s, kind, cam.pos, d, best, h, normal, object);
-        A.normal[3 * idx] = normal.x;
-        A.normal[3 * idx + 1] = normal.y;
-        A.normal[3 * idx + 2] = normal.z;
-        if (A.object_id) A.object_id[idx] = object;
-    } else if (A.object_id) {
-        A.object_id[idx] = found ? object_of(A.s, kind, h) : OBJECT_NONE;
+        if (found) surface(Scene(), kind, cam.pos, d, best, h, normal, object);
+        normals[3 * idx] = normal.x;
+        normals[3 * idx + 1] = normal.y;
+        normals[3 * idx + 2] = normal.z;
+        if (object_id) object_id[idx] = object;
+    } else if (object_id) {
+        object_id[idx] = found ? object_of(Scene(), kind, h) : OBJECT_NONE;
     }
 }
 
@@ -1030,7 +1095,7 @@ __global__ __launch_bounds__(256, BLOCKS) void render_kernel(const RenderArgs A)
     NGX_PAIR_LDS(L);
     const long long tile = wave_tile(A.xcd_remap, A.total_tiles);
     if (tile >= A.total_tiles) return;
-    render_tile<WALK>(A, L, tile);
+    render_tile<WALK>(L, tile);
 }
 
 // Persistent: a fixed grid whose wavefronts take tiles until none are left. The tiles are cut into eight
@@ -1076,7 +1141,7 @@ __device__ __forceinline__ void take_tiles(int *counters, const long long total,
 template <int WALK, int BLOCKS>
 __global__ __launch_bounds__(256, BLOCKS) void render_persistent_kernel(const RenderArgs A) {
     NGX_PAIR_LDS(L);
-    take_tiles(A.tile_counters, A.total_tiles, [&](const long long tile) { render_tile<WALK>(A, L, tile); });
+    take_tiles(A.tile_counters, A.total_tiles, [&](const long long tile) { render_tile<WALK>(L, tile); });
 }
 
 __global__ void zero_counters_kernel(int *c) {
@@ -1107,7 +1172,7 @@ __global__ __launch_bounds__(256) void render_stats_kernel(const RenderArgs A, i
     WaveStats stats;
     for (int k = 0; k < ST_COUNT; ++k) stats.c[k] = 0;
     stats.add(ST_VALID, popc64(ballot(valid)));
-    scene_hit<WALK>(A.s, L, world, cam.pos, d, ballot(valid), best, h, stats);
+    scene_hit<WALK>(Scene(), L, world, cam.pos, d, ballot(valid), best, h, stats);
     int mine = 0;
     for (int k = 0; k < ST_COUNT; ++k) mine = lane == k ? stats.c[k] : mine;
     if (lane < ST_COUNT) out[(size_t)tile * ST_COUNT + lane] = mine;
@@ -1173,12 +1238,12 @@ __device__ __forceinline__ float light_factor(const float4 q, const float4 dir, 
 
 // Whether anything lies between o and o + max_dist d, for the lanes in live (render_core.h:146-160).
 template <int WALK, class Walk = Occlusion>
-__device__ __forceinline__ bool occluded(const TraceScene &S, PairLds *L, const int world, const float3 o, const float3 d,
+__device__ __forceinline__ bool occluded(const Scene S, PairLds *L, const int world, const float3 o, const float3 d,
                                          const uint64_t live, const float max_dist) {
     const bool mine = in_mask(live);
     bool blocked = false;
-    for (int i = 0; i < S.sphere_count; ++i) {
-        const float4 sp = sload4(S.spheres + i);
+    for (int i = 0; i < S.sphere_count(); ++i) {
+        const float4 sp = sload4(S.spheres() + i);
         const float3 Lc = sub3(xyz(sp), o);
         const float tca = dot3(Lc, d);
         const float r2 = sp.w * sp.w;
@@ -1190,10 +1255,10 @@ __device__ __forceinline__ bool occluded(const TraceScene &S, PairLds *L, const 
         if (t >= 0.0f && t < max_dist) blocked = true;
     }
     if (fabsf(d.y) > 1e-3f) {
-        const float dist = (S.floor_y - o.y) / d.y;
+        const float dist = (S.floor_y() - o.y) / d.y;
         if (dist > 0.0f && dist < max_dist) {
             const float3 pt = add3(o, mul3(d, dist));
-            if (fabsf(pt.x) < S.floor_hx && pt.z > S.floor_zmin && pt.z < S.floor_zmax) blocked = true;
+            if (fabsf(pt.x) < S.floor_hx() && pt.z > S.floor_zmin() && pt.z < S.floor_zmax()) blocked = true;
         }
     }
     // the walk limited to max_dist, stopping each ray at its first hit: it finds a hit exactly when the
@@ -1205,11 +1270,11 @@ __device__ __forceinline__ bool occluded(const TraceScene &S, PairLds *L, const 
         Walk stats;
         if (WALK != WALK_LANES) {
             const int lane = lane_id();
-            L->hit_inst[lane] = -1;
+            L->hit[lane].x = -1;
             wave_lds_order();
             trace_world<blas_mode<WALK>()>(S, L, world, o, d, rest, best, h, stats);
             wave_lds_order();
-            if (in_mask(rest) && L->hit_inst[lane] >= 0) blocked = true;
+            if (in_mask(rest) && L->hit[lane].x >= 0) blocked = true;
         } else {
             h.inst = -1;
             trace_world_lanes(S, world, o, d, in_mask(rest), best, h, stats);
@@ -1283,9 +1348,9 @@ __device__ __forceinline__ void hit_material(const RgbArgs &G, const int kind, c
     const ShadeScene &E = G.shade;
     point = add3(o, mul3(d, best));
     int object;
-    surface(A.s, kind, o, d, best, h, normal, object);
+    surface(Scene(), kind, o, d, best, h, normal, object);
     if (kind == OBJECT_INSTANCE) {
-        const float4 *mp = E.instance_materials + 2 * (size_t)A.s.inst[h.inst].tmpl;
+        const float4 *mp = E.instance_materials + 2 * (size_t)Scene().inst()[h.inst].tmpl;
         m0 = mp[0];
         m1 = mp[1];
     } else if (kind == OBJECT_FLOOR) {
@@ -1367,7 +1432,7 @@ __device__ __forceinline__ void shade_hit(const RgbArgs &G, PairLds *L, const in
         // a wave with no lane needing a shadow ray skips the walk
         const uint64_t shadow = ballot(need);
         if (!shadow) continue;
-        const bool blocked = occluded<WALK, Shadow>(A.s, L, world, offset_origin(point, normal, light_dir), light_dir, shadow,
+        const bool blocked = occluded<WALK, Shadow>(Scene(), L, world, offset_origin(point, normal, light_dir), light_dir, shadow,
                                                     light_distance);
         if (need && !blocked) {
             diffuse = add3(diffuse, cd);
@@ -1411,7 +1476,7 @@ __device__ __forceinline__ void rgb_tile(const RgbArgs &G, PairLds *L, const lon
             LaneHit h;
             ShadeRays stats;
             int kind = OBJECT_NONE;
-            if (depth <= MAX_BOUNCES) kind = scene_hit<WALK>(A.s, L, p.world, o, d, ballot(active), best, h, stats);
+            if (depth <= MAX_BOUNCES) kind = scene_hit<WALK>(Scene(), L, p.world, o, d, ballot(active), best, h, stats);
             shade_hit<WALK, Occlusion>(G, L, p.world, kind, best, h, active, o, d, rng, radiance, throughput);
         }
         sum = add3(sum, radiance);
@@ -1450,8 +1515,8 @@ __device__ __forceinline__ void rgb_hit_tile(const RgbArgs &G, PairLds *L, const
     const float3 d = camera_ray_at(cam, A.fov_scale, A.aspect, (float)p.x + jx, (float)p.y + jy, A.width, A.height);
     float best;
     LaneHit h;
-    NoStats stats;
-    const int kind = scene_hit<WALK>(A.s, L, p.world, cam.pos, d, ballot(p.valid), best, h, stats);
+    CameraRays stats;
+    const int kind = scene_hit<WALK>(Scene(), L, p.world, cam.pos, d, ballot(p.valid), best, h, stats);
     if (!p.valid) return;
     G.hits[p.index] = make_int4(__float_as_int(best), kind, h.inst, h.tri);
     if (G.hit_uv != nullptr) G.hit_uv[p.index] = kind == OBJECT_INSTANCE ? make_float2(h.u, h.v) : make_float2(0.0f, 0.0f);
@@ -1536,7 +1601,7 @@ __device__ __forceinline__ void rgb_shade_one_light_tile(const RgbArgs &G, PairL
     const uint64_t shadow = ballot(need);
     bool blocked = false;
     if (shadow)
-        blocked = occluded<WALK, OcclusionTwoChild>(G.r.s, L, q.p.world, offset_origin(point, normal, light_dir), light_dir, shadow,
+        blocked = occluded<WALK, OcclusionTwoChild>(Scene(), L, q.p.world, offset_origin(point, normal, light_dir), light_dir, shadow,
                                                     light_distance);
     if (q.p.valid) store_rgb(G, q.p.index, need && !blocked ? lit_bytes : dark_bytes);
 }
@@ -1563,62 +1628,77 @@ __global__ __launch_bounds__(256, BLOCKS) void rgb_shade_kernel(const RgbArgs G)
 // 6 workgroups (24 wavefronts) per compute unit, at most 84 VGPRs: the ray queries wait on memory more than the
 // render does, and a sixth wavefront per SIMD hides more of it (lidar_sweeps 22.7 -> 21.5 ms; 7 gives 22.6)
 // (built at 5, 6 and 7 for the packet and hybrid walks, the autotuner picking; the per-lane walk's at 6)
+struct QueryRay {
+    long long i;  // the ray's place in the caller's arrays
+    float3 o, d;
+    bool ok;      // its direction can be normalized
+};
+// The ray of a slot: the slot itself, or the world's ray at that place in the direction order. The arguments are read
+// again here, so a ray is read twice, before its walk and for its results, rather than held in seven registers between.
+__device__ __forceinline__ QueryRay query_ray(const long long slot, const int world) {
+    const auto &A = kernel_args<RayArgs>();
+    const int *const order = in_global(A.order);
+    QueryRay q;
+    q.i = order ? (long long)world * A.rays_per_world + order[slot] : slot;
+    const float *const po = in_global(A.origins) + 3 * q.i, *const pd = in_global(A.dirs) + 3 * q.i;
+    q.o = mk3(po[0], po[1], po[2]);
+    q.d = mk3(pd[0], pd[1], pd[2]);
+    const float len2 = dot3(q.d, q.d);
+    q.ok = len2 > 1e-30f && len2 < 1e30f;
+    if (q.ok) q.d = mul3(q.d, rcp_rn(sqrtf(len2)));
+    return q;
+}
+__device__ __forceinline__ void store_ray(const long long slot, const int world, const int kind, const float best, const LaneHit &h) {
+    const QueryRay q = query_ray(slot, world);
+    const auto &A = kernel_args<RayArgs>();
+    const bool found = kind != OBJECT_NONE && best <= A.max_distance;
+    float3 normal = mk3(0.0f, 0.0f, 0.0f);
+    int object = OBJECT_NONE;
+    if (found) surface(Scene(), kind, q.o, q.d, best, h, normal, object);
+    in_global(A.distance)[q.i] = found ? best : __int_as_float(0x7f800000);
+    float *const n = in_global(A.normal) + 3 * q.i;
+    n[0] = normal.x;
+    n[1] = normal.y;
+    n[2] = normal.z;
+    in_global(A.object_id)[q.i] = object;
+}
+
 template <int WALK, int BLOCKS>
 __global__ __launch_bounds__(256, BLOCKS) void ray_kernel(const RayArgs A) {
     NGX_PAIR_LDS(L);
     const long long base = wave_tile(A.xcd_remap, 0) * 64;
     if (base >= A.count) return;
-    const int lane = lane_id();
-    const long long slot = base + lane;
+    const long long slot = base + lane_id();
     const bool valid = slot < A.count;
     const int world = valid ? (int)(slot / A.rays_per_world) : -1;
-    // the ray this lane traces: the slot itself, or the world's ray at that place in the direction order
-    const long long i = valid && A.order ? (long long)world * A.rays_per_world + A.order[slot] : slot;
     float3 o = mk3(0.0f, 0.0f, 0.0f), d = mk3(0.0f, 0.0f, 1.0f);
     bool ok = false;
-    if (valid) {
-        o = mk3(A.origins[3 * i], A.origins[3 * i + 1], A.origins[3 * i + 2]);
-        d = mk3(A.dirs[3 * i], A.dirs[3 * i + 1], A.dirs[3 * i + 2]);
-        const float len2 = dot3(d, d);
-        ok = len2 > 1e-30f && len2 < 1e30f;
-        if (ok) d = mul3(d, rcp_rn(sqrtf(len2)));
-    }
-    float best = 1e30f;
     LaneHit h;
     h.inst = -1;
     h.tri = -1;
-    int kind = OBJECT_NONE;
+    if (valid) {
+        const QueryRay q = query_ray(slot, world);
+        o = q.o;
+        d = q.d;
+        ok = q.ok;
+        if (!ok) store_ray(slot, world, OBJECT_NONE, 0.0f, h);
+    }
+    float best;
+    NoStats stats;
     if (WALK != WALK_LANES) {
         uint64_t pending = ballot(ok);
         while (pending != 0) {
             const int w = __builtin_amdgcn_readlane(world, first_lane(pending));
             const uint64_t mine = ballot(ok && world == w);
-            float b;
-            LaneHit hh;
-            NoStats stats;
-            const int k = scene_hit<WALK>(A.s, L, w, o, d, mine, b, hh, stats);
-            if (in_mask(mine)) {
-                best = b;
-                h = hh;
-                kind = k;
-            }
+            const int kind = scene_hit<WALK>(Scene(), L, w, o, d, mine, best, h, stats);
+            if (in_mask(mine)) store_ray(slot, w, kind, best, h);
             pending &= ~mine;
         }
     } else {
         // each lane walks its own world
-        NoStats stats;
-        kind = scene_hit<WALK_LANES>(A.s, L, world, o, d, ballot(ok), best, h, stats);
+        const int kind = scene_hit<WALK_LANES>(Scene(), L, world, o, d, ballot(ok), best, h, stats);
+        if (ok) store_ray(slot, world, kind, best, h);
     }
-    if (!valid) return;
-    const bool found = ok && kind != OBJECT_NONE && best <= A.max_distance;
-    float3 normal = mk3(0.0f, 0.0f, 0.0f);
-    int object = OBJECT_NONE;
-    if (found) surface(A.s, kind, o, d, best, h, normal, object);
-    A.distance[i] = found ? best : __int_as_float(0x7f800000);
-    A.normal[3 * i] = normal.x;
-    A.normal[3 * i + 1] = normal.y;
-    A.normal[3 * i + 2] = normal.z;
-    A.object_id[i] = object;
 }
 
 // ------------------------------------------------------------------------------ backward --
@@ -1629,16 +1709,16 @@ __global__ __launch_bounds__(256, BLOCKS) void ray_kernel(const RayArgs A) {
 // a = dL/dt * n / n.d; the projection onto the raw quaternion is applied once per body afterwards.
 
 // The 7 gradient terms of one lane's hit: returns false when the hit does not depend on a body pose.
-__device__ __forceinline__ bool hit_pose_terms(const TraceScene &S, const int world, const int bodies_per_world,
+__device__ __forceinline__ bool hit_pose_terms(const Scene S, const int world, const int bodies_per_world,
                                                const int *body_of_instance, const float *local_rot_scale, const float *body_poses,
                                                const float3 o, const float3 d, const LaneHit &h, const float dl_dt,
                                                int &body, float g[7]) {
-    const InstanceRec &rec = S.inst[h.inst];
+    const InstanceRec &rec = S.inst()[h.inst];
     body = body_of_instance[rec.tmpl];
     if (body < 0) return false;
     const float3 r0 = xyz(rec.inv[0]), r1 = xyz(rec.inv[1]), r2 = xyz(rec.inv[2]);
     float3 v0, e1, e2;
-    load_tri(S.tris, (size_t)h.tri, v0, e1, e2);
+    load_tri(S.tris(), (size_t)h.tri, v0, e1, e2);
     const float3 nl = cross3(e1, e2);
     const float3 n = add3(add3(mul3(r0, nl.x), mul3(r1, nl.y)), mul3(r2, nl.z));
     const float nd = dot3(n, d);
@@ -1717,13 +1797,13 @@ __global__ __launch_bounds__(64 * BWD_WAVES, BLOCKS) void depth_backward_kernel(
         const float bound = want ? (depth / cosf_) * (1.0f + 1e-5f) + 1e-6f : 0.0f;
         float best;
         LaneHit h;
-        NoStats stats;
-        const int kind = scene_hit<WALK>(A.s, L, world, cam.pos, d, ballot(want), best, h, stats, bound);
+        CameraRays stats;
+        const int kind = scene_hit<WALK>(Scene(), L, world, cam.pos, d, ballot(want), best, h, stats, bound);
         int body = -1;
         float g[7] = {0, 0, 0, 0, 0, 0, 0};
         bool has = false;
         if (want && kind == OBJECT_INSTANCE)
-            has = hit_pose_terms(A.s, world, B, A.body_of_instance, A.local_rot_scale, A.body_poses, cam.pos, d, h, gd * cosf_, body, g);
+            has = hit_pose_terms(Scene(), world, B, A.body_of_instance, A.local_rot_scale, A.body_poses, cam.pos, d, h, gd * cosf_, body, g);
         wave_accumulate(has, body, g, acc);
     }
     __syncthreads();
@@ -1762,12 +1842,12 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void range_backward_kernel(const Ra
         float best;
         LaneHit h;
         NoStats stats;
-        const int kind = scene_hit<WALK>(A.s, L, world, o, d, ballot(want), best, h, stats, bound);
+        const int kind = scene_hit<WALK>(Scene(), L, world, o, d, ballot(want), best, h, stats, bound);
         int body = -1;
         float g[7] = {0, 0, 0, 0, 0, 0, 0};
         bool has = false;
         if (want && kind == OBJECT_INSTANCE)
-            has = hit_pose_terms(A.s, world, B, A.body_of_instance, A.local_rot_scale, A.body_poses, o, d, h, gd, body, g);
+            has = hit_pose_terms(Scene(), world, B, A.body_of_instance, A.local_rot_scale, A.body_poses, o, d, h, gd, body, g);
         wave_accumulate(has, body, g, acc);
     }
     __syncthreads();
