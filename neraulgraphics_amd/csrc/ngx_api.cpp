@@ -178,7 +178,7 @@ struct ngx_ctx {
     long long ray_in_cap = 0;
     float *d_hit_dist = nullptr, *d_hit_normal = nullptr;
     int32_t *d_hit_id = nullptr;
-    uint32_t *d_ray_keys = nullptr;     // the direction order's scratch: 2 x rays (cell and index in one word)
+    uint32_t *d_ray_keys = nullptr;     // the direction order's scratch (it grows with the rays a world)
     int *d_ray_vals = nullptr;          // the direction order: rays
     long long ray_cap = 0;
     float *d_partial = nullptr;
@@ -995,7 +995,7 @@ ngx_status ngx_cast_rays_batch(ngx_ctx *ctx, const float *origins, const float *
             device_alloc(ctx->d_hit_dist, (size_t)count);
             device_alloc(ctx->d_hit_normal, 3 * (size_t)count);
             device_alloc(ctx->d_hit_id, (size_t)count);
-            device_alloc(ctx->d_ray_keys, 2 * (size_t)count);
+            device_alloc(ctx->d_ray_keys, ngx::ray_order_scratch_words(rays_per_world, ctx->worlds));
             device_alloc(ctx->d_ray_vals, (size_t)count);
             ctx->ray_cap = count;
         }

@@ -242,8 +242,9 @@ struct BigBuildScratch {
 };
 
 // Per world, a stable order of its rays by direction cell, for coherent wavefronts: keys is scratch of
-// 2 x rays_per_world x worlds words, vals receives the order (rays_per_world x worlds), and *order is vals.
+// ray_order_scratch_words words, vals receives the order (rays_per_world x worlds), and *order is vals.
 constexpr int RAY_ORDER_MAX_RAYS = 262144;
+size_t ray_order_scratch_words(int rays_per_world, int worlds);
 hipError_t launch_ray_order(const float *dirs, int rays_per_world, int worlds, uint32_t *keys, int *vals, int **order,
                             hipStream_t stream);
 

@@ -97,7 +97,7 @@ extern "C" ngx_status ngx_debug_ray_order(int32_t device_id, const float *direct
     float *d = nullptr;
     uint32_t *keys = nullptr;
     int *vals = nullptr, *out = nullptr;
-    bool ok = hipMalloc(&d, 3 * n * sizeof(float)) == hipSuccess && hipMalloc(&keys, 2 * n * sizeof(uint32_t)) == hipSuccess &&
+    bool ok = hipMalloc(&d, 3 * n * sizeof(float)) == hipSuccess && hipMalloc(&keys, ngx::ray_order_scratch_words(rays_per_world, worlds) * sizeof(uint32_t)) == hipSuccess &&
               hipMalloc(&vals, n * sizeof(int)) == hipSuccess;
     if (!ok) {
         hipFree(d);

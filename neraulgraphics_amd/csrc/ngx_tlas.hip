@@ -644,21 +644,27 @@ __global__ __launch_bounds__(256) void big_write_kernel(const TlasBuildArgs A, c
 //
 // A query's rays come in the caller's order; a LiDAR's consecutive rays fan out over many degrees, so a
 // wavefront of 64 of them shares little of either tree. Each world's rays are put in a stable order of a
-// 12-bit direction cell (octahedral map of the direction, 64 x 64 cells, Morton order) by one workgroup per
-// world. Up to 65,536 rays a world, one counting sort: each of the workgroup's 16 wavefronts takes a contiguous
-// sixteenth of the world's rays, counts their cells into its own row of 16-bit counters (4096 cells x 16 wavefronts =
-// 128 KB of LDS) and keeps each cell in 2 bytes of scratch; one scan of the counters in cell-major, wavefront-minor
-// order gives each (cell, wavefront) its first place; each wavefront then reads its cells back and writes its rays'
-// indices in ray order, a ray's rank among the equal cells of its 64 from ballots: a stable sort by cell, reading
-// each direction once (16 bytes a ray of traffic where the radix sort moved 40; lidar_sweeps 1.20 -> 0.57 ms). Above
-// 65,536 rays, a stable LSD radix sort over chunks of 1024 rays in three passes of 4-bit digits, through global
-// memory; both give the one stable order. The tracer then gives a wavefront 64 consecutive rays of that order;
-// results still go to each ray's own place. In the radix sort a ray's cell and its index travel as one 32-bit word
-// (cell above bit 20, index below), so a pass moves 4 bytes a ray; the last pass writes the index alone.
-constexpr int RAY_ORDER_MAX_CHUNKS = RAY_ORDER_MAX_RAYS / 1024;
-constexpr int RAY_ORDER_INDEX_BITS = 20;
-static_assert(RAY_ORDER_MAX_RAYS <= (1 << RAY_ORDER_INDEX_BITS), "a world's ray index fits below the cell");
+// 12-bit direction cell (octahedral map of the direction, 64 x 64 cells, Morton order) by a counting sort; the
+// tracer then gives a wavefront 64 consecutive rays of that order, and results still go to each ray's own place.
+//
+// One workgroup orders a world (or a segment of one, below): each of its wavefronts takes a contiguous part of the
+// rays, counts their cells into its own row of 16-bit counters in LDS (4096 cells x 16 wavefronts = 128 KB) and keeps
+// each cell in 2 bytes of scratch; the counters are scanned in cell-major, wavefront-minor order, which gives each
+// (cell, wavefront) its first place; each wavefront then reads its cells back and writes its rays' indices in ray
+// order, a ray's rank among the equal cells of its 64 from ballots. 16 bytes a ray of traffic.
+//
+// Where there are fewer worlds than the chip has room for, or more rays than 16-bit places number, a world is cut into
+// segments of 4096 rays: one kernel counts each segment's cells, one sums each cell's counts over the segments, and one
+// orders each segment as above, from the cells' places and the segments' within them.
+// One world of 262,144 rays: 21 us, where a radix sort by one workgroup took 2,000; of 65,536 rays: 20 us, where one
+// workgroup takes 140. 96 worlds of 65,536 rays: 108 us against 150; at 128 worlds, half the compute units, the extra pass
+// costs what the spreading saves, and every segment has 4096 cells to clear and scan, so worlds of few rays keep to one.
+constexpr int RAY_ORDER_CELLS = 4096;
 constexpr int RAY_ORDER_ONE_PASS_MAX_RAYS = 65536;
+constexpr int RAY_ORDER_SEGMENT = 4096;
+constexpr int RAY_ORDER_SEGMENTED_MIN_RAYS = 8192;
+constexpr int RAY_ORDER_SEGMENTED_MAX_WORLDS = 96;
+constexpr int RAY_ORDER_FEW_RAYS = 2048, RAY_ORDER_FEW_RAYS_MANY_WORLDS = 4096, RAY_ORDER_MANY_WORLDS = 512;
 
 // tile_digit for a BITS-bit digit: the digit of each key of a 1024-key tile, its rank among the equal digits of
 // its wave, and how many of its wave share the digit (valid for the rank-0 lane).
@@ -699,141 +705,176 @@ __device__ __forceinline__ uint32_t direction_cell(const float x, const float y,
     return (spread6(qu) << 1) | spread6(qv);
 }
 
-// The one-pass order of up to 65,536 rays a world (see above); cells is scratch of one 16-bit cell a ray.
-__global__ __launch_bounds__(1024) void ray_order_one_pass_kernel(const float *dirs, const int R, uint16_t *cells, int *order) {
-    constexpr int NW = 16, CELLS = 4096;
-    // per (cell, wavefront), cell-major: first how many of the wavefront's rays fall in the cell, then where the next
-    // of them goes. A count is at most 4096 and a place below R <= 65,536, so 16 bits hold either; the scan's
-    // running sum runs in 32 bits (past the last occupied slot it may reach R, and those slots are never read).
-    __shared__ uint16_t slot[CELLS * NW];
-    __shared__ int wave_tot[NW];
+// The counters of a workgroup's wavefronts: per (cell, wavefront), cell-major, first how many of the wavefront's rays
+// fall in the cell, then where the next of them goes.
+template <int NW>
+struct RayOrderShared {
+    // a count is at most 4096 and a place below 65,536, so 16 bits hold either; the scan's running sum runs in 32 bits
+    // (past the last occupied slot it may reach 65,536, and those slots are never read)
+    alignas(16) uint16_t slot[RAY_ORDER_CELLS * NW];
+    int wave_tot[NW];
+};
+
+template <int NW>
+__device__ __forceinline__ void ray_order_clear(RayOrderShared<NW> &sh) {
+    uint4 *p = reinterpret_cast<uint4 *>(sh.slot);
+    for (int i = threadIdx.x; i < RAY_ORDER_CELLS * NW / 8; i += 64 * NW) p[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+// Counts a ray in its wavefront's counter of cell c: a 32-bit word holds the counters of two neighbouring wavefronts,
+// and a count stays below 2^16, so adding 1 to a wavefront's own half never carries into the other.
+template <int NW>
+__device__ __forceinline__ void ray_order_count(RayOrderShared<NW> &sh, const uint32_t c, const int wave) {
+    atomicAdd(&reinterpret_cast<uint32_t *>(sh.slot)[(c * NW + wave) >> 1], 1u << (16 * (wave & 1)));
+}
+// Turns a cell's counts into places from `start` on, wavefront after wavefront, and returns the cell's count. The
+// counters of a cell are read and written 4 at a time: lanes take neighbouring cells.
+template <int NW>
+__device__ __forceinline__ int ray_order_places(RayOrderShared<NW> &sh, const int cell, const int start) {
+    ushort4 *p = reinterpret_cast<ushort4 *>(sh.slot + cell * NW);
+    int run = start;
+    for (int k = 0; k < NW / 4; ++k) {
+        ushort4 n = p[k];
+        const ushort4 c = n;
+        n.x = (uint16_t)run; run += c.x;
+        n.y = (uint16_t)run; run += c.y;
+        n.z = (uint16_t)run; run += c.z;
+        n.w = (uint16_t)run; run += c.w;
+        p[k] = n;
+    }
+    return run - start;
+}
+// The number of rays counted in a cell.
+template <int NW>
+__device__ __forceinline__ int ray_order_total(const RayOrderShared<NW> &sh, const int cell) {
+    const ushort4 *p = reinterpret_cast<const ushort4 *>(sh.slot + cell * NW);
+    int sum = 0;
+    for (int k = 0; k < NW / 4; ++k) sum += p[k].x + p[k].y + p[k].z + p[k].w;
+    return sum;
+}
+// The place of a ray of cell c (RAY_ORDER_CELLS: no ray) among its wavefront's, in ray order.
+template <int NW>
+__device__ __forceinline__ int ray_order_place(RayOrderShared<NW> &sh, const bool has, const uint32_t c, const int wave) {
+    uint32_t digit;
+    int rank, cnt, place = 0;
+    tile_digit_bits<12>(has, c, 0, digit, rank, cnt);
+    if (has) place = (int)sh.slot[c * NW + wave] + rank;
+    // every lane has read its cell's place before the cell's first lane moves it on (one wavefront's LDS accesses
+    // complete in order)
+    if (has && rank == 0) sh.slot[c * NW + wave] = (uint16_t)(place + cnt);
+    return place;
+}
+
+// The order of up to 65,536 rays a world, a workgroup of NW wavefronts a world; cells is scratch of one 16-bit cell a
+// ray. What bounds it is the counters' share of LDS (one workgroup of 16 wavefronts fits a compute unit) and, for few
+// rays, clearing and scanning them: there a quarter as many wavefronts take a quarter of the
+// counters (64 worlds of 1,081 rays: 11 us against 15; 1,024 worlds of 4,096 rays, four workgroups a compute unit: 39 us
+// against 71; but 64 such worlds 26 us against 20, each wavefront having four times the rays).
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void ray_order_one_pass_kernel(const float *dirs, const int R, uint16_t *cells, int *order) {
+    __shared__ RayOrderShared<NW> sh;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const size_t base = (size_t)blockIdx.x * R;
     const int seg = (R + NW - 1) / NW;
     const int first = wave * seg, end = min(first + seg, R);
-    uint32_t *slot32 = reinterpret_cast<uint32_t *>(slot);
-    for (int i = tid; i < CELLS * NW / 2; i += 1024) slot32[i] = 0u;
+    ray_order_clear(sh);
     __syncthreads();
-    // each ray's cell, kept for the second sweep, and counted: a 32-bit word holds the counters of two neighbouring
-    // wavefronts, and a count stays below 2^16, so adding 1 to a wavefront's own half never carries into the other
     for (int i = first + lane; i < end; i += 64) {
         const float *p = dirs + 3 * (base + i);
         const uint32_t c = direction_cell(p[0], p[1], p[2]);
         cells[base + i] = (uint16_t)c;
-        atomicAdd(&slot32[(c * NW + wave) >> 1], 1u << (16 * (wave & 1)));
+        ray_order_count(sh, c, wave);
     }
     __syncthreads();
-    // exclusive scan of the 65,536 slots: each thread sums 64 consecutive ones, the threads' sums are scanned, then
-    // each thread writes its slots' starts
-    {
-        constexpr int SPAN = CELLS * NW / 1024;
-        const int s0 = tid * SPAN;
-        int sum = 0;
-        for (int k = 0; k < SPAN; ++k) sum += slot[s0 + k];
-        const int incl = wave_prefix_sum(sum);
-        if (lane == 63) wave_tot[wave] = incl;
+    // the cells in order, a thread a cell, the workgroup's threads at a time
+    int carry = 0;
+    for (int c0 = 0; c0 < RAY_ORDER_CELLS; c0 += 64 * NW) {
+        const int n = ray_order_total(sh, c0 + tid);
+        const int incl = wave_prefix_sum(n);
+        if (lane == 63) sh.wave_tot[wave] = incl;
         __syncthreads();
-        int run = incl - sum;
-        for (int wv = 0; wv < wave; ++wv) run += wave_tot[wv];
-        for (int k = 0; k < SPAN; ++k) {
-            const int n = slot[s0 + k];
-            slot[s0 + k] = (uint16_t)run;
-            run += n;
+        int start = carry + incl - n;
+        for (int wv = 0; wv < NW; ++wv) {
+            if (wv < wave) start += sh.wave_tot[wv];
+            carry += sh.wave_tot[wv];
         }
+        ray_order_places(sh, c0 + tid, start);
+        __syncthreads();
     }
-    __syncthreads();
-    // the rays again, in the same order: each one's place is its cell's next place in this wavefront plus its rank
-    // among the equal cells of its 64
     for (int at = first; at < end; at += 64) {
         const int i = at + lane;
         const bool has = i < end;
-        const uint32_t c = has ? cells[base + i] : (uint32_t)CELLS;
-        uint32_t digit;
-        int rank, cnt;
-        tile_digit_bits<12>(has, c, 0, digit, rank, cnt);
-        int dest = 0;
-        if (c < CELLS) dest = (int)slot[c * NW + wave] + rank;
-        // every lane has read its cell's place before the cell's first lane moves it on (one wavefront's LDS
-        // accesses complete in order)
-        if (c < CELLS && rank == 0) slot[c * NW + wave] = (uint16_t)(dest + cnt);
-        if (c < CELLS) order[base + dest] = i;
+        const uint32_t c = has ? cells[base + i] : (uint32_t)RAY_ORDER_CELLS;
+        const int place = ray_order_place(sh, has, c, wave);
+        if (has) order[base + place] = i;
     }
 }
 
-template <int BITS, int MAX_CHUNKS>
-__global__ __launch_bounds__(1024) void ray_order_kernel(const float *dirs, const int R, uint32_t *ka, uint32_t *kb, int *order) {
-    constexpr int NW = 16, NB = 1 << BITS, PASSES = 12 / BITS;
-    static_assert(PASSES * BITS == 12 && NB * NW <= 1024, "12-bit keys in whole digits, one histogram entry a thread");
-    __shared__ int counts[NB * MAX_CHUNKS];
-    __shared__ int hist[NB * NW];
-    __shared__ int wave_tot[NW];
-    __shared__ int carry;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const size_t base = (size_t)blockIdx.x * R;
-    const int chunks = (R + 1023) / 1024;
-    for (int i = tid; i < R; i += 1024) {
+// Segmented worlds, first kernel: each ray's cell, and how many of the segment's rays fall in each cell.
+__global__ __launch_bounds__(1024) void ray_order_count_kernel(const float *dirs, const int R, const int segments, uint16_t *cells,
+                                                               uint32_t *counts) {
+    __shared__ uint32_t hist[RAY_ORDER_CELLS];
+    const int world = blockIdx.x / segments, s = blockIdx.x % segments;
+    const size_t base = (size_t)world * R;
+    const int end = min((s + 1) * RAY_ORDER_SEGMENT, R);
+    for (int c = threadIdx.x; c < RAY_ORDER_CELLS; c += 1024) hist[c] = 0u;
+    __syncthreads();
+    for (int i = s * RAY_ORDER_SEGMENT + threadIdx.x; i < end; i += 1024) {
         const float *p = dirs + 3 * (base + i);
-        ka[base + i] = (direction_cell(p[0], p[1], p[2]) << RAY_ORDER_INDEX_BITS) | (uint32_t)i;
+        const uint32_t c = direction_cell(p[0], p[1], p[2]);
+        cells[base + i] = (uint16_t)c;
+        atomicAdd(&hist[c], 1u);
     }
     __syncthreads();
-    uint32_t *ks = ka, *kd = kb;
-    for (int pass = 0; pass < PASSES; ++pass) {
-        const int shift = RAY_ORDER_INDEX_BITS + BITS * pass;
-        const bool last = pass == PASSES - 1;
-        for (int c = 0; c < chunks; ++c) {
-            const int i = c * 1024 + tid;
-            const bool has = i < R;
-            if (tid < NB * NW) hist[tid] = 0;
-            __syncthreads();
-            uint32_t digit;
-            int rank, cnt;
-            tile_digit_bits<BITS>(has, has ? ks[base + i] : 0u, shift, digit, rank, cnt);
-            if (has && rank == 0) hist[digit * NW + wave] = cnt;
-            __syncthreads();
-            if (tid < NB) {
-                int sum = 0;
-                for (int wv = 0; wv < NW; ++wv) sum += hist[tid * NW + wv];
-                counts[tid * chunks + c] = sum;
-            }
-            __syncthreads();
-        }
-        // exclusive scan of the counts in digit-major order
-        const int total = NB * chunks;
-        if (tid == 0) carry = 0;
-        __syncthreads();
-        for (int b0 = 0; b0 < total; b0 += 1024) {
-            const int cin = carry;
-            const int idx = b0 + tid;
-            const int x = idx < total ? counts[idx] : 0;
-            int incl = wave_prefix_sum(x);
-            if (lane == 63) wave_tot[wave] = incl;
-            __syncthreads();
-            for (int wv = 0; wv < wave; ++wv) incl += wave_tot[wv];
-            __syncthreads();
-            if (idx < total) counts[idx] = cin + incl - x;
-            if (tid == 1023) carry = cin + incl;
-            __syncthreads();
-        }
-        for (int c = 0; c < chunks; ++c) {
-            const int i = c * 1024 + tid;
-            const bool has = i < R;
-            const uint32_t k = has ? ks[base + i] : 0u;
-            if (tid < NB * NW) hist[tid] = 0;
-            __syncthreads();
-            uint32_t digit;
-            int rank, cnt;
-            tile_digit_bits<BITS>(has, k, shift, digit, rank, cnt);
-            if (has && rank == 0) hist[digit * NW + wave] = cnt;
-            __syncthreads();
-            block_exclusive_scan(hist, NB * NW, wave_tot);
-            if (has) {
-                const int dest = counts[digit * chunks + c] + hist[digit * NW + wave] - hist[digit * NW] + rank;
-                if (last) order[base + dest] = (int)(k & ((1u << RAY_ORDER_INDEX_BITS) - 1u));
-                else kd[base + dest] = k;
-            }
-            __syncthreads();
-        }
-        uint32_t *tk = ks; ks = kd; kd = tk;
+    uint32_t *out = counts + (size_t)blockIdx.x * RAY_ORDER_CELLS;
+    for (int c = threadIdx.x; c < RAY_ORDER_CELLS; c += 1024) out[c] = hist[c];
+}
+
+// Second kernel: a world's counts [segment][cell] become how many of the cell's rays the segments before hold, and
+// totals how many there are in all. A thread a cell, 16 workgroups a world.
+__global__ __launch_bounds__(256) void ray_order_sum_kernel(const int segments, uint32_t *counts, uint32_t *totals) {
+    const int world = blockIdx.x / (RAY_ORDER_CELLS / 256), cell = blockIdx.x % (RAY_ORDER_CELLS / 256) * 256 + threadIdx.x;
+    uint32_t *c = counts + (size_t)world * segments * RAY_ORDER_CELLS + cell;
+    uint32_t run = 0;
+#pragma unroll 16
+    for (int s = 0; s < segments; ++s) {
+        const uint32_t n = c[(size_t)s * RAY_ORDER_CELLS];
+        c[(size_t)s * RAY_ORDER_CELLS] = run;
+        run += n;
+    }
+    totals[(size_t)world * RAY_ORDER_CELLS + cell] = run;
+}
+
+// Third kernel: each segment's rays to their places, 16 wavefronts of 256 rays.
+__global__ __launch_bounds__(1024) void ray_order_segment_kernel(const int R, const int segments, const uint16_t *cells,
+                                                                 const uint32_t *before, const uint32_t *totals, int *order) {
+    constexpr int NW = 16, STEPS = RAY_ORDER_SEGMENT / (64 * NW);
+    __shared__ RayOrderShared<NW> sh;
+    __shared__ uint32_t start[RAY_ORDER_CELLS];  // the first place of the segment's rays of each cell
+    const int world = blockIdx.x / segments, s = blockIdx.x % segments;
+    const size_t base = (size_t)world * R;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int first = s * RAY_ORDER_SEGMENT + wave * 64 * STEPS + lane;
+    uint32_t c[STEPS];
+    for (int k = 0; k < STEPS; ++k) c[k] = first + 64 * k < R ? cells[base + first + 64 * k] : (uint32_t)RAY_ORDER_CELLS;
+    const uint4 n = reinterpret_cast<const uint4 *>(totals + (size_t)world * RAY_ORDER_CELLS)[tid];
+    const uint4 mine = reinterpret_cast<const uint4 *>(before + (size_t)blockIdx.x * RAY_ORDER_CELLS)[tid];
+    ray_order_clear(sh);
+    const int sum = (int)(n.x + n.y + n.z + n.w);
+    const int incl = wave_prefix_sum(sum);
+    if (lane == 63) sh.wave_tot[wave] = incl;
+    __syncthreads();
+    for (int k = 0; k < STEPS; ++k)
+        if (c[k] < RAY_ORDER_CELLS) ray_order_count(sh, c[k], wave);
+    uint32_t at = (uint32_t)(incl - sum);
+    for (int wv = 0; wv < wave; ++wv) at += (uint32_t)sh.wave_tot[wv];
+    reinterpret_cast<uint4 *>(start)[tid] = make_uint4(at + mine.x, at + n.x + mine.y, at + n.x + n.y + mine.z, at + n.x + n.y + n.z + mine.w);
+    __syncthreads();
+    for (int cell = tid; cell < RAY_ORDER_CELLS; cell += 1024) ray_order_places(sh, cell, 0);
+    __syncthreads();
+    for (int k = 0; k < STEPS; ++k) {
+        const bool has = c[k] < RAY_ORDER_CELLS;
+        const int place = ray_order_place(sh, has, c[k], wave);
+        if (has) order[base + start[c[k]] + place] = first + 64 * k;
     }
 }
 
@@ -869,14 +910,35 @@ hipError_t launch_tlas_build_big(const TlasBuildArgs &a, const BigBuildScratch &
     return hipGetLastError();
 }
 
+static bool ray_order_segmented(const int rays_per_world, const int worlds) {
+    return rays_per_world > RAY_ORDER_ONE_PASS_MAX_RAYS ||
+           (rays_per_world >= RAY_ORDER_SEGMENTED_MIN_RAYS && worlds <= RAY_ORDER_SEGMENTED_MAX_WORLDS);
+}
+
+size_t ray_order_scratch_words(const int rays_per_world, const int worlds) {
+    // a cell in 2 bytes a ray; segmented, a word a cell for each world and for each segment, at most one of them broken
+    const size_t n = (size_t)rays_per_world * worlds;
+    const size_t cells = (n + 7) / 8 * 4;
+    const size_t segments = ((size_t)rays_per_world + RAY_ORDER_SEGMENT - 1) / RAY_ORDER_SEGMENT;
+    return ray_order_segmented(rays_per_world, worlds) ? cells + (1 + segments) * worlds * RAY_ORDER_CELLS : cells;
+}
+
 hipError_t launch_ray_order(const float *dirs, const int rays_per_world, const int worlds, uint32_t *keys, int *vals, int **order,
                             hipStream_t stream) {
     if (rays_per_world <= 0 || rays_per_world > RAY_ORDER_MAX_RAYS || worlds <= 0) return hipErrorInvalidValue;
     const size_t n = (size_t)rays_per_world * worlds;
-    if (rays_per_world <= RAY_ORDER_ONE_PASS_MAX_RAYS) {
-        ray_order_one_pass_kernel<<<worlds, 1024, 0, stream>>>(dirs, rays_per_world, reinterpret_cast<uint16_t *>(keys), vals);
+    uint16_t *const cells = reinterpret_cast<uint16_t *>(keys);
+    if (ray_order_segmented(rays_per_world, worlds)) {
+        const int segments = (rays_per_world + RAY_ORDER_SEGMENT - 1) / RAY_ORDER_SEGMENT;
+        uint32_t *const totals = keys + (n + 7) / 8 * 4;  // past the cells, on 16 bytes
+        uint32_t *const counts = totals + (size_t)worlds * RAY_ORDER_CELLS;
+        ray_order_count_kernel<<<worlds * segments, 1024, 0, stream>>>(dirs, rays_per_world, segments, cells, counts);
+        ray_order_sum_kernel<<<worlds * (RAY_ORDER_CELLS / 256), 256, 0, stream>>>(segments, counts, totals);
+        ray_order_segment_kernel<<<worlds * segments, 1024, 0, stream>>>(rays_per_world, segments, cells, counts, totals, vals);
+    } else if (rays_per_world <= (worlds >= RAY_ORDER_MANY_WORLDS ? RAY_ORDER_FEW_RAYS_MANY_WORLDS : RAY_ORDER_FEW_RAYS)) {
+        ray_order_one_pass_kernel<4><<<worlds, 256, 0, stream>>>(dirs, rays_per_world, cells, vals);
     } else {
-        ray_order_kernel<4, RAY_ORDER_MAX_CHUNKS><<<worlds, 1024, 0, stream>>>(dirs, rays_per_world, keys, keys + n, vals);
+        ray_order_one_pass_kernel<16><<<worlds, 1024, 0, stream>>>(dirs, rays_per_world, cells, vals);
     }
     *order = vals;
     return hipGetLastError();

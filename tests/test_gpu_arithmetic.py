@@ -84,3 +84,21 @@ def test_ray_order_is_the_stable_order_of_direction_cells(gpu):
             assert np.array_equal(np.sort(order[w]), np.arange(rays)), (worlds, rays, w)
             assert np.array_equal(order[w], np.argsort(cells, kind="stable")), (worlds, rays, w)
         assert np.array_equal(order[1], np.arange(rays))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("worlds,rays", [(1, 1), (3, 63), (2, 2048), (2, 2049), (512, 4096), (2, 4097), (3, 8191), (1, 8192), (2, 8193),
+                                         (1, 12288), (97, 8192), (1, 65536), (1, 65537), (2, 131071), (1, 262144)])
+def test_ray_order_at_the_edges_of_its_kernels(gpu, worlds, rays):
+    """The same order where one workgroup a world gives way to a smaller one and to segments of 4096 rays: the sizes on
+    either side of each line, whole and broken segments, and as many worlds as take one workgroup each again."""
+    import numpy as np
+    from neraulgraphics_amd import _lib
+    rng = np.random.default_rng(rays + worlds)
+    d = rng.normal(size=(worlds, rays, 3)).astype(np.float32)
+    d[:, ::3] *= np.float32([0.02, 0.02, 1.0])  # a third of them crowded into a few cells
+    order = np.full((worlds, rays), -1, np.int32)
+    print(f"ray order: {worlds} worlds x {rays} rays", flush=True)
+    _lib.check(_lib.load().ngx_debug_ray_order(0, np.ascontiguousarray(d).ctypes.data, rays, worlds, order.ctypes.data))
+    for w in range(worlds):
+        assert np.array_equal(order[w], np.argsort(_direction_cells(d[w]), kind="stable")), w
