@@ -124,9 +124,12 @@ struct ngx_ctx {
     int *d_blas_parent = nullptr;
     int *d_blas_wide_node = nullptr;
     // deforming meshes (ngx_set_mesh_vertices)
-    float *d_vertices = nullptr;        // every mesh's vertices, 3 floats each
-    int *d_tri_verts = nullptr, *d_node_parent = nullptr, *d_node_wide = nullptr, *d_node_arrivals = nullptr;
-    std::vector<int> mesh_vertex_base, mesh_vertex_count, mesh_node_base, mesh_node_count, mesh_tri_base, mesh_tri_count;
+    float *d_vertices = nullptr;        // every mesh's vertices, 3 floats each: where new ones from the host land
+    int *d_tri_verts = nullptr, *d_refit_levels = nullptr;
+    ngx::RefitEntry *d_refit_entries = nullptr;
+    ngx::RefitTreelet *d_refit_treelets = nullptr;
+    std::vector<std::vector<ngx::host::RefitLayer>> refit_layers;  // per mesh
+    std::vector<int> mesh_vertex_base, mesh_vertex_count, mesh_tri_count;
     std::vector<uint8_t> mesh_has_normals;
     bool top_level_stale = false;       // a mesh moved since the last pose update
     ngx::SkipNode *d_skip = nullptr;
@@ -206,7 +209,7 @@ struct ngx_ctx {
 
     ~ngx_ctx() {
         int *ints[] = {d_world_off, d_tmpl_mesh, d_roots, d_body_of_instance, d_dbg_sorted_ids, d_blas_parent, d_blas_wide_node, d_wide_parent,
-                       d_tri_verts, d_node_parent, d_node_wide, d_node_arrivals,
+                       d_tri_verts, d_refit_levels,
                        d_geom_of_instance, d_tile_counters, d_mesh_skip_root, d_mesh_tris, d_overflow};
         for (int *p : ints) if (p) (void)hipFree(p);
         float *floats[] = {d_vertices, d_mesh_bounds, d_matrices, d_matrix_stage, d_local_pose, d_scale, d_local_rot_scale, d_body_stage,
@@ -215,7 +218,7 @@ struct ngx_ctx {
         for (float *p : floats) if (p) (void)hipFree(p);
         void *others[] = {d_root_at_end, d_blas_wide, d_mesh_roots, d_tris, d_attrs, d_spheres, d_inst, d_nodes, d_wide,
                           d_id, d_hit_id, d_dbg_keys, d_dbg_sorted_keys, d_skip, d_ray_keys, d_ray_vals, d_inst_mat, d_sphere_mat,
-                          d_lights, d_rgb, d_rgb_hits, d_rgb_uv, big.key[0], big.key[1], big.val[0], big.val[1],
+                          d_lights, d_rgb, d_refit_entries, d_refit_treelets, d_rgb_hits, d_rgb_uv, big.key[0], big.key[1], big.val[0], big.val[1],
                           big.box, big.node_box, big.left, big.right, big.parent, big.arrivals, big.bounds, big.tile_counts};
         for (void *p : others) if (p) (void)hipFree(p);
         if (ev0) (void)hipEventDestroy(ev0);
@@ -494,17 +497,15 @@ ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out) {
             upload(c.d_mesh_skip_root, built.roots.data(), built.roots.size());
             upload(c.d_vertices, s.vertices, 3 * (size_t)s.vertex_offsets[s.mesh_count]);
             upload(c.d_tri_verts, built.tri_verts.data(), built.tri_verts.size());
-            upload(c.d_node_parent, built.node_parent.data(), built.node_parent.size());
-            upload(c.d_node_wide, built.node_wide.data(), built.node_wide.size());
-            device_alloc(c.d_node_arrivals, built.nodes.size());
+            upload(c.d_refit_levels, built.refit_levels.data(), built.refit_levels.size());
+            upload(c.d_refit_entries, built.refit_entries.data(), built.refit_entries.size());
+            upload(c.d_refit_treelets, built.refit_treelets.data(), built.refit_treelets.size());
+            c.refit_layers = built.refit_layers;
             for (int m = 0; m < s.mesh_count; ++m) {
                 c.mesh_vertex_base.push_back(s.vertex_offsets[m]);
                 c.mesh_vertex_count.push_back(s.vertex_offsets[m + 1] - s.vertex_offsets[m]);
                 c.mesh_has_normals.push_back(s.normals && s.mesh_has_normals && s.mesh_has_normals[m] ? 1 : 0);
             }
-            c.mesh_node_base = built.node_base;
-            c.mesh_node_count = built.node_count;
-            c.mesh_tri_base = built.tri_base;
             c.mesh_tri_count = built.tri_counts;
             upload(c.d_mesh_tris, built.tri_counts.data(), built.tri_counts.size());
             for (const int t : built.tri_counts) c.max_mesh_tris = std::max(c.max_mesh_tris, t);
@@ -760,27 +761,24 @@ ngx_status ngx_set_mesh_vertices(ngx_ctx *ctx, const int32_t mesh, const float *
         if (ctx->mesh_tri_count[mesh] == 0) return;
         ctx->set_device();
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        float *dst = ctx->d_vertices + 3 * (size_t)ctx->mesh_vertex_base[mesh];
-        HIP_CHECK(hipMemcpyAsync(dst, vertices, n * sizeof(float),
-                                 memory == NGX_MEM_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice, s));
         ngx::MeshRefitArgs a{};
-        a.vertices = dst;
+        a.vertices = vertices;
+        if (memory == NGX_MEM_HOST) {
+            float *dst = ctx->d_vertices + 3 * (size_t)ctx->mesh_vertex_base[mesh];
+            HIP_CHECK(hipMemcpyAsync(dst, vertices, n * sizeof(float), hipMemcpyHostToDevice, s));
+            a.vertices = dst;
+        }
         a.vertex_base = ctx->mesh_vertex_base[mesh];
         a.tri_verts = ctx->d_tri_verts;
-        a.tri_base = ctx->mesh_tri_base[mesh];
-        a.tri_count = ctx->mesh_tri_count[mesh];
         a.tris = ctx->d_tris;
         a.skip = ctx->d_skip + 1;
-        a.node_parent = ctx->d_node_parent;
-        a.node_wide = ctx->d_node_wide;
         a.wide = ctx->d_blas_wide;
-        a.node_base = ctx->mesh_node_base[mesh];
-        a.node_count = ctx->mesh_node_count[mesh];
-        a.root = ctx->mesh_node_base[mesh];
-        a.arrivals = ctx->d_node_arrivals;
+        a.treelets = ctx->d_refit_treelets;
+        a.entries = ctx->d_refit_entries;
+        a.levels = ctx->d_refit_levels;
         a.mesh_root = ctx->d_mesh_roots + mesh;
         a.mesh_bounds = ctx->d_mesh_bounds + 6 * (size_t)mesh;
-        HIP_CHECK(ngx::launch_mesh_refit(a, s));
+        for (const ngx::host::RefitLayer &layer : ctx->refit_layers[mesh]) HIP_CHECK(ngx::launch_mesh_refit(a, layer.first, layer.count, s));
         ctx->top_level_stale = true;
     });
 }

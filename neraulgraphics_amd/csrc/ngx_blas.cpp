@@ -148,6 +148,70 @@ int sah_build(const Box *bounds, const int n, const int max_leaf, std::vector<Bl
     return static_cast<int>(nodes.size());
 }
 
+// Cuts every mesh's tree into treelets, the lowest first: a treelet is a largest subtree of at most `most` nodes, and
+// once a layer's treelets are taken out the tree above them is cut the same way, until the root is in one. The lowest
+// layer's treelets are small enough to be a few hundred for a large mesh (a workgroup each); a small tree is one.
+static void plan_refits(const std::vector<int> &wide_index, BuiltMeshes &out) {
+    const std::vector<BlasNode> &nodes = out.nodes;
+    std::vector<int> size(nodes.size()), slot(nodes.size(), -1), height(nodes.size());
+    std::vector<uint8_t> done(nodes.size(), 0);
+    for (size_t m = 0; m < out.roots.size(); ++m) {
+        const int base = out.roots[m], end = m + 1 < out.roots.size() ? out.roots[m + 1] : static_cast<int>(nodes.size());
+        std::vector<RefitLayer> layers;
+        int most = REFIT_TREELET_NODES;
+        if (end - base > most) most = std::min(512, std::max(128, (end - base) / 256));
+        while (!done[base]) {
+            // the nodes left below each node: children come after their parent
+            for (int i = end - 1; i >= base; --i)
+                size[i] = done[i] ? 0 : nodes[i].count > 0 ? 1 : 1 + size[nodes[i].a] + size[nodes[i].a + 1];
+            RefitLayer layer{static_cast<int>(out.refit_treelets.size()), 0};
+            for (int root = base; root < end; ++root) {
+                if (done[root] || size[root] > most || (root != base && size[out.node_parent[root]] <= most)) continue;
+                std::vector<int> members{root};
+                for (size_t k = 0; k < members.size(); ++k) {
+                    const BlasNode &n = nodes[members[k]];
+                    for (int c = 0; n.count == 0 && c < 2; ++c)
+                        if (!done[n.a + c]) members.push_back(n.a + c);
+                }
+                int levels = 0;
+                for (size_t k = members.size(); k-- > 0;) {
+                    const int i = members[k];
+                    height[i] = 0;
+                    for (int c = 0; nodes[i].count == 0 && c < 2; ++c)
+                        if (!done[nodes[i].a + c]) height[i] = std::max(height[i], 1 + height[nodes[i].a + c]);
+                    levels = std::max(levels, height[i] + 1);
+                }
+                std::stable_sort(members.begin(), members.end(), [&](const int x, const int y) { return height[x] < height[y]; });
+                out.refit_treelets.push_back(RefitTreelet{static_cast<int>(out.refit_entries.size()),
+                                                          static_cast<int>(out.refit_levels.size()), levels, root == base ? 1 : 0});
+                for (size_t k = 0; k < members.size(); ++k) {
+                    if (k == 0 || height[members[k]] != height[members[k - 1]]) out.refit_levels.push_back(static_cast<int>(k));
+                    slot[members[k]] = static_cast<int>(k);
+                    const BlasNode &n = nodes[members[k]];
+                    RefitEntry e{members[k], n.a, n.count, -1};
+                    if (n.count == 0) {
+                        e.wide = wide_index[members[k]];
+                        e.left = done[n.a] ? ~n.a : slot[n.a];
+                        e.right = done[n.a + 1] ? ~(n.a + 1) : slot[n.a + 1];
+                    }
+                    out.refit_entries.push_back(e);
+                }
+                out.refit_levels.push_back(static_cast<int>(members.size()));
+                ++layer.count;
+            }
+            // taken out only now: a treelet's children are its own or an earlier layer's
+            for (int t = layer.first; t < layer.first + layer.count; ++t) {
+                const RefitTreelet &tr = out.refit_treelets[t];
+                const int n = out.refit_levels[tr.level_first + tr.levels];
+                for (int k = 0; k < n; ++k) done[out.refit_entries[tr.first + k].node] = 1;
+            }
+            layers.push_back(layer);
+            most = REFIT_TREELET_NODES;
+        }
+        out.refit_layers.push_back(layers);
+    }
+}
+
 void build_meshes(const MeshInput &in, BuiltMeshes &out) {
     out = BuiltMeshes{};
     bool any_normals = false;
@@ -174,9 +238,6 @@ void build_meshes(const MeshInput &in, BuiltMeshes &out) {
         const int node_base = static_cast<int>(out.nodes.size());
         const int tri_base = static_cast<int>(out.triangles.size() / 12);
         out.roots.push_back(node_base);
-        out.node_base.push_back(node_base);
-        out.node_count.push_back(static_cast<int>(tree.size()));
-        out.tri_base.push_back(tri_base);
         out.bounds.push_back(Box{{tree[0].lo[0], tree[0].lo[1], tree[0].lo[2]}, {tree[0].hi[0], tree[0].hi[1], tree[0].hi[2]}});
         for (BlasNode node : tree) {
             node.a += node.count > 0 ? tri_base : node_base;
@@ -210,7 +271,6 @@ void build_meshes(const MeshInput &in, BuiltMeshes &out) {
     for (size_t i = 0; i < out.nodes.size(); ++i)
         if (out.nodes[i].count == 0) wide_index[i] = wide_count++;
     out.wide.resize(static_cast<size_t>(wide_count));
-    out.node_wide = wide_index;
     out.node_parent.assign(out.nodes.size(), -1);
     for (size_t i = 0; i < out.nodes.size(); ++i)
         if (out.nodes[i].count == 0) out.node_parent[out.nodes[i].a] = out.node_parent[out.nodes[i].a + 1] = static_cast<int>(i);
@@ -298,6 +358,7 @@ void build_meshes(const MeshInput &in, BuiltMeshes &out) {
         child_ref(root, out.roots[m], mr.ref, mr.count);
         out.mesh_roots.push_back(mr);
     }
+    plan_refits(wide_index, out);
 }
 
 bool transform_ok(const float *m) {

@@ -87,6 +87,21 @@ struct alignas(64) SkipNode {
 };
 static_assert(sizeof(SkipNode) == 64, "64-byte skip node");
 
+// How a mesh's bottom level is refitted to new vertices: its tree is cut into treelets of at most REFIT_TREELET_NODES
+// nodes, a workgroup each, whose boxes are made level by level from the leaves. An entry is a node of a treelet: a leaf
+// (wide < 0) with its first triangle and their count, or an interior node with its wide node and its children, each
+// the child's entry within the treelet or ~ the node of a treelet made before. A treelet's entries are in order of
+// level, its root last.
+constexpr int REFIT_TREELET_NODES = 1024;
+struct alignas(16) RefitEntry {
+    int32_t node, left, right, wide;
+};
+struct RefitTreelet {
+    int32_t first;               // its entries
+    int32_t level_first, levels; // where each level's entries start, levels + 1 values, relative to first
+    int32_t is_root;             // the mesh's root is this treelet's
+};
+
 // ------------------------------------------------------------------ float3 arithmetic --
 
 __device__ __forceinline__ float3 mk3(float x, float y, float z) { return make_float3(x, y, z); }

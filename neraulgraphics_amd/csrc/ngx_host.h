@@ -21,6 +21,11 @@ struct MeshInput {
     const uint8_t *has_normals;
 };
 
+// Treelets that can be refitted side by side.
+struct RefitLayer {
+    int first, count;
+};
+
 struct BuiltMeshes {
     std::vector<BlasNode> nodes;      // the reference's layout, global indices
     std::vector<float> triangles;     // 12 floats each: v0, e1, e2
@@ -36,8 +41,10 @@ struct BuiltMeshes {
     // for refitting a mesh to new vertices on the device (ngx_set_mesh_vertices)
     std::vector<int> tri_verts;       // per packed triangle: its three vertices, global indices
     std::vector<int> node_parent;     // per node of `nodes`: its parent, -1 at a mesh's root
-    std::vector<int> node_wide;       // per node of `nodes`: its wide node, -1 for a leaf
-    std::vector<int> node_base, node_count, tri_base;  // per mesh
+    std::vector<RefitEntry> refit_entries;
+    std::vector<int> refit_levels;
+    std::vector<RefitTreelet> refit_treelets;
+    std::vector<std::vector<RefitLayer>> refit_layers;  // per mesh: its treelets, each layer's from those before
 };
 
 // Binned SAH build (src/bvh.cpp:46-174). Returns the node count.

@@ -256,18 +256,17 @@ struct MeshRefitArgs {
     const float *vertices;    // the mesh's vertices, 3 floats each
     int vertex_base;          // global index of its first vertex (tri_verts holds global indices)
     const int *tri_verts;     // per packed triangle: its three vertices
-    int tri_base, tri_count;  // the mesh's packed triangles
     float *tris;              // packed triangles, 9 floats each
-    SkipNode *skip;           // per node: the box written here first
-    const int *node_parent;   // per node, -1 at the root
-    const int *node_wide;     // per node: its wide node, -1 for a leaf
+    SkipNode *skip;           // every node's box is written here
     WideNode *wide;
-    int node_base, node_count, root;
-    int *arrivals;            // per node, zeroed by the launch
+    const RefitTreelet *treelets;
+    const RefitEntry *entries;
+    const int *levels;
     MeshRoot *mesh_root;      // the mesh's
     float *mesh_bounds;       // the mesh's 6 floats (lo, hi): the top-level build's local box
 };
-hipError_t launch_mesh_refit(const MeshRefitArgs &a, hipStream_t stream);
+// One layer of the mesh's treelets, first .. first + count - 1; the layers in order.
+hipError_t launch_mesh_refit(const MeshRefitArgs &a, int first, int count, hipStream_t stream);
 
 // The RGB picture; with a.r.tile_counters set and compute_units > 0, from a persistent grid as launch_render.
 hipError_t launch_rgb(const RgbArgs &a, hipStream_t stream, int compute_units = 0);

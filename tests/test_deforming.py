@@ -78,3 +78,26 @@ def test_refits_refuse_bad_input(gpu):
     with pytest.raises(ValueError, match="values"):
         r.set_mesh_vertices(1, bad[:-1])
     r.render(cfg["cameras"], cfg["fov"], depth=True)  # nothing moved: still renders
+
+
+@pytest.mark.parametrize("nx,ny", [(1, 1), (2, 1), (17, 15), (18, 15), (40, 25), (96, 64)])
+def test_refits_of_trees_of_one_and_of_several_treelets(gpu, oracle, nx, ny):
+    """Meshes of one leaf, of one treelet (up to 1024 nodes), just over it, and of many: moved vertices give the image of
+    the deformed mesh built afresh, and the original vertices give back the first image bit for bit."""
+    import torch
+    cfg = workloads.make("one_world_icospheres")
+    mesh = ng.geometry.make_grid(nx, ny, 2.0, 1.5, 0.1, seed=nx)
+    cfg["meshes"] = [mesh]
+    r = workloads.make_renderer(cfg)
+    before = r.render(cfg["cameras"], cfg["fov"], depth=True, object_ids=True)
+    moved = _wave(mesh)
+    r.set_mesh_vertices(0, torch.from_numpy(moved).cuda())
+    r.set_instance_transforms(cfg["matrices"])
+    out = r.render(cfg["cameras"], cfg["fov"], depth=True, object_ids=True)
+    compare_images(dict(depth=out["depth"], object_id=out["object_ids"]),
+                   forward(dict(cfg, meshes=[ng.Mesh(moved, mesh.indices)]), oracle), f"grid {nx} x {ny}")
+    r.set_mesh_vertices(0, mesh.vertices)
+    r.set_instance_transforms(cfg["matrices"])
+    again = r.render(cfg["cameras"], cfg["fov"], depth=True, object_ids=True)
+    assert np.array_equal(again["depth"].view(np.uint32), before["depth"].view(np.uint32))
+    assert np.array_equal(again["object_ids"], before["object_ids"])
