@@ -111,6 +111,8 @@ struct ngx_ctx {
     int small_max = 0;                // the largest world built by one workgroup
     std::vector<int> big_worlds;      // worlds built by the device-wide path
     ngx::BigBuildScratch big{};
+    ngx::BigWorld *d_big_worlds = nullptr;
+    ngx::BigTile *d_big_sort_tiles = nullptr, *d_big_node_tiles = nullptr;
     std::vector<int> counts, world_off;
     int sphere_count = 0;
     float floor[4] = {0, 0, 0, 0};
@@ -219,7 +221,7 @@ struct ngx_ctx {
         void *others[] = {d_root_at_end, d_blas_wide, d_mesh_roots, d_tris, d_attrs, d_spheres, d_inst, d_nodes, d_wide,
                           d_id, d_hit_id, d_dbg_keys, d_dbg_sorted_keys, d_skip, d_ray_keys, d_ray_vals, d_inst_mat, d_sphere_mat,
                           d_lights, d_rgb, d_refit_entries, d_refit_treelets, d_rgb_hits, d_rgb_uv, big.key[0], big.key[1], big.val[0], big.val[1],
-                          big.box, big.node_box, big.left, big.right, big.parent, big.arrivals, big.bounds, big.tile_counts};
+                          big.box, big.span, big.across, big.bounds, d_big_worlds, d_big_sort_tiles, d_big_node_tiles};
         for (void *p : others) if (p) (void)hipFree(p);
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
@@ -325,8 +327,8 @@ struct ngx_ctx {
     }
 
     void build(const ngx::TlasBuildArgs &a, hipStream_t stream) const {
-        HIP_CHECK(ngx::launch_tlas_build(a, small_max, stream));
-        for (const int w : big_worlds) HIP_CHECK(ngx::launch_tlas_build_big(a, big, w, world_off[w], counts[w], stream));
+        if (small_max > 0) HIP_CHECK(ngx::launch_tlas_build(a, small_max, stream));  // an empty world stays as it was created
+        if (!big_worlds.empty()) HIP_CHECK(ngx::launch_tlas_build_big(a, big, stream));
     }
 
     void build_from_matrices(const float *matrices_wp12, hipStream_t stream) {
@@ -550,21 +552,36 @@ ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out) {
             device_alloc(c.d_wide_parent, std::max<size_t>(1, (size_t)c.total - 1));
             if (!c.big_worlds.empty()) {
                 ngx::BigBuildScratch &b = c.big;
-                b.capacity = 0;
-                for (const int w : c.big_worlds) b.capacity = std::max(b.capacity, counts[w]);
-                const size_t cap = (size_t)b.capacity, tiles = (cap + 1023) / 1024;
-                for (int k = 0; k < 2; ++k) {
-                    device_alloc(b.key[k], cap);
-                    device_alloc(b.val[k], cap);
+                std::vector<ngx::BigWorld> big;
+                std::vector<ngx::BigTile> sort_tiles, node_tiles;
+                int largest = 0, base = 0;
+                for (const int w : c.big_worlds) {
+                    const int slot = (int)big.size(), n = counts[w];
+                    big.push_back(ngx::BigWorld{w, c.world_off[w], n, base});
+                    for (int i = 0; i < n; i += ngx::BIG_SORT_TILE) sort_tiles.push_back(ngx::BigTile{slot, i});
+                    for (int i = 0; i < n; i += ngx::BIG_NODE_TILE) node_tiles.push_back(ngx::BigTile{slot, i});
+                    base += n;
+                    largest = std::max(largest, n);
                 }
-                device_alloc(b.box, 6 * cap);
-                device_alloc(b.node_box, 6 * cap);
-                device_alloc(b.left, cap);
-                device_alloc(b.right, cap);
-                device_alloc(b.parent, 2 * cap);
-                device_alloc(b.arrivals, cap);
-                device_alloc(b.bounds, 6);
-                device_alloc(b.tile_counts, 16 * tiles);
+                upload(c.d_big_worlds, big.data(), big.size());
+                upload(c.d_big_sort_tiles, sort_tiles.data(), sort_tiles.size());
+                upload(c.d_big_node_tiles, node_tiles.data(), node_tiles.size());
+                b.capacity = base;
+                b.largest = largest;
+                b.worlds = c.d_big_worlds;
+                b.sort_tiles = c.d_big_sort_tiles;
+                b.node_tiles = c.d_big_node_tiles;
+                b.sort_tile_count = (int)sort_tiles.size();
+                b.node_tile_count = (int)node_tiles.size();
+                for (int k = 0; k < 2; ++k) {
+                    device_alloc(b.key[k], (size_t)base);
+                    device_alloc(b.val[k], (size_t)base);
+                }
+                device_alloc(b.box, 6 * (size_t)base);
+                device_alloc(b.span, 3 * (size_t)base);
+                device_alloc(b.across, (size_t)base);
+                device_alloc(b.bounds, 6 * big.size());
+                HIP_CHECK(ngx::reset_big_bounds(b, (int)big.size()));
             }
             // nodes that join worlds are never written by a build: give them a fixed value once
             HIP_CHECK(hipMemset(c.d_nodes, 0, sizeof(ngx::TlasNode) * (2 * (size_t)c.total - 1)));

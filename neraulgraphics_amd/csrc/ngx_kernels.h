@@ -228,18 +228,28 @@ hipError_t noalloc_scratch(float **out);
 // workgroup per world; larger worlds are skipped.
 hipError_t launch_tlas_build(const TlasBuildArgs &a, int max_count, hipStream_t stream);
 
-// Scratch of the device-wide build of one large world, sized for `capacity` instances.
+// The worlds of more than WORKGROUP_BUILD_MAX instances, built together: each one's place in the batch and in the
+// scratch, and the tiles its instances are cut into.
+struct BigWorld {
+    int world, first, n;  // the world's number, its first instance and how many it has
+    int base;             // its first element in the scratch arrays
+};
+struct BigTile {
+    int world, first;     // which of the large worlds, and the tile's first instance of it
+};
 struct BigBuildScratch {
-    int capacity;
+    int capacity;              // the large worlds' instances
+    int largest;               // the largest of them
+    const BigWorld *worlds;
+    const BigTile *sort_tiles, *node_tiles;  // of 1024 and of 256 instances
+    int sort_tile_count, node_tile_count;
     uint32_t *key[2], *val[2]; // [capacity] each
     float *box;                // [6][capacity]: instance boxes by template index, lo xyz then hi xyz
-    float *node_box;           // [6][capacity]: internal node boxes by local index
-    int *left, *right;         // [capacity]
-    int *parent;               // [2 * capacity]
-    int *arrivals;             // [capacity]
-    int *bounds;               // [6]: centre bounds as ordered ints
-    int *tile_counts;          // [16 * ceil(capacity / 1024)]
+    float4 *span;              // [capacity][3]: by sorted place, the box of the leaves of its tile up to it, and from it on
+    int4 *across;              // [capacity]: an internal node that spans tiles (children, first and last leaf), or -1
+    int *bounds;               // [worlds][6]: centre bounds as ordered ints, reset by the build that used them
 };
+constexpr int BIG_SORT_TILE = 1024, BIG_NODE_TILE = 256;
 
 // Per world, a stable order of its rays by direction cell, for coherent wavefronts: keys is scratch of
 // ray_order_scratch_words words, vals receives the order (rays_per_world x worlds), and *order is vals.
@@ -248,8 +258,9 @@ size_t ray_order_scratch_words(int rays_per_world, int worlds);
 hipError_t launch_ray_order(const float *dirs, int rays_per_world, int worlds, uint32_t *keys, int *vals, int **order,
                             hipStream_t stream);
 
-// Builds world `world` (instances first .. first+n-1, n > 1) with grid-wide kernels.
-hipError_t launch_tlas_build_big(const TlasBuildArgs &a, const BigBuildScratch &s, int world, int first, int n, hipStream_t stream);
+// Builds the large worlds with grid-wide kernels; reset_big_bounds readies the bounds for the first build.
+hipError_t launch_tlas_build_big(const TlasBuildArgs &a, const BigBuildScratch &s, hipStream_t stream);
+hipError_t reset_big_bounds(const BigBuildScratch &s, int worlds);
 // The RGB picture of every view, one 64-pixel tile per wavefront.
 // A mesh's bottom level refitted to new vertices (ngx_refit.hip).
 struct MeshRefitArgs {

@@ -93,6 +93,25 @@ def test_large_worlds_build_and_render_as_the_reference_algorithm(gpu, oracle):
     assert rep["hits"] > 1000
 
 
+@pytest.mark.parametrize("counts", [[1025], [1280, 1281], [2048, 3, 2049, 0, 1026], [5000, 1025], [32768, 1500], [32769]])
+@pytest.mark.parametrize("crowded", [False, True], ids=["spread", "crowded"])
+def test_large_world_builds_at_the_edges_of_their_tiles(gpu, oracle, counts, crowded):
+    """Large worlds are built together in tiles of 1024 (sort) and 256 (boxes) leaves, up to 32 sorted runs merged at
+    once: worlds just over a tile or a merge, several at a time with small and empty ones between. Crowded, most keys are
+    equal, so only positions tell them apart; twice, since a build readies the next one's bounds."""
+    _say(f"large-world build edges: counts {counts}, crowded {crowded}")
+    cfg = workloads.scattered(len(counts), max(counts), counts=counts, spread=30.0, width=16, height=16)
+    if crowded:
+        cfg["matrices"] = cfg["matrices"].copy()
+        cfg["matrices"].reshape(len(counts), -1, 12)[:, 5:, 3::4] = np.float32([0.5, -0.25, -20.0])
+    r = workloads.make_renderer(cfg)
+    r.keep_build_intermediates(True)
+    r.set_instance_transforms(cfg["matrices"])
+    r.set_instance_transforms(cfg["matrices"])
+    ref = forward(cfg, oracle, outputs=())
+    _check_build(r, ref, ref["world_off"])
+
+
 @pytest.mark.parametrize("worlds,per", [(1, 20000), (300, 40)])
 def test_morton_trees_see_what_the_sah_trees_see(gpu, oracle, worlds, per):
     """tests/test_batch.cpp:335-371: 20,000 instances in one world and 300 worlds of 40, rendered through this
