@@ -292,6 +292,44 @@ struct ngx_ctx {
 
     void set_device() const { HIP_CHECK(hipSetDevice(device)); }
 
+    // How many rays a wavefront takes. A launch of few wavefronts leaves most of the chip idle, and each of them walks
+    // the union of its 64 rays' paths, one dependent node read after the other; with fewer rays a wavefront there are
+    // more of them, each walks less, and the lanes without a ray take subtrees off those that have one. Full wavefronts
+    // do the least work in all, so the line is where the chip fills up: lanes by wavefronts of 64 rays per compute unit
+    // (mixed meshes, us a step: 64 wavefronts 86 with 64 lanes, 60 with 8; 1,024: 89, 79 with 8, 74 with 16; 2,048: 145,
+    // 124 with 16; 4,096: 99, 96 with 32; 8,192: 116, 121 with 32). Worlds whose top level is large walk longer (20,000
+    // instances, 84 wavefronts: 600 with 64 lanes, 261 with 8, 208 with 4), and so do paths of several segments and
+    // samples (`deep`; 432 wavefronts: 3,393 with 64, 1,940 with 8, 1,824 with 4; 6,912: 4,550, 4,111 with 32).
+    // Where a ray meets two triangles of one object at the same distance (through their shared edge) it keeps whichever
+    // the wavefront tests first; between full and part wavefronts that differs for one ray in 10^7 to 10^8, but for one
+    // in 10^6 on a mesh of very many small triangles, where outputs that show it (normals) keep to full wavefronts.
+    int wave_lanes(const long long rays, const bool normals, const bool deep) const {
+        if (walk() == 0 || (normals && max_mesh_tris > FINE_MESH_TRIANGLES)) return 64;
+        const long long waves = (rays + 63) / 64, cus = std::max(1, compute_units);
+        if (deep) return waves <= 2 * cus ? 4 : waves <= 8 * cus ? 8 : waves <= 16 * cus ? 16 : waves <= 32 * cus ? 32 : 64;
+        if (max_count > ngx::WORKGROUP_BUILD_MAX && waves <= 2 * cus) return 4;
+        return waves <= 2 * cus ? 8 : waves <= 8 * cus ? 16 : waves <= 24 * cus ? 32 : 64;
+    }
+    static constexpr int FINE_MESH_TRIANGLES = 10000;
+
+    // The tiles of a picture: `shape` pixels wide and 64 in all, the longer side halved until a tile has `lanes` pixels.
+    void set_tiles(ngx::RenderArgs &a, const int lanes, const int shape) const {
+        a.tile_w = shape;
+        a.tile_h = 64 / shape;
+        while (a.tile_w * a.tile_h > lanes) {
+            if (a.tile_h >= a.tile_w) a.tile_h /= 2;
+            else a.tile_w /= 2;
+        }
+        a.tile_w_log2 = 0;
+        while ((1 << a.tile_w_log2) < a.tile_w) ++a.tile_w_log2;
+        a.tiles_x = (width + a.tile_w - 1) / a.tile_w;
+        a.tiles_per_view = a.tiles_x * ((height + a.tile_h - 1) / a.tile_h);
+        a.total_tiles = (long long)a.tiles_per_view * views;
+        a.by_tiles_per_view = ngx::fast_divide_by(a.tiles_per_view);
+        a.by_tiles_x = ngx::fast_divide_by(a.tiles_x);
+        a.by_cameras = ngx::fast_divide_by(cpw);
+    }
+
     ngx::RenderArgs render_args(const float *cams, const float fov) const {
         ngx::RenderArgs a{};
         a.s = trace_scene();
@@ -302,11 +340,7 @@ struct ngx_ctx {
         a.height = height;
         a.cameras_per_world = cpw;
         a.views = views;
-        a.tile_w = tile_w;
-        a.tile_h = 64 / tile_w;
-        a.tiles_x = (width + a.tile_w - 1) / a.tile_w;
-        a.tiles_per_view = a.tiles_x * ((height + a.tile_h - 1) / a.tile_h);
-        a.total_tiles = (long long)a.tiles_per_view * views;
+        set_tiles(a, 64, tile_w);
         a.xcd_remap = xcd_remap;
         a.walk = walk();
         a.tile_counters = persistent ? d_tile_counters : nullptr;
@@ -916,23 +950,11 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
             cams = ctx->d_cam_stage;
         }
         ngx::RenderArgs a = ctx->render_args(cams, fov);
-        a.fov_scale = std::tan(fov * 0.5f);
-        a.aspect = (float)ctx->width / (float)ctx->height;
-        a.width = ctx->width;
-        a.height = ctx->height;
-        a.cameras_per_world = ctx->cpw;
-        a.views = ctx->views;
-        a.tile_w = ctx->tile_w;
-        a.tile_h = 64 / ctx->tile_w;
-        a.tiles_x = (ctx->width + a.tile_w - 1) / a.tile_w;
-        a.tiles_per_view = a.tiles_x * ((ctx->height + a.tile_h - 1) / a.tile_h);
-        a.total_tiles = (long long)a.tiles_per_view * ctx->views;
         a.depth = (outputs & NGX_OUTPUT_DEPTH) ? ctx->d_depth : nullptr;
         a.normal = (outputs & NGX_OUTPUT_NORMAL) ? ctx->d_normal : nullptr;
         a.object_id = (outputs & NGX_OUTPUT_OBJECT_ID) ? ctx->d_id : nullptr;
-        a.xcd_remap = ctx->xcd_remap;
-        a.walk = ctx->walk();
         a.blocks = ctx->render_blocks;
+        ctx->set_tiles(a, ctx->wave_lanes((long long)pixels, (outputs & (NGX_OUTPUT_NORMAL | NGX_OUTPUT_RGB)) != 0, false), ctx->tile_w);
         uint8_t *rgb = nullptr;
         if (outputs & NGX_OUTPUT_RGB) {
             if (!ctx->d_rgb) device_alloc(ctx->d_rgb, 3 * pixels);
@@ -964,6 +986,7 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
                 g.hit_uv = ctx->d_attrs ? ctx->d_rgb_uv : nullptr;
                 HIP_CHECK(ngx::launch_rgb_two_pass(g, ctx->render_blocks, s, ctx->compute_units));
             } else {
+                ctx->set_tiles(g.r, ctx->wave_lanes((long long)pixels, true, spp > 1 || !ctx->shade_no_bounce), ctx->tile_w);
                 HIP_CHECK(ngx::launch_rgb(g, s, ctx->persistent ? ctx->compute_units : 0));
             }
             ctx->last_rgb_passes = two_pass ? 2 : 1;
@@ -1025,6 +1048,7 @@ ngx_status ngx_cast_rays_batch(ngx_ctx *ctx, const float *origins, const float *
         a.normal = ctx->d_hit_normal;
         a.object_id = ctx->d_hit_id;
         a.walk = ctx->walk_rays();
+        a.lanes = ctx->wave_lanes(count, true, false);
         a.blocks = ctx->ray_blocks;
         const bool timed = !ctx->capturing(s);
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev0, s));
@@ -1058,9 +1082,13 @@ void pose_backward_depth(ngx_ctx *ctx, const float *body_poses, const float *cam
                                   " bodies per world; the binding has " + std::to_string(ctx->bodies));
     require(body_poses && cams12 && depth && grad_depth && grad_out, "device arrays must not be null");
     require(fov > 0.0f && fov < 3.14159265f, "fov must be between 0 and pi radians, got " + std::to_string(fov));
-    // enough workgroups to fill the GPU: each view's tiles are split over `parts` workgroups of 4 waves
-    const int tiles = ((ctx->width + 7) / 8) * ((ctx->height + 7) / 8);
-    const int parts = std::max(1, std::min(16, tiles / 8));
+    // enough workgroups to fill the GPU: each view's tiles are split over `parts` workgroups of 4 waves; where there are
+    // few views, over as many as there are tiles for, if their partial sums fit
+    ngx::RenderArgs grid = ctx->render_args(cams12, fov);
+    ctx->set_tiles(grid, ctx->wave_lanes((long long)ctx->views * ctx->width * ctx->height, true, false), 8);
+    const int few = std::max(1, std::min(16, ((ctx->width + 7) / 8) * ((ctx->height + 7) / 8) / 8));
+    int parts = std::max(few, std::min((grid.tiles_per_view + 3) / 4, 8 * ctx->compute_units / ctx->views));
+    if (no_alloc && (size_t)ctx->views * parts * ctx->bodies * 7 > ngx::NOALLOC_SCRATCH_FLOATS) parts = few;
     const size_t need = (size_t)ctx->views * parts * ctx->bodies * 7;
     if (no_alloc)
         require(need <= ngx::NOALLOC_SCRATCH_FLOATS,
@@ -1094,6 +1122,10 @@ void pose_backward_depth(ngx_ctx *ctx, const float *body_poses, const float *cam
     a.body_of_instance = ctx->d_body_of_instance;
     a.local_rot_scale = ctx->d_local_rot_scale;
     a.body_poses = body_poses;
+    a.tile_w_log2 = grid.tile_w_log2;
+    a.tile_h = grid.tile_h;
+    a.tiles_x = grid.tiles_x;
+    a.tiles = grid.tiles_per_view;
     a.parts = parts;
     a.partial = partial;
     a.walk = ctx->walk();
@@ -1136,7 +1168,11 @@ ngx_status ngx_pose_backward_range(ngx_ctx *ctx, const float *body_poses, const 
         ctx->set_device();
         const hipStream_t s = static_cast<hipStream_t>(stream);
         const int chunks = std::max(1, std::min(64, rays_per_world / 4096));
-        const size_t need = (size_t)ctx->worlds * chunks * ctx->bodies * 7;
+        // a chunk's rays are taken in groups of `lanes` from its first on; few chunks are split over more workgroups
+        const int lanes = ctx->wave_lanes((long long)rays_per_world * ctx->worlds, true, false);
+        const int groups = ((rays_per_world + chunks - 1) / chunks + lanes - 1) / lanes;
+        const int split = std::max(1, std::min((groups + 3) / 4, (int)(8ll * ctx->compute_units / ((long long)ctx->worlds * chunks))));
+        const size_t need = (size_t)ctx->worlds * chunks * split * ctx->bodies * 7;
         if (need > ctx->partial_cap) {
             HIP_CHECK(hipStreamSynchronize(s));
             device_alloc(ctx->d_partial, need);
@@ -1149,6 +1185,8 @@ ngx_status ngx_pose_backward_range(ngx_ctx *ctx, const float *body_poses, const 
         a.dirs = directions;
         a.rays_per_world = rays_per_world;
         a.chunks = chunks;
+        a.split = split;
+        a.lanes = lanes;
         a.walk = ctx->walk_rays();
         a.max_distance = max_distance;
         a.distance = distance;
@@ -1164,7 +1202,7 @@ ngx_status ngx_pose_backward_range(ngx_ctx *ctx, const float *body_poses, const 
         HIP_CHECK(ngx::launch_range_backward(a, s));
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev1, s));
         ctx->timed = timed;
-        ngx::PoseGradFinishArgs f{ctx->worlds, ctx->bodies, chunks, ctx->d_partial, body_poses, grad_out};
+        ngx::PoseGradFinishArgs f{ctx->worlds, ctx->bodies, chunks * split, ctx->d_partial, body_poses, grad_out};
         HIP_CHECK(ngx::launch_pose_grad_finish(f, s));
         ctx->last_stream = s;
     });

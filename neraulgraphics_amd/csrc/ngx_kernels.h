@@ -98,14 +98,28 @@ constexpr int SHARE_STACK = 128;
 // indices stay below 2^25; a tree over n triangles has fewer than 2n nodes, so at most 2^24 triangles over all meshes.
 constexpr long long MAX_TRIANGLES = 1ll << 24;
 
+// Division of n < 2^31 by a divisor known on the host, as a multiplication: n / d = n * mul >> shift, with shift 31 more
+// than d's bits and mul = 2^shift / d rounded up (the rounding is below one part in 2^31, so it never shows).
+struct FastDivide {
+    uint32_t mul, shift;
+};
+inline FastDivide fast_divide_by(const int d) {
+    FastDivide f{0, 31};
+    while ((1ll << (f.shift - 31)) < d) ++f.shift;
+    f.mul = (uint32_t)(((1ull << f.shift) + (uint64_t)d - 1) / (uint64_t)d);
+    return f;
+}
+
 struct RenderArgs {
     TraceScene s;
     const float *cams;         // [views][12]
     float fov_scale;           // tanf(fov / 2), computed on the host as the reference's CPU backend does
     float aspect;              // width / height
     int width, height, cameras_per_world, views;
-    int tile_w, tile_h, tiles_x, tiles_per_view;
+    // a wavefront's tile: tile_w (a power of two) x tile_h pixels, at most 64; tiles are numbered view-major
+    int tile_w, tile_w_log2, tile_h, tiles_x, tiles_per_view;
     long long total_tiles;
+    FastDivide by_tiles_per_view, by_tiles_x, by_cameras;  // for tile numbers below 2^31
     float *depth;              // [views][H][W] or null
     float *normal;             // [views][H][W][3] or null
     int32_t *object_id;        // [views][H][W] or null
@@ -159,6 +173,7 @@ struct RayArgs {
     int walk;
     const int *order;          // null, or per world the order to trace its rays in (indices within the world)
     int xcd_remap;             // 1: each XCD takes a contiguous range of the waves
+    int lanes;                 // rays a wavefront takes: 64, or fewer where there are few
     int blocks;                // the kernel variant (0: the default)
 };
 
@@ -174,6 +189,7 @@ struct DepthBackwardArgs {
     const int *body_of_instance;     // [P]
     const float *local_rot_scale;    // [P][12]: Rl diag(s) | pl, the instance in its body's frame
     const float *body_poses;   // [worlds][bodies][7], the poses the tree was built from
+    int tile_w_log2, tile_h, tiles_x, tiles;  // a view's tiles, a wavefront each (as RenderArgs)
     int parts;                 // workgroups per view, each taking every parts-th group of tiles
     float *partial;            // [views][parts][bodies][7]
     int walk;                  // the re-trace's walk, as the forward's
@@ -184,7 +200,9 @@ struct RangeBackwardArgs {
     TraceScene s;
     const float *origins, *dirs;
     int rays_per_world;
-    int chunks;                // per world
+    int chunks;                // per world: equal runs of its rays
+    int split;                 // workgroups per chunk, each taking every split-th group of rays
+    int lanes;                 // rays a wavefront takes
     float max_distance;
     const float *distance;     // the forward's distances
     const float *grad_distance;
@@ -193,7 +211,7 @@ struct RangeBackwardArgs {
     const float *local_rot_scale;
     const float *body_poses;
     int worlds;
-    float *partial;            // [worlds][chunks][bodies][7]
+    float *partial;            // [worlds][chunks][split][bodies][7]
     int walk;
 };
 

@@ -1041,33 +1041,56 @@ __device__ __forceinline__ long long wave_tile(const int xcd_remap, const long l
 // LDS of the packet walk's triangle batches: one PairLds per wavefront of a 256-thread workgroup.
 #define NGX_PAIR_LDS(name) __shared__ PairLds name##_all[4]; PairLds *name = WALK != WALK_LANES ? &name##_all[threadIdx.x >> 6] : nullptr
 
+// A lane's pixel in its wavefront's tile of one view. Args: RenderArgs, or the same in the kernel arguments' segment.
+struct TilePixel {
+    int view, x, y, world;
+    bool valid;
+    size_t index;  // into [views][H][W]
+};
+template <class Divide>
+__device__ __forceinline__ int fast_divide(const int n, const Divide &by) { return (int)(((uint64_t)(uint32_t)n * by.mul) >> by.shift); }
+template <class Args>
+__device__ __forceinline__ TilePixel tile_pixel(const Args &A, const long long tile) {
+    const int lane = lane_id();
+    TilePixel p;
+    int t, ty;
+    if (A.total_tiles <= INT32_MAX) {
+        p.view = fast_divide((int)tile, A.by_tiles_per_view);
+        t = (int)tile - p.view * A.tiles_per_view;
+        ty = fast_divide(t, A.by_tiles_x);
+        p.world = fast_divide(p.view, A.by_cameras);
+    } else {
+        p.view = (int)(tile / A.tiles_per_view);
+        t = (int)(tile - (long long)p.view * A.tiles_per_view);
+        ty = t / A.tiles_x;
+        p.world = p.view / A.cameras_per_world;
+    }
+    p.x = (t - ty * A.tiles_x) * A.tile_w + (lane & (A.tile_w - 1));
+    p.y = ty * A.tile_h + (lane >> A.tile_w_log2);
+    p.valid = lane < A.tile_w * A.tile_h && p.x < A.width && p.y < A.height;
+    p.index = ((size_t)p.view * A.height + p.y) * A.width + p.x;
+    return p;
+}
+
 // One 64-pixel tile of one view: camera ray per lane, closest hit, depth / normal / object ID.
 template <int WALK>
 __device__ __forceinline__ void render_tile(PairLds *L, const long long tile) {
-    const int lane = lane_id();
     float3 d;
     Cam cam;
-    int view, x, y, world;
-    bool valid;
+    TilePixel p;
     {
         const auto &A = kernel_args<RenderArgs>();
-        view = (int)(tile / A.tiles_per_view);
-        const int t = (int)(tile % A.tiles_per_view);
-        const int tx = t % A.tiles_x, ty = t / A.tiles_x;
-        x = tx * A.tile_w + lane % A.tile_w;
-        y = ty * A.tile_h + lane / A.tile_w;
-        valid = x < A.width && y < A.height;
-        world = view / A.cameras_per_world;
-        cam = load_camera(A.cams + 12 * (size_t)view);
-        d = pixel_ray(cam, A.fov_scale, A.aspect, x, y, A.width, A.height);
+        p = tile_pixel(A, tile);
+        cam = load_camera(A.cams + 12 * (size_t)p.view);
+        d = pixel_ray(cam, A.fov_scale, A.aspect, p.x, p.y, A.width, A.height);
     }
     float best;
     LaneHit h;
     CameraRays stats;
-    const int kind = scene_hit<WALK>(Scene(), L, world, cam.pos, d, ballot(valid), best, h, stats);
-    if (!valid) return;
+    const int kind = scene_hit<WALK>(Scene(), L, p.world, cam.pos, d, ballot(p.valid), best, h, stats);
+    if (!p.valid) return;
     const auto &A = kernel_args<RenderArgs>();
-    const size_t idx = ((size_t)view * A.height + y) * A.width + x;
+    const size_t idx = p.index;
     const bool found = kind != OBJECT_NONE;
     float *const depth = in_global(A.depth), *const normals = in_global(A.normal);
     int32_t *const object_id = in_global(A.object_id);
@@ -1158,15 +1181,11 @@ __global__ __launch_bounds__(256) void render_stats_kernel(const RenderArgs A, i
     const long long tile = wave_tile(A.xcd_remap, A.total_tiles);
     if (tile >= A.total_tiles) return;
     const int lane = lane_id();
-    const int view = (int)(tile / A.tiles_per_view);
-    const int t = (int)(tile % A.tiles_per_view);
-    const int tx = t % A.tiles_x, ty = t / A.tiles_x;
-    const int x = tx * A.tile_w + lane % A.tile_w;
-    const int y = ty * A.tile_h + lane / A.tile_w;
-    const bool valid = x < A.width && y < A.height;
-    const int world = view / A.cameras_per_world;
-    const Cam cam = load_camera(A.cams + 12 * (size_t)view);
-    const float3 d = pixel_ray(cam, A.fov_scale, A.aspect, x, y, A.width, A.height);
+    const TilePixel p = tile_pixel(A, tile);
+    const bool valid = p.valid;
+    const int world = p.world;
+    const Cam cam = load_camera(A.cams + 12 * (size_t)p.view);
+    const float3 d = pixel_ray(cam, A.fov_scale, A.aspect, p.x, p.y, A.width, A.height);
     float best;
     LaneHit h;
     WaveStats stats;
@@ -1300,24 +1319,6 @@ __device__ __forceinline__ float srgb_channel(const float v) {
     return x <= 0.0031308f ? 12.92f * x : 1.055f * exp2f(__log2f(x) * (1.0f / 2.4f)) - 0.055f;
 }
 
-// A wavefront's pixels: an 8x8 (or tile_w x 64 / tile_w) tile of one view.
-struct TilePixel {
-    int view, x, y, world;
-    bool valid;
-    size_t index;  // into [views][H][W]
-};
-__device__ __forceinline__ TilePixel tile_pixel(const RenderArgs &A, const long long tile) {
-    const int lane = lane_id();
-    TilePixel p;
-    p.view = (int)(tile / A.tiles_per_view);
-    const int tt = (int)(tile % A.tiles_per_view);
-    p.x = (tt % A.tiles_x) * A.tile_w + lane % A.tile_w;
-    p.y = (tt / A.tiles_x) * A.tile_h + lane / A.tile_w;
-    p.valid = p.x < A.width && p.y < A.height;
-    p.world = p.view / A.cameras_per_world;
-    p.index = ((size_t)p.view * A.height + p.y) * A.width + p.x;
-    return p;
-}
 // The pixel's random stream, seeded by the pixel and the frame (geom_dev.h:122-126).
 __device__ __forceinline__ uint32_t pixel_stream(const RenderArgs &A, const TilePixel &p, const int frame) {
     return pcg_hash((uint32_t)(p.y * A.width + p.x) ^ pcg_hash((uint32_t)frame + 1u));
@@ -1666,10 +1667,10 @@ __device__ __forceinline__ void store_ray(const long long slot, const int world,
 template <int WALK, int BLOCKS>
 __global__ __launch_bounds__(256, BLOCKS) void ray_kernel(const RayArgs A) {
     NGX_PAIR_LDS(L);
-    const long long base = wave_tile(A.xcd_remap, 0) * 64;
+    const long long base = wave_tile(A.xcd_remap, 0) * A.lanes;
     if (base >= A.count) return;
     const long long slot = base + lane_id();
-    const bool valid = slot < A.count;
+    const bool valid = lane_id() < A.lanes && slot < A.count;
     const int world = valid ? (int)(slot / A.rays_per_world) : -1;
     float3 o = mk3(0.0f, 0.0f, 0.0f), d = mk3(0.0f, 0.0f, 1.0f);
     bool ok = false;
@@ -1783,10 +1784,10 @@ __global__ __launch_bounds__(64 * BWD_WAVES, BLOCKS) void depth_backward_kernel(
     for (int i = lane; i < B * 7; i += 64) acc[i] = 0.0f;
     const int world = view / A.cameras_per_world;
     const Cam cam = load_camera(A.cams + 12 * (size_t)view);
-    const int tiles_x = (A.width + 7) / 8, tiles_y = (A.height + 7) / 8;
-    for (int t = part * BWD_WAVES + wave; t < tiles_x * tiles_y; t += A.parts * BWD_WAVES) {
-        const int x = (t % tiles_x) * 8 + (lane & 7), y = (t / tiles_x) * 8 + (lane >> 3);
-        const bool valid = x < A.width && y < A.height;
+    for (int t = part * BWD_WAVES + wave; t < A.tiles; t += A.parts * BWD_WAVES) {
+        const int ty = t / A.tiles_x, row = lane >> A.tile_w_log2;
+        const int x = ((t - ty * A.tiles_x) << A.tile_w_log2) + (lane & ((1 << A.tile_w_log2) - 1)), y = ty * A.tile_h + row;
+        const bool valid = row < A.tile_h && x < A.width && y < A.height;
         const size_t idx = ((size_t)view * A.height + (valid ? y : 0)) * A.width + (valid ? x : 0);
         const float3 d = pixel_ray(cam, A.fov_scale, A.aspect, x, y, A.width, A.height);
         const float depth = valid ? A.depth[idx] : 0.0f;
@@ -1818,7 +1819,8 @@ template <int WALK>
 __global__ __launch_bounds__(64 * BWD_WAVES) void range_backward_kernel(const RangeBackwardArgs A) {
     extern __shared__ float acc_all[];
     NGX_PAIR_LDS(L);
-    const int world = blockIdx.x / A.chunks, chunk = blockIdx.x % A.chunks;
+    const int piece = blockIdx.x / A.split, part = blockIdx.x % A.split;
+    const int world = piece / A.chunks, chunk = piece % A.chunks;
     const int wave = uniform(threadIdx.x >> 6), lane = lane_id();
     const int B = A.bodies_per_world;
     float *acc = acc_all + (size_t)wave * B * 7;
@@ -1826,9 +1828,9 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void range_backward_kernel(const Ra
     const int R = A.rays_per_world;
     const int per = (R + A.chunks - 1) / A.chunks;
     const int r0 = chunk * per, r1 = min(R, r0 + per);
-    for (int r = r0 + wave * 64; r < r1; r += 64 * BWD_WAVES) {
+    for (int r = r0 + (part * BWD_WAVES + wave) * A.lanes; r < r1; r += A.split * BWD_WAVES * A.lanes) {
         const int ri = r + lane;
-        const bool valid = ri < r1;
+        const bool valid = lane < A.lanes && ri < r1;
         const size_t i = (size_t)world * R + (valid ? ri : r0);
         float3 o = mk3(A.origins[3 * i], A.origins[3 * i + 1], A.origins[3 * i + 2]);
         float3 d = mk3(A.dirs[3 * i], A.dirs[3 * i + 1], A.dirs[3 * i + 2]);
@@ -1854,21 +1856,27 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void range_backward_kernel(const Ra
     for (int i = threadIdx.x; i < B * 7; i += blockDim.x) {
         float s = 0.0f;
         for (int wv = 0; wv < BWD_WAVES; ++wv) s += acc_all[(size_t)wv * B * 7 + i];
-        A.partial[((size_t)world * A.chunks + chunk) * B * 7 + i] = s;
+        A.partial[(size_t)blockIdx.x * B * 7 + i] = s;
     }
 }
 
-// Sums the parts of each world in order, then projects the unit-quaternion gradient onto the raw
-// quaternion: d unit / d q = (I - u u^T) / |q|.
-__global__ void pose_grad_finish_kernel(const PoseGradFinishArgs A) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= A.worlds * A.bodies_per_world) return;
-    const int w = i / A.bodies_per_world, b = i % A.bodies_per_world;
+// Sums the parts of each body, then projects the unit-quaternion gradient onto the raw quaternion: d unit / d q =
+// (I - u u^T) / |q|. Eight lanes a body, each taking every eighth part in order, their sums added pairwise: a fixed order.
+constexpr int FINISH_LANES = 8;
+__global__ __launch_bounds__(256) void pose_grad_finish_kernel(const PoseGradFinishArgs A) {
+    const int bodies = A.worlds * A.bodies_per_world;
+    const int i = (blockIdx.x * blockDim.x + threadIdx.x) / FINISH_LANES, part = threadIdx.x % FINISH_LANES;
     float g[7] = {0, 0, 0, 0, 0, 0, 0};
-    for (int p = 0; p < A.parts; ++p) {
-        const float *src = A.partial + (((size_t)w * A.parts + p) * A.bodies_per_world + b) * 7;
-        for (int k = 0; k < 7; ++k) g[k] += src[k];
+    if (i < bodies) {
+        const int w = i / A.bodies_per_world, b = i % A.bodies_per_world;
+        for (int p = part; p < A.parts; p += FINISH_LANES) {
+            const float *src = A.partial + (((size_t)w * A.parts + p) * A.bodies_per_world + b) * 7;
+            for (int k = 0; k < 7; ++k) g[k] += src[k];
+        }
     }
+    for (int o = 1; o < FINISH_LANES; o <<= 1)
+        for (int k = 0; k < 7; ++k) g[k] += __shfl_xor(g[k], o, 64);
+    if (i >= bodies || part != 0) return;
     const float *bp = A.body_poses + 7 * (size_t)i;
     const float q[4] = {bp[3], bp[4], bp[5], bp[6]};
     const float qn = sqrtf(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
@@ -2043,7 +2051,8 @@ hipError_t launch_rgb_two_pass(const RgbArgs &a, const int hit_blocks, hipStream
 
 hipError_t launch_rays(const RayArgs &a, hipStream_t stream) {
     if (a.count <= 0) return hipSuccess;
-    const long long waves = (a.count + 63) / 64;
+    if (a.lanes < 1 || a.lanes > 64) return hipErrorInvalidValue;
+    const long long waves = (a.count + a.lanes - 1) / a.lanes;
     const long long blocks = (waves + 3) / 4;
 #define NGX_LAUNCH(W, B) ray_kernel<W, B><<<(unsigned)blocks, 256, 0, stream>>>(a)
     if (a.walk == WALK_SHARED) {
@@ -2071,9 +2080,10 @@ hipError_t launch_depth_backward(const DepthBackwardArgs &a, hipStream_t stream)
 
 hipError_t launch_range_backward(const RangeBackwardArgs &a, hipStream_t stream) {
     if (a.worlds <= 0 || a.chunks <= 0) return hipSuccess;
+    if (a.split < 1 || a.lanes < 1 || a.lanes > 64) return hipErrorInvalidValue;
     if (a.bodies_per_world <= 0 || a.bodies_per_world > BACKWARD_MAX_BODIES) return hipErrorInvalidValue;
     const size_t lds = sizeof(float) * BWD_WAVES * 7 * (size_t)a.bodies_per_world;
-#define NGX_LAUNCH(W) range_backward_kernel<W><<<a.worlds * a.chunks, 64 * BWD_WAVES, lds, stream>>>(a)
+#define NGX_LAUNCH(W) range_backward_kernel<W><<<a.worlds * a.chunks * a.split, 64 * BWD_WAVES, lds, stream>>>(a)
     switch (a.walk) {
     case WALK_LANES: NGX_LAUNCH(WALK_LANES); break;
     case WALK_HYBRID: NGX_LAUNCH(WALK_HYBRID); break;
@@ -2087,7 +2097,8 @@ hipError_t launch_range_backward(const RangeBackwardArgs &a, hipStream_t stream)
 hipError_t launch_pose_grad_finish(const PoseGradFinishArgs &a, hipStream_t stream) {
     const int n = a.worlds * a.bodies_per_world;
     if (n <= 0) return hipSuccess;
-    pose_grad_finish_kernel<<<(n + 255) / 256, 256, 0, stream>>>(a);
+    if (n > INT32_MAX / FINISH_LANES - 256) return hipErrorInvalidValue;
+    pose_grad_finish_kernel<<<(n * FINISH_LANES + 255) / 256, 256, 0, stream>>>(a);
     return hipGetLastError();
 }
 

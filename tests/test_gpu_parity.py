@@ -1008,3 +1008,40 @@ def test_rgb_known_answers_on_the_device(gpu, oracle):
     env2 = ng.Environment(color_up=(0.3, 0.6, 0.1), color_down=(0.3, 0.6, 0.1))
     m = gpu_rgb(scene(floor=mirror, cam=down, env=env2), floor=mirror, env=env2)
     assert np.all(m.reshape(-1, 3) == srgb_byte(np.array((0.3, 0.6, 0.1), np.float32)))
+
+
+@pytest.mark.parametrize("worlds", [1, 7, 9, 33, 97, 401])
+def test_small_launches_see_what_full_wavefronts_see(gpu, worlds):
+    """Launches of few wavefronts give each fewer rays (4 to 32 lanes of 64, by how many there are) and split the
+    backwards over more workgroups; the worlds they draw look as they do in a batch large enough for full wavefronts."""
+    import torch
+    full = workloads.make("posed_bodies", worlds=1600)
+    _say(f"part wavefronts: {worlds} worlds against the same of 1600")
+    rng = np.random.default_rng(5)
+    dirs = rng.normal(size=(1600, 77, 3)).astype(np.float32) * np.float32([0.4, 0.4, 1.0]) - np.float32([0, 0, 2])
+    origins = np.repeat(full["cameras"].reshape(-1, 3, 4)[:, None, :, 3], 77, axis=1)
+    seeds = rng.normal(size=(1600, 64, 64)).astype(np.float32), rng.normal(size=(1600, 77)).astype(np.float32)
+
+    def run(n):
+        cfg = dict(full, worlds=n)
+        for k in ("cameras", "body_poses"):
+            cfg[k] = full[k][:n]
+        r = workloads.make_renderer(cfg)
+        up = lambda a: torch.from_numpy(np.ascontiguousarray(a[:n])).cuda()  # noqa: E731
+        poses, cams, o, d = up(full["body_poses"]), up(full["cameras"]), up(origins), up(dirs)
+        out = {k: v.clone() for k, v in r.render(cams, cfg["fov"], depth=True, object_ids=True, zero_copy=True).items()}
+        rgb = r.render(cams, cfg["fov"], 2, rgb=True, zero_copy=True)["rgb"].clone()
+        hits = {k: v.clone() for k, v in r.cast_rays(o, d, 50.0).items()}
+        gd = r.pose_backward_depth(poses, cams, cfg["fov"], out["depth"], up(seeds[0]))
+        gr = r.pose_backward_range(poses, o, d, 50.0, hits["distance"], up(seeds[1]))
+        return {k: v[:worlds].cpu().numpy() for k, v in dict(out, rgb=rgb, **{"ray_" + k: v for k, v in hits.items()}, gd=gd, gr=gr).items()}
+
+    small, large = run(worlds), run(1600)
+    for k in ("object_ids", "ray_object_id"):
+        assert np.array_equal(small[k], large[k]), k
+    # the same triangle tests in another order: equal but for ties, of which a picture of these meshes has next to none
+    for k in ("depth", "ray_distance", "ray_normal", "rgb"):
+        assert np.mean(small[k] != large[k]) < 1e-5, k
+    # sums of up to 4096 pixels' terms, grouped otherwise: their rounding, against the largest gradient
+    for k in ("gd", "gr"):
+        assert np.abs(small[k] - large[k]).max() <= 1e-4 * np.abs(large[k]).max(), k
