@@ -122,7 +122,8 @@ struct ngx_ctx {
     uint8_t *d_root_at_end = nullptr;
     int *d_tmpl_mesh = nullptr;
     float *d_mesh_bounds = nullptr;
-    ngx::WideNode *d_blas_wide = nullptr;
+    ngx::WideNode *d_blas_wide = nullptr, *d_blas_octants = nullptr;
+    int octant_nodes = 0;
     int *d_blas_parent = nullptr;
     int *d_blas_wide_node = nullptr;
     // deforming meshes (ngx_set_mesh_vertices)
@@ -218,7 +219,7 @@ struct ngx_ctx {
                            d_geom_scale, d_geom_stage, d_depth, d_normal, d_cam_stage, d_ray_o, d_ray_d, d_hit_dist, d_hit_normal, d_partial, d_dbg_aabb,
                            d_dbg_world_bounds};
         for (float *p : floats) if (p) (void)hipFree(p);
-        void *others[] = {d_root_at_end, d_blas_wide, d_mesh_roots, d_tris, d_attrs, d_spheres, d_inst, d_nodes, d_wide,
+        void *others[] = {d_root_at_end, d_blas_wide, d_blas_octants, d_mesh_roots, d_tris, d_attrs, d_spheres, d_inst, d_nodes, d_wide,
                           d_id, d_hit_id, d_dbg_keys, d_dbg_sorted_keys, d_skip, d_ray_keys, d_ray_vals, d_inst_mat, d_sphere_mat,
                           d_lights, d_rgb, d_refit_entries, d_refit_treelets, d_rgb_hits, d_rgb_uv, big.key[0], big.key[1], big.val[0], big.val[1],
                           big.box, big.span, big.across, big.bounds, d_big_worlds, d_big_sort_tiles, d_big_node_tiles};
@@ -238,6 +239,8 @@ struct ngx_ctx {
         s.inst = d_inst;
         s.mesh_roots = d_mesh_roots;
         s.blas_wide = d_blas_wide;
+        s.blas_octants = d_blas_octants;
+        s.octant_nodes = octant_nodes;
         s.tris = d_tris;
         s.attrs = d_attrs;
         s.sphere_count = sphere_count;
@@ -518,6 +521,14 @@ ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out) {
             }
             upload(c.d_blas_wide, built.wide.data(), built.wide.size() ? built.wide.size() : 0);
             if (!c.d_blas_wide) device_alloc(c.d_blas_wide, 1);
+            if (!built.wide.empty() && 8 * sizeof(ngx::WideNode) * built.wide.size() <= ngx::OCTANT_COPIES_MAX_BYTES) {
+                c.octant_nodes = (int)built.wide.size();
+                std::vector<ngx::WideNode> copies;
+                copies.reserve(8 * built.wide.size());
+                for (int o = 0; o < 8; ++o)
+                    for (const ngx::WideNode &n : built.wide) copies.push_back(n.for_octant(o, o * c.octant_nodes));
+                upload(c.d_blas_octants, copies.data(), copies.size());
+            }
             upload(c.d_blas_parent, built.wide_parent.data(), built.wide_parent.size());
             if (!c.d_blas_parent) device_alloc(c.d_blas_parent, 1);
             upload(c.d_blas_wide_node, built.wide_node.data(), built.wide_node.size());
@@ -824,6 +835,8 @@ ngx_status ngx_set_mesh_vertices(ngx_ctx *ctx, const int32_t mesh, const float *
         a.tris = ctx->d_tris;
         a.skip = ctx->d_skip + 1;
         a.wide = ctx->d_blas_wide;
+        a.octants = ctx->d_blas_octants;
+        a.octant_nodes = ctx->octant_nodes;
         a.treelets = ctx->d_refit_treelets;
         a.entries = ctx->d_refit_entries;
         a.levels = ctx->d_refit_levels;

@@ -52,6 +52,21 @@ struct alignas(64) WideNode {
         plane[axis][1] = lo;
         plane[axis][3] = hi;
     }
+    // The node as rays of an octant read it, the octant's copies of a tree's nodes starting at `base`: per axis the near
+    // planes first, and references to the octant's copies.
+    __host__ __device__ WideNode for_octant(const int octant, const int base) const {
+        WideNode n = *this;
+        for (int ax = 0; ax < 3; ++ax)
+            if ((octant >> ax) & 1) {
+                n.plane[ax][0] = plane[ax][2];
+                n.plane[ax][1] = plane[ax][3];
+                n.plane[ax][2] = plane[ax][0];
+                n.plane[ax][3] = plane[ax][1];
+            }
+        if (left >= 0) n.left += base;
+        if (right >= 0) n.right += base;
+        return n;
+    }
 };
 static_assert(sizeof(WideNode) == 64, "64-byte wide node");
 
@@ -140,7 +155,9 @@ __device__ __forceinline__ float safe_nonzero(const float x) { return fabsf(x) <
 __device__ __forceinline__ float3 safe_inverse(const float3 d) {
     const float3 s = mk3(safe_nonzero(d.x), safe_nonzero(d.y), safe_nonzero(d.z));
     float3 r = mk3(rcp_in_range(s.x), rcp_in_range(s.y), rcp_in_range(s.z));
-    if (__builtin_expect(fmaxf(fmaxf(fabsf(s.x), fabsf(s.y)), fabsf(s.z)) >= 0x1p126f, 0)) r = mk3(1.0f / s.x, 1.0f / s.y, 1.0f / s.z);
+    const bool beyond = fmaxf(fmaxf(fabsf(s.x), fabsf(s.y)), fabsf(s.z)) >= 0x1p126f;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(beyond) != 0, 0))
+        r = beyond ? mk3(1.0f / s.x, 1.0f / s.y, 1.0f / s.z) : r;
     return r;
 }
 
@@ -179,6 +196,20 @@ __device__ __forceinline__ bool box_hit(const float lx, const float ly, const fl
     return tn <= tf;
 }
 
+// box_hit with each axis' near and far plane told apart beforehand by the sign of the ray's inverse direction (never
+// zero): near gives the smaller of the two products and far the larger, since rounding keeps order, so the decision and
+// tn are box_hit's.
+__device__ __forceinline__ bool box_hit_ordered(const float nx, const float ny, const float nz, const float fx, const float fy,
+                                                const float fz, const float3 o, const float3 inv_d, const float lim, float &tn) {
+    tn = fmaxf(fmaxf((nx - o.x) * inv_d.x, (ny - o.y) * inv_d.y), fmaxf((nz - o.z) * inv_d.z, 0.0f));
+    const float tf = min_quiet(fminf(fminf((fx - o.x) * inv_d.x, (fy - o.y) * inv_d.y), (fz - o.z) * inv_d.z), lim);
+    return tn <= tf;
+}
+// The octant of a ray by the signs of its inverse direction: bit k set where it is negative along axis k.
+__device__ __forceinline__ int ray_octant(const float3 inv_d) {
+    return (int)((__float_as_uint(inv_d.x) >> 31) | (__float_as_uint(inv_d.y) >> 31) << 1 | (__float_as_uint(inv_d.z) >> 31) << 2);
+}
+
 // Triangle j of the packed array (v0, e1, e2: 9 floats).
 __device__ __forceinline__ void load_tri(const float *tris, const size_t j, float3 &v0, float3 &e1, float3 &e2) {
     const float *p = tris + 9 * j;
@@ -189,13 +220,15 @@ __device__ __forceinline__ void load_tri(const float *tris, const size_t j, floa
 
 // Two-sided Moller-Trumbore (mesh_dev.h:80-99), triangle given as v0, e1, e2.
 // Every condition is worked out and the lot taken together: an early way out for some of a wave's lanes saves the others
-// nothing and costs a change of the execution mask. A lane that fails the first condition may hold any values after it.
+// nothing and costs a change of the execution mask. A lane that fails the first condition may hold any values after it, and a lane that is
+// not in use any throughout.
 __device__ __forceinline__ bool triangle_hit(const float3 v0, const float3 e1, const float3 e2, const float3 o, const float3 d,
-                                             const float tmax, float &t, float &bu, float &bv) {
+                                             const float tmax, float &t, float &bu, float &bv, const bool use = true) {
     const float3 p = cross3(d, e2);
     const float det = dot3(e1, p);
     float inv_det = rcp_in_range(det);
-    if (__builtin_expect(!(fabsf(det) < 0x1p126f), 0)) inv_det = 1.0f / det;
+    const bool beyond = use & !(fabsf(det) < 0x1p126f);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(beyond) != 0, 0)) inv_det = beyond ? 1.0f / det : inv_det;
     const float3 s = sub3(o, v0);
     const float u = dot3(s, p) * inv_det;
     const float3 q = cross3(s, e1);
@@ -203,7 +236,7 @@ __device__ __forceinline__ bool triangle_hit(const float3 v0, const float3 e1, c
     t = dot3(e2, q) * inv_det;
     bu = u;
     bv = v;
-    return !(fabsf(det) < 1e-14f) & !(u < 0.0f) & !(u > 1.0f) & !(v < 0.0f) & !(u + v > 1.0f) & (t > 0.0f) & (t < tmax);
+    return use & !(fabsf(det) < 1e-14f) & !(u < 0.0f) & !(u > 1.0f) & !(v < 0.0f) & !(u + v > 1.0f) & (t > 0.0f) & (t < tmax);
 }
 
 // ------------------------------------------------------------------ wave primitives --

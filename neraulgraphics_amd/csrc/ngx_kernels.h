@@ -72,6 +72,8 @@ struct TraceScene {
     const InstanceRec *inst;
     const MeshRoot *mesh_roots;
     const WideNode *blas_wide;
+    const WideNode *blas_octants; // the bottom level once per ray octant, [8][octant_nodes], or null
+    int octant_nodes;          // bottom-level wide nodes when there are octant copies, else 0
     const float *tris;         // 9 floats per triangle: v0, e1, e2 (packed: the walks fetch 36 bytes a triangle)
     const float4 *attrs;       // 4 per triangle (normals + flags) or null
     int sphere_count;
@@ -87,6 +89,12 @@ struct TraceScene {
     int share_cap;             // entries of the LDS stack the two-child shared walk gives subtrees to, 1..128 (128;
                                // lower only to test the lanes' own stacks, which take the rest)
 };
+
+// The bottom level is copied once per ray octant, near planes first, while the copies take at most this many bytes: a
+// two-child step then needs no minimum and maximum per pair of planes, 12 of its 58 vector instructions (4096 worlds
+// 128x128: 7.01 -> 6.73 ms, 64x64: 1.081 -> 1.044 ms, three meshes of 2,332 triangles). Larger trees would lose more to
+// the caches than that saves: an XCD's L2 is 4 MB, and rays of all octants are under way at once.
+constexpr size_t OCTANT_COPIES_MAX_BYTES = (size_t)2 << 20;
 
 // The walks' depth limits: a wave-uniform stack of WALK_STACK entries per level for the packet walk, a 64-bit trail per
 // level for the per-lane walk.
@@ -288,6 +296,8 @@ struct MeshRefitArgs {
     float *tris;              // packed triangles, 9 floats each
     SkipNode *skip;           // every node's box is written here
     WideNode *wide;
+    WideNode *octants;        // the octant copies, octant_nodes each, or null
+    int octant_nodes;
     const RefitTreelet *treelets;
     const RefitEntry *entries;
     const int *levels;

@@ -68,6 +68,8 @@ __global__ __launch_bounds__(256) void refit_treelet_kernel(const MeshRefitArgs 
                     lo[ax] = fminf(child[0][ax], child[1][ax]);
                     hi[ax] = fmaxf(child[0][3 + ax], child[1][3 + ax]);
                 }
+                if (A.octants)
+                    for (int o = 0; o < 8; ++o) A.octants[(size_t)o * A.octant_nodes + e.wide] = w.for_octant(o, o * A.octant_nodes);
             }
             SkipNode &n = A.skip[e.node];
             for (int ax = 0; ax < 3; ++ax) {

@@ -13,11 +13,13 @@
 // (mesh_dev.h:98), so the result equals the per-ray walk's except where two surfaces meet the ray at the
 // same distance.
 //
-// What bounds these kernels is instruction issue, of vector, scalar and branch instructions together (the 4096-world
-// 128x128 render: 5.66 G vector, 3.36 G scalar and 0.83 G branch instructions; its time follows their sum), so the
-// walks are written for few instructions a visit: arguments read where they are used, wave-uniform stacks in vector
-// registers, a triangle test without early ways out, one range check for three reciprocals, selects where both sides
-// are cheap. Together 8.44 -> 7.69 ms there, 13.7 -> 13.2 ms for 67 M LiDAR rays.
+// What bounds these kernels is instruction issue, the scalar side of it first: a SIMD starts a scalar instruction or a
+// branch every 4.4 cycles and a vector one every 2.4 (add, multiply, move) to 4 (minimum, compare, select, fused), all
+// measured with 8 wavefronts, and the 4096-world 128x128 render issued 3.36 G scalar, 0.83 G branch and 5.66 G vector
+// instructions in 8.44 ms: the scalar unit was busy nearly throughout. So the walks are written for few scalar
+// instructions a visit: arguments read where they are used and the walk's pointers once, wave-uniform stacks in vector
+// registers, masked instructions without a branch around them (NGX_LIKELY), lanes that drop out by their limit rather
+// than by a mask, rare cases tested once for the wave. 8.44 -> 6.73 ms there, 13.7 -> 12.7 ms for 67 M LiDAR rays.
 #include <cstddef>
 #include <mutex>
 #include "ngx_kernels.h"
@@ -28,6 +30,11 @@ static __device__ __align__(256) float scratch[ngx::NOALLOC_SCRATCH_FLOATS];
 
 namespace ngx {
 namespace {
+
+// A condition some lane of the wave almost always meets: the compiler then leaves out the branch it would otherwise put
+// before the masked instructions, to skip them when no lane does.
+#define NGX_LIKELY(x) __builtin_expect_with_probability((x), 1, 0.9999)
+#define NGX_UNLIKELY(x) __builtin_expect_with_probability((x), 0, 0.9999)
 
 struct LaneHit {
     int inst;
@@ -52,7 +59,20 @@ template <class T>
 __device__ __forceinline__ T *in_global(T *p) { return (T *)(__attribute__((address_space(1))) T *)p; }
 
 // The scene of the running kernel, whose arguments begin with a TraceScene.
+// What every visit reads is held in registers for the walk.
 struct Scene {
+    const InstanceRec *inst_;
+    const MeshRoot *mesh_roots_;
+    const float *tris_;
+    __device__ __forceinline__ Scene() {
+        const auto &A = kernel_args<TraceScene>();
+        inst_ = in_global(A.inst);
+        mesh_roots_ = in_global(A.mesh_roots);
+        tris_ = in_global(A.tris);
+    }
+    __device__ __forceinline__ const InstanceRec *inst() const { return inst_; }
+    __device__ __forceinline__ const MeshRoot *mesh_roots() const { return mesh_roots_; }
+    __device__ __forceinline__ const float *tris() const { return tris_; }
 #define NGX_SCENE_POINTER(type, name) \
     __device__ __forceinline__ type *name() const { return in_global(kernel_args<TraceScene>().name); }
 #define NGX_SCENE_VALUE(type, name) \
@@ -62,10 +82,9 @@ struct Scene {
     NGX_SCENE_POINTER(const int, blas_parent)
     NGX_SCENE_POINTER(const int, blas_wide_node)
     NGX_SCENE_POINTER(const int, roots)
-    NGX_SCENE_POINTER(const InstanceRec, inst)
-    NGX_SCENE_POINTER(const MeshRoot, mesh_roots)
     NGX_SCENE_POINTER(const WideNode, blas_wide)
-    NGX_SCENE_POINTER(const float, tris)
+    NGX_SCENE_POINTER(const WideNode, blas_octants)
+    NGX_SCENE_VALUE(int, octant_nodes)
     NGX_SCENE_POINTER(const float4, attrs)
     NGX_SCENE_POINTER(const float4, spheres)
     NGX_SCENE_POINTER(const SkipNode, skip)
@@ -157,15 +176,15 @@ __device__ __forceinline__ Wide load_wide(const WideNode *nodes, const int index
 // order as the floats do). That is what testing the triangles one by one with a strict "closer than"
 // keeps (mesh_dev.h:98, :186-199). A ray's limit is not lowered until its batch is tested, so a few
 // more boxes may be entered; that costs time, not correctness.
-// 3,328 bytes a wavefront.
+// 4,608 bytes a wavefront.
 struct PairLds {
-    int pair[64];                  // ray lane | triangle << 6
+    int pair[128];                 // ray lane | triangle << 6; the upper half takes writes that count for nothing
     unsigned long long best[64];   // per ray lane: distance bits << 32 | pair number
     int4 hit[64];                  // per ray lane: instance (-1: none), triangle and barycentrics of its closest hit so far
     // the per-lane bottom-level walk's shared work: subtrees given away (ray lane | node << 6), and a ring of
     // leaves waiting for their triangle tests (first triangle; ray lane | count << 6)
     int share[128];
-    int2 leaf[128];
+    int2 leaf[256];
 };
 
 // v of the lane whose number is in bits 2 to 7 of four_times_lane.
@@ -193,25 +212,26 @@ __device__ __forceinline__ int write_lane(const int v, const int lane, const int
 // three instructions and waits for nothing.
 struct WaveStack {
     int ref, lo, hi;
-    int sp;
-    __device__ __forceinline__ WaveStack() : ref(0), lo(0), hi(0), sp(0) {}
+    int sp, deepest;
+    __device__ __forceinline__ WaveStack() : ref(0), lo(0), hi(0), sp(0), deepest(0) {}
     // Depth bounds keep sp below WALK_STACK (a top-level tree has fewer than 64 levels below a world's root, and the
-    // host refuses bottom-level trees deeper than 60). A tree that breaks them anyway loses the entry that does not
-    // fit, and the walk reports it through the scene's overflow flag, which the host turns into an error.
+    // host refuses bottom-level trees deeper than 60). A tree that breaks them anyway loses an entry, and the walk
+    // reports it at its end through the scene's overflow flag, which the host turns into an error.
     __device__ __forceinline__ void push(const int r, const uint64_t m) {
-        if (__builtin_expect(sp >= WALK_STACK, 0)) {
-            if (lane_id() == 0) *Scene().overflow() = 1;
-            return;
-        }
-        ref = write_lane(r, sp, ref);
-        lo = write_lane((int)(uint32_t)m, sp, lo);
-        hi = write_lane((int)(uint32_t)(m >> 32), sp, hi);
-        ++sp;
+        const int at = min(sp, WALK_STACK - 1);
+        ref = write_lane(r, at, ref);
+        lo = write_lane((int)(uint32_t)m, at, lo);
+        hi = write_lane((int)(uint32_t)(m >> 32), at, hi);
+        deepest = max(deepest, ++sp);
+        sp = min(sp, WALK_STACK);
     }
     __device__ __forceinline__ void pop(int &r, uint64_t &m) {
         --sp;
         r = __builtin_amdgcn_readlane(ref, sp);
         m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, sp) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, sp);
+    }
+    __device__ __forceinline__ void report() const {
+        if (NGX_UNLIKELY(deepest > WALK_STACK) && lane_id() == 0) *Scene().overflow() = 1;
     }
 };
 static_assert(WALK_STACK <= 64, "an entry a lane");
@@ -226,27 +246,26 @@ __device__ __forceinline__ void flush_pairs(const Scene S, PairLds *L, int &pair
     const int lane = lane_id();
     L->best[lane] = ((unsigned long long)__float_as_uint(tmax) << 32) | 0xffffffffull;
     wave_lds_order();
-    const bool act = lane < pairs;
     const int e = L->pair[lane];
-    const int r = e & 63;
+    const int r = e & 63, src = e << 2;
     float3 po = lo;
-    if (!Stats::kOneOrigin) po = mk3(__shfl(lo.x, r, 64), __shfl(lo.y, r, 64), __shfl(lo.z, r, 64));
-    const float3 pd = mk3(__shfl(ld.x, r, 64), __shfl(ld.y, r, 64), __shfl(ld.z, r, 64));
-    const float pt = __shfl(tmax, r, 64);
+    if (!Stats::kOneOrigin) po = mk3(lane_read(lo.x, src), lane_read(lo.y, src), lane_read(lo.z, src));
+    const float3 pd = mk3(lane_read(ld.x, src), lane_read(ld.y, src), lane_read(ld.z, src));
+    const float pt = lane_read(tmax, src);
+    float3 v0 = mk3(unknown_f(), unknown_f(), unknown_f()), e1 = mk3(unknown_f(), unknown_f(), unknown_f()),
+           e2 = mk3(unknown_f(), unknown_f(), unknown_f());
+    const bool act = lane < pairs;
     pairs = 0;
-    float t = 0.0f, bu = 0.0f, bv = 0.0f;
-    bool found = false;
-    if (act) {
-        float3 v0, e1, e2;
-        load_tri(S.tris(), (uint32_t)e >> 6, v0, e1, e2);
-        found = triangle_hit(v0, e1, e2, po, pd, pt, t, bu, bv);
-    }
+    if (NGX_LIKELY(act)) load_tri(S.tris(), (uint32_t)e >> 6, v0, e1, e2);
+    float t, bu, bv;
+    const bool found = triangle_hit(v0, e1, e2, po, pd, pt, t, bu, bv, act);
     if (ballot(found) == 0) return;
     const unsigned long long mine = ((unsigned long long)__float_as_uint(t) << 32) | (unsigned)lane;
-    if (found) atomicMin(&L->best[r], mine);
+    if (NGX_LIKELY(found)) atomicMin(&L->best[r], mine);
     wave_lds_order();
     // the pair that won writes its ray's hit; it is kept in LDS, not registers, until the walk is over
-    if (found && L->best[r] == mine) L->hit[r] = make_int4(inst, (int)((uint32_t)e >> 6), __float_as_int(bu), __float_as_int(bv));
+    if (NGX_LIKELY(found && L->best[r] == mine))
+        L->hit[r] = make_int4(inst, (int)((uint32_t)e >> 6), __float_as_int(bu), __float_as_int(bv));
     const unsigned long long b = L->best[lane];
     tmax = !Stats::kAnyHit ? __uint_as_float((unsigned)(b >> 32)) : (unsigned)b != 0xffffffffu ? -1.0f : tmax;
     wave_lds_order();
@@ -288,7 +307,7 @@ __device__ __forceinline__ void add_leaf(const Scene S, PairLds *L, int &pairs, 
 // pairs wait, and at the end; after each batch every walking lane re-reads its ray's closest distance. Every
 // node a ray enters is walked by exactly one lane, so each ray's closest hit is its own. (The RGB kernel walks so;
 // the other kernels use the two-child walk further below, which shares its work the same way.)
-constexpr int SHARE_CAP = SHARE_STACK, LEAF_RING = 128;
+constexpr int SHARE_CAP = SHARE_STACK, LEAF_RING = 256;
 // Queued leaves that trigger a batch of triangle tests (at most 64 pairs a batch; fewer leaves wait for more).
 #ifndef NGX_LEAF_BATCH
 #define NGX_LEAF_BATCH 64
@@ -305,37 +324,31 @@ __device__ __forceinline__ void test_queued_leaves(const Scene S, PairLds *L, in
     const int lane = lane_id();
     while (count > 0) {
         wave_lds_order();
-        const int avail = min(count, 64);
-        const bool mine = lane < avail;
-        const int slot = (head + lane) & (LEAF_RING - 1);
-        const int2 queued_leaf = L->leaf[slot];
-        const int rc = mine ? queued_leaf.y : 0;
-        const int first = queued_leaf.x;
+        const int2 leaf = L->leaf[(head + lane) & (LEAF_RING - 1)];  // what is past the queued ones is masked out
+        const int rc = lane < count ? leaf.y : 0, first = leaf.x;
         const int c = rc >> 6;
-        const int c0 = __builtin_amdgcn_readlane(c, 0);
-        if (c0 > 64) {
+        const int incl = wave_prefix_sum(c);
+        const uint64_t take = ballot(lane < count && incl <= 64);
+        if (NGX_UNLIKELY(take == 0)) {
             // a leaf of more than 64 triangles (the tree's leaves hold 4, unless a mesh has many coincident
             // triangles): its next 64, the rest stays queued
             const int ray0 = __builtin_amdgcn_readlane(rc, 0) & 63, first0 = __builtin_amdgcn_readlane(first, 0);
+            const int c0 = __builtin_amdgcn_readlane(c, 0);
             wave_lds_order();
             L->pair[lane] = ray0 | ((first0 + lane) << 6);
-            if (lane == 0) {
-                L->leaf[head] = make_int2(first0 + 64, ray0 | ((c0 - 64) << 6));
-            }
+            if (lane == 0) L->leaf[head] = make_int2(first0 + 64, ray0 | ((c0 - 64) << 6));
             int pairs = 64;
             flush_pairs(S, L, pairs, g, lo, ld, tmax, stats);
             continue;
         }
-        const int incl = wave_prefix_sum(c);
-        const bool take = mine && incl <= 64;
-        const int taken = popc64(ballot(take));  // at least the first leaf, which holds 64 triangles at most
-        const int pairs_total = __builtin_amdgcn_readlane(incl, taken - 1);
-        if (!FORCE && pairs_total < 64 && count < 64) break;
-        if (take) {
-            const int ray = rc & 63;
-            for (int k = 0; k < c; ++k) L->pair[incl - c + k] = ray | ((first + k) << 6);
-        }
-        int pairs = pairs_total;
+        const int taken = popc64(take);
+        int pairs = __builtin_amdgcn_readlane(incl, taken - 1);
+        if (!FORCE && count < 64 && pairs < 64) break;
+        // each leaf's pairs from its place on; what a lane has no pair for goes to the upper half
+        const int at = in_mask(take) ? incl - c : 64, n = in_mask(take) ? c : 0, pair0 = (rc & 63) | (first << 6);
+        for (int k = 0; k < 4; ++k) L->pair[k < n ? at + k : 64 + lane] = pair0 + (k << 6);
+        if (NGX_UNLIKELY(ballot(n > 4) != 0))
+            for (int k = 4; k < n; ++k) L->pair[at + k] = pair0 + (k << 6);
         flush_pairs(S, L, pairs, g, lo, ld, tmax, stats);
         head = (head + taken) & (LEAF_RING - 1);
         count -= taken;
@@ -443,45 +456,51 @@ __device__ void walk_shared(const Scene S, PairLds *L, const int g, int top, con
 // takes the newest given subtree (with its ray's mesh-space data read from the ray's lane). A lane's own entries lie on
 // one path down a tree, one a level at most, and the host refuses bottom-level trees of WALK_STACK levels or more, so
 // WALK_STACK entries hold them. Leaves are queued and tested in batches as in the walk above.
-template <class Stats>
+// ORDERED: the nodes are the octant copies, an item's node in its ray's octant's, so near and far planes are known.
+template <bool ORDERED, class Stats>
 __device__ void walk_shared_two_child(const Scene S, PairLds *L, const int g, int top, const float3 lo,
                                       const float3 ld, const float3 inv_ld, float &tmax, Stats &stats) {
     int head = 0, queued = 0;
     // A lane's work as the stacks hold it, ray lane | node << 6 (so its upper bits are the node's byte offset), or
-    // negative: idle. Lane reads take the low bits of 4 x a lane number, so work << 2 reads the ray's lane.
+    // negative: idle. Lane reads take the low bits of 4 x a lane number, so work << 2 reads the ray's lane. An idle
+    // lane's limit is negative, so it enters no box.
     int work = -1;
     float3 wlo = lo, winv = inv_ld;
-    float wlim = box_limit(tmax);
+    float wlim = -1.0f;
     int own[WALK_STACK];
-    int own_n = 0;
-    const char *const nodes = reinterpret_cast<const char *>(S.blas_wide());
+    int own_n = 0, own_total = 0;  // the lane's own entries, and the wave's
+    const char *const nodes = reinterpret_cast<const char *>(ORDERED ? S.blas_octants() : S.blas_wide());
     const int share_cap = S.share_cap();
-    while (true) {
-        uint64_t busy = ballot(work >= 0);
-        const uint64_t resume = ~busy & ballot(own_n > 0);
-        if (~busy != 0 && (top | (int)(resume != 0)) != 0) {
-            const uint64_t takers = ~(busy | resume);
+    uint64_t busy = 0;
+    do {
+        if ((top | own_total) != 0 && ~busy != 0) {
+            uint64_t takers = ~busy;
+            if (NGX_UNLIKELY(own_total != 0)) {
+                const uint64_t resume = takers & ballot(own_n > 0);
+                if (in_mask(resume)) work = own[--own_n];
+                own_total -= popc64(resume);
+                takers &= ~resume;
+            }
             const int n = min(popc64(takers), top);
             const int rk = rank_in(takers);
             wave_lds_order();
-            if (in_mask(takers) && rk < n) work = L->share[top - 1 - rk];
-            if (in_mask(resume)) work = own[--own_n];
+            if (NGX_LIKELY(in_mask(takers) && rk < n)) work = L->share[top - 1 - rk];
             top -= n;
             const int src = work << 2;
             if (!Stats::kOneOrigin) wlo = mk3(lane_read(lo.x, src), lane_read(lo.y, src), lane_read(lo.z, src));
             winv = mk3(lane_read(inv_ld.x, src), lane_read(inv_ld.y, src), lane_read(inv_ld.z, src));
-            wlim = min_quiet(lane_read(tmax, src), BELOW_NO_HIT);
+            const float limit = min_quiet(lane_read(tmax, src), BELOW_NO_HIT);
+            wlim = work >= 0 ? limit : -1.0f;
             busy = ballot(work >= 0);
         }
-        if (busy == 0) break;
         stats.add(ST_BLAS_NODES, 1);
         stats.add(ST_BLAS_LANES, popc64(busy));
-        // idle lanes test whatever their registers hold, and their results are masked out
+        // idle lanes test whatever their registers hold
         float4 f0 = make_float4(unknown_f(), unknown_f(), unknown_f(), unknown_f());
         float4 f1 = make_float4(unknown_f(), unknown_f(), unknown_f(), unknown_f());
         float4 f2 = make_float4(unknown_f(), unknown_f(), unknown_f(), unknown_f());
         int4 f3 = make_int4(unknown_i(), unknown_i(), unknown_i(), unknown_i());
-        if (in_mask(busy)) {
+        if (NGX_LIKELY(in_mask(busy))) {
             // a 32-bit byte offset from the array's base (node indices stay below 2^25)
             const float4 *np = reinterpret_cast<const float4 *>(nodes + ((uint32_t)work & ~63u));
             f0 = np[0];
@@ -490,51 +509,48 @@ __device__ void walk_shared_two_child(const Scene S, PairLds *L, const int g, in
             f3 = *reinterpret_cast<const int4 *>(np + 3);
         }
         float dl, dr;
-        const uint64_t hl = busy & ballot(box_hit(f0.x, f1.x, f2.x, f0.z, f1.z, f2.z, wlo, winv, wlim, dl));
-        const uint64_t hr = busy & ballot(box_hit(f0.y, f1.y, f2.y, f0.w, f1.w, f2.w, wlo, winv, wlim, dr));
+        const uint64_t hl = ballot(ORDERED ? box_hit_ordered(f0.x, f1.x, f2.x, f0.z, f1.z, f2.z, wlo, winv, wlim, dl)
+                                           : box_hit(f0.x, f1.x, f2.x, f0.z, f1.z, f2.z, wlo, winv, wlim, dl));
+        const uint64_t hr = ballot(ORDERED ? box_hit_ordered(f0.y, f1.y, f2.y, f0.w, f1.w, f2.w, wlo, winv, wlim, dr)
+                                           : box_hit(f0.y, f1.y, f2.y, f0.w, f1.w, f2.w, wlo, winv, wlim, dr));
         const uint64_t lleaf = ballot(f3.x < 0), rleaf = ballot(f3.y < 0);
         const uint64_t ll = hl & lleaf, rl = hr & rleaf;    // leaves entered
         const uint64_t li = hl & ~lleaf, ri = hr & ~rleaf;  // interior children entered
+        const int ray = work & 63;
         if ((ll | rl) != 0) {
-            const int nl = popc64(ll), nr = popc64(rl);
-            // a step queues at most 128 leaves, so the ring holds them once what waits is tested
-            if (__builtin_expect(queued + nl + nr > LEAF_RING, 0)) {
-                test_queued_leaves<true>(S, L, head, queued, g, lo, ld, tmax, stats);
-                wlim = min_quiet(lane_read(tmax, work << 2), BELOW_NO_HIT);
-            }
-            const int ray = work & 63;
-            if (in_mask(ll)) L->leaf[(head + queued + rank_in(ll)) & (LEAF_RING - 1)] = make_int2(~f3.x, ray | (f3.z << 6));
-            if (in_mask(rl)) L->leaf[(head + queued + nl + rank_in(rl)) & (LEAF_RING - 1)] = make_int2(~f3.y, ray | (f3.w << 6));
+            // fewer than 64 wait and a step queues at most 128, so the ring holds them
+            const int tail = head + queued, nl = popc64(ll), nr = popc64(rl);
+            if (NGX_LIKELY(in_mask(ll))) L->leaf[(tail + rank_in(ll)) & (LEAF_RING - 1)] = make_int2(~f3.x, ray | (f3.z << 6));
+            if (NGX_LIKELY(in_mask(rl))) L->leaf[(tail + nl + rank_in(rl)) & (LEAF_RING - 1)] = make_int2(~f3.y, ray | (f3.w << 6));
             queued += nl + nr;
         }
         // on to the nearer of the interior children entered (the left one when they are as near)
         const uint64_t go_left = li & (~ri | ballot(dl <= dr));
         const uint64_t both = li & ri;
-        const int ray = work & 63;
         const int near = in_mask(go_left) ? f3.x : f3.y;
         if (both != 0) {
             const int far = ray | ((in_mask(go_left) ? f3.y : f3.x) << 6);
             // the lowest-ranked lanes fill the shared stack's room; the others keep their far child
             const int room = share_cap - top, rk = rank_in(both), n = popc64(both);
-            if (n <= room) {
-                if (in_mask(both)) L->share[top + rk] = far;
-                top += n;
-            } else {
-                const uint64_t given = both & ballot(rk < room);
-                if (in_mask(given)) L->share[top + rk] = far;
-                top += popc64(given);
-                if (in_mask(both & ~given)) {
-                    if (own_n < WALK_STACK) own[own_n++] = far;
-                    else *S.overflow() = 1;
-                }
+            const bool gives = rk < room;
+            if (NGX_LIKELY(in_mask(both) && gives)) L->share[top + rk] = far;
+            top += min(n, room);
+            if (NGX_UNLIKELY(n > room)) {
+                const bool keeps = in_mask(both) && !gives, fits = own_n < WALK_STACK;
+                if (keeps && fits) own[own_n++] = far;
+                if (keeps && !fits) *S.overflow() = 1;
+                own_total += popc64(ballot(keeps && fits));
             }
         }
-        work = in_mask(li | ri) ? ray | (near << 6) : -1;
+        busy = li | ri;
+        work = in_mask(busy) ? ray | (near << 6) : -1;
+        wlim = in_mask(busy) ? wlim : -1.0f;
         if (queued >= NGX_LEAF_BATCH) {
             test_queued_leaves<false>(S, L, head, queued, g, lo, ld, tmax, stats);
-            wlim = min_quiet(lane_read(tmax, work << 2), BELOW_NO_HIT);
+            const float limit = min_quiet(lane_read(tmax, work << 2), BELOW_NO_HIT);
+            wlim = in_mask(busy) ? limit : -1.0f;
         }
-    }
+    } while ((busy | (uint64_t)(uint32_t)(top | own_total)) != 0);
     test_queued_leaves<true>(S, L, head, queued, g, lo, ld, tmax, stats);
 }
 
@@ -543,7 +559,7 @@ __device__ void walk_shared_two_child(const Scene S, PairLds *L, const int g, in
 template <bool LANES, class Stats>
 __device__ __forceinline__ void walk_packet(const Scene S, PairLds *L, const int g, const int root_ref, const uint64_t root_mask,
                                             const float3 lo, const float3 ld, const float3 inv_d, float &tmax, LaneHit &h,
-                                            int &shared, Stats &stats) {
+                                            const int octant_base, int &shared, Stats &stats) {
     int pairs = 0;
     WaveStack st;
     const WideNode *const nodes = S.blas_wide();
@@ -588,7 +604,7 @@ __device__ __forceinline__ void walk_packet(const Scene S, PairLds *L, const int
             if (next_mask != 0 && next_ref >= 0) {
                 const int n = popc64(next_mask);
                 if (!LANES || !Stats::kHandoff || n > NGX_HANDOFF_LANES || shared + n > SHARE_CAP) break;
-                share_subtree(L, shared, next_mask, Stats::kTwoChild ? next_ref : S.blas_wide_node()[next_ref]);
+                share_subtree(L, shared, next_mask, Stats::kTwoChild ? octant_base + next_ref : S.blas_wide_node()[next_ref]);
             } else if (next_mask != 0) {
                 add_leaf(S, L, pairs, ~next_ref, next_count, next_mask, g, lo, ld, tmax, h, stats);
             }
@@ -612,6 +628,7 @@ __device__ __forceinline__ void walk_packet(const Scene S, PairLds *L, const int
         cm = next_mask;
     }
     flush_pairs(S, L, pairs, g, lo, ld, tmax, stats);
+    st.report();
 }
 
 // One instance for the lanes in mask: the ray moved into mesh space (mesh_dev.h:164-171, direction not
@@ -655,12 +672,15 @@ __device__ void visit_instance(const Scene S, PairLds *L, const int g, const uin
         flush_pairs(S, L, pairs, g, lo, ld, tmax, stats);
         return;
     }
-    // the two-child layout starts below the root's box
-    if (lanes) share_subtree(L, shared, root_mask, root_ref);
-    else if (BLAS != 2) walk_packet<LANES>(S, L, g, root_ref, root_mask, lo, ld, inv_d, tmax, h, shared, stats);
+    // the two-child layout starts below the root's box; with octant copies, each ray in its octant's
+    const int octant_nodes = LANES && Stats::kTwoChild ? S.octant_nodes() : 0;
+    const int octant_base = octant_nodes * ray_octant(inv_d);
+    if (lanes) share_subtree(L, shared, root_mask, octant_base + root_ref);
+    else if (BLAS != 2) walk_packet<LANES>(S, L, g, root_ref, root_mask, lo, ld, inv_d, tmax, h, octant_base, shared, stats);
     if (LANES && shared > 0) {
-        if constexpr (Stats::kTwoChild) walk_shared_two_child(S, L, g, shared, lo, ld, inv_d, tmax, stats);
-        else walk_shared(S, L, g, shared, lo, ld, inv_d, tmax, stats);
+        if constexpr (!Stats::kTwoChild) walk_shared(S, L, g, shared, lo, ld, inv_d, tmax, stats);
+        else if (octant_nodes > 0) walk_shared_two_child<true>(S, L, g, shared, lo, ld, inv_d, tmax, stats);
+        else walk_shared_two_child<false>(S, L, g, shared, lo, ld, inv_d, tmax, stats);
     }
 }
 
@@ -686,31 +706,37 @@ __device__ void trace_world(const Scene S, PairLds *L, const int world, const fl
     int next_ref = root >= first_leaf ? ~(root - first_leaf) : root;
     uint64_t next_mask = live;
     while (true) {
-        while (next_mask == 0 || next_ref < 0) {
-            if (next_mask != 0) {
-                visit_instance<BLAS>(S, L, ~next_ref, next_mask, ov, d, tmax, h, stats);
-                lim = min_quiet(tmax, BELOW_NO_HIT);
+        if (next_mask != 0) {
+            if (next_ref >= 0) {
+                const Wide w = load_wide(nodes, next_ref);
+                stats.add(ST_TLAS_NODES, 1);
+                stats.add(ST_TLAS_LANES, popc64(next_mask));
+                float dl, dr;
+                const uint64_t ml = next_mask & ballot(box_hit(w.l_lo[0], w.l_lo[1], w.l_lo[2], w.l_hi[0], w.l_hi[1], w.l_hi[2], ov, inv_d, lim, dl));
+                const uint64_t mr = next_mask & ballot(box_hit(w.r_lo[0], w.r_lo[1], w.r_lo[2], w.r_hi[0], w.r_hi[1], w.r_hi[2], ov, inv_d, lim, dr));
+                if (mr == 0) {
+                    next_ref = w.left;
+                    next_mask = ml;
+                } else if (ml == 0) {
+                    next_ref = w.right;
+                    next_mask = mr;
+                } else {
+                    // a lane is nearer the left child when it enters only the left, or the left no later than the right
+                    const uint64_t near_left = ml & (~mr | ballot(dl <= dr));
+                    const bool left_first = 2 * popc64(near_left) >= popc64(ml | mr);
+                    next_ref = left_first ? w.left : w.right;
+                    next_mask = left_first ? ml : mr;
+                    st.push(left_first ? w.right : w.left, left_first ? mr : ml);
+                }
+                continue;
             }
-            if (st.sp == 0) return;
-            st.pop(next_ref, next_mask);
+            visit_instance<BLAS>(S, L, ~next_ref, next_mask, ov, d, tmax, h, stats);
+            lim = min_quiet(tmax, BELOW_NO_HIT);
         }
-        const Wide w = load_wide(nodes, next_ref);
-        stats.add(ST_TLAS_NODES, 1);
-        stats.add(ST_TLAS_LANES, popc64(next_mask));
-        float dl, dr;
-        const uint64_t ml = next_mask & ballot(box_hit(w.l_lo[0], w.l_lo[1], w.l_lo[2], w.l_hi[0], w.l_hi[1], w.l_hi[2], ov, inv_d, lim, dl));
-        const uint64_t mr = next_mask & ballot(box_hit(w.r_lo[0], w.r_lo[1], w.r_lo[2], w.r_hi[0], w.r_hi[1], w.r_hi[2], ov, inv_d, lim, dr));
-        next_ref = ml != 0 ? w.left : w.right;
-        next_mask = ml != 0 ? ml : mr;
-        if (ml != 0 && mr != 0) {
-            // a lane is nearer the left child when it enters only the left, or the left no later than the right
-            const uint64_t near_left = ml & (~mr | ballot(dl <= dr));
-            const bool left_first = 2 * popc64(near_left) >= popc64(ml | mr);
-            next_ref = left_first ? w.left : w.right;
-            next_mask = left_first ? ml : mr;
-            st.push(left_first ? w.right : w.left, left_first ? mr : ml);
-        }
+        if (st.sp == 0) break;
+        st.pop(next_ref, next_mask);
     }
+    st.report();
 }
 
 // ------------------------------------------------------------------------------ per-lane walk --
