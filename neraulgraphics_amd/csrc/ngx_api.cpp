@@ -122,15 +122,16 @@ struct ngx_ctx {
     uint8_t *d_root_at_end = nullptr;
     int *d_tmpl_mesh = nullptr;
     float *d_mesh_bounds = nullptr;
-    ngx::WideNode *d_blas_wide = nullptr, *d_blas_octants = nullptr;
+    ngx::WideNode *d_blas_wide = nullptr;  // and the octant copies after it, octant_nodes each
+    const ngx::WideNode *octants() const { return octant_nodes > 0 ? d_blas_wide + octant_nodes : nullptr; }
     int octant_nodes = 0;
     int *d_blas_parent = nullptr;
     int *d_blas_wide_node = nullptr;
     // deforming meshes (ngx_set_mesh_vertices)
     float *d_vertices = nullptr;        // every mesh's vertices, 3 floats each: where new ones from the host land
-    int *d_tri_verts = nullptr, *d_refit_levels = nullptr;
-    ngx::RefitEntry *d_refit_entries = nullptr;
-    ngx::RefitTreelet *d_refit_treelets = nullptr;
+    int *d_tri_verts = nullptr;
+    int *d_refit = nullptr;             // how meshes are refitted: the entries, then the treelets, then their levels
+    size_t refit_entries = 0, refit_treelets = 0;
     std::vector<std::vector<ngx::host::RefitLayer>> refit_layers;  // per mesh
     std::vector<int> mesh_vertex_base, mesh_vertex_count, mesh_tri_count;
     std::vector<uint8_t> mesh_has_normals;
@@ -207,21 +208,22 @@ struct ngx_ctx {
     int render_blocks = 0, rgb_blocks = 0, ray_blocks = 0, backward_blocks = 0;
     int rgb_two_pass = 1;
     int compute_units = 0;              // sizes the persistent launch
-    int *d_tile_counters = nullptr;
+    int *d_tile_counters = nullptr;     // TILE_COUNTER_SETS sets
+    char *d_view_tables = nullptr;      // ViewTables' arrays, in d_wide's allocation after the nodes, or null
     int *d_overflow = nullptr;          // set by a walk whose stack would pass its capacity; read by ngx_synchronize
 
     ~ngx_ctx() {
         int *ints[] = {d_world_off, d_tmpl_mesh, d_roots, d_body_of_instance, d_dbg_sorted_ids, d_blas_parent, d_blas_wide_node, d_wide_parent,
-                       d_tri_verts, d_refit_levels,
+                       d_tri_verts, d_refit,
                        d_geom_of_instance, d_tile_counters, d_mesh_skip_root, d_mesh_tris, d_overflow};
         for (int *p : ints) if (p) (void)hipFree(p);
         float *floats[] = {d_vertices, d_mesh_bounds, d_matrices, d_matrix_stage, d_local_pose, d_scale, d_local_rot_scale, d_body_stage,
                            d_geom_scale, d_geom_stage, d_depth, d_normal, d_cam_stage, d_ray_o, d_ray_d, d_hit_dist, d_hit_normal, d_partial, d_dbg_aabb,
                            d_dbg_world_bounds};
         for (float *p : floats) if (p) (void)hipFree(p);
-        void *others[] = {d_root_at_end, d_blas_wide, d_blas_octants, d_mesh_roots, d_tris, d_attrs, d_spheres, d_inst, d_nodes, d_wide,
+        void *others[] = {d_root_at_end, d_blas_wide, d_mesh_roots, d_tris, d_attrs, d_spheres, d_inst, d_nodes, d_wide,
                           d_id, d_hit_id, d_dbg_keys, d_dbg_sorted_keys, d_skip, d_ray_keys, d_ray_vals, d_inst_mat, d_sphere_mat,
-                          d_lights, d_rgb, d_refit_entries, d_refit_treelets, d_rgb_hits, d_rgb_uv, big.key[0], big.key[1], big.val[0], big.val[1],
+                          d_lights, d_rgb, d_rgb_hits, d_rgb_uv, big.key[0], big.key[1], big.val[0], big.val[1],
                           big.box, big.span, big.across, big.bounds, d_big_worlds, d_big_sort_tiles, d_big_node_tiles};
         for (void *p : others) if (p) (void)hipFree(p);
         if (ev0) (void)hipEventDestroy(ev0);
@@ -239,7 +241,7 @@ struct ngx_ctx {
         s.inst = d_inst;
         s.mesh_roots = d_mesh_roots;
         s.blas_wide = d_blas_wide;
-        s.blas_octants = d_blas_octants;
+        s.blas_octants = octants();
         s.octant_nodes = octant_nodes;
         s.tris = d_tris;
         s.attrs = d_attrs;
@@ -314,6 +316,7 @@ struct ngx_ctx {
         return waves <= 2 * cus ? 8 : waves <= 8 * cus ? 16 : waves <= 24 * cus ? 32 : 64;
     }
     static constexpr int FINE_MESH_TRIANGLES = 10000;
+    static constexpr int TILE_COUNTER_SETS = 3;  // a frame's launches one after the other: depth, hits or RGB, shading
 
     // The tiles of a picture: `shape` pixels wide and 64 in all, the longer side halved until a tile has `lanes` pixels.
     void set_tiles(ngx::RenderArgs &a, const int lanes, const int shape) const {
@@ -348,6 +351,64 @@ struct ngx_ctx {
         a.walk = walk();
         a.tile_counters = persistent ? d_tile_counters : nullptr;
         return a;
+    }
+
+    // The view tables' arrays, the cameras first (each a multiple of 16 bytes): 336 bytes an instance and camera, beside some
+    // 300 that a built instance takes.
+    size_t view_table_instances() const { return (size_t)cpw * (size_t)total; }
+    size_t view_tables_bytes() const {
+        return 4 * sizeof(float4) * (size_t)views +
+               view_table_instances() * (ngx::VIEW_OCTANTS * sizeof(ngx::WideNode) + ngx::VIEW_INSTANCE_FLOAT4S * sizeof(float4)) +
+               sizeof(float) * ((size_t)width + height + 2 * ngx::PIXEL_PAD);
+    }
+    // A launch makes them where it gains by them. They cost some 0.15 ns an instance and a few microseconds, and save a
+    // wavefront of a full chip a tenth of its instructions: 4096 worlds of 128 instances at 128x128 6.90 -> 6.79 ms, of 32 at
+    // 64x64 1.110 -> 1.105, 1,024 lit pictures 7.64 -> 7.40; but one world of 16 (512 tiles) 48.5 -> 49.4 us.
+    // Re-traces of a backward, which are bounded by the forward's depth, do not gain (depth gradient 702 -> 708 us).
+    static constexpr size_t VIEW_TABLES_MAX_BYTES = (size_t)1 << 30;
+    static constexpr int VIEW_TABLES_MAX_VIEWS = 1 << 22;
+    static constexpr long long VIEW_TABLES_MIN_TILES = 4096, VIEW_TABLES_MAX_INSTANCES_PER_TILE = 4;
+    bool view_tables_pay(const long long tiles) const {
+        return tiles >= VIEW_TABLES_MIN_TILES && (long long)view_table_instances() <= VIEW_TABLES_MAX_INSTANCES_PER_TILE * tiles;
+    }
+    // Whether any launch of the context may make them: its tiles have 4 pixels or more.
+    bool view_tables_of_use() const {
+        return views <= VIEW_TABLES_MAX_VIEWS && view_tables_bytes() <= VIEW_TABLES_MAX_BYTES &&
+               view_tables_pay((long long)views * width * height / 4);
+    }
+
+    // Makes a launch's view tables, where it has some, and zeroes its sets of tile counters.
+    void prepare_views(ngx::ViewTables &t, const float *cams, const float fov, const long long tiles, const int counter_sets, hipStream_t s) {
+        ngx::ViewTableArgs v{};
+        if (d_view_tables && packet && view_tables_pay(tiles)) {
+            char *p = d_view_tables;
+            t.cams = reinterpret_cast<float4 *>(p);
+            p += 4 * sizeof(float4) * (size_t)views;
+            t.nodes = reinterpret_cast<ngx::WideNode *>(p);
+            p += ngx::VIEW_OCTANTS * sizeof(ngx::WideNode) * view_table_instances();
+            t.inst = reinterpret_cast<float4 *>(p);
+            p += ngx::VIEW_INSTANCE_FLOAT4S * sizeof(float4) * view_table_instances();
+            t.pixels = reinterpret_cast<float *>(p);
+            v.t = t;
+        }
+        v.counters = d_tile_counters;
+        v.counter_sets = counter_sets;
+        v.cams = cams;
+        v.views = views;
+        v.cameras_per_world = cpw;
+        v.width = width;
+        v.height = height;
+        v.fov_scale = std::tan(fov * 0.5f);
+        v.aspect = (float)width / (float)height;
+        v.world_off = d_world_off;
+        v.root_at_end = d_root_at_end;
+        v.tlas_wide = d_wide;
+        v.inst = d_inst;
+        v.mesh_roots = d_mesh_roots;
+        v.total = total;
+        v.max_count = max_count;
+        v.lane_min_tris = lane_min_tris;
+        HIP_CHECK(ngx::launch_view_tables(v, s));
     }
 
     // The kernels' walk: per-lane, packet, or packet with the bottom level of meshes of lane_min_tris or more
@@ -496,7 +557,7 @@ ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out) {
             c.compute_units = std::max(1, prop.multiProcessorCount);
         }
         HIP_CHECK(ngx::noalloc_scratch(&c.d_noalloc_scratch));
-        device_alloc(c.d_tile_counters, (size_t)ngx::TILE_COUNTER_INTS);
+        device_alloc(c.d_tile_counters, (size_t)ngx_ctx::TILE_COUNTER_SETS * ngx::TILE_COUNTER_INTS);
         device_alloc(c.d_overflow, 1);
         HIP_CHECK(hipMemset(c.d_overflow, 0, sizeof(int)));
         HIP_CHECK(hipEventCreate(&c.ev0));
@@ -519,16 +580,15 @@ ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out) {
                     fail(NGX_DEVICE_ERROR, "a bottom-level tree is " + std::to_string(deepest) + " levels deep; the walks hold " +
                                                std::to_string(ngx::WALK_STACK - 1));
             }
-            upload(c.d_blas_wide, built.wide.data(), built.wide.size() ? built.wide.size() : 0);
-            if (!c.d_blas_wide) device_alloc(c.d_blas_wide, 1);
-            if (!built.wide.empty() && 8 * sizeof(ngx::WideNode) * built.wide.size() <= ngx::OCTANT_COPIES_MAX_BYTES) {
-                c.octant_nodes = (int)built.wide.size();
-                std::vector<ngx::WideNode> copies;
-                copies.reserve(8 * built.wide.size());
+            const size_t wide_count = built.wide.size();
+            if (wide_count > 0 && 8 * sizeof(ngx::WideNode) * wide_count <= ngx::OCTANT_COPIES_MAX_BYTES) {
+                c.octant_nodes = (int)wide_count;
+                built.wide.reserve(9 * wide_count);
                 for (int o = 0; o < 8; ++o)
-                    for (const ngx::WideNode &n : built.wide) copies.push_back(n.for_octant(o, o * c.octant_nodes));
-                upload(c.d_blas_octants, copies.data(), copies.size());
+                    for (size_t i = 0; i < wide_count; ++i) built.wide.push_back(built.wide[i].for_octant(o, o * c.octant_nodes));
             }
+            upload(c.d_blas_wide, built.wide.data(), built.wide.size());
+            if (!c.d_blas_wide) device_alloc(c.d_blas_wide, 1);
             upload(c.d_blas_parent, built.wide_parent.data(), built.wide_parent.size());
             if (!c.d_blas_parent) device_alloc(c.d_blas_parent, 1);
             upload(c.d_blas_wide_node, built.wide_node.data(), built.wide_node.size());
@@ -544,9 +604,17 @@ ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out) {
             upload(c.d_mesh_skip_root, built.roots.data(), built.roots.size());
             upload(c.d_vertices, s.vertices, 3 * (size_t)s.vertex_offsets[s.mesh_count]);
             upload(c.d_tri_verts, built.tri_verts.data(), built.tri_verts.size());
-            upload(c.d_refit_levels, built.refit_levels.data(), built.refit_levels.size());
-            upload(c.d_refit_entries, built.refit_entries.data(), built.refit_entries.size());
-            upload(c.d_refit_treelets, built.refit_treelets.data(), built.refit_treelets.size());
+            {
+                constexpr size_t E = sizeof(ngx::RefitEntry) / sizeof(int), T = sizeof(ngx::RefitTreelet) / sizeof(int);
+                c.refit_entries = built.refit_entries.size();
+                c.refit_treelets = built.refit_treelets.size();
+                std::vector<int> plan(E * c.refit_entries + T * c.refit_treelets + built.refit_levels.size());
+                int *const p = plan.data();
+                std::memcpy(p, built.refit_entries.data(), sizeof(ngx::RefitEntry) * c.refit_entries);
+                std::memcpy(p + E * c.refit_entries, built.refit_treelets.data(), sizeof(ngx::RefitTreelet) * c.refit_treelets);
+                std::copy(built.refit_levels.begin(), built.refit_levels.end(), p + E * c.refit_entries + T * c.refit_treelets);
+                upload(c.d_refit, p, plan.size());
+            }
             c.refit_layers = built.refit_layers;
             for (int m = 0; m < s.mesh_count; ++m) {
                 c.mesh_vertex_base.push_back(s.vertex_offsets[m]);
@@ -593,7 +661,11 @@ ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out) {
             device_alloc(c.d_matrix_stage, 12 * (size_t)s.worlds * s.instances_per_world);
             device_alloc(c.d_inst, (size_t)c.total);
             device_alloc(c.d_nodes, 2 * (size_t)c.total - 1);
-            device_alloc(c.d_wide, std::max<size_t>(1, (size_t)c.total - 1));
+            const size_t wide_nodes = std::max<size_t>(1, (size_t)c.total - 1);
+            if (c.view_tables_of_use() &&
+                try_device_alloc(c.d_wide, wide_nodes + (c.view_tables_bytes() + sizeof(ngx::WideNode) - 1) / sizeof(ngx::WideNode)))
+                c.d_view_tables = reinterpret_cast<char *>(c.d_wide + wide_nodes);
+            else device_alloc(c.d_wide, wide_nodes);
             device_alloc(c.d_wide_parent, std::max<size_t>(1, (size_t)c.total - 1));
             if (!c.big_worlds.empty()) {
                 ngx::BigBuildScratch &b = c.big;
@@ -835,11 +907,11 @@ ngx_status ngx_set_mesh_vertices(ngx_ctx *ctx, const int32_t mesh, const float *
         a.tris = ctx->d_tris;
         a.skip = ctx->d_skip + 1;
         a.wide = ctx->d_blas_wide;
-        a.octants = ctx->d_blas_octants;
+        a.octants = const_cast<ngx::WideNode *>(ctx->octants());
         a.octant_nodes = ctx->octant_nodes;
-        a.treelets = ctx->d_refit_treelets;
-        a.entries = ctx->d_refit_entries;
-        a.levels = ctx->d_refit_levels;
+        a.entries = reinterpret_cast<const ngx::RefitEntry *>(ctx->d_refit);
+        a.treelets = reinterpret_cast<const ngx::RefitTreelet *>(a.entries + ctx->refit_entries);
+        a.levels = reinterpret_cast<const int *>(a.treelets + ctx->refit_treelets);
         a.mesh_root = ctx->d_mesh_roots + mesh;
         a.mesh_bounds = ctx->d_mesh_bounds + 6 * (size_t)mesh;
         for (const ngx::host::RefitLayer &layer : ctx->refit_layers[mesh]) HIP_CHECK(ngx::launch_mesh_refit(a, layer.first, layer.count, s));
@@ -975,6 +1047,7 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
         }
         const bool timed = !ctx->capturing(s);
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev0, s));
+        ctx->prepare_views(a.tables, cams, fov, a.total_tiles, ctx->persistent ? ngx_ctx::TILE_COUNTER_SETS : 0, s);
         if (a.depth || a.normal || a.object_id) HIP_CHECK(ngx::launch_render(a, s, ctx->persistent ? ctx->compute_units : 0));
         if (rgb) {
             ngx::RgbArgs g{};
@@ -982,7 +1055,7 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
             g.r.depth = nullptr;
             g.r.normal = nullptr;
             g.r.object_id = nullptr;
-            g.r.tile_counters = ctx->persistent ? ctx->d_tile_counters : nullptr;
+            g.r.tile_counters = ctx->persistent ? ctx->d_tile_counters + ngx::TILE_COUNTER_INTS : nullptr;
             g.shade = ctx->shade;
             g.rgb = rgb;
             g.spp = spp;

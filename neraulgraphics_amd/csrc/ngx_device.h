@@ -316,5 +316,15 @@ __device__ __forceinline__ int4 sload4i(const int4 *p) {
     const v4i v = *(const const_v4i *)((uintptr_t)p);
     return make_int4(v.x, v.y, v.z, v.w);
 }
+// 4 or 16 floats at a 32-bit offset past a wave-uniform base, which the load adds by itself.
+typedef float v16f __attribute__((ext_vector_type(16), aligned(16)));
+typedef __attribute__((address_space(4))) const v16f const_v16f;
+__device__ __forceinline__ float4 sload4_at(const void *base, const uint32_t offset) {
+    const v4f v = *(const const_v4f *)((__attribute__((address_space(4))) const char *)(uintptr_t)base + offset);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ v16f sload16_at(const void *base, const uint32_t offset) {
+    return *(const const_v16f *)((__attribute__((address_space(4))) const char *)(uintptr_t)base + offset);
+}
 
 }  // namespace ngx

@@ -118,8 +118,27 @@ inline FastDivide fast_divide_by(const int d) {
     return f;
 }
 
+// What a launch of camera rays reads of its views, made by launch_view_tables before it: a view's rays share their
+// origin, so its camera, the top level's boxes about it and each instance's rows and origin are worked out once, not once
+// a wavefront. The nodes are kept per octant of ray directions, near planes first, for the first VIEW_OCTANTS octants
+// that a view's rays may have (looking about along an axis they have four; a wavefront whose rays have several octants,
+// or one that is not kept, walks the tree itself). All null: not made.
+constexpr int VIEW_OCTANTS = 4;
+constexpr int VIEW_NO_OCTANTS = -1;
+struct ViewTables {
+    float4 *cams;              // [views][4]: position and, four bits an octant, where its nodes are (15: nowhere); right; up; forward
+    WideNode *nodes;           // [cameras_per_world][VIEW_OCTANTS][total]
+    float4 *inst;              // [cameras_per_world][total][VIEW_INSTANCE_FLOAT4S]
+    float *pixels;             // the image plane's x of each column, PIXEL_PAD more, then its y of each row, PIXEL_PAD more
+};
+// per instance: its three rows, each with the mesh-space origin's component; the root box's planes about that origin and
+// the root's reference; and in the last word the triangles of a root that is a leaf, or whether it is walked lane by lane
+constexpr int VIEW_INSTANCE_FLOAT4S = 5;
+constexpr int PIXEL_PAD = 64;  // tiles reach past the image by less
+
 struct RenderArgs {
     TraceScene s;
+    ViewTables tables;
     const float *cams;         // [views][12]
     float fov_scale;           // tanf(fov / 2), computed on the host as the reference's CPU backend does
     float aspect;              // width / height
@@ -133,7 +152,7 @@ struct RenderArgs {
     int32_t *object_id;        // [views][H][W] or null
     int xcd_remap;             // 1: consecutive tiles stay on one XCD
     int walk;                  // 0 per-lane, 1 packet, 2 packet with fine meshes lane by lane
-    int *tile_counters;        // persistent mode (non-null): TILE_COUNTER_INTS ints, zeroed by the launch
+    int *tile_counters;        // persistent mode (non-null): TILE_COUNTER_INTS ints, zero (launch_view_tables)
     int blocks;                // the kernel variant: workgroups per compute unit it is built for (0: the walk's default)
 };
 
@@ -307,15 +326,33 @@ struct MeshRefitArgs {
 // One layer of the mesh's treelets, first .. first + count - 1; the layers in order.
 hipError_t launch_mesh_refit(const MeshRefitArgs &a, int first, int count, hipStream_t stream);
 
-// The RGB picture; with a.r.tile_counters set and compute_units > 0, from a persistent grid as launch_render.
+// The RGB picture; with a.r.tile_counters set and compute_units > 0, from a persistent grid as launch_render. The
+// two-pass picture takes two sets of counters, one after the other.
 hipError_t launch_rgb(const RgbArgs &a, hipStream_t stream, int compute_units = 0);
 // One sample a pixel, no surface reflective enough to bounce, persistent launch, packet or hybrid walk: the hit pass,
 // then the shading pass; the same bytes as launch_rgb.
 hipError_t launch_rgb_two_pass(const RgbArgs &a, int hit_blocks, hipStream_t stream, int compute_units);
 
+// Zeroes `counter_sets` sets of tile counters (or none, null) and makes the view tables, unless t.cams is null.
+struct ViewTableArgs {
+    ViewTables t;
+    int *counters;
+    int counter_sets;
+    const float *cams;         // [views][12]
+    int views, cameras_per_world, width, height;
+    float fov_scale, aspect;
+    const int *world_off;      // [worlds + 1]
+    const uint8_t *root_at_end;
+    const WideNode *tlas_wide;
+    const InstanceRec *inst;
+    const MeshRoot *mesh_roots;
+    int total, max_count;      // instances in all, and of the largest world
+    int lane_min_tris;
+};
+hipError_t launch_view_tables(const ViewTableArgs &a, hipStream_t stream);
+
 // Renders every view; with a.tile_counters set and compute_units > 0, a fixed grid of as many workgroups as the
-// device holds at once takes tiles from per-XCD counters until none are left (the counters are zeroed by this
-// call first).
+// device holds at once takes tiles from per-XCD counters until none are left.
 hipError_t launch_render(const RenderArgs &a, hipStream_t stream, int compute_units = 0);
 hipError_t launch_rays(const RayArgs &a, hipStream_t stream);
 hipError_t launch_depth_backward(const DepthBackwardArgs &a, hipStream_t stream);

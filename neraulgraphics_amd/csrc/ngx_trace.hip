@@ -20,6 +20,7 @@
 // instructions a visit: arguments read where they are used and the walk's pointers once, wave-uniform stacks in vector
 // registers, masked instructions without a branch around them (NGX_LIKELY), lanes that drop out by their limit rather
 // than by a mask, rare cases tested once for the wave. 8.44 -> 6.73 ms there, 13.7 -> 12.7 ms for 67 M LiDAR rays.
+#include <algorithm>
 #include <cstddef>
 #include <mutex>
 #include "ngx_kernels.h"
@@ -121,8 +122,13 @@ struct NoStats {
     __device__ __forceinline__ void add(int, int) {}
 };
 // Camera rays: every ray of the wave starts at the camera, so what an instance makes of the origin is one point for the
-// wave, held in scalar registers.
-struct CameraRays {
+// wave, held in scalar registers, and the view's tables may hold the top level about it.
+struct ViewOfRays {
+    const WideNode *nodes = nullptr;  // the view's copies of the top level (VIEW_OCTANTS times total), where `octants` says
+    const float4 *inst = nullptr;     // the view's instances, or null
+    int octants = VIEW_NO_OCTANTS;
+};
+struct CameraRays : ViewOfRays {
     static constexpr bool kAnyHit = false, kHandoff = true, kTwoChild = true, kOneOrigin = true;
     __device__ __forceinline__ void add(int, int) {}
 };
@@ -141,7 +147,7 @@ struct OcclusionTwoChild {
     __device__ __forceinline__ void add(int, int) {}
 };
 #ifdef NGX_TRACE_STATS
-struct WaveStats {
+struct WaveStats : ViewOfRays {
     static constexpr bool kAnyHit = false, kHandoff = true, kTwoChild = true, kOneOrigin = true;
     int c[ST_COUNT];
     __device__ __forceinline__ void add(const int k, const int v) { c[k] += v; }
@@ -208,6 +214,14 @@ __device__ __forceinline__ int rank_in(const uint64_t mask) {
 extern "C" __device__ __attribute__((const)) int ngx_write_lane(int v, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 __device__ __forceinline__ int write_lane(const int v, const int lane, const int old) { return ngx_write_lane(v, lane, old); }
 
+// A wave-uniform value in a scalar register, whose origin the compiler then does not see: it would otherwise compare counts
+// of lanes as 64-bit numbers in vector registers, and keep conditions as lane masks.
+__device__ __forceinline__ int as_scalar(int v) {
+    v = uniform(v);
+    asm("" : "+s"(v));
+    return v;
+}
+
 // A wave-uniform stack of (node reference, lane mask) in three vector registers, entry k in lane k: a push or a pop is
 // three instructions and waits for nothing.
 struct WaveStack {
@@ -225,13 +239,21 @@ struct WaveStack {
         deepest = max(deepest, ++sp);
         sp = min(sp, WALK_STACK);
     }
+    // The same where m may be empty, which pushes nothing: the entry is written and not counted. The caller keeps `deepest`.
+    __device__ __forceinline__ void push_some(const int r, const uint64_t m) {
+        const int at = sp & 63;
+        ref = write_lane(r, at, ref);
+        lo = write_lane((int)(uint32_t)m, at, lo);
+        hi = write_lane((int)(uint32_t)(m >> 32), at, hi);
+        sp += as_scalar(min(popc64(m), 1));
+    }
     __device__ __forceinline__ void pop(int &r, uint64_t &m) {
         --sp;
         r = __builtin_amdgcn_readlane(ref, sp);
         m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, sp) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, sp);
     }
     __device__ __forceinline__ void report() const {
-        if (NGX_UNLIKELY(deepest > WALK_STACK) && lane_id() == 0) *Scene().overflow() = 1;
+        if (NGX_UNLIKELY(deepest >= WALK_STACK) && lane_id() == 0) *Scene().overflow() = 1;
     }
 };
 static_assert(WALK_STACK <= 64, "an entry a lane");
@@ -631,6 +653,17 @@ __device__ __forceinline__ void walk_packet(const Scene S, PairLds *L, const int
     st.report();
 }
 
+template <class Stats>
+__device__ __forceinline__ bool has_view(const Stats &stats) {
+    if constexpr (Stats::kOneOrigin) return stats.inst != nullptr;
+    return false;
+}
+template <class Stats>
+__device__ __forceinline__ const float4 *view_instances(const Stats &stats) {
+    if constexpr (Stats::kOneOrigin) return stats.inst;
+    return nullptr;
+}
+
 // One instance for the lanes in mask: the ray moved into mesh space (mesh_dev.h:164-171, direction not
 // renormalized so t is shared), then the mesh's own tree.
 // BLAS: how bottom levels are walked: 0 as a packet; 1 lane by lane for meshes of lane_min_tris triangles or more,
@@ -641,26 +674,46 @@ __device__ void visit_instance(const Scene S, PairLds *L, const int g, const uin
                                const float3 d, float &tmax, LaneHit &h, Stats &stats) {
     stats.add(ST_INSTANCES, 1);
     stats.add(ST_INSTANCE_LANES, popc64(mask));
-    const float4 *rp = reinterpret_cast<const float4 *>(S.inst() + g);
-    const float4 r0 = sload4(rp), r1 = sload4(rp + 1), r2 = sload4(rp + 2);
-    const int4 meta = sload4i(reinterpret_cast<const int4 *>(rp + 3));
-    float3 lo = mk3(dot3(xyz(r0), o) + r0.w, dot3(xyz(r1), o) + r1.w, dot3(xyz(r2), o) + r2.w);
-    if (Stats::kOneOrigin) lo = mk3(uniform_f(lo.x), uniform_f(lo.y), uniform_f(lo.z));
-    const float3 ld = mk3(dot3(xyz(r0), d), dot3(xyz(r1), d), dot3(xyz(r2), d));
-    const float3 inv_d = safe_inverse(ld);
-    const float4 *mp = reinterpret_cast<const float4 *>(S.mesh_roots() + meta.x);
-    const float4 m0 = sload4(mp), m1 = sload4(mp + 1);
+    float3 lo, ld, inv_d;
     float root_t;
-    const uint64_t root_mask = mask & ballot(box_hit(m0.x, m0.y, m0.z, m1.x, m1.y, m1.z, lo, inv_d, box_limit(tmax), root_t));
+    uint64_t root_mask;
+    int root_ref, root_count, skip_root = 0;
+    bool lanes;
+    if (Stats::kOneOrigin && has_view(stats)) {
+        const float4 *const table = view_instances(stats);
+        const uint32_t at = (uint32_t)g * (uint32_t)(VIEW_INSTANCE_FLOAT4S * sizeof(float4));
+        const v16f r = sload16_at(table, at);
+        const float4 m1 = sload4_at(table, at + 64);
+        lo = mk3(r[3], r[7], r[11]);
+        ld = mk3(dot3(mk3(r[0], r[1], r[2]), d), dot3(mk3(r[4], r[5], r[6]), d), dot3(mk3(r[8], r[9], r[10]), d));
+        inv_d = safe_inverse(ld);
+        root_mask = mask & ballot(box_hit(r[12], r[13], r[14], m1.x, m1.y, m1.z, mk3(0.0f, 0.0f, 0.0f), inv_d, box_limit(tmax), root_t));
+        root_ref = __float_as_int(r[15]);
+        root_count = __float_as_int(m1.w);
+        lanes = BLAS == 2 || (BLAS == 1 && root_ref >= 0 && root_count != 0);
+    } else {
+        const float4 *rp = reinterpret_cast<const float4 *>((Stats::kOneOrigin ? Scene().inst() : S.inst()) + g);
+        const float4 r0 = sload4(rp), r1 = sload4(rp + 1), r2 = sload4(rp + 2);
+        const int4 meta = sload4i(reinterpret_cast<const int4 *>(rp + 3));
+        lo = mk3(dot3(xyz(r0), o) + r0.w, dot3(xyz(r1), o) + r1.w, dot3(xyz(r2), o) + r2.w);
+        if (Stats::kOneOrigin) lo = mk3(uniform_f(lo.x), uniform_f(lo.y), uniform_f(lo.z));
+        ld = mk3(dot3(xyz(r0), d), dot3(xyz(r1), d), dot3(xyz(r2), d));
+        inv_d = safe_inverse(ld);
+        const float4 *mp = reinterpret_cast<const float4 *>((Stats::kOneOrigin ? Scene().mesh_roots() : S.mesh_roots()) + meta.x);
+        const float4 m0 = sload4(mp), m1 = sload4(mp + 1);
+        root_mask = mask & ballot(box_hit(m0.x, m0.y, m0.z, m1.x, m1.y, m1.z, lo, inv_d, box_limit(tmax), root_t));
+        root_ref = __float_as_int(m0.w);
+        root_count = __float_as_int(m1.w);
+        skip_root = meta.w;
+        lanes = BLAS == 2 || (BLAS == 1 && meta.z >= S.lane_min_tris());
+    }
     if (root_mask == 0) return;
     stats.add(ST_INSTANCE_ROOT_LANES, popc64(root_mask));
     int shared = 0;  // subtrees given to the shared per-lane walk
     constexpr bool LANES = BLAS != 0;
-    const int root_ref = __float_as_int(m0.w);
-    const bool lanes = BLAS == 2 || (BLAS == 1 && meta.z >= S.lane_min_tris());
     if constexpr (!Stats::kTwoChild) {
         if (lanes) {
-            share_subtree(L, shared, root_mask, meta.w);
+            share_subtree(L, shared, root_mask, skip_root);
             walk_shared(S, L, g, shared, lo, ld, inv_d, tmax, stats);
             return;
         }
@@ -668,7 +721,7 @@ __device__ void visit_instance(const Scene S, PairLds *L, const int g, const uin
     if (root_ref < 0) {
         // a mesh of one leaf, tested as a batch
         int pairs = 0;
-        add_leaf(S, L, pairs, ~root_ref, __float_as_int(m1.w), root_mask, g, lo, ld, tmax, h, stats);
+        add_leaf(S, L, pairs, ~root_ref, root_count, root_mask, g, lo, ld, tmax, h, stats);
         flush_pairs(S, L, pairs, g, lo, ld, tmax, stats);
         return;
     }
@@ -684,6 +737,23 @@ __device__ void visit_instance(const Scene S, PairLds *L, const int g, const uin
     }
 }
 
+// From a top-level node to its nearer child, the farther one pushed, for the lanes in `mask`; l and r are the lanes whose
+// rays enter each child's box, and nearer those that enter the left one no later. A lane is nearer the left child when it
+// enters only the left, or the left no later than the right; the left child is first when it is nearer for half the lanes
+// that enter either.
+template <class Stats>
+__device__ __forceinline__ void enter_children(WaveStack &st, const uint64_t l, const uint64_t r, const uint64_t nearer, const int left,
+                                               const int right, int &ref, uint64_t &mask, Stats &stats) {
+    stats.add(ST_TLAS_NODES, 1);
+    stats.add(ST_TLAS_LANES, popc64(mask));
+    const uint64_t ml = mask & l, mr = mask & r;
+    const uint64_t near_left = ml & (~mr | nearer);
+    const int more = as_scalar(popc64(near_left)) - as_scalar(popc64((ml | mr) & ~near_left));
+    st.push_some(more >= 0 ? right : left, more >= 0 ? mr : ml);
+    ref = more >= 0 ? left : right;
+    mask = more >= 0 ? ml : mr;
+}
+
 // The closest instance hit in one world for the lanes in live (mesh_dev.h:177-205). tmax is each lane's
 // distance to beat on entry and its closest distance on return.
 template <int BLAS, class Stats>
@@ -692,45 +762,54 @@ __device__ void trace_world(const Scene S, PairLds *L, const int world, const fl
     if (live == 0) return;
     const int root = uniform(S.roots()[world]);
     if (root < 0) return;
-    // the origin in vector registers: for camera rays it is the same in every lane
-    const float3 ov = in_vgpr3(o);
     const float3 inv_d = safe_inverse(d);
     float lim = box_limit(tmax);
     // One entry is pushed per level at most. Below a world's root every level fixes at least one more bit
     // of a Morton code (30 bits) or, among equal codes, of the leaves' positions (at most ceil(log2 n) + 1
     // bits over n consecutive positions): fewer than 64 levels for any n < 2^31, so 64 entries do.
     WaveStack st;
-    const WideNode *const nodes = S.tlas_wide();
+    const WideNode *nodes = S.tlas_wide();
+    int ordered = 0;  // the nodes are the view's, about its camera, for the octant all the rays have
+    if constexpr (Stats::kOneOrigin) {
+        if (stats.octants != VIEW_NO_OCTANTS) {
+            const int octant = ray_octant(inv_d), all = __builtin_amdgcn_readlane(octant, first_lane(live));
+            const int slot = (stats.octants >> (4 * all)) & 15;
+            if (slot < VIEW_OCTANTS && (ballot(octant != all) & live) == 0) {
+                ordered = 1;
+                nodes = stats.nodes + (size_t)slot * (size_t)S.total();
+            }
+        }
+    }
     const int first_leaf = S.total() - 1;
     // what to visit next: a node, or below zero an instance (a one-instance world's root is one)
     int next_ref = root >= first_leaf ? ~(root - first_leaf) : root;
     uint64_t next_mask = live;
     while (true) {
-        if (next_mask != 0) {
-            if (next_ref >= 0) {
-                const Wide w = load_wide(nodes, next_ref);
-                stats.add(ST_TLAS_NODES, 1);
-                stats.add(ST_TLAS_LANES, popc64(next_mask));
-                float dl, dr;
-                const uint64_t ml = next_mask & ballot(box_hit(w.l_lo[0], w.l_lo[1], w.l_lo[2], w.l_hi[0], w.l_hi[1], w.l_hi[2], ov, inv_d, lim, dl));
-                const uint64_t mr = next_mask & ballot(box_hit(w.r_lo[0], w.r_lo[1], w.r_lo[2], w.r_hi[0], w.r_hi[1], w.r_hi[2], ov, inv_d, lim, dr));
-                if (mr == 0) {
-                    next_ref = w.left;
-                    next_mask = ml;
-                } else if (ml == 0) {
-                    next_ref = w.right;
-                    next_mask = mr;
-                } else {
-                    // a lane is nearer the left child when it enters only the left, or the left no later than the right
-                    const uint64_t near_left = ml & (~mr | ballot(dl <= dr));
-                    const bool left_first = 2 * popc64(near_left) >= popc64(ml | mr);
-                    next_ref = left_first ? w.left : w.right;
-                    next_mask = left_first ? ml : mr;
-                    st.push(left_first ? w.right : w.left, left_first ? mr : ml);
-                }
-                continue;
+        // down to an instance, or to where no lane enters either child
+        if (next_ref >= 0) {
+            if (Stats::kOneOrigin && ordered != 0) {
+                do {
+                    const v16f w = sload16_at(nodes, (uint32_t)next_ref * (uint32_t)sizeof(WideNode));
+                    const float3 about = mk3(0.0f, 0.0f, 0.0f);
+                    float dl, dr;
+                    const uint64_t l = ballot(box_hit_ordered(w[0], w[4], w[8], w[2], w[6], w[10], about, inv_d, lim, dl));
+                    const uint64_t r = ballot(box_hit_ordered(w[1], w[5], w[9], w[3], w[7], w[11], about, inv_d, lim, dr));
+                    enter_children(st, l, r, ballot(dl <= dr), __float_as_int(w[12]), __float_as_int(w[13]), next_ref, next_mask, stats);
+                } while (as_scalar(next_mask != 0 ? next_ref : -1) >= 0);
+            } else {
+                const float3 ov = in_vgpr3(o);  // for camera rays the origin is scalars, as the nodes' planes are
+                do {
+                    const Wide w = load_wide(nodes, next_ref);
+                    float dl, dr;
+                    const uint64_t l = ballot(box_hit(w.l_lo[0], w.l_lo[1], w.l_lo[2], w.l_hi[0], w.l_hi[1], w.l_hi[2], ov, inv_d, lim, dl));
+                    const uint64_t r = ballot(box_hit(w.r_lo[0], w.r_lo[1], w.r_lo[2], w.r_hi[0], w.r_hi[1], w.r_hi[2], ov, inv_d, lim, dr));
+                    enter_children(st, l, r, ballot(dl <= dr), w.left, w.right, next_ref, next_mask, stats);
+                } while (as_scalar(next_mask != 0 ? next_ref : -1) >= 0);
             }
-            visit_instance<BLAS>(S, L, ~next_ref, next_mask, ov, d, tmax, h, stats);
+            st.deepest = max(st.deepest, st.sp);
+        }
+        if (next_mask != 0) {
+            visit_instance<BLAS>(S, L, ~next_ref, next_mask, o, d, tmax, h, stats);
             lim = min_quiet(tmax, BELOW_NO_HIT);
         }
         if (st.sp == 0) break;
@@ -1040,13 +1119,39 @@ __device__ __forceinline__ Cam load_camera(const float *m12) {
     return cam;
 }
 
+// A view's camera, from its tables or, where there are none, its matrix; with the tables its rays walk.
+// Args: RenderArgs, or the same in the kernel arguments' segment.
+template <class Args>
+__device__ __forceinline__ Cam camera_of(const Args &A, const int view, const int world, ViewOfRays &rays) {
+    if (A.tables.cams == nullptr) return load_camera(in_global(A.cams) + 12 * (size_t)view);
+    const float4 *p = A.tables.cams + 4 * (size_t)view;
+    const float4 a = sload4(p), b = sload4(p + 1), c = sload4(p + 2), e = sload4(p + 3);
+    const size_t first = (size_t)(view - world * A.cameras_per_world) * (size_t)A.s.total;
+    rays.octants = __float_as_int(a.w);
+    rays.nodes = A.tables.nodes + VIEW_OCTANTS * first;
+    rays.inst = A.tables.inst + VIEW_INSTANCE_FLOAT4S * first;
+    return Cam{xyz(a), xyz(b), xyz(c), xyz(e)};
+}
+
 // camera_ray (device_scene.h:114-119) through a pixel's centre.
+__device__ __forceinline__ float plane_x(const float px, const int width, const float fov_scale, const float aspect) {
+    return (2.0f * px / (float)width - 1.0f) * fov_scale * aspect;
+}
+__device__ __forceinline__ float plane_y(const float py, const int height, const float fov_scale) {
+    return -(2.0f * py / (float)height - 1.0f) * fov_scale;
+}
+__device__ __forceinline__ float3 plane_ray(const Cam &c, const float sx, const float sy) {
+    return normalize3(add3(add3(mul3(c.right, sx), mul3(c.up, sy)), c.fwd));
+}
 __device__ __forceinline__ float3 pixel_ray(const Cam &c, const float fov_scale, const float aspect, const int x, const int y,
                                             const int width, const int height) {
-    const float px = (float)x + 0.5f, py = (float)y + 0.5f;
-    const float sx = (2.0f * px / (float)width - 1.0f) * fov_scale * aspect;
-    const float sy = -(2.0f * py / (float)height - 1.0f) * fov_scale;
-    return normalize3(add3(add3(mul3(c.right, sx), mul3(c.up, sy)), c.fwd));
+    return plane_ray(c, plane_x((float)x + 0.5f, width, fov_scale, aspect), plane_y((float)y + 0.5f, height, fov_scale));
+}
+template <class Args>
+__device__ __forceinline__ float3 pixel_ray_of(const Args &A, const Cam &c, const int x, const int y) {
+    if (A.tables.cams == nullptr) return pixel_ray(c, A.fov_scale, A.aspect, x, y, A.width, A.height);
+    const float *const px = in_global(A.tables.pixels);
+    return plane_ray(c, px[(uint32_t)x], px[(uint32_t)(A.width + PIXEL_PAD + y)]);
 }
 
 // The tile of a wave: tiles are numbered view-major, and with xcd_remap consecutive workgroups, which
@@ -1104,15 +1209,15 @@ __device__ __forceinline__ void render_tile(PairLds *L, const long long tile) {
     float3 d;
     Cam cam;
     TilePixel p;
+    CameraRays stats;
     {
         const auto &A = kernel_args<RenderArgs>();
         p = tile_pixel(A, tile);
-        cam = load_camera(A.cams + 12 * (size_t)p.view);
-        d = pixel_ray(cam, A.fov_scale, A.aspect, p.x, p.y, A.width, A.height);
+        cam = camera_of(A, p.view, p.world, stats);
+        d = pixel_ray_of(A, cam, p.x, p.y);
     }
     float best;
     LaneHit h;
-    CameraRays stats;
     const int kind = scene_hit<WALK>(Scene(), L, p.world, cam.pos, d, ballot(p.valid), best, h, stats);
     if (!p.valid) return;
     const auto &A = kernel_args<RenderArgs>();
@@ -1193,8 +1298,87 @@ __global__ __launch_bounds__(256, BLOCKS) void render_persistent_kernel(const Re
     take_tiles(A.tile_counters, A.total_tiles, [&](const long long tile) { render_tile<WALK>(L, tile); });
 }
 
-__global__ void zero_counters_kernel(int *c) {
-    if (threadIdx.x < 8 * COUNTER_SLICES) c[threadIdx.x * COUNTER_STRIDE] = 0;
+// The view tables: a wavefront a view and a run of its world's instances. Bound by the copies it writes, about 340 bytes an
+// instance and view (541,000 instances in 4,096 views: 80 us, 2.3 TB/s; the launch it goes before is 6.4 ms and 4 to 5%
+// shorter for them). Node copies hold the lower of a pair of planes as near whatever the node holds, so that a box turned
+// inside out, or one with a plane that is no number, is entered by the rays that entered it before.
+__global__ __launch_bounds__(64) void view_tables_kernel(const ViewTableArgs A, const int runs) {
+    const int first = blockIdx.x * 64 + threadIdx.x, step = gridDim.x * 64;
+    for (int i = first; i < A.counter_sets * 8 * COUNTER_SLICES; i += step) A.counters[(size_t)i * COUNTER_STRIDE] = 0;
+    if (A.t.cams == nullptr) return;
+    const int columns = A.width + PIXEL_PAD;
+    for (int i = first; i < columns + A.height + PIXEL_PAD; i += step)
+        A.t.pixels[i] = i < columns ? plane_x((float)i + 0.5f, A.width, A.fov_scale, A.aspect)
+                                    : plane_y((float)(i - columns) + 0.5f, A.height, A.fov_scale);
+    const int view = blockIdx.x / runs, run = blockIdx.x % runs;
+    const int world = view / A.cameras_per_world, camera = view - world * A.cameras_per_world;
+    const Cam cam = load_camera(A.cams + 12 * (size_t)view);
+    // The octants of the view's rays: along an axis the directions before normalization are linear over the image, so
+    // the corners tell which signs it has.
+    bool below[3] = {false, false, false}, above[3] = {false, false, false};
+    for (int corner = 0; corner < 4; ++corner) {
+        const float sx = (corner & 1 ? A.aspect : -A.aspect) * A.fov_scale, sy = corner & 2 ? A.fov_scale : -A.fov_scale;
+        const float3 d = add3(add3(mul3(cam.right, sx), mul3(cam.up, sy)), cam.fwd);
+        const float along[3] = {d.x, d.y, d.z};
+        for (int ax = 0; ax < 3; ++ax) {
+            below[ax] |= along[ax] < 0.0f;
+            above[ax] |= !(along[ax] < 0.0f);
+        }
+    }
+    int octants = 0, kept = 0, of_slot = 0;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+        bool seen = kept < VIEW_OCTANTS;
+        for (int ax = 0; ax < 3; ++ax) seen &= (o >> ax) & 1 ? below[ax] : above[ax];
+        octants |= (seen ? kept : 15) << (4 * o);
+        if (seen) of_slot |= o << (4 * kept++);
+    }
+    if (run == 0 && threadIdx.x < 4) {
+        const float3 v = threadIdx.x == 0 ? cam.pos : threadIdx.x == 1 ? cam.right : threadIdx.x == 2 ? cam.up : cam.fwd;
+        A.t.cams[4 * (size_t)view + threadIdx.x] = make_float4(v.x, v.y, v.z, threadIdx.x == 0 ? __int_as_float(octants) : 0.0f);
+    }
+    const int base = A.world_off[world], count = A.world_off[world + 1] - base;
+    const int no_node = A.root_at_end[world] ? 0 : count - 1;  // the world's run of nodes has one unused
+    const size_t at = (size_t)camera * (size_t)A.total;
+    const float origin[3] = {cam.pos.x, cam.pos.y, cam.pos.z};
+    for (int k = run * 64 + threadIdx.x; k < count; k += runs * 64) {
+        const size_t g = (size_t)base + k;
+        if (k != no_node) {
+            const WideNode node = A.tlas_wide[g];
+            float low[3][2], high[3][2];
+            for (int ax = 0; ax < 3; ++ax)
+                for (int side = 0; side < 2; ++side) {
+                    const float p = node.plane[ax][side] - origin[ax], q = node.plane[ax][2 + side] - origin[ax];
+                    low[ax][side] = fminf(p, q);
+                    high[ax][side] = fmaxf(p, q);
+                }
+            for (int slot = 0; slot < kept; ++slot) {
+                const int o = of_slot >> (4 * slot);
+                WideNode n;
+                for (int ax = 0; ax < 3; ++ax)
+                    for (int side = 0; side < 2; ++side) {
+                        const bool down = (o >> ax) & 1;
+                        n.plane[ax][side] = down ? high[ax][side] : low[ax][side];
+                        n.plane[ax][2 + side] = down ? low[ax][side] : high[ax][side];
+                    }
+                n.left = node.left;
+                n.right = node.right;
+                n.left_count = n.right_count = 1;
+                A.t.nodes[VIEW_OCTANTS * at + (size_t)slot * (size_t)A.total + g] = n;
+            }
+        }
+        const InstanceRec rec = A.inst[g];
+        const MeshRoot root = A.mesh_roots[rec.mesh];
+        float4 *const out = A.t.inst + VIEW_INSTANCE_FLOAT4S * (at + g);
+        float lo[3];
+        for (int ax = 0; ax < 3; ++ax) {
+            lo[ax] = dot3(xyz(rec.inv[ax]), cam.pos) + rec.inv[ax].w;
+            out[ax] = make_float4(rec.inv[ax].x, rec.inv[ax].y, rec.inv[ax].z, lo[ax]);
+        }
+        out[3] = make_float4(root.lo[0] - lo[0], root.lo[1] - lo[1], root.lo[2] - lo[2], __int_as_float(root.ref));
+        out[4] = make_float4(root.hi[0] - lo[0], root.hi[1] - lo[1], root.hi[2] - lo[2],
+                             __int_as_float(root.ref < 0 ? root.count : rec.mesh_tris >= A.lane_min_tris ? 1 : 0));
+    }
 }
 
 #ifdef NGX_TRACE_STATS
@@ -1210,11 +1394,11 @@ __global__ __launch_bounds__(256) void render_stats_kernel(const RenderArgs A, i
     const TilePixel p = tile_pixel(A, tile);
     const bool valid = p.valid;
     const int world = p.world;
-    const Cam cam = load_camera(A.cams + 12 * (size_t)p.view);
-    const float3 d = pixel_ray(cam, A.fov_scale, A.aspect, p.x, p.y, A.width, A.height);
+    WaveStats stats;
+    const Cam cam = camera_of(A, p.view, world, stats);
+    const float3 d = pixel_ray_of(A, cam, p.x, p.y);
     float best;
     LaneHit h;
-    WaveStats stats;
     for (int k = 0; k < ST_COUNT; ++k) stats.c[k] = 0;
     stats.add(ST_VALID, popc64(ballot(valid)));
     scene_hit<WALK>(Scene(), L, world, cam.pos, d, ballot(valid), best, h, stats);
@@ -1488,7 +1672,8 @@ template <int WALK>
 __device__ __forceinline__ void rgb_tile(const RgbArgs &G, PairLds *L, const long long tile) {
     const RenderArgs &A = G.r;
     const TilePixel p = tile_pixel(A, tile);
-    const Cam cam = load_camera(A.cams + 12 * (size_t)p.view);
+    ViewOfRays view;
+    const Cam cam = camera_of(A, p.view, p.world, view);
     uint32_t rng = pixel_stream(A, p, G.frame);
     float3 sum = mk3(0.0f, 0.0f, 0.0f);
     for (int sample = 0; sample < G.spp; ++sample) {
@@ -1536,13 +1721,13 @@ template <int WALK>
 __device__ __forceinline__ void rgb_hit_tile(const RgbArgs &G, PairLds *L, const long long tile) {
     const RenderArgs &A = G.r;
     const TilePixel p = tile_pixel(A, tile);
-    const Cam cam = load_camera(A.cams + 12 * (size_t)p.view);
+    CameraRays stats;
+    const Cam cam = camera_of(A, p.view, p.world, stats);
     uint32_t rng = pixel_stream(A, p, G.frame);
     const float jx = rand01(rng), jy = rand01(rng);
     const float3 d = camera_ray_at(cam, A.fov_scale, A.aspect, (float)p.x + jx, (float)p.y + jy, A.width, A.height);
     float best;
     LaneHit h;
-    CameraRays stats;
     const int kind = scene_hit<WALK>(Scene(), L, p.world, cam.pos, d, ballot(p.valid), best, h, stats);
     if (!p.valid) return;
     G.hits[p.index] = make_int4(__float_as_int(best), kind, h.inst, h.tri);
@@ -1562,7 +1747,8 @@ __device__ __forceinline__ ShadeStart shade_start(const RgbArgs &G, const long l
     const RenderArgs &A = G.r;
     ShadeStart q;
     q.p = tile_pixel(A, tile);
-    const Cam cam = load_camera(A.cams + 12 * (size_t)q.p.view);
+    ViewOfRays view;
+    const Cam cam = camera_of(A, q.p.view, q.p.world, view);
     q.rng = pixel_stream(A, q.p, G.frame);
     const float jx = rand01(q.rng), jy = rand01(q.rng);
     q.o = cam.pos;
@@ -1950,13 +2136,33 @@ static int persistent_grid(const int compute_units, const long long tiles) {
     return capped_grid((per_cu * compute_units + 7) / 8 * 8, tiles);
 }
 
+// The persistent hybrid walk by default: where the bottom levels have octant copies it is built for 8 workgroups per compute
+// unit (64 VGPRs, a few spilled), which hide more of each other's waits (4096 mixed worlds 128x128: 6.79 ms at 7, 6.50 at
+// 8; 64x64: 1.119 and 1.088; RGB + depth + ID: 7.40 and 7.24), and where they are too large for them, and their nodes come
+// from further away, for 7 (a deforming mesh of 138,000 triangles: 397 us at 7, 415 at 8).
+static bool eight_blocks(const RenderArgs &a, const int blocks) { return blocks == 0 && a.walk == WALK_HYBRID && a.s.octant_nodes > 0; }
+
+hipError_t launch_view_tables(const ViewTableArgs &a, hipStream_t stream) {
+    if (a.t.cams == nullptr) {
+        if (a.counters == nullptr || a.counter_sets <= 0) return hipSuccess;
+        view_tables_kernel<<<std::min(a.counter_sets * 8 * COUNTER_SLICES / 64, 64), 64, 0, stream>>>(a, 1);
+        return hipGetLastError();
+    }
+    if (a.views < 1 || a.total < 1 || (a.counter_sets > 0 && a.counters == nullptr)) return hipErrorInvalidValue;
+    // a wavefront a view for every 64 instances of the largest world, and no more than fill the chip several times over
+    const int runs = std::max(1, std::min((a.max_count + 63) / 64, 65536 / a.views));
+    if ((long long)a.views * runs > INT32_MAX / 64) return hipErrorInvalidValue;  // thread numbers are 31 bits
+    view_tables_kernel<<<a.views * runs, 64, 0, stream>>>(a, runs);
+    return hipGetLastError();
+}
+
 hipError_t launch_render(const RenderArgs &a, hipStream_t stream, const int compute_units) {
     if (a.total_tiles <= 0) return hipSuccess;
     if (a.tile_counters && compute_units > 0) {
         if (a.total_tiles >= INT32_MAX / 2) return hipErrorInvalidValue;
-        zero_counters_kernel<<<1, 8 * COUNTER_SLICES, 0, stream>>>(a.tile_counters);
 #define NGX_LAUNCH(W, B) render_persistent_kernel<W, B><<<persistent_grid<W, B>(compute_units, a.total_tiles), 256, 0, stream>>>(a)
-        NGX_BY_VARIANT3(a.walk, a.blocks, RENDER_BLOCKS_DEFAULT, 1, 5, 6, 7, NGX_LAUNCH)
+        if (eight_blocks(a, a.blocks)) NGX_LAUNCH(WALK_HYBRID, 8);
+        else NGX_BY_VARIANT3(a.walk, a.blocks, RENDER_BLOCKS_DEFAULT, 1, 5, 6, 7, NGX_LAUNCH)
 #undef NGX_LAUNCH
         return hipGetLastError();
     }
@@ -2012,7 +2218,6 @@ hipError_t launch_rgb(const RgbArgs &a, hipStream_t stream, const int compute_un
     if (a.spp < 1 || a.shade.light_count < 0 || a.shade.light_count > MAX_LIGHTS) return hipErrorInvalidValue;
     if (a.r.tile_counters && compute_units > 0) {
         if (a.r.total_tiles >= INT32_MAX / 2) return hipErrorInvalidValue;
-        zero_counters_kernel<<<1, 8 * COUNTER_SLICES, 0, stream>>>(a.r.tile_counters);
 #define NGX_LAUNCH(W, B) rgb_persistent_kernel<W, B><<<rgb_persistent_grid<W, B>(compute_units, a.r.total_tiles), 256, 0, stream>>>(a)
         NGX_RGB_VARIANT(a.r.walk, a.blocks, NGX_LAUNCH)
 #undef NGX_LAUNCH
@@ -2055,16 +2260,17 @@ hipError_t launch_rgb_two_pass(const RgbArgs &a, const int hit_blocks, hipStream
         a.r.tile_counters == nullptr || compute_units <= 0 || a.r.walk == WALK_LANES || a.r.total_tiles >= INT32_MAX / 2)
         return hipErrorInvalidValue;
     const bool hybrid = a.r.walk == WALK_HYBRID;
-    zero_counters_kernel<<<1, 8 * COUNTER_SLICES, 0, stream>>>(a.r.tile_counters);
 #define NGX_LAUNCH(W, B) rgb_hit_kernel<W, B><<<resident_grid<rgb_hit_kernel<W, B>>(compute_units, a.r.total_tiles), 256, 0, stream>>>(a)
-    switch (hit_blocks ? hit_blocks : RENDER_BLOCKS_DEFAULT) {
+    switch (hit_blocks ? hit_blocks : eight_blocks(a.r, 0) ? 8 : RENDER_BLOCKS_DEFAULT) {
+    case 8: NGX_LAUNCH(WALK_HYBRID, 8); break;
     case 5: if (hybrid) NGX_LAUNCH(WALK_HYBRID, 5); else NGX_LAUNCH(WALK_PACKET, 5); break;
     case 6: if (hybrid) NGX_LAUNCH(WALK_HYBRID, 6); else NGX_LAUNCH(WALK_PACKET, 6); break;
     default: if (hybrid) NGX_LAUNCH(WALK_HYBRID, 7); else NGX_LAUNCH(WALK_PACKET, 7); break;
     }
 #undef NGX_LAUNCH
-    zero_counters_kernel<<<1, 8 * COUNTER_SLICES, 0, stream>>>(a.r.tile_counters);
-#define NGX_LAUNCH(W, B) launch_shade<W, B>(a, stream, compute_units)
+    RgbArgs shade = a;
+    shade.r.tile_counters += TILE_COUNTER_INTS;
+#define NGX_LAUNCH(W, B) launch_shade<W, B>(shade, stream, compute_units)
     switch (a.blocks ? a.blocks : a.shade.light_count == 1 ? SHADE_ONE_LIGHT_BLOCKS_DEFAULT : SHADE_BLOCKS_DEFAULT) {
     case 4: if (hybrid) NGX_LAUNCH(WALK_HYBRID, 4); else NGX_LAUNCH(WALK_PACKET, 4); break;
     case 5: if (hybrid) NGX_LAUNCH(WALK_HYBRID, 5); else NGX_LAUNCH(WALK_PACKET, 5); break;

@@ -1045,3 +1045,39 @@ def test_small_launches_see_what_full_wavefronts_see(gpu, worlds):
     # sums of up to 4096 pixels' terms, grouped otherwise: their rounding, against the largest gradient
     for k in ("gd", "gr"):
         assert np.abs(small[k] - large[k]).max() <= 1e-4 * np.abs(large[k]).max(), k
+
+
+@pytest.mark.parametrize("cameras,spread", [(1, 0.0), (3, 0.0), (1, 1.0), (3, 1.0)])
+def test_views_with_and_without_their_tables(gpu, cameras, spread):
+    """A launch of 4096 tiles or more has its cameras, top levels and instances laid out per view (the top level for four
+    octants of ray directions); one of fewer has not. Cameras that look along the axes and across several octants, inside
+    boxes and out, in ragged worlds of 0 to 6 instances, with the same worlds in both."""
+    import torch
+    from neraulgraphics_amd.batch import BatchRenderer
+    from neraulgraphics_amd.geometry import Instance, make_box, make_icosphere
+    worlds = {1: (4100, 600), 3: (1400, 300)}[cameras]
+    _say(f"view tables: {worlds} worlds of {cameras} cameras of 8x8")
+    rng = np.random.default_rng(3)
+    n, W = 6, worlds[0]
+    counts = rng.integers(0, n + 1, size=W).astype(np.int32)
+    q = rng.normal(size=(W, n, 3, 3))
+    m = np.concatenate([np.linalg.qr(q)[0] * rng.uniform(0.3, 1.5, size=(W, n, 1, 1)), rng.uniform(-3, 3, size=(W, n, 3, 1))], axis=-1)
+    turn = np.eye(3)[:, rng.permuted(np.tile(np.arange(3), (W * cameras, 1)), axis=1)].transpose(1, 0, 2) * rng.choice([-1, 1], size=(W * cameras, 1, 3))
+    if spread:
+        turn = turn @ np.linalg.qr(rng.normal(size=(W * cameras, 3, 3)))[0]
+    c = np.concatenate([turn, rng.uniform(-2, 2, size=(W * cameras, 3, 1))], axis=-1).reshape(-1, 12).astype(np.float32)
+
+    def run(k):
+        r = BatchRenderer(8, 8, k, cameras, meshes=[make_box((1, 1, 1)), make_icosphere(1.0, 2)],
+                          instances=[Instance(i % 2) for i in range(n)], instances_in_world=counts[:k])
+        r.set_instance_transforms(torch.from_numpy(np.ascontiguousarray(m[:k], np.float32)).cuda())
+        cams = c[:k * cameras]
+        seen = [r.render(cams, fov, depth=True, object_ids=True, normals=True) for fov in (0.3, 1.0, 2.6)]
+        return {f"{k} {i}": np.array(v).reshape(-1)[:worlds[1] * cameras * 64 * np.array(v).reshape(-1).size // (len(cams) * 64)]
+                for i, s in enumerate(seen) for k, v in s.items()}
+
+    few, many = run(worlds[1]), run(W)
+    assert sum(np.isfinite(v).sum() for k, v in many.items() if k.startswith("depth")) > 1000
+    # the same arithmetic on the same worlds; only how many rays a wavefront takes may break a tie otherwise
+    for k, v in few.items():
+        assert np.mean(v != many[k]) < 1e-5, k
