@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <cstddef>
 #include <mutex>
+#include <type_traits>
 #include "ngx_kernels.h"
 
 // Partial sums of ngx_pose_backward_depth_noalloc, which allocates nothing: NOALLOC_SCRATCH_FLOATS floats
@@ -112,11 +113,9 @@ enum StatIndex { ST_TLAS_NODES, ST_TLAS_LANES, ST_INSTANCES, ST_INSTANCE_LANES, 
 // The same type also says whether the walk is an occlusion test (kAnyHit): then a ray's limit drops below zero
 // at its first hit, so its lane leaves every box after it and the walk ends as soon as every ray is blocked or
 // done; whether a ray is blocked is all that is read (mesh_dev.h:208-227 stops at the first hit too).
-// kHandoff says whether the hybrid walk may hand thin subtrees to the shared per-lane walk; the RGB kernel, whose
-// registers are already spent on shading, walks without it. kTwoChild says which shared per-lane walk runs: the one
-// testing both children of a node a step (depth, IDs, ray queries, the backward), or the one-box-a-step walk of the
-// skip layout, which needs fewer registers (the RGB kernel, whose spills the other raises: body_worlds RGB 34.7 ->
-// 44.4 ms, where the depth kernel gains 10.1 -> 9.3 ms and the LiDAR query 21.1 -> 16.4 ms).
+// kHandoff says whether the hybrid walk may hand thin subtrees to the shared per-lane walk, and kTwoChild which shared
+// per-lane walk runs: the one testing both children of a node a step, or the one-box-a-step walk of the skip layout, which
+// needs fewer registers and is left for one-pass pictures of full wavefronts.
 struct NoStats {
     static constexpr bool kAnyHit = false, kHandoff = true, kTwoChild = true, kOneOrigin = false;
     __device__ __forceinline__ void add(int, int) {}
@@ -132,17 +131,16 @@ struct CameraRays : ViewOfRays {
     static constexpr bool kAnyHit = false, kHandoff = true, kTwoChild = true, kOneOrigin = true;
     __device__ __forceinline__ void add(int, int) {}
 };
-struct ShadeRays {
+struct OneBoxRays {
     static constexpr bool kAnyHit = false, kHandoff = false, kTwoChild = false, kOneOrigin = false;
     __device__ __forceinline__ void add(int, int) {}
 };
-struct Occlusion {
+struct OneBoxOcclusion {
     static constexpr bool kAnyHit = true, kHandoff = false, kTwoChild = false, kOneOrigin = false;
     __device__ __forceinline__ void add(int, int) {}
 };
-// Shadow rays of the two-pass picture, whose second pass holds no primary walk: the depth kernel's walk, stopping
-// each ray at its first hit (body_worlds RGB + depth + ID 26.9 ms a step with the one-box-a-step walk here, 26.1 so).
-struct OcclusionTwoChild {
+// Shadow rays: the depth kernel's walk, stopping each ray at its first hit.
+struct Occlusion {
     static constexpr bool kAnyHit = true, kHandoff = true, kTwoChild = true, kOneOrigin = false;
     __device__ __forceinline__ void add(int, int) {}
 };
@@ -327,8 +325,8 @@ __device__ __forceinline__ void add_leaf(const Scene S, PairLds *L, int &pairs, 
 // read from the rays' own lanes. So the few rays that enter an instance keep the whole wave busy. Leaves are
 // queued, and their triangles are tested in batches of up to 64 (ray, triangle) pairs once 64 leaves or 64
 // pairs wait, and at the end; after each batch every walking lane re-reads its ray's closest distance. Every
-// node a ray enters is walked by exactly one lane, so each ray's closest hit is its own. (The RGB kernel walks so;
-// the other kernels use the two-child walk further below, which shares its work the same way.)
+// node a ray enters is walked by exactly one lane, so each ray's closest hit is its own. (OneBoxRays walk so;
+// the others use the two-child walk further below, which shares its work the same way.)
 constexpr int SHARE_CAP = SHARE_STACK, LEAF_RING = 256;
 // Queued leaves that trigger a batch of triangle tests (at most 64 pairs a batch; fewer leaves wait for more).
 #ifndef NGX_LEAF_BATCH
@@ -1466,7 +1464,7 @@ __device__ __forceinline__ float light_factor(const float4 q, const float4 dir, 
 }
 
 // Whether anything lies between o and o + max_dist d, for the lanes in live (render_core.h:146-160).
-template <int WALK, class Walk = Occlusion>
+template <int WALK, class Walk>
 __device__ __forceinline__ bool occluded(const Scene S, PairLds *L, const int world, const float3 o, const float3 d,
                                          const uint64_t live, const float max_dist) {
     const bool mine = in_mask(live);
@@ -1668,8 +1666,11 @@ __device__ __forceinline__ void shade_hit(const RgbArgs &G, PairLds *L, const in
 // packet walk, is 3.1 ms at 4 and 4.2 at 6).
 // The packet and hybrid walks' RGB kernels are built at 4, 5, 6 and 7 workgroups per compute unit, the per-lane
 // walk's at 4; the autotuner picks.
-template <int WALK>
+// TWO_CHILD: with the two-child walk below instances (OneBoxRays otherwise).
+template <int WALK, bool TWO_CHILD>
 __device__ __forceinline__ void rgb_tile(const RgbArgs &G, PairLds *L, const long long tile) {
+    using Rays = std::conditional_t<TWO_CHILD, NoStats, OneBoxRays>;
+    using Shadows = std::conditional_t<TWO_CHILD, Occlusion, OneBoxOcclusion>;
     const RenderArgs &A = G.r;
     const TilePixel p = tile_pixel(A, tile);
     ViewOfRays view;
@@ -1686,10 +1687,10 @@ __device__ __forceinline__ void rgb_tile(const RgbArgs &G, PairLds *L, const lon
         for (int depth = 0; ballot(active); ++depth) {
             float best = 0.0f;
             LaneHit h;
-            ShadeRays stats;
+            Rays stats;
             int kind = OBJECT_NONE;
             if (depth <= MAX_BOUNCES) kind = scene_hit<WALK>(Scene(), L, p.world, o, d, ballot(active), best, h, stats);
-            shade_hit<WALK, Occlusion>(G, L, p.world, kind, best, h, active, o, d, rng, radiance, throughput);
+            shade_hit<WALK, Shadows>(G, L, p.world, kind, best, h, active, o, d, rng, radiance, throughput);
         }
         sum = add3(sum, radiance);
     }
@@ -1701,15 +1702,15 @@ __global__ __launch_bounds__(256, BLOCKS) void rgb_kernel(const RgbArgs G) {
     NGX_PAIR_LDS(L);
     const long long tile = wave_tile(G.r.xcd_remap, G.r.total_tiles);
     if (tile >= G.r.total_tiles) return;
-    rgb_tile<WALK>(G, L, tile);
+    rgb_tile<WALK, false>(G, L, tile);
 }
 
 // The same tiles from a fixed grid taking them from the per-XCD slice counters, as the persistent depth
 // kernel does.
-template <int WALK, int BLOCKS>
+template <int WALK, int BLOCKS, bool TWO_CHILD = false>
 __global__ __launch_bounds__(256, BLOCKS) void rgb_persistent_kernel(const RgbArgs G) {
     NGX_PAIR_LDS(L);
-    take_tiles(G.r.tile_counters, G.r.total_tiles, [&](const long long tile) { rgb_tile<WALK>(G, L, tile); });
+    take_tiles(G.r.tile_counters, G.r.total_tiles, [&](const long long tile) { rgb_tile<WALK, TWO_CHILD>(G, L, tile); });
 }
 
 // The picture in two passes, for one sample a pixel where no surface reflects (every reflectivity below
@@ -1780,7 +1781,7 @@ __device__ __forceinline__ void rgb_shade_tile(const RgbArgs &G, PairLds *L, con
     float3 radiance = mk3(0.0f, 0.0f, 0.0f);
     float throughput = 1.0f;
     bool active = q.p.valid;
-    shade_hit<WALK, OcclusionTwoChild>(G, L, q.p.world, q.kind, q.best, q.h, active, q.o, q.d, q.rng, radiance, throughput);
+    shade_hit<WALK, Occlusion>(G, L, q.p.world, q.kind, q.best, q.h, active, q.o, q.d, q.rng, radiance, throughput);
     if (q.p.valid) write_rgb(G, q.p.index, add3(mk3(0.0f, 0.0f, 0.0f), radiance));
 }
 
@@ -1814,7 +1815,7 @@ __device__ __forceinline__ void rgb_shade_one_light_tile(const RgbArgs &G, PairL
     const uint64_t shadow = ballot(need);
     bool blocked = false;
     if (shadow)
-        blocked = occluded<WALK, OcclusionTwoChild>(Scene(), L, q.p.world, offset_origin(point, normal, light_dir), light_dir, shadow,
+        blocked = occluded<WALK, Occlusion>(Scene(), L, q.p.world, offset_origin(point, normal, light_dir), light_dir, shadow,
                                                     light_distance);
     if (q.p.valid) store_rgb(G, q.p.index, need && !blocked ? lit_bytes : dark_bytes);
 }
@@ -2188,11 +2189,12 @@ hipError_t launch_render_stats(const RenderArgs &a, int *out, hipStream_t stream
 }
 #endif
 
-template <int WALK, int BLOCKS>
-static int rgb_persistent_grid(const int compute_units, const long long tiles) {
+
+template <auto KERNEL>
+static int resident_grid(const int compute_units, const long long tiles) {
     static const int per_cu = [] {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, rgb_persistent_kernel<WALK, BLOCKS>, 256, 0) != hipSuccess || n < 1) n = 1;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, KERNEL, 256, 0) != hipSuccess || n < 1) n = 1;
         return n;
     }();
     return capped_grid((per_cu * compute_units + 7) / 8 * 8, tiles);
@@ -2218,8 +2220,15 @@ hipError_t launch_rgb(const RgbArgs &a, hipStream_t stream, const int compute_un
     if (a.spp < 1 || a.shade.light_count < 0 || a.shade.light_count > MAX_LIGHTS) return hipErrorInvalidValue;
     if (a.r.tile_counters && compute_units > 0) {
         if (a.r.total_tiles >= INT32_MAX / 2) return hipErrorInvalidValue;
-#define NGX_LAUNCH(W, B) rgb_persistent_kernel<W, B><<<rgb_persistent_grid<W, B>(compute_units, a.r.total_tiles), 256, 0, stream>>>(a)
-        NGX_RGB_VARIANT(a.r.walk, a.blocks, NGX_LAUNCH)
+#define NGX_LAUNCH(W, B) rgb_persistent_kernel<W, B><<<resident_grid<rgb_persistent_kernel<W, B>>(compute_units, a.r.total_tiles), 256, 0, stream>>>(a)
+        // The two-child walk, built for few workgroups without spills, is the faster one at every size (16 worlds of 40
+        // mirrors at 96x72, 4 samples: 2,215 us with the one-box walk, 1,650 so; 256 worlds 128x128: 3.20 ms and 2.33). But
+        // where two surfaces meet a ray at the same distance the walks may keep different ones (20 of 16.8 M pixels of
+        // 1,024 mirror worlds), so launches of full wavefronts keep the one-box walk's picture.
+        if (a.r.walk == WALK_HYBRID && a.blocks == 0 && a.r.tile_w * a.r.tile_h < 64)
+            rgb_persistent_kernel<WALK_HYBRID, RGB_TWO_CHILD_BLOCKS, true>
+                <<<resident_grid<rgb_persistent_kernel<WALK_HYBRID, RGB_TWO_CHILD_BLOCKS, true>>(compute_units, a.r.total_tiles), 256, 0, stream>>>(a);
+        else NGX_RGB_VARIANT(a.r.walk, a.blocks, NGX_LAUNCH)
 #undef NGX_LAUNCH
         return hipGetLastError();
     }
@@ -2228,16 +2237,6 @@ hipError_t launch_rgb(const RgbArgs &a, hipStream_t stream, const int compute_un
     NGX_RGB_VARIANT(a.r.walk, a.blocks, NGX_LAUNCH)
 #undef NGX_LAUNCH
     return hipGetLastError();
-}
-
-template <auto KERNEL>
-static int resident_grid(const int compute_units, const long long tiles) {
-    static const int per_cu = [] {
-        int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, KERNEL, 256, 0) != hipSuccess || n < 1) n = 1;
-        return n;
-    }();
-    return capped_grid((per_cu * compute_units + 7) / 8 * 8, tiles);
 }
 
 // The two-pass picture, persistent launches of the packet and hybrid walks only: the hit pass built like the depth
