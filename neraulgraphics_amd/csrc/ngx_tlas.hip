@@ -10,10 +10,12 @@
 //   place     body pose (FP64, instances.cpp:137-164) -> matrix, inverse (cuda_tlas.cuh:35-47),
 //             8-corner world box, the world's centre bounds (cuda_tlas.cuh:69-96)
 //   keys      30-bit Morton code of the box centre (cuda_tlas.cuh:99-115)
-//   sort      stable LSD radix sort, 4-bit digits, ranks from wave ballots (multisplit), staged in LDS
+//   sort      stable LSD radix sort, 4-bit digits, ranks from wave ballots (multisplit), staged in LDS; a world of one
+//             wavefront by counting the keys before each
 //   hierarchy Karras 2012 per node, equal keys told apart by their GLOBAL positions exactly as the
 //             reference's common_prefix does (cuda_tlas.cuh:119-124)
-//   boxes     bottom-up union with LDS arrival counters (the fit_boxes climb, cuda_tlas.cuh:179-196)
+//   boxes     bottom-up union with LDS arrival counters (the fit_boxes climb, cuda_tlas.cuh:179-196); in a world of
+//             one wavefront, of the runs of leaves that a node's children cover
 //   write     the reference's node layout at the reference's node indices, plus the 64-byte wide
 //             nodes the tracer reads
 //
@@ -93,14 +95,20 @@ __device__ __forceinline__ void invert_affine(const float *m, float *out) {
     }
 }
 
-__device__ __forceinline__ int wave_min(int v) {
-    for (int o = 32; o >= 1; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-    return v;
+// A wavefront's least and greatest value, every lane active: one DPP instruction a stage, as wave_prefix_sum's, and a lane
+// shifted in from outside the row keeps its own.
+template <class Pick>
+__device__ __forceinline__ int wave_pick(int v, const Pick &pick) {
+    v = pick(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+    v = pick(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xf, 0xf, false));  // row_shr:2
+    v = pick(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xf, 0xf, false));  // row_shr:4
+    v = pick(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xf, 0xf, false));  // row_shr:8
+    v = pick(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    v = pick(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return __builtin_amdgcn_readlane(v, 63);
 }
-__device__ __forceinline__ int wave_max(int v) {
-    for (int o = 32; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-    return v;
-}
+__device__ __forceinline__ int wave_min(const int v) { return wave_pick(v, [](const int x, const int y) { return min(x, y); }); }
+__device__ __forceinline__ int wave_max(const int v) { return wave_pick(v, [](const int x, const int y) { return max(x, y); }); }
 
 // Exclusive scan of data[0 .. count) in place, count <= blockDim.x; wave_tot has one slot per wave.
 __device__ void block_exclusive_scan(int *data, const int count, int *wave_tot) {
@@ -120,6 +128,11 @@ __device__ void block_exclusive_scan(int *data, const int count, int *wave_tot) 
 // Places instance i of world w (global index g): its matrix as given or composed from its body, the
 // inverse the tracer reads, and its world box (the 8 corners of the mesh box, cuda_tlas.cuh:69-96).
 __device__ void place_instance(const TlasBuildArgs &A, const int w, const int i, const int g, float lo[3], float hi[3]) {
+    // the mesh's values first, so their loads, one after another, run beside the pose's
+    const int mesh = A.tmpl_mesh[i];
+    float lb[6];
+    for (int k = 0; k < 6; ++k) lb[k] = A.mesh_bounds[6 * mesh + k];
+    const int mesh_tris = A.mesh_tris[mesh], skip_root = A.mesh_skip_root[mesh];
     float m[12];
     if (A.source == SOURCE_BODIES) {
         const int b = A.body_of_instance[i];
@@ -147,18 +160,16 @@ __device__ void place_instance(const TlasBuildArgs &A, const int w, const int i,
     mo[2] = make_float4(m[8], m[9], m[10], m[11]);
     float inv[12];
     invert_affine(m, inv);
-    const int mesh = A.tmpl_mesh[i];
     InstanceRec rec;
     rec.inv[0] = make_float4(inv[0], inv[1], inv[2], inv[3]);
     rec.inv[1] = make_float4(inv[4], inv[5], inv[6], inv[7]);
     rec.inv[2] = make_float4(inv[8], inv[9], inv[10], inv[11]);
     rec.mesh = mesh;
     rec.tmpl = i;
-    rec.mesh_tris = A.mesh_tris[mesh];
-    rec.skip_root = A.mesh_skip_root[mesh];
+    rec.mesh_tris = mesh_tris;
+    rec.skip_root = skip_root;
     A.inst[g] = rec;
 
-    const float *lb = A.mesh_bounds + 6 * mesh;
     for (int ax = 0; ax < 3; ++ax) { lo[ax] = 1e30f; hi[ax] = -1e30f; }
     for (int corner = 0; corner < 8; ++corner) {
         const float p[3] = {(corner & 1) ? lb[3] : lb[0], (corner & 2) ? lb[4] : lb[1], (corner & 4) ? lb[5] : lb[2]};
@@ -290,6 +301,11 @@ struct BuildShared {
     int world_bounds[6];
 };
 
+// A world's build is a chain of dependent steps; what bounds it is their latency, since even thousands of worlds give a
+// SIMD few wavefronts. Worlds of at most 64 instances, one wavefront each, sort by counting (eight digit passes before) and
+// make boxes of runs of leaves (a climb with an atomic at every node before): one world of 16 13.5 -> 7.7 us, 64 of 32
+// posed by bodies 17.3 -> 11.2, 4,096 of 32 28 -> 19. Both take n or log n steps and as many LDS reads a lane as a
+// wavefront has lanes, so larger worlds keep the passes and the climb.
 template <int MAXN>
 __global__ __launch_bounds__(MAXN) void tlas_build_kernel(const TlasBuildArgs A) {
     __shared__ BuildShared<MAXN> sh;
@@ -334,18 +350,34 @@ __global__ __launch_bounds__(MAXN) void tlas_build_kernel(const TlasBuildArgs A)
     __syncthreads();
 
     // ---- keys
+    uint32_t mine = ~0u;
     if (has) {
         const float lo[3] = {sh.box_lo[0][tid], sh.box_lo[1][tid], sh.box_lo[2][tid]};
         const float hi[3] = {sh.box_hi[0][tid], sh.box_hi[1][tid], sh.box_hi[2][tid]};
         const uint32_t morton = morton_code(lo, hi, sh.world_bounds);
+        mine = morton;
         sh.key[0][tid] = morton;
         sh.val[0][tid] = (uint32_t)tid;
         if (A.dbg_keys) A.dbg_keys[a + tid] = ((uint64_t)w << 32) | morton;
     }
 
     // ---- sort
-    sort_keys<MAXN>(sh.key, sh.val, sh.hist, sh.wave_tot, has);
     // eight passes end in buffer 0
+    if constexpr (MAXN > 64) sort_keys<MAXN>(sh.key, sh.val, sh.hist, sh.wave_tot, has);
+    else {
+        // one wavefront counts, for each of its keys, those that come before it
+        int rank = 0;
+        for (int j = 0; j < n; ++j) {
+            const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, j);
+            rank += other < mine + (j < tid ? 1u : 0u) ? 1 : 0;
+        }
+        __syncthreads();
+        if (has) {
+            sh.key[0][rank] = mine;
+            sh.val[0][rank] = (uint32_t)tid;
+        }
+        __syncthreads();
+    }
     const uint32_t *key = sh.key[0];
     const uint32_t *val = sh.val[0];
     if (has) {
@@ -371,8 +403,8 @@ __global__ __launch_bounds__(MAXN) void tlas_build_kernel(const TlasBuildArgs A)
     for (int i = tid; i < 2 * n - 1; i += MAXN) sh.parent[i] = -1;
     if (tid < n - 1) sh.arrivals[tid] = 0;
     __syncthreads();
+    int l = 0, r = 0, first = 0, last = 0;
     if (tid < n - 1) {
-        int l, r, first, last;
         karras_node(tid, n, a, key, l, r, first, last);
         sh.left[tid] = l;
         sh.right[tid] = r;
@@ -381,7 +413,53 @@ __global__ __launch_bounds__(MAXN) void tlas_build_kernel(const TlasBuildArgs A)
     }
     __syncthreads();
 
-    // ---- boxes, bottom up: the second of two children to arrive at a node computes its box
+    // ---- boxes
+    const int root_index = A.root_at_end[w] ? a + n - 1 : a;
+    if constexpr (MAXN <= 64) {
+        // One wavefront: a node's children cover the leaves first .. split and split + 1 .. last, and each is the union of
+        // two runs of 2^k leaves. The unions of all runs of 2^k leaves are made for one k after another, in the place of
+        // the leaves' boxes, and each child taken as its k comes up: six steps at most, whatever the tree's depth.
+        float box[6], child[2][6];
+        const int id = has ? (int)val[tid] : 0;
+        for (int ax = 0; ax < 3; ++ax) {
+            box[ax] = sh.box_lo[ax][id];
+            box[3 + ax] = sh.box_hi[ax][id];
+        }
+        __syncthreads();
+        const int split = l >= n - 1 ? l - (n - 1) : l;
+        const int from[2] = {first, split + 1}, to[2] = {split, last};
+        for (int k = 0; (1 << k) < n; ++k) {
+            for (int ax = 0; ax < 3; ++ax) {
+                sh.box_lo[ax][tid] = box[ax];
+                sh.box_hi[ax][tid] = box[3 + ax];
+            }
+            __syncthreads();
+            for (int c = 0; c < 2; ++c) {
+                const int length = to[c] - from[c] + 1;
+                if (tid < n - 1 && (length >> k) == 1) {
+                    const int other = to[c] + 1 - (1 << k);
+                    for (int ax = 0; ax < 3; ++ax) {
+                        child[c][ax] = fminf(sh.box_lo[ax][from[c]], sh.box_lo[ax][other]);
+                        child[c][3 + ax] = fmaxf(sh.box_hi[ax][from[c]], sh.box_hi[ax][other]);
+                    }
+                }
+            }
+            const int next = min(tid + (1 << k), n - 1);
+            for (int ax = 0; ax < 3; ++ax) {
+                box[ax] = fminf(box[ax], sh.box_lo[ax][next]);
+                box[3 + ax] = fmaxf(box[3 + ax], sh.box_hi[ax][next]);
+            }
+            __syncthreads();
+        }
+        if (tid == 0) A.roots[w] = root_index;
+        if (tid < n - 1) {
+            const int gi = tid == 0 ? root_index : a + tid, parent = sh.parent[tid];
+            write_interior(A, gi, n, a, l, r, child[0], child[1], [&](const int k) { return (int)val[k]; });
+            A.wide_parent[gi] = parent < 0 ? -1 : (parent == 0 ? root_index : a + parent);
+        }
+        return;
+    }
+    // bottom up: the second of two children to arrive at a node computes its box
     if (has) {
         int node = n - 1 + tid;
         while (true) {
@@ -389,7 +467,8 @@ __global__ __launch_bounds__(MAXN) void tlas_build_kernel(const TlasBuildArgs A)
             if (p < 0) break;
             const int prior = __hip_atomic_fetch_add(&sh.arrivals[p], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
             if (prior == 0) break;
-            const int l = sh.left[p], r = sh.right[p];
+            l = sh.left[p];
+            r = sh.right[p];
             for (int ax = 0; ax < 3; ++ax) {
                 const float llo = l >= n - 1 ? sh.box_lo[ax][val[l - (n - 1)]] : sh.node_lo[ax][l];
                 const float lhi = l >= n - 1 ? sh.box_hi[ax][val[l - (n - 1)]] : sh.node_hi[ax][l];
@@ -404,10 +483,11 @@ __global__ __launch_bounds__(MAXN) void tlas_build_kernel(const TlasBuildArgs A)
     __syncthreads();
 
     // ---- write the interior nodes in both layouts
-    const int root_index = A.root_at_end[w] ? a + n - 1 : a;
     if (tid == 0) A.roots[w] = root_index;
     if (tid < n - 1) {
-        const int l = sh.left[tid], r = sh.right[tid], parent = sh.parent[tid];
+        l = sh.left[tid];
+        r = sh.right[tid];
+        const int parent = sh.parent[tid];
         float lbox[6], rbox[6];
         for (int ax = 0; ax < 3; ++ax) {
             lbox[ax] = l >= n - 1 ? sh.box_lo[ax][val[l - (n - 1)]] : sh.node_lo[ax][l];

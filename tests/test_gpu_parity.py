@@ -112,6 +112,23 @@ def test_large_world_builds_at_the_edges_of_their_tiles(gpu, oracle, counts, cro
     _check_build(r, ref, ref["world_off"])
 
 
+@pytest.mark.parametrize("crowded", [False, True], ids=["spread", "crowded"])
+def test_worlds_of_one_wavefront_build_at_every_size(gpu, oracle, crowded):
+    """Worlds of up to 64 instances are built by one wavefront, which sorts by counting and makes a child's box of two
+    runs of 2^k leaves: every size from 0 to 64. Crowded, most keys are equal, so only positions tell them apart."""
+    counts = list(range(65))
+    _say(f"one-wavefront builds, crowded {crowded}")
+    cfg = workloads.scattered(len(counts), max(counts), counts=counts, spread=30.0, width=16, height=16)
+    if crowded:
+        cfg["matrices"] = cfg["matrices"].copy()
+        cfg["matrices"].reshape(len(counts), -1, 12)[:, 5:, 3::4] = np.float32([0.5, -0.25, -20.0])
+    r = workloads.make_renderer(cfg)
+    r.keep_build_intermediates(True)
+    r.set_instance_transforms(cfg["matrices"])
+    ref = forward(cfg, oracle, outputs=())
+    _check_build(r, ref, ref["world_off"])
+
+
 @pytest.mark.parametrize("worlds,per", [(1, 20000), (300, 40)])
 def test_morton_trees_see_what_the_sah_trees_see(gpu, oracle, worlds, per):
     """tests/test_batch.cpp:335-371: 20,000 instances in one world and 300 worlds of 40, rendered through this
