@@ -209,6 +209,7 @@ struct ngx_ctx {
     int rgb_two_pass = 1;
     int compute_units = 0;              // sizes the persistent launch
     int *d_tile_counters = nullptr;     // TILE_COUNTER_SETS sets
+    int counter_set = 0;                // which of the first two the next persistent launch takes; it is zero
     char *d_view_tables = nullptr;      // ViewTables' arrays, in d_wide's allocation after the nodes, or null
     int *d_overflow = nullptr;          // set by a walk whose stack would pass its capacity; read by ngx_synchronize
 
@@ -316,7 +317,26 @@ struct ngx_ctx {
         return waves <= 2 * cus ? 8 : waves <= 8 * cus ? 16 : waves <= 24 * cus ? 32 : 64;
     }
     static constexpr int FINE_MESH_TRIANGLES = 10000;
-    static constexpr int TILE_COUNTER_SETS = 3;  // a frame's launches one after the other: depth, hits or RGB, shading
+    // Two sets of tile counters that launches take in turn, each zeroing the other's. A captured launch is replayed with
+    // the set it was captured with, so a captured frame's (depth, hits or RGB, shading) have one each, zeroed in the graph.
+    static constexpr int CAPTURED_COUNTER_SETS = 3, TILE_COUNTER_SETS = 2 + CAPTURED_COUNTER_SETS;
+    int *counters(const int set) const { return d_tile_counters + (size_t)set * ngx::TILE_COUNTER_INTS; }
+    // Before and after a frame's launches. A frame that an error left half launched may have taken a set without the
+    // next being zeroed.
+    bool frame_open = false;
+    void open_frame(const bool captured, hipStream_t s) {
+        if (captured || !persistent) return;
+        if (frame_open) HIP_CHECK(hipMemsetAsync(d_tile_counters, 0, 2 * sizeof(int) * (size_t)ngx::TILE_COUNTER_INTS, s));
+        frame_open = true;
+    }
+    void close_frame() { frame_open = false; }
+    // The counters of a frame's launch number `launch`, and those it zeroes.
+    void take_counters(int *&now, int *&next, const int launch, const bool captured) {
+        now = next = nullptr;
+        if (!persistent) return;
+        now = counters(captured ? 2 + launch : counter_set);
+        next = captured ? nullptr : counters(counter_set ^= 1);
+    }
 
     // The tiles of a picture: `shape` pixels wide and 64 in all, the longer side halved until a tile has `lanes` pixels.
     void set_tiles(ngx::RenderArgs &a, const int lanes, const int shape) const {
@@ -349,7 +369,6 @@ struct ngx_ctx {
         set_tiles(a, 64, tile_w);
         a.xcd_remap = xcd_remap;
         a.walk = walk();
-        a.tile_counters = persistent ? d_tile_counters : nullptr;
         return a;
     }
 
@@ -391,7 +410,7 @@ struct ngx_ctx {
             t.pixels = reinterpret_cast<float *>(p);
             v.t = t;
         }
-        v.counters = d_tile_counters;
+        v.counters = counters(2);
         v.counter_sets = counter_sets;
         v.cams = cams;
         v.views = views;
@@ -558,6 +577,7 @@ ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out) {
         }
         HIP_CHECK(ngx::noalloc_scratch(&c.d_noalloc_scratch));
         device_alloc(c.d_tile_counters, (size_t)ngx_ctx::TILE_COUNTER_SETS * ngx::TILE_COUNTER_INTS);
+        HIP_CHECK(hipMemset(c.d_tile_counters, 0, sizeof(int) * ngx_ctx::TILE_COUNTER_SETS * (size_t)ngx::TILE_COUNTER_INTS));
         device_alloc(c.d_overflow, 1);
         HIP_CHECK(hipMemset(c.d_overflow, 0, sizeof(int)));
         HIP_CHECK(hipEventCreate(&c.ev0));
@@ -713,8 +733,8 @@ ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out) {
                 std::memcpy(&start[12 * (size_t)w * s.instances_per_world], s.instance_transforms, sizeof(float) * 12 * s.instances_per_world);
             HIP_CHECK(hipMemcpy(c.d_matrix_stage, start.data(), start.size() * sizeof(float), hipMemcpyHostToDevice));
             c.build_from_matrices(c.d_matrix_stage, nullptr);
-            HIP_CHECK(hipDeviceSynchronize());
         }
+        HIP_CHECK(hipDeviceSynchronize());
         *out = ctx.release();
     });
 }
@@ -1047,15 +1067,19 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
         }
         const bool timed = !ctx->capturing(s);
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev0, s));
-        ctx->prepare_views(a.tables, cams, fov, a.total_tiles, ctx->persistent ? ngx_ctx::TILE_COUNTER_SETS : 0, s);
-        if (a.depth || a.normal || a.object_id) HIP_CHECK(ngx::launch_render(a, s, ctx->persistent ? ctx->compute_units : 0));
+        ctx->open_frame(!timed, s);
+        ctx->prepare_views(a.tables, cams, fov, a.total_tiles, ctx->persistent && !timed ? ngx_ctx::CAPTURED_COUNTER_SETS : 0, s);
+        if (a.depth || a.normal || a.object_id) {
+            ctx->take_counters(a.tile_counters, a.next_counters, 0, !timed);
+            HIP_CHECK(ngx::launch_render(a, s, ctx->persistent ? ctx->compute_units : 0));
+        }
         if (rgb) {
             ngx::RgbArgs g{};
             g.r = a;
             g.r.depth = nullptr;
             g.r.normal = nullptr;
             g.r.object_id = nullptr;
-            g.r.tile_counters = ctx->persistent ? ctx->d_tile_counters + ngx::TILE_COUNTER_INTS : nullptr;
+            ctx->take_counters(g.r.tile_counters, g.r.next_counters, 1, !timed);
             g.shade = ctx->shade;
             g.rgb = rgb;
             g.spp = spp;
@@ -1070,13 +1094,16 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
             if (two_pass) {
                 g.hits = ctx->d_rgb_hits;
                 g.hit_uv = ctx->d_attrs ? ctx->d_rgb_uv : nullptr;
-                HIP_CHECK(ngx::launch_rgb_two_pass(g, ctx->render_blocks, s, ctx->compute_units));
+                int *shade_counters, *shade_next;
+                ctx->take_counters(shade_counters, shade_next, 2, !timed);
+                HIP_CHECK(ngx::launch_rgb_two_pass(g, ctx->render_blocks, s, ctx->compute_units, shade_counters, shade_next));
             } else {
                 ctx->set_tiles(g.r, ctx->wave_lanes((long long)pixels, true, spp > 1 || !ctx->shade_no_bounce), ctx->tile_w);
                 HIP_CHECK(ngx::launch_rgb(g, s, ctx->persistent ? ctx->compute_units : 0));
             }
             ctx->last_rgb_passes = two_pass ? 2 : 1;
         }
+        if (timed) ctx->close_frame();
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev1, s));
         ctx->timed = timed;
         ctx->last_stream = s;

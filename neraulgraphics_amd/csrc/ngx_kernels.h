@@ -152,7 +152,8 @@ struct RenderArgs {
     int32_t *object_id;        // [views][H][W] or null
     int xcd_remap;             // 1: consecutive tiles stay on one XCD
     int walk;                  // 0 per-lane, 1 packet, 2 packet with fine meshes lane by lane
-    int *tile_counters;        // persistent mode (non-null): TILE_COUNTER_INTS ints, zero (launch_view_tables)
+    int *tile_counters;        // persistent mode (non-null): TILE_COUNTER_INTS ints, zero when the launch begins
+    int *next_counters;        // another set, which the launch zeroes for the next one (or null)
     int blocks;                // the kernel variant: workgroups per compute unit it is built for (0: the walk's default)
 };
 
@@ -326,12 +327,11 @@ struct MeshRefitArgs {
 // One layer of the mesh's treelets, first .. first + count - 1; the layers in order.
 hipError_t launch_mesh_refit(const MeshRefitArgs &a, int first, int count, hipStream_t stream);
 
-// The RGB picture; with a.r.tile_counters set and compute_units > 0, from a persistent grid as launch_render. The
-// two-pass picture takes two sets of counters, one after the other.
+// The RGB picture; with a.r.tile_counters set and compute_units > 0, from a persistent grid as launch_render.
 hipError_t launch_rgb(const RgbArgs &a, hipStream_t stream, int compute_units = 0);
 // One sample a pixel, no surface reflective enough to bounce, persistent launch, packet or hybrid walk: the hit pass,
-// then the shading pass; the same bytes as launch_rgb.
-hipError_t launch_rgb_two_pass(const RgbArgs &a, int hit_blocks, hipStream_t stream, int compute_units);
+// then the shading pass, which takes its tiles from shade_counters and zeroes shade_next; the same bytes as launch_rgb.
+hipError_t launch_rgb_two_pass(const RgbArgs &a, int hit_blocks, hipStream_t stream, int compute_units, int *shade_counters, int *shade_next);
 
 // Zeroes `counter_sets` sets of tile counters (or none, null) and makes the view tables, unless t.cams is null.
 struct ViewTableArgs {

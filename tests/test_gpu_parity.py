@@ -1098,3 +1098,43 @@ def test_views_with_and_without_their_tables(gpu, cameras, spread):
     # the same arithmetic on the same worlds; only how many rays a wavefront takes may break a tie otherwise
     for k, v in few.items():
         assert np.mean(v != many[k]) < 1e-5, k
+
+
+def test_frames_of_one_to_three_launches_in_any_order_and_from_a_graph(gpu):
+    """Persistent launches take their tiles from two sets of counters in turn, each zeroing the other's; a captured frame
+    has sets of its own. Frames of one launch (depth), two (hits, then shading) and three, of one or two samples a pixel,
+    one after the other and between replays of a captured frame of three, are the ones first drawn."""
+    import torch
+    from neraulgraphics_amd.batch import BatchRenderer
+    from neraulgraphics_amd.geometry import Instance, Light, make_icosphere
+    _say("tile counters in turn")
+    W = 40
+    rng = np.random.default_rng(2)
+    r = BatchRenderer(48, 40, W, meshes=[make_icosphere(1.0, 2)], instances=[Instance(0)] * 5, lights=[Light((5.0, 12.0, 6.0))])
+    m = np.tile(np.eye(3, 4, dtype=np.float32), (W, 5, 1, 1))
+    m[..., 3] = rng.uniform(-3, 3, size=(W, 5, 3)) - [0, 0, 6]
+    r.set_instance_transforms(torch.from_numpy(m).cuda())
+    cams = torch.from_numpy(np.tile(np.eye(3, 4, dtype=np.float32).reshape(1, 12), (W, 1))).cuda()
+    frames = [dict(depth=True), dict(rgb=True), dict(rgb=True, depth=True, object_ids=True), dict(rgb=True, samples_per_pixel=2)]
+
+    def draw(k):
+        return r.render(cams, 1.0, zero_copy=True, **frames[k])
+
+    want = []
+    for k in range(4):
+        want.append({n: v.clone() for n, v in draw(k).items()})
+    assert torch.isfinite(want[0]["depth"]).sum() > 1000
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        held = draw(2)
+    for k in rng.integers(0, 5, size=40):
+        if k == 4:
+            for v in held.values():
+                v.zero_()
+            g.replay()
+            got, k = held, 2
+        else:
+            got = draw(int(k))
+        for n, v in want[k].items():
+            assert torch.equal(got[n], v), (int(k), n)
