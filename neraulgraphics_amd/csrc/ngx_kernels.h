@@ -255,11 +255,18 @@ struct PoseGradFinishArgs {
 constexpr int RENDER_BLOCKS[] = {5, 6, 7}, RENDER_BLOCKS_DEFAULT = 7;
 constexpr int RGB_BLOCKS[] = {4, 5, 6, 7}, RGB_BLOCKS_DEFAULT_PACKET = 4, RGB_BLOCKS_DEFAULT_HYBRID = 7, RGB_TWO_CHILD_BLOCKS = 4;
 // The two-pass picture's shading pass by default: 4 workgroups per compute unit, the build without spills (the reference's
-// falling-bodies scene, hybrid walk: 4.97 ms a frame for 32 bodies at 128x128 against 5.84 at 5), and 5 for the build
-// for one light, which holds less across its shadow walk (the same scene: 4.75 ms at 5, 5.01 at 4, 4.86 at 6)
-constexpr int SHADE_BLOCKS_DEFAULT = 4, SHADE_ONE_LIGHT_BLOCKS_DEFAULT = 5;
+// falling-bodies scene, hybrid walk: 4.97 ms a frame for 32 bodies at 128x128 against 5.84 at 5). The build for one light,
+// which holds less across its shadow walk: 6 where worlds have SHADE_MANY_INSTANCES or more on average, whose shadow walks
+// are long and wait for each other's, and 5 below, where the shading around them weighs more and a build of 6 spills in it
+// (1,024 pictures 128x128 of 8, 16, 32, 64, 128 instances: 763, 1043, 1547, 2318, 3617 us at 5, 766, 1029, 1505, 2241, 3471
+// at 6; 4,096 of 8 falling bodies at 64x64 638.6 and 648.9)
+constexpr int SHADE_BLOCKS_DEFAULT = 4, SHADE_ONE_LIGHT_BLOCKS_FEW = 5, SHADE_ONE_LIGHT_BLOCKS_MANY = 6, SHADE_MANY_INSTANCES = 16;
 constexpr int RAY_BLOCKS[] = {5, 6, 7}, RAY_BLOCKS_DEFAULT = 6;
-constexpr int BACKWARD_BLOCKS[] = {4, 5, 6}, BACKWARD_BLOCKS_DEFAULT = 5;
+// The depth backward by default: 6, where its workgroups' LDS (the pair tables and 112 bytes a body) lets 6 run on a compute
+// unit, else 5 (1,024 views 64x64, forward and backward: of 32 bodies 696 us at 5, 654 at 6, 646 at 7; of 64 bodies 1062,
+// 1017 and 1038; 512 views 96x96 of 48 bodies 890, 846 and 865).
+constexpr int BACKWARD_BLOCKS[] = {4, 5, 6}, BACKWARD_BLOCKS_MOST_LDS = 5;
+constexpr int BACKWARD_FEW_BODIES = (160 * 1024 / 6 - 4 * 4608) / 112;
 
 // The pose backward sums gradients per body in LDS: at most this many bodies per world.
 constexpr int BACKWARD_MAX_BODIES = 256;

@@ -255,6 +255,7 @@ struct WaveStack {
     }
 };
 static_assert(WALK_STACK <= 64, "an entry a lane");
+static_assert(sizeof(PairLds) == 4608, "as BACKWARD_FEW_BODIES counts it");
 
 // Tests the queued pairs of instance inst, whose mesh-space ray is (lo, ld) in each ray's lane.
 template <class Stats>
@@ -1986,9 +1987,8 @@ __device__ __forceinline__ void wave_accumulate(const bool has, const int body, 
 
 constexpr int BWD_WAVES = 4;
 
-// 5 workgroups of 4 wavefronts per compute unit (at most 100 VGPRs; posed_bodies forward + backward 746k -> 794k
-// images/s; 6 gives 781k)
-// (built at 4, 5 and 6 for the packet and hybrid walks, the autotuner picking; the per-lane walk's at 5)
+// Built for 4, 5 and 6 workgroups per compute unit (BLOCKS) for the packet and hybrid walks, the autotuner picking, and the
+// per-lane walk's for 5.
 template <int WALK, int BLOCKS>
 __global__ __launch_bounds__(64 * BWD_WAVES, BLOCKS) void depth_backward_kernel(const DepthBackwardArgs A) {
     extern __shared__ float acc_all[];  // [BWD_WAVES][bodies][7]
@@ -2263,6 +2263,7 @@ hipError_t launch_rgb_two_pass(const RgbArgs &a, const int hit_blocks, hipStream
         a.r.tile_counters == nullptr || compute_units <= 0 || a.r.walk == WALK_LANES || a.r.total_tiles >= INT32_MAX / 2)
         return hipErrorInvalidValue;
     const bool hybrid = a.r.walk == WALK_HYBRID;
+    const bool many = (long long)a.r.s.total * a.r.cameras_per_world >= (long long)SHADE_MANY_INSTANCES * a.r.views;
 #define NGX_LAUNCH(W, B) rgb_hit_kernel<W, B><<<resident_grid<rgb_hit_kernel<W, B>>(compute_units, a.r.total_tiles), 256, 0, stream>>>(a)
     switch (hit_blocks ? hit_blocks : eight_blocks(a.r, 0) ? 8 : RENDER_BLOCKS_DEFAULT) {
     case 8: NGX_LAUNCH(WALK_HYBRID, 8); break;
@@ -2275,7 +2276,7 @@ hipError_t launch_rgb_two_pass(const RgbArgs &a, const int hit_blocks, hipStream
     shade.r.tile_counters = shade_counters;
     shade.r.next_counters = shade_next;
 #define NGX_LAUNCH(W, B) launch_shade<W, B>(shade, stream, compute_units)
-    switch (a.blocks ? a.blocks : a.shade.light_count == 1 ? SHADE_ONE_LIGHT_BLOCKS_DEFAULT : SHADE_BLOCKS_DEFAULT) {
+    switch (a.blocks ? a.blocks : a.shade.light_count != 1 ? SHADE_BLOCKS_DEFAULT : many ? SHADE_ONE_LIGHT_BLOCKS_MANY : SHADE_ONE_LIGHT_BLOCKS_FEW) {
     case 4: if (hybrid) NGX_LAUNCH(WALK_HYBRID, 4); else NGX_LAUNCH(WALK_PACKET, 4); break;
     case 5: if (hybrid) NGX_LAUNCH(WALK_HYBRID, 5); else NGX_LAUNCH(WALK_PACKET, 5); break;
     case 6: if (hybrid) NGX_LAUNCH(WALK_HYBRID, 6); else NGX_LAUNCH(WALK_PACKET, 6); break;
@@ -2309,7 +2310,8 @@ hipError_t launch_depth_backward(const DepthBackwardArgs &a, hipStream_t stream)
     if (a.bodies_per_world <= 0 || a.bodies_per_world > BACKWARD_MAX_BODIES) return hipErrorInvalidValue;
     const size_t lds = sizeof(float) * BWD_WAVES * 7 * (size_t)a.bodies_per_world;
 #define NGX_LAUNCH(W, B) depth_backward_kernel<W, B><<<a.views * a.parts, 64 * BWD_WAVES, lds, stream>>>(a)
-    NGX_BY_VARIANT3(a.walk, a.blocks, BACKWARD_BLOCKS_DEFAULT, 5, 4, 5, 6, NGX_LAUNCH)
+    const int blocks = a.bodies_per_world <= BACKWARD_FEW_BODIES ? 6 : BACKWARD_BLOCKS_MOST_LDS;
+    NGX_BY_VARIANT3(a.walk, a.blocks, blocks, 5, 4, 5, 6, NGX_LAUNCH)
 #undef NGX_LAUNCH
     return hipGetLastError();
 }
