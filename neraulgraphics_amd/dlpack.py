@@ -3,11 +3,12 @@
 The capsule's manager keeps its owner (the renderer) alive until the consumer releases the tensor, which
 is how the reference's Python edge hands out its buffers (python/bindings.cpp:192-202)."""
 import ctypes
+import functools
 
 import numpy as np
 
 kDLROCM = 10
-_CODES = {np.dtype(np.float32): (2, 32), np.dtype(np.int32): (0, 32), np.dtype(np.uint8): (1, 8)}
+_CODES = {np.float32: (2, 32), np.int32: (0, 32), np.uint8: (1, 8)}
 
 
 class DLDevice(ctypes.Structure):
@@ -44,25 +45,25 @@ _PyCapsule_New.restype = ctypes.py_object
 _PyCapsule_New.argtypes = [ctypes.c_void_p, ctypes.c_char_p, ctypes.c_void_p]
 
 
+_SHAPE = [ctypes.c_int64 * n for n in range(6)]
+
+
 def capsule(pointer, shape, dtype, device_id, owner):
     """A 'dltensor' capsule viewing `pointer` (device memory) as a C-contiguous array."""
-    code, bits = _CODES[np.dtype(dtype)]
-    shp = (ctypes.c_int64 * len(shape))(*shape)
-    mt = DLManagedTensor()
-    mt.dl_tensor.data = pointer
-    mt.dl_tensor.device = DLDevice(kDLROCM, device_id)
-    mt.dl_tensor.ndim = len(shape)
-    mt.dl_tensor.dtype = DLDataType(code, bits, 1)
-    mt.dl_tensor.shape = shp
-    mt.dl_tensor.strides = None
-    mt.dl_tensor.byte_offset = 0
-    mt.manager_ctx = None
-    mt.deleter = _release
+    code, bits = _CODES.get(dtype) or _CODES[np.dtype(dtype).type]
+    n = len(shape)
+    shp = _SHAPE[n](*shape) if n < len(_SHAPE) else (ctypes.c_int64 * n)(*shape)
+    mt = DLManagedTensor((pointer, (kDLROCM, device_id), n, (code, bits, 1), shp, None, 0), None, _release)
     address = ctypes.addressof(mt)
     _live[address] = (mt, shp, owner)
     return _PyCapsule_New(address, b"dltensor", None)
 
 
-def to_torch(pointer, shape, dtype, device_id, owner):
+@functools.lru_cache(maxsize=None)
+def _from_dlpack():
     from torch.utils.dlpack import from_dlpack
-    return from_dlpack(capsule(pointer, shape, dtype, device_id, owner))
+    return from_dlpack
+
+
+def to_torch(pointer, shape, dtype, device_id, owner):
+    return _from_dlpack()(capsule(pointer, shape, dtype, device_id, owner))
