@@ -301,21 +301,25 @@ struct ngx_ctx {
     // How many rays a wavefront takes. A launch of few wavefronts leaves most of the chip idle, and each of them walks
     // the union of its 64 rays' paths, one dependent node read after the other; with fewer rays a wavefront there are
     // more of them, each walks less, and the lanes without a ray take subtrees off those that have one. Full wavefronts
-    // do the least work in all, so the line is where the chip fills up: lanes by wavefronts of 64 rays per compute unit
-    // (mixed meshes, us a step: 64 wavefronts 86 with 64 lanes, 60 with 8; 1,024: 89, 79 with 8, 74 with 16; 2,048: 145,
-    // 124 with 16; 4,096: 99, 96 with 32; 8,192: 116, 121 with 32). Worlds whose top level is large walk longer (20,000
-    // instances, 84 wavefronts: 600 with 64 lanes, 261 with 8, 208 with 4), and so do paths of several segments and
-    // samples (`deep`; 432 wavefronts: 3,393 with 64, 1,940 with 8, 1,824 with 4; 6,912: 4,550, 4,111 with 32).
-    // Where a ray meets two triangles of one object at the same distance (through their shared edge) it keeps whichever
-    // the wavefront tests first; between full and part wavefronts that differs for one ray in 10^7 to 10^8, but for one
-    // in 10^6 on a mesh of very many small triangles, where outputs that show it (normals) keep to full wavefronts.
-    int wave_lanes(const long long rays, const bool normals, const bool deep) const {
-        if (walk() == 0 || (normals && max_mesh_tris > FINE_MESH_TRIANGLES)) return 64;
+    // do the least work in all (mixed meshes, us a step: 64 wavefronts of 64 rays 86 with 64 lanes, 60 with 8; 1,024: 89, 79
+    // with 8, 74 with 16; 2,048: 145, 124 with 16; 8,192: 116, 121 with 32). Worlds whose top level is large walk longer
+    // (20,000 instances, 84 wavefronts: 600 with 64 lanes, 261 with 8, 208 with 4), and so do paths of several segments and
+    // samples (`paths` above 1; 432 wavefronts: 3,393 with 64, 1,940 with 8, 1,824 with 4).
+    // Where a ray meets two triangles at the same distance (through the edge they share) it keeps whichever the wavefront
+    // tests first, and with fewer rays a wavefront that may be the other one: for one ray in 10^7 or so where the output shows
+    // which triangle it was (`shown`: normals, colours, gradients), in 3 x 10^7 where it shows the object alone, in 10^6 on a
+    // mesh of very many small triangles. So part wavefronts are for launches of so few rays (`paths` times `rays`) that
+    // hardly one of a hundred launches holds such a ray; shadow rays do not count, since whether one is blocked does not
+    // depend on the order.
+    int wave_lanes(const long long rays, const bool shown, const long long paths = 1) const {
+        if (walk() == 0 || (shown && max_mesh_tris > FINE_MESH_TRIANGLES)) return 64;
+        if (rays > (shown ? PART_WAVE_MAX_SHOWN : PART_WAVE_MAX_RAYS) / paths) return 64;
         const long long waves = (rays + 63) / 64, cus = std::max(1, compute_units);
-        if (deep) return waves <= 2 * cus ? 4 : waves <= 8 * cus ? 8 : waves <= 16 * cus ? 16 : waves <= 32 * cus ? 32 : 64;
+        if (paths > 1) return waves <= 2 * cus ? 4 : 8;
         if (max_count > ngx::WORKGROUP_BUILD_MAX && waves <= 2 * cus) return 4;
-        return waves <= 2 * cus ? 8 : waves <= 8 * cus ? 16 : waves <= 24 * cus ? 32 : 64;
+        return waves <= 2 * cus ? 8 : 16;
     }
+    static constexpr long long PART_WAVE_MAX_SHOWN = 65536, PART_WAVE_MAX_RAYS = 131072;
     static constexpr int FINE_MESH_TRIANGLES = 10000;
     // Two sets of tile counters that launches take in turn, each zeroing the other's. A captured launch is replayed with
     // the set it was captured with, so a captured frame's (depth, hits or RGB, shading) have one each, zeroed in the graph.
@@ -1059,7 +1063,7 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
         a.normal = (outputs & NGX_OUTPUT_NORMAL) ? ctx->d_normal : nullptr;
         a.object_id = (outputs & NGX_OUTPUT_OBJECT_ID) ? ctx->d_id : nullptr;
         a.blocks = ctx->render_blocks;
-        ctx->set_tiles(a, ctx->wave_lanes((long long)pixels, (outputs & (NGX_OUTPUT_NORMAL | NGX_OUTPUT_RGB)) != 0, false), ctx->tile_w);
+        ctx->set_tiles(a, ctx->wave_lanes((long long)pixels, (outputs & (NGX_OUTPUT_NORMAL | NGX_OUTPUT_RGB)) != 0), ctx->tile_w);
         uint8_t *rgb = nullptr;
         if (outputs & NGX_OUTPUT_RGB) {
             if (!ctx->d_rgb) device_alloc(ctx->d_rgb, 3 * pixels);
@@ -1098,7 +1102,7 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
                 ctx->take_counters(shade_counters, shade_next, 2, !timed);
                 HIP_CHECK(ngx::launch_rgb_two_pass(g, ctx->render_blocks, s, ctx->compute_units, shade_counters, shade_next));
             } else {
-                ctx->set_tiles(g.r, ctx->wave_lanes((long long)pixels, true, spp > 1 || !ctx->shade_no_bounce), ctx->tile_w);
+                ctx->set_tiles(g.r, ctx->wave_lanes((long long)pixels, true, (ctx->shade_no_bounce ? 1ll : 2ll) * spp), ctx->tile_w);
                 HIP_CHECK(ngx::launch_rgb(g, s, ctx->persistent ? ctx->compute_units : 0));
             }
             ctx->last_rgb_passes = two_pass ? 2 : 1;
@@ -1161,7 +1165,7 @@ ngx_status ngx_cast_rays_batch(ngx_ctx *ctx, const float *origins, const float *
         a.normal = ctx->d_hit_normal;
         a.object_id = ctx->d_hit_id;
         a.walk = ctx->walk_rays();
-        a.lanes = ctx->wave_lanes(count, true, false);
+        a.lanes = ctx->wave_lanes(count, true);
         a.blocks = ctx->ray_blocks;
         const bool timed = !ctx->capturing(s);
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev0, s));
@@ -1198,7 +1202,7 @@ void pose_backward_depth(ngx_ctx *ctx, const float *body_poses, const float *cam
     // enough workgroups to fill the GPU: each view's tiles are split over `parts` workgroups of 4 waves; where there are
     // few views, over as many as there are tiles for, if their partial sums fit
     ngx::RenderArgs grid = ctx->render_args(cams12, fov);
-    ctx->set_tiles(grid, ctx->wave_lanes((long long)ctx->views * ctx->width * ctx->height, true, false), 8);
+    ctx->set_tiles(grid, ctx->wave_lanes((long long)ctx->views * ctx->width * ctx->height, true), 8);
     const int few = std::max(1, std::min(16, ((ctx->width + 7) / 8) * ((ctx->height + 7) / 8) / 8));
     int parts = std::max(few, std::min((grid.tiles_per_view + 3) / 4, 8 * ctx->compute_units / ctx->views));
     if (no_alloc && (size_t)ctx->views * parts * ctx->bodies * 7 > ngx::NOALLOC_SCRATCH_FLOATS) parts = few;
@@ -1282,7 +1286,7 @@ ngx_status ngx_pose_backward_range(ngx_ctx *ctx, const float *body_poses, const 
         const hipStream_t s = static_cast<hipStream_t>(stream);
         const int chunks = std::max(1, std::min(64, rays_per_world / 4096));
         // a chunk's rays are taken in groups of `lanes` from its first on; few chunks are split over more workgroups
-        const int lanes = ctx->wave_lanes((long long)rays_per_world * ctx->worlds, true, false);
+        const int lanes = ctx->wave_lanes((long long)rays_per_world * ctx->worlds, true);
         const int groups = ((rays_per_world + chunks - 1) / chunks + lanes - 1) / lanes;
         const int split = std::max(1, std::min((groups + 3) / 4, (int)(8ll * ctx->compute_units / ((long long)ctx->worlds * chunks))));
         const size_t need = (size_t)ctx->worlds * chunks * split * ctx->bodies * 7;

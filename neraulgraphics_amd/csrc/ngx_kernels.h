@@ -253,7 +253,7 @@ struct PoseGradFinishArgs {
 // The variants each kernel is built in, by workgroups of 256 threads per compute unit (its register budget
 // follows: 512 / (blocks x 4 / 4 SIMDs) registers a lane). 0 in a trace configuration picks the default.
 constexpr int RENDER_BLOCKS[] = {5, 6, 7}, RENDER_BLOCKS_DEFAULT = 7;
-constexpr int RGB_BLOCKS[] = {4, 5, 6, 7}, RGB_BLOCKS_DEFAULT_PACKET = 4, RGB_BLOCKS_DEFAULT_HYBRID = 7, RGB_TWO_CHILD_BLOCKS = 4;
+constexpr int RGB_BLOCKS[] = {4, 5, 6, 7}, RGB_BLOCKS_DEFAULT_PACKET = 4, RGB_BLOCKS_DEFAULT_HYBRID = 7, RGB_TWO_CHILD_BLOCKS = 4, RGB_FEW_INSTANCES = 96;
 // The two-pass picture's shading pass by default: 4 workgroups per compute unit, the build without spills (the reference's
 // falling-bodies scene, hybrid walk: 4.97 ms a frame for 32 bodies at 128x128 against 5.84 at 5). The build for one light,
 // which holds less across its shadow walk: 6 where worlds have SHADE_MANY_INSTANCES or more on average, whose shadow walks

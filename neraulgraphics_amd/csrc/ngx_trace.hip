@@ -135,11 +135,8 @@ struct OneBoxRays {
     static constexpr bool kAnyHit = false, kHandoff = false, kTwoChild = false, kOneOrigin = false;
     __device__ __forceinline__ void add(int, int) {}
 };
-struct OneBoxOcclusion {
-    static constexpr bool kAnyHit = true, kHandoff = false, kTwoChild = false, kOneOrigin = false;
-    __device__ __forceinline__ void add(int, int) {}
-};
-// Shadow rays: the depth kernel's walk, stopping each ray at its first hit.
+// Shadow rays: the two-child walk, stopping each ray at its first hit. Whether a ray is blocked does not depend on the order
+// in which boxes and triangles are tested.
 struct Occlusion {
     static constexpr bool kAnyHit = true, kHandoff = true, kTwoChild = true, kOneOrigin = false;
     __device__ __forceinline__ void add(int, int) {}
@@ -1664,17 +1661,12 @@ __device__ __forceinline__ void shade_hit(const RgbArgs &G, PairLds *L, const in
     }
 }
 
-// Workgroups per compute unit the RGB kernels are compiled for: 4 (16 wavefronts, at most 128 VGPRs) for the
-// packet and per-lane walks, 7 (at most 72 VGPRs, many more spills) for the hybrid walk, whose scenes have more
-// latency to hide (body_worlds RGB: 25.7 ms at 5, 24.3 at 6, 23.5 at 7, 33.0 at 8; the 8-body falling-bodies scene,
-// packet walk, is 3.1 ms at 4 and 4.2 at 6).
 // The packet and hybrid walks' RGB kernels are built at 4, 5, 6 and 7 workgroups per compute unit, the per-lane
 // walk's at 4; the autotuner picks.
-// TWO_CHILD: with the two-child walk below instances (OneBoxRays otherwise).
+// TWO_CHILD: the paths themselves with the two-child walk below instances, as the shadow rays (OneBoxRays otherwise).
 template <int WALK, bool TWO_CHILD>
 __device__ __forceinline__ void rgb_tile(const RgbArgs &G, PairLds *L, const long long tile) {
     using Rays = std::conditional_t<TWO_CHILD, NoStats, OneBoxRays>;
-    using Shadows = std::conditional_t<TWO_CHILD, Occlusion, OneBoxOcclusion>;
     const RenderArgs &A = G.r;
     const TilePixel p = tile_pixel(A, tile);
     ViewOfRays view;
@@ -1694,7 +1686,7 @@ __device__ __forceinline__ void rgb_tile(const RgbArgs &G, PairLds *L, const lon
             Rays stats;
             int kind = OBJECT_NONE;
             if (depth <= MAX_BOUNCES) kind = scene_hit<WALK>(Scene(), L, p.world, o, d, ballot(active), best, h, stats);
-            shade_hit<WALK, Shadows>(G, L, p.world, kind, best, h, active, o, d, rng, radiance, throughput);
+            shade_hit<WALK, Occlusion>(G, L, p.world, kind, best, h, active, o, d, rng, radiance, throughput);
         }
         sum = add3(sum, radiance);
     }
@@ -2203,13 +2195,18 @@ static int resident_grid(const int compute_units, const long long tiles) {
     return capped_grid((per_cu * compute_units + 7) / 8 * 8, tiles);
 }
 
-// The RGB kernels' variants: 4, 5, 6 or 7 workgroups per compute unit for the packet and hybrid walks, 4 for the
-// per-lane walk; defaults 4 for the packet walk and 7 for the hybrid walk.
+// The RGB kernels' variants: 4, 5, 6 or 7 workgroups per compute unit for the packet and hybrid walks, 4 for the per-lane
+// walk; by default 4 for the packet walk, and for the hybrid walk 4, which spills nothing, or 7 in worlds of many instances,
+// whose walks are long and wait for each other's (two or four samples: 64 worlds of 64 mirrors 6.73 ms at 4, 6.75 at 5, 7.29
+// at 7; 256 worlds of 40 instances 2.84, 2.97, 3.07; 1,024 worlds of 256 mirrors 219.7, 201.5, 192.2).
+static int rgb_hybrid_blocks(const RenderArgs &a) {
+    return (long long)a.s.total * a.cameras_per_world > (long long)RGB_FEW_INSTANCES * a.views ? RGB_BLOCKS_DEFAULT_HYBRID : 4;
+}
 #define NGX_RGB_VARIANT(walk, blocks, launch) \
     switch (walk) { \
     case WALK_LANES: launch(WALK_LANES, 4); break; \
     case WALK_HYBRID: \
-        switch (blocks ? blocks : RGB_BLOCKS_DEFAULT_HYBRID) { case 4: launch(WALK_HYBRID, 4); break; \
+        switch (blocks ? blocks : rgb_hybrid_blocks(a.r)) { case 4: launch(WALK_HYBRID, 4); break; \
             case 5: launch(WALK_HYBRID, 5); break; case 6: launch(WALK_HYBRID, 6); break; default: launch(WALK_HYBRID, 7); break; } \
         break; \
     default: \
@@ -2224,10 +2221,9 @@ hipError_t launch_rgb(const RgbArgs &a, hipStream_t stream, const int compute_un
     if (a.r.tile_counters && compute_units > 0) {
         if (a.r.total_tiles >= INT32_MAX / 2) return hipErrorInvalidValue;
 #define NGX_LAUNCH(W, B) rgb_persistent_kernel<W, B><<<resident_grid<rgb_persistent_kernel<W, B>>(compute_units, a.r.total_tiles), 256, 0, stream>>>(a)
-        // The two-child walk, built for few workgroups without spills, is the faster one at every size (16 worlds of 40
-        // mirrors at 96x72, 4 samples: 2,215 us with the one-box walk, 1,650 so; 256 worlds 128x128: 3.20 ms and 2.33). But
-        // where two surfaces meet a ray at the same distance the walks may keep different ones (20 of 16.8 M pixels of
-        // 1,024 mirror worlds), so launches of full wavefronts keep the one-box walk's picture.
+        // Part wavefronts take the two-child walk for the paths too (one world of 8 mirrors at 48x48: 183 us with the one-box
+        // walk, 160 so). Where two surfaces meet a ray at the same distance the walks may keep different ones (20 of 16.8 M
+        // pixels of 1,024 mirror worlds), so launches of full wavefronts keep the one-box walk's.
         if (a.r.walk == WALK_HYBRID && a.blocks == 0 && a.r.tile_w * a.r.tile_h < 64)
             rgb_persistent_kernel<WALK_HYBRID, RGB_TWO_CHILD_BLOCKS, true>
                 <<<resident_grid<rgb_persistent_kernel<WALK_HYBRID, RGB_TWO_CHILD_BLOCKS, true>>(compute_units, a.r.total_tiles), 256, 0, stream>>>(a);
