@@ -314,7 +314,6 @@ hipError_t launch_ray_order(const float *dirs, int rays_per_world, int worlds, u
 // Builds the large worlds with grid-wide kernels; reset_big_bounds readies the bounds for the first build.
 hipError_t launch_tlas_build_big(const TlasBuildArgs &a, const BigBuildScratch &s, hipStream_t stream);
 hipError_t reset_big_bounds(const BigBuildScratch &s, int worlds);
-// The RGB picture of every view, one 64-pixel tile per wavefront.
 // A mesh's bottom level refitted to new vertices (ngx_refit.hip).
 struct MeshRefitArgs {
     const float *vertices;    // the mesh's vertices, 3 floats each

@@ -19,7 +19,8 @@
 // instructions in 8.44 ms: the scalar unit was busy nearly throughout. So the walks are written for few scalar
 // instructions a visit: arguments read where they are used and the walk's pointers once, wave-uniform stacks in vector
 // registers, masked instructions without a branch around them (NGX_LIKELY), lanes that drop out by their limit rather
-// than by a mask, rare cases tested once for the wave. 8.44 -> 6.73 ms there, 13.7 -> 12.7 ms for 67 M LiDAR rays.
+// than by a mask, rare cases tested once for the wave. 8.44 -> 6.3 ms there, now at 4.3 G vector, 2.6 G scalar and 0.57 G
+// branch instructions; 13.7 -> 12.5 ms for 67 M LiDAR rays.
 #include <algorithm>
 #include <cstddef>
 #include <mutex>
@@ -1262,7 +1263,7 @@ __global__ __launch_bounds__(256, BLOCKS) void render_kernel(const RenderArgs A)
 constexpr int PERSISTENT_CHUNK = NGX_PERSISTENT_CHUNK;
 
 // The first workgroup zeroes `next`, the counters of the launch after this one, which spares that launch a kernel to
-// do so before it (a step of one small world: 43 us with one, 40 so).
+// do so before it (a step of one small world: 44.1 us with one, 42.1 so).
 template <class Work>
 __device__ __forceinline__ void take_tiles(int *counters, int *next, const long long total, Work &&work) {
     if (blockIdx.x == 0 && next != nullptr && threadIdx.x < 8 * COUNTER_SLICES) next[threadIdx.x * COUNTER_STRIDE] = 0;
@@ -2239,8 +2240,8 @@ hipError_t launch_rgb(const RgbArgs &a, hipStream_t stream, const int compute_un
 }
 
 // The two-pass picture, persistent launches of the packet and hybrid walks only: the hit pass built like the depth
-// kernel (5, 6 or 7 workgroups per compute unit: hit_blocks, 0 for the default), the shading pass like the RGB
-// kernel (4 to 7: a.blocks, 0 for 4).
+// kernel (5, 6 or 7 workgroups per compute unit: hit_blocks, 0 for the default, 8 as eight_blocks says), the shading pass
+// for 4 to 7 (a.blocks, 0 for the default).
 // The shading pass, built for one light where the scene has one.
 template <int WALK, int BLOCKS>
 static void launch_shade(const RgbArgs &a, hipStream_t stream, const int compute_units) {
