@@ -10,12 +10,12 @@
 //   place     body pose (FP64, instances.cpp:137-164) -> matrix, inverse (cuda_tlas.cuh:35-47),
 //             8-corner world box, the world's centre bounds (cuda_tlas.cuh:69-96)
 //   keys      30-bit Morton code of the box centre (cuda_tlas.cuh:99-115)
-//   sort      stable LSD radix sort, 4-bit digits, ranks from wave ballots (multisplit), staged in LDS; a world of one
-//             wavefront by counting the keys before each
+//   sort      stable LSD radix sort, 4-bit digits, ranks from wave ballots (multisplit), staged in LDS; worlds of
+//             up to 256 instances by counting the keys before each
 //   hierarchy Karras 2012 per node, equal keys told apart by their GLOBAL positions exactly as the
 //             reference's common_prefix does (cuda_tlas.cuh:119-124)
-//   boxes     bottom-up union with LDS arrival counters (the fit_boxes climb, cuda_tlas.cuh:179-196); in a world of
-//             one wavefront, of the runs of leaves that a node's children cover
+//   boxes     bottom-up union with LDS arrival counters (the fit_boxes climb, cuda_tlas.cuh:179-196); in worlds
+//             of up to 256 instances, of the runs of leaves that a node's children cover
 //   write     the reference's node layout at the reference's node indices, plus the 64-byte wide
 //             nodes the tracer reads
 //
@@ -286,12 +286,14 @@ __device__ __forceinline__ void sort_keys(uint32_t (&key)[2][MAXN], uint32_t (&v
     }
 }
 
+constexpr int COUNTED_BUILD_MAX = 256;
+
 template <int MAXN>
 struct BuildShared {
     static constexpr int NW = MAXN / 64;
     float box_lo[3][MAXN], box_hi[3][MAXN];    // instance boxes by template index
     float node_lo[3][MAXN], node_hi[3][MAXN];  // interior nodes by local index
-    uint32_t key[2][MAXN];
+    alignas(16) uint32_t key[2][MAXN];
     uint32_t val[2][MAXN];
     int left[MAXN], right[MAXN], arrivals[MAXN];
     int parent[2 * MAXN];
@@ -302,10 +304,10 @@ struct BuildShared {
 };
 
 // A world's build is a chain of dependent steps; what bounds it is their latency, since even thousands of worlds give a
-// SIMD few wavefronts. Worlds of at most 64 instances, one wavefront each, sort by counting (eight digit passes before) and
-// make boxes of runs of leaves (a climb with an atomic at every node before): one world of 16 13.5 -> 7.7 us, 64 of 32
-// posed by bodies 17.3 -> 11.2, 4,096 of 32 28 -> 19. Both take n or log n steps and as many LDS reads a lane as a
-// wavefront has lanes, so larger worlds keep the passes and the climb.
+// SIMD few wavefronts. Worlds of at most COUNTED_BUILD_MAX instances sort by counting (eight digit passes before) and make
+// boxes of runs of leaves (a climb with an atomic at every node before): one world of 16 13.5 -> 7.7 us, 64 of 32 posed by
+// bodies 17.3 -> 11.2, 4,096 of 32 28 -> 19; a step of one world of 100 85 -> 79, of 200 101 -> 96, of 512 of 128 392 -> 385.
+// Counting takes n steps a key, so larger worlds keep the passes, and the climb.
 template <int MAXN>
 __global__ __launch_bounds__(MAXN) void tlas_build_kernel(const TlasBuildArgs A) {
     __shared__ BuildShared<MAXN> sh;
@@ -363,13 +365,22 @@ __global__ __launch_bounds__(MAXN) void tlas_build_kernel(const TlasBuildArgs A)
 
     // ---- sort
     // eight passes end in buffer 0
-    if constexpr (MAXN > 64) sort_keys<MAXN>(sh.key, sh.val, sh.hist, sh.wave_tot, has);
+    if constexpr (MAXN > COUNTED_BUILD_MAX) sort_keys<MAXN>(sh.key, sh.val, sh.hist, sh.wave_tot, has);
     else {
-        // one wavefront counts, for each of its keys, those that come before it
+        // each thread counts the keys that come before its own: from the wavefront's registers, or from LDS, four at a time
         int rank = 0;
-        for (int j = 0; j < n; ++j) {
-            const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, j);
-            rank += other < mine + (j < tid ? 1u : 0u) ? 1 : 0;
+        if constexpr (MAXN <= 64) {
+            for (int j = 0; j < n; ++j)
+                rank += (uint32_t)__builtin_amdgcn_readlane((int)mine, j) < mine + (j < tid ? 1u : 0u) ? 1 : 0;
+        } else {
+            if (!has) sh.key[0][tid] = ~0u;
+            __syncthreads();
+            const uint4 *const four = reinterpret_cast<const uint4 *>(sh.key[0]);
+            for (int j = 0; j < n; j += 4) {
+                const uint4 other = four[j / 4];
+                rank += (other.x < mine + (j < tid ? 1u : 0u) ? 1 : 0) + (other.y < mine + (j + 1 < tid ? 1u : 0u) ? 1 : 0) +
+                        (other.z < mine + (j + 2 < tid ? 1u : 0u) ? 1 : 0) + (other.w < mine + (j + 3 < tid ? 1u : 0u) ? 1 : 0);
+            }
         }
         __syncthreads();
         if (has) {
@@ -415,10 +426,10 @@ __global__ __launch_bounds__(MAXN) void tlas_build_kernel(const TlasBuildArgs A)
 
     // ---- boxes
     const int root_index = A.root_at_end[w] ? a + n - 1 : a;
-    if constexpr (MAXN <= 64) {
-        // One wavefront: a node's children cover the leaves first .. split and split + 1 .. last, and each is the union of
+    if constexpr (MAXN <= COUNTED_BUILD_MAX) {
+        // A node's children cover the leaves first .. split and split + 1 .. last, and each is the union of
         // two runs of 2^k leaves. The unions of all runs of 2^k leaves are made for one k after another, in the place of
-        // the leaves' boxes, and each child taken as its k comes up: six steps at most, whatever the tree's depth.
+        // the leaves' boxes, and each child taken as its k comes up: eight steps at most, whatever the tree's depth.
         float box[6], child[2][6];
         const int id = has ? (int)val[tid] : 0;
         for (int ax = 0; ax < 3; ++ax) {

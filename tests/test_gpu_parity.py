@@ -112,12 +112,13 @@ def test_large_world_builds_at_the_edges_of_their_tiles(gpu, oracle, counts, cro
     _check_build(r, ref, ref["world_off"])
 
 
+@pytest.mark.parametrize("counts", [list(range(65)), [128, 0, 1, 2, 63, 64, 65, 100, 127], [256, 129, 3, 191, 192, 193, 255, 128, 64]],
+                         ids=["64", "128", "256"])
 @pytest.mark.parametrize("crowded", [False, True], ids=["spread", "crowded"])
-def test_worlds_of_one_wavefront_build_at_every_size(gpu, oracle, crowded):
-    """Worlds of up to 64 instances are built by one wavefront, which sorts by counting and makes a child's box of two
-    runs of 2^k leaves: every size from 0 to 64. Crowded, most keys are equal, so only positions tell them apart."""
-    counts = list(range(65))
-    _say(f"one-wavefront builds, crowded {crowded}")
+def test_worlds_built_by_counting_at_the_edges_of_their_sizes(gpu, oracle, counts, crowded):
+    """Batches of worlds of up to 256 instances sort by counting and make a child's box of two runs of 2^k leaves, in
+    workgroups of 64, 128 and 256. Crowded, most keys are equal, so only positions tell them apart."""
+    _say(f"builds by counting, up to {max(counts)}, crowded {crowded}")
     cfg = workloads.scattered(len(counts), max(counts), counts=counts, spread=30.0, width=16, height=16)
     if crowded:
         cfg["matrices"] = cfg["matrices"].copy()
