@@ -489,7 +489,9 @@ __device__ void walk_shared_two_child(const Scene S, PairLds *L, const int g, in
     int own[WALK_STACK];
     int own_n = 0, own_total = 0;  // the lane's own entries, and the wave's
     const char *const nodes = reinterpret_cast<const char *>(ORDERED ? S.blas_octants() : S.blas_wide());
-    const int share_cap = S.share_cap();
+    // A packet may have given more subtrees (up to SHARE_CAP) than a lowered capacity: what the first step's 64 takers leave
+    // still lies on the shared stack, so its room is never negative.
+    const int share_cap = max(S.share_cap(), top - 64);
     uint64_t busy = 0;
     do {
         if ((top | own_total) != 0 && ~busy != 0) {

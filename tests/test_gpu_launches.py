@@ -1,0 +1,48 @@
+"""What a launch may not depend on: capacities, kernel variants, what other calls of the context ran before it or run
+beside it."""
+import numpy as np
+import pytest
+
+from neraulgraphics_amd import _lib
+from neraulgraphics_amd.batch import BatchRenderer
+from neraulgraphics_amd.geometry import Instance, make_grid, make_icosphere
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(*a):
+    print(*a, flush=True)
+
+
+def _eyes(n, z=0.0):
+    c = np.tile(np.eye(3, 4, dtype=np.float32), (n, 1, 1))
+    c[:, 2, 3] = z
+    return c.reshape(n, 12)
+
+
+@pytest.mark.parametrize("subdivisions,grid,lane_min", [(3, (38, 20), 1400), (5, (200, 75), 25000)],
+                         ids=["with octant copies", "without"])
+def test_packets_that_give_many_subtrees_under_a_lowered_share_capacity(gpu, subdivisions, grid, lane_min):
+    """A mesh below lane_min_triangles is walked as a packet, which gives subtrees that few rays enter to the shared
+    per-lane walk: up to 128 at once, whatever the capacity of its stack. Cut to 1, 3 and 100 entries, images are those of
+    the default capacity."""
+    _say(f"share capacity against a packet's subtrees: {subdivisions} subdivisions")
+    worlds = 40
+    r = BatchRenderer(64, 64, worlds, meshes=[make_icosphere(1.0, subdivisions), make_grid(*grid, 1.0, 1.0, 0.1, seed=3)],
+                      instances=[Instance(0)] * 6 + [Instance(1)])
+    rng = np.random.default_rng(5)
+    m = np.tile(np.eye(3, 4, dtype=np.float32), (worlds, 7, 1, 1))
+    m[..., :3] *= rng.uniform(0.4, 1.2, size=(worlds, 7, 1, 1)).astype(np.float32)
+    m[..., 3] = rng.uniform(-2, 2, size=(worlds, 7, 3)) - [0, 0, 5]
+    r.set_instance_transforms(m)
+    r.set_trace_config(lane_min_triangles=lane_min)
+    want = r.render(_eyes(worlds), 1.0, depth=True, object_ids=True, normals=True)
+    assert np.isfinite(want["depth"]).mean() > 0.2
+    for entries in (1, 3, 100):
+        _lib.check(r._lib.ngx_debug_set_share_capacity(r._h, entries))
+        got = r.render(_eyes(worlds), 1.0, depth=True, object_ids=True, normals=True)
+        r.synchronize()
+        # the same triangles tested in another order: equal but for rays through a shared edge, 1 in 10^6
+        off = {k: int(np.sum(np.asarray(got[k]) != np.asarray(want[k]))) for k in want}
+        _say(f"{entries} entries: values that differ {off}")
+        assert off["depth"] <= 4 and off["object_ids"] <= 4 and off["normals"] <= 12, (entries, off)
