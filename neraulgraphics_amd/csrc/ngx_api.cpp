@@ -97,6 +97,17 @@ void upload(T *&ptr, const T *src, const size_t count) {
     if (count) HIP_CHECK(hipMemcpy(ptr, src, count * sizeof(T), hipMemcpyHostToDevice));
 }
 
+// Whether p is memory of GPU `device` itself, which its kernels may read where it is. A pointer that HIP does not know, or
+// knows as another GPU's or the host's, is not: a copy reaches it whatever a kernel could.
+bool on_device(const void *p, const int device) {
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == device;
+}
+
 template <class T>
 void release(T *&ptr) {
     if (ptr) (void)hipFree(ptr);
@@ -921,9 +932,9 @@ ngx_status ngx_set_mesh_vertices(ngx_ctx *ctx, const int32_t mesh, const float *
         const hipStream_t s = static_cast<hipStream_t>(stream);
         ngx::MeshRefitArgs a{};
         a.vertices = vertices;
-        if (memory == NGX_MEM_HOST) {
+        if (memory == NGX_MEM_HOST || !on_device(vertices, ctx->device)) {
             float *dst = ctx->d_vertices + 3 * (size_t)ctx->mesh_vertex_base[mesh];
-            HIP_CHECK(hipMemcpyAsync(dst, vertices, n * sizeof(float), hipMemcpyHostToDevice, s));
+            HIP_CHECK(hipMemcpyAsync(dst, vertices, n * sizeof(float), memory == NGX_MEM_HOST ? hipMemcpyHostToDevice : hipMemcpyDefault, s));
             a.vertices = dst;
         }
         a.vertex_base = ctx->mesh_vertex_base[mesh];

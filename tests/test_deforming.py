@@ -101,3 +101,59 @@ def test_refits_of_trees_of_one_and_of_several_treelets(gpu, oracle, nx, ny):
     again = r.render(cfg["cameras"], cfg["fov"], depth=True, object_ids=True)
     assert np.array_equal(again["depth"].view(np.uint32), before["depth"].view(np.uint32))
     assert np.array_equal(again["object_ids"], before["object_ids"])
+
+
+def _images_of(r, cfg):
+    r.set_instance_transforms(cfg["matrices"])
+    out = r.render(cfg["cameras"], cfg["fov"], depth=True, object_ids=True)
+    return np.asarray(out["depth"]).view(np.uint32), np.asarray(out["object_ids"])
+
+
+@pytest.mark.parametrize("where", ["pinned host memory", "another GPU"])
+def test_vertices_that_lie_elsewhere_are_copied_first(gpu, where):
+    """Vertices given as device memory that is not the context's GPU's own (pinned host memory, another GPU's) are copied to
+    it before they are read: the images are those of the same vertices on the GPU."""
+    import ctypes
+    import torch
+    from neraulgraphics_amd import _lib
+    if where == "another GPU" and torch.cuda.device_count() < 2:
+        pytest.skip("one GPU")
+    cfg = workloads.make("one_world_icospheres")
+    mesh = cfg["meshes"][0]
+    moved = _wave(mesh)
+    r = workloads.make_renderer(cfg)
+    r.set_mesh_vertices(0, torch.from_numpy(moved).cuda())
+    want = _images_of(r, cfg)
+    r.set_mesh_vertices(0, mesh.vertices)
+    assert not np.array_equal(_images_of(r, cfg)[0], want[0])
+    if where == "another GPU":
+        r.set_mesh_vertices(0, torch.from_numpy(moved).to("cuda:1"))
+    else:
+        held = torch.empty(moved.shape, dtype=torch.float32, pin_memory=True)
+        held.copy_(torch.from_numpy(moved))
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        _lib.check(r._lib.ngx_set_mesh_vertices(r._h, 0, ctypes.c_void_p(held.data_ptr()), _lib.NGX_MEM_DEVICE, stream))
+        torch.cuda.synchronize()
+    got = _images_of(r, cfg)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+def test_a_captured_refit_reads_the_vertices_at_replay(gpu):
+    """A refit captured into a graph with vertices on the GPU reads what they hold when it is replayed."""
+    import torch
+    cfg = workloads.make("one_world_icospheres")
+    mesh = cfg["meshes"][0]
+    r = workloads.make_renderer(cfg)
+    before = _images_of(r, cfg)
+    vertices = torch.from_numpy(_wave(mesh)).cuda()
+    r.set_mesh_vertices(0, vertices)
+    moved = _images_of(r, cfg)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        r.set_mesh_vertices(0, vertices)
+    for values, want in ((mesh.vertices, before), (_wave(mesh), moved), (mesh.vertices, before)):
+        vertices.copy_(torch.from_numpy(np.ascontiguousarray(values)))
+        graph.replay()
+        got = _images_of(r, cfg)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
