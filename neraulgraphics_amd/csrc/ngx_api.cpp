@@ -12,6 +12,7 @@
 #include "../../include/ngx_backend.h"
 #include "ngx_host.h"
 #include "ngx_kernels.h"
+#include "ngx_turns.h"
 
 static_assert(ngx::BACKWARD_MAX_BODIES == NGX_BACKWARD_MAX_BODIES, "the header states the backward's body limit");
 static_assert(ngx::MAX_TRIANGLES == NGX_MAX_TRIANGLES, "the header states the triangle limit");
@@ -220,7 +221,6 @@ struct ngx_ctx {
     int rgb_two_pass = 1;
     int compute_units = 0;              // sizes the persistent launch
     int *d_tile_counters = nullptr;     // TILE_COUNTER_SETS sets
-    int counter_set = 0;                // which of the first two the next persistent launch takes; it is zero
     char *d_view_tables = nullptr;      // ViewTables' arrays, in d_wide's allocation after the nodes, or null
     int *d_overflow = nullptr;          // set by a walk whose stack would pass its capacity; read by ngx_synchronize
 
@@ -336,21 +336,18 @@ struct ngx_ctx {
     // the set it was captured with, so a captured frame's (depth, hits or RGB, shading) have one each, zeroed in the graph.
     static constexpr int CAPTURED_COUNTER_SETS = 3, TILE_COUNTER_SETS = 2 + CAPTURED_COUNTER_SETS;
     int *counters(const int set) const { return d_tile_counters + (size_t)set * ngx::TILE_COUNTER_INTS; }
-    // Before and after a frame's launches. A frame that an error left half launched may have taken a set without the
-    // next being zeroed.
-    bool frame_open = false;
-    void open_frame(const bool captured, hipStream_t s) {
-        if (captured || !persistent) return;
-        if (frame_open) HIP_CHECK(hipMemsetAsync(d_tile_counters, 0, 2 * sizeof(int) * (size_t)ngx::TILE_COUNTER_INTS, s));
-        frame_open = true;
+    ngx::CounterTurns turns;
+    // Before the launches of a frame that takes the two sets in turn.
+    void ready_counters(hipStream_t s) {
+        if (turns.dirty) HIP_CHECK(hipMemsetAsync(d_tile_counters, 0, 2 * sizeof(int) * (size_t)ngx::TILE_COUNTER_INTS, s));
+        turns.dirty = false;
     }
-    void close_frame() { frame_open = false; }
     // The counters of a frame's launch number `launch`, and those it zeroes.
     void take_counters(int *&now, int *&next, const int launch, const bool captured) {
         now = next = nullptr;
         if (!persistent) return;
-        now = counters(captured ? 2 + launch : counter_set);
-        next = captured ? nullptr : counters(counter_set ^= 1);
+        now = counters(captured ? 2 + launch : turns.set);
+        next = captured ? nullptr : counters(turns.set ^= 1);
     }
 
     // The tiles of a picture: `shape` pixels wide and 64 in all, the longer side halved until a tile has `lanes` pixels.
@@ -1082,7 +1079,9 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
         }
         const bool timed = !ctx->capturing(s);
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev0, s));
-        ctx->open_frame(!timed, s);
+        const bool in_turn = timed && ctx->persistent;
+        if (in_turn) ctx->ready_counters(s);
+        ngx::CounterTurns::Frame launches(in_turn ? &ctx->turns : nullptr);
         ctx->prepare_views(a.tables, cams, fov, a.total_tiles, ctx->persistent && !timed ? ngx_ctx::CAPTURED_COUNTER_SETS : 0, s);
         if (a.depth || a.normal || a.object_id) {
             ctx->take_counters(a.tile_counters, a.next_counters, 0, !timed);
@@ -1118,7 +1117,7 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
             }
             ctx->last_rgb_passes = two_pass ? 2 : 1;
         }
-        if (timed) ctx->close_frame();
+        launches.close();
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev1, s));
         ctx->timed = timed;
         ctx->last_stream = s;
