@@ -191,7 +191,9 @@ ngx_status ngx_set_shading(ngx_ctx *ctx, const ngx_shading *shading);
 /* Backend::render_batch (src/backend.h:67-68); checks of src/batch.cpp:146-162. views x 12 camera-to-world
  * floats (OpenGL convention). NGX_OUTPUT_RGB draws the classic picture (spp jittered samples a pixel, seeded
  * by pixel and frame, src/render_core.h:251-263), 3 bytes a pixel; depth, normal and ID do not depend on spp
- * or frame. */
+ * or frame. A context's frames share its scratch memory: one queued on another stream than the last starts when that
+ * is done (but for launches that are not persistent, see ngx_trace_config, which share none). Replays of captured frames
+ * are the caller's to keep from overlapping each other and the context's other frames. */
 ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory, float fov, int32_t spp,
                             uint32_t outputs, int32_t frame, void *stream, ngx_batch_frame *out);
 

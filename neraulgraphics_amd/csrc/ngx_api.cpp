@@ -212,6 +212,7 @@ struct ngx_ctx {
 
     // timing and tuning
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    hipEvent_t timed_until = nullptr;   // what was last timed from ev0 ends here: ev1, or frame_done
     bool timed = false;
     hipStream_t last_stream = nullptr;
     int tile_w = 8, xcd_remap = 1, packet = 1, pair_limit = 64, persistent = 1, lane_min_tris = 300, sort_rays = 1;
@@ -240,6 +241,7 @@ struct ngx_ctx {
         for (void *p : others) if (p) (void)hipFree(p);
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
+        if (frame_done) (void)hipEventDestroy(frame_done);
     }
 
     ngx::TraceScene trace_scene() const {
@@ -337,8 +339,33 @@ struct ngx_ctx {
     static constexpr int CAPTURED_COUNTER_SETS = 3, TILE_COUNTER_SETS = 2 + CAPTURED_COUNTER_SETS;
     int *counters(const int set) const { return d_tile_counters + (size_t)set * ngx::TILE_COUNTER_INTS; }
     ngx::CounterTurns turns;
+    // Frames drawn by persistent launches share these sets, the view tables and the picture's hit records, so one on another
+    // stream than the last waits for it. Its end is an event of its own, since ev1 moves on with other calls.
+    hipEvent_t frame_done = nullptr;
+    hipStream_t frame_stream = nullptr;
+    bool frame_drawn = false;
+    // Where a frame ends on its stream, be it by an error. Null: a frame that shares nothing.
+    struct FrameEnd {
+        ngx_ctx *c;
+        hipStream_t s;
+        FrameEnd(ngx_ctx *ctx, hipStream_t stream) : c(ctx), s(stream) {
+            if (!c) return;
+            c->frame_stream = s;
+            c->frame_drawn = true;
+        }
+        void record() {
+            const ngx_ctx *const ctx = c;
+            c = nullptr;
+            HIP_CHECK(hipEventRecord(ctx->frame_done, s));
+        }
+        ~FrameEnd() {
+            if (c) (void)hipEventRecord(c->frame_done, s);
+        }
+    };
     // Before the launches of a frame that takes the two sets in turn.
-    void ready_counters(hipStream_t s) {
+    void ready_frame(hipStream_t s) {
+        // the per-thread default stream is a different one in every thread
+        if (frame_drawn && (s != frame_stream || s == hipStreamPerThread)) HIP_CHECK(hipStreamWaitEvent(s, frame_done, 0));
         if (turns.dirty) HIP_CHECK(hipMemsetAsync(d_tile_counters, 0, 2 * sizeof(int) * (size_t)ngx::TILE_COUNTER_INTS, s));
         turns.dirty = false;
     }
@@ -395,7 +422,8 @@ struct ngx_ctx {
     // A launch makes them where it gains by them. They cost some 0.15 ns an instance and a few microseconds, and save a
     // wavefront of a full chip a tenth of its instructions: 4096 worlds of 128 instances at 128x128 6.90 -> 6.79 ms, of 32 at
     // 64x64 1.110 -> 1.105, 1,024 lit pictures 7.64 -> 7.40; but one world of 16 (512 tiles) 48.5 -> 49.4 us.
-    // Re-traces of a backward, which are bounded by the forward's depth, do not gain (depth gradient 702 -> 708 us).
+    // Re-traces of a backward, which are bounded by the forward's depth, do not gain (depth gradient 702 -> 708 us). A context
+    // has one set of them, so only persistent launches, which wait for each other, use them: frames of the others may overlap.
     static constexpr size_t VIEW_TABLES_MAX_BYTES = (size_t)1 << 30;
     static constexpr int VIEW_TABLES_MAX_VIEWS = 1 << 22;
     static constexpr long long VIEW_TABLES_MIN_TILES = 4096, VIEW_TABLES_MAX_INSTANCES_PER_TILE = 4;
@@ -411,7 +439,7 @@ struct ngx_ctx {
     // Makes a launch's view tables, where it has some, and zeroes its sets of tile counters.
     void prepare_views(ngx::ViewTables &t, const float *cams, const float fov, const long long tiles, const int counter_sets, hipStream_t s) {
         ngx::ViewTableArgs v{};
-        if (d_view_tables && packet && view_tables_pay(tiles)) {
+        if (d_view_tables && packet && persistent && view_tables_pay(tiles)) {
             char *p = d_view_tables;
             t.cams = reinterpret_cast<float4 *>(p);
             p += 4 * sizeof(float4) * (size_t)views;
@@ -594,6 +622,7 @@ ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out) {
         HIP_CHECK(hipMemset(c.d_overflow, 0, sizeof(int)));
         HIP_CHECK(hipEventCreate(&c.ev0));
         HIP_CHECK(hipEventCreate(&c.ev1));
+        HIP_CHECK(hipEventCreate(&c.frame_done));
 
         if (s.sphere_count > 0) upload(c.d_spheres, reinterpret_cast<const float4 *>(s.spheres), (size_t)s.sphere_count);
         if (c.total > 0) {
@@ -1080,8 +1109,9 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
         const bool timed = !ctx->capturing(s);
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev0, s));
         const bool in_turn = timed && ctx->persistent;
-        if (in_turn) ctx->ready_counters(s);
+        if (in_turn) ctx->ready_frame(s);
         ngx::CounterTurns::Frame launches(in_turn ? &ctx->turns : nullptr);
+        ngx_ctx::FrameEnd end(in_turn ? ctx : nullptr, s);
         ctx->prepare_views(a.tables, cams, fov, a.total_tiles, ctx->persistent && !timed ? ngx_ctx::CAPTURED_COUNTER_SETS : 0, s);
         if (a.depth || a.normal || a.object_id) {
             ctx->take_counters(a.tile_counters, a.next_counters, 0, !timed);
@@ -1118,8 +1148,10 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
             ctx->last_rgb_passes = two_pass ? 2 : 1;
         }
         launches.close();
-        if (timed) HIP_CHECK(hipEventRecord(ctx->ev1, s));
+        if (in_turn) end.record();
+        else if (timed) HIP_CHECK(hipEventRecord(ctx->ev1, s));
         ctx->timed = timed;
+        ctx->timed_until = in_turn ? ctx->frame_done : ctx->ev1;
         ctx->last_stream = s;
         *out = ngx_batch_frame{NGX_MEM_DEVICE, ctx->device, ctx->views, ctx->width, ctx->height, rgb, a.depth, a.normal, a.object_id};
     });
@@ -1190,6 +1222,7 @@ ngx_status ngx_cast_rays_batch(ngx_ctx *ctx, const float *origins, const float *
         HIP_CHECK(ngx::launch_rays(a, s));
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev1, s));
         ctx->timed = timed;
+        ctx->timed_until = ctx->ev1;
         ctx->last_stream = s;
         *out = ngx_ray_hits{NGX_MEM_DEVICE, ctx->device, (int32_t)count, ctx->d_hit_dist, ctx->d_hit_normal, ctx->d_hit_id};
     });
@@ -1263,6 +1296,7 @@ void pose_backward_depth(ngx_ctx *ctx, const float *body_poses, const float *cam
     HIP_CHECK(ngx::launch_depth_backward(a, s));
     if (timed) HIP_CHECK(hipEventRecord(ctx->ev1, s));
     ctx->timed = timed;
+    ctx->timed_until = ctx->ev1;
     ngx::PoseGradFinishArgs f{ctx->worlds, ctx->bodies, ctx->cpw * parts, partial, body_poses, grad_out};
     HIP_CHECK(ngx::launch_pose_grad_finish(f, s));
     ctx->last_stream = s;
@@ -1329,6 +1363,7 @@ ngx_status ngx_pose_backward_range(ngx_ctx *ctx, const float *body_poses, const 
         HIP_CHECK(ngx::launch_range_backward(a, s));
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev1, s));
         ctx->timed = timed;
+        ctx->timed_until = ctx->ev1;
         ngx::PoseGradFinishArgs f{ctx->worlds, ctx->bodies, chunks * split, ctx->d_partial, body_poses, grad_out};
         HIP_CHECK(ngx::launch_pose_grad_finish(f, s));
         ctx->last_stream = s;
@@ -1361,7 +1396,7 @@ ngx_status ngx_synchronize(ngx_ctx *ctx) {
 float ngx_last_kernel_ms(ngx_ctx *ctx) {
     if (!ctx || !ctx->timed) return 0.0f;
     float ms = 0.0f;
-    if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) != hipSuccess) {
+    if (hipEventElapsedTime(&ms, ctx->ev0, ctx->timed_until) != hipSuccess) {
         (void)hipGetLastError();
         return 0.0f;
     }

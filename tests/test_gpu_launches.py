@@ -5,7 +5,7 @@ import pytest
 
 from neraulgraphics_amd import _lib
 from neraulgraphics_amd.batch import BatchRenderer
-from neraulgraphics_amd.geometry import Instance, make_grid, make_icosphere
+from neraulgraphics_amd.geometry import Instance, Light, make_grid, make_icosphere
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +46,38 @@ def test_packets_that_give_many_subtrees_under_a_lowered_share_capacity(gpu, sub
         off = {k: int(np.sum(np.asarray(got[k]) != np.asarray(want[k]))) for k in want}
         _say(f"{entries} entries: values that differ {off}")
         assert off["depth"] <= 4 and off["object_ids"] <= 4 and off["normals"] <= 12, (entries, off)
+
+
+def test_frames_on_several_streams_wait_for_each_other(gpu):
+    """Frames of one context share their tile counters, view tables and hit records: a frame on another stream than the last
+    starts after it, so frames queued on three streams at once with no order between them, and those queued after them, are
+    the ones drawn alone. The same where the launches are not persistent, which share nothing."""
+    import torch
+    _say("frames on three streams")
+    worlds = 600
+    rng = np.random.default_rng(6)
+    r = BatchRenderer(64, 64, worlds, meshes=[make_icosphere(1.0, 2)], instances=[Instance(0)] * 6,
+                      lights=[Light((5.0, 12.0, 6.0), intensity=1.0, radius=0.5)])
+    m = np.tile(np.eye(3, 4, dtype=np.float32), (worlds, 6, 1, 1))
+    m[..., 3] = rng.uniform(-3, 3, size=(worlds, 6, 3)) - [0, 0, 6]
+    r.set_instance_transforms(torch.from_numpy(m).cuda())
+    cams = [torch.from_numpy(_eyes(worlds, z)).cuda() for z in (0.0, 0.4, 0.8)]
+    outputs = [dict(depth=True), dict(normals=True), dict(rgb=True)]  # buffers of their own
+    for persistent in (True, False):
+        r.set_trace_config(persistent=persistent)
+        want = []
+        for k in range(3):
+            want.append({n: v.clone() for n, v in r.render(cams[k], 1.0, zero_copy=True, **outputs[k]).items()})
+            torch.cuda.synchronize()
+        assert torch.isfinite(want[0]["depth"]).sum() > 1000
+        streams = [torch.cuda.Stream() for _ in range(3)]
+        for order in rng.integers(0, 3, size=(12, 5)):
+            got = {}
+            for k in order:
+                with torch.cuda.stream(streams[k]):
+                    got[int(k)] = r.render(cams[k], 1.0, zero_copy=True, **outputs[k])
+            torch.cuda.synchronize()
+            assert r.last_kernel_ms > 0
+            for k, out in got.items():
+                for n, v in want[k].items():
+                    assert torch.equal(out[n], v), (persistent, list(order), k, n)
