@@ -278,7 +278,7 @@ typedef struct {
      * the RGB kernel 4, 5, 6 or 7 (default 4 for the packet walk, 7 for the hybrid one; the two-pass picture's hit pass
      * takes render_blocks and its shading pass rgb_blocks, default 5 for a scene of one light and 4 otherwise), the
      * ray-query kernel 5, 6 or 7 (default 6), the depth backward 4, 5 or 6 (default 5). The per-lane walk has one
-     * variant of each. */
+     * variant of each, and so has the RGB kernel for pictures of few rays, whose wavefronts take 4 to 16 of them. */
     int32_t render_blocks, rgb_blocks, ray_blocks, backward_blocks;
     int32_t rgb_two_pass;
 } ngx_trace_config;

@@ -1696,12 +1696,12 @@ __device__ __forceinline__ void rgb_tile(const RgbArgs &G, PairLds *L, const lon
     if (p.valid) write_rgb(G, p.index, sum);
 }
 
-template <int WALK, int BLOCKS>
+template <int WALK, int BLOCKS, bool TWO_CHILD = false>
 __global__ __launch_bounds__(256, BLOCKS) void rgb_kernel(const RgbArgs G) {
     NGX_PAIR_LDS(L);
     const long long tile = wave_tile(G.r.xcd_remap, G.r.total_tiles);
     if (tile >= G.r.total_tiles) return;
-    rgb_tile<WALK, false>(G, L, tile);
+    rgb_tile<WALK, TWO_CHILD>(G, L, tile);
 }
 
 // The same tiles from a fixed grid taking them from the per-XCD slice counters, as the persistent depth
@@ -2221,13 +2221,15 @@ static int rgb_hybrid_blocks(const RenderArgs &a) {
 hipError_t launch_rgb(const RgbArgs &a, hipStream_t stream, const int compute_units) {
     if (a.r.total_tiles <= 0) return hipSuccess;
     if (a.spp < 1 || a.shade.light_count < 0 || a.shade.light_count > MAX_LIGHTS) return hipErrorInvalidValue;
+    // Part wavefronts take the two-child walk for the paths too (one world of 8 mirrors at 48x48: 183 us with the one-box
+    // walk, 160 so). Where two surfaces meet a ray at the same distance the walks may keep different ones (20 of 16.8 M
+    // pixels of 1,024 mirror worlds), so launches of full wavefronts keep the one-box walk's, and the walk follows from the
+    // tile alone: whatever variant is asked for (a.blocks), part wavefronts have this one build, persistent or not.
+    const bool two_child = a.r.walk == WALK_HYBRID && a.r.tile_w * a.r.tile_h < 64;
     if (a.r.tile_counters && compute_units > 0) {
         if (a.r.total_tiles >= INT32_MAX / 2) return hipErrorInvalidValue;
 #define NGX_LAUNCH(W, B) rgb_persistent_kernel<W, B><<<resident_grid<rgb_persistent_kernel<W, B>>(compute_units, a.r.total_tiles), 256, 0, stream>>>(a)
-        // Part wavefronts take the two-child walk for the paths too (one world of 8 mirrors at 48x48: 183 us with the one-box
-        // walk, 160 so). Where two surfaces meet a ray at the same distance the walks may keep different ones (20 of 16.8 M
-        // pixels of 1,024 mirror worlds), so launches of full wavefronts keep the one-box walk's.
-        if (a.r.walk == WALK_HYBRID && a.blocks == 0 && a.r.tile_w * a.r.tile_h < 64)
+        if (two_child)
             rgb_persistent_kernel<WALK_HYBRID, RGB_TWO_CHILD_BLOCKS, true>
                 <<<resident_grid<rgb_persistent_kernel<WALK_HYBRID, RGB_TWO_CHILD_BLOCKS, true>>(compute_units, a.r.total_tiles), 256, 0, stream>>>(a);
         else NGX_RGB_VARIANT(a.r.walk, a.blocks, NGX_LAUNCH)
@@ -2236,7 +2238,8 @@ hipError_t launch_rgb(const RgbArgs &a, hipStream_t stream, const int compute_un
     }
     const long long blocks = (a.r.total_tiles + 3) / 4;
 #define NGX_LAUNCH(W, B) rgb_kernel<W, B><<<(unsigned)blocks, 256, 0, stream>>>(a)
-    NGX_RGB_VARIANT(a.r.walk, a.blocks, NGX_LAUNCH)
+    if (two_child) rgb_kernel<WALK_HYBRID, RGB_TWO_CHILD_BLOCKS, true><<<(unsigned)blocks, 256, 0, stream>>>(a);
+    else NGX_RGB_VARIANT(a.r.walk, a.blocks, NGX_LAUNCH)
 #undef NGX_LAUNCH
     return hipGetLastError();
 }

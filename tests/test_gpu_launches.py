@@ -5,7 +5,7 @@ import pytest
 
 from neraulgraphics_amd import _lib
 from neraulgraphics_amd.batch import BatchRenderer
-from neraulgraphics_amd.geometry import Instance, Light, make_grid, make_icosphere
+from neraulgraphics_amd.geometry import Instance, Light, Material, Mesh, make_grid, make_icosphere
 
 pytestmark = pytest.mark.gpu
 
@@ -81,3 +81,42 @@ def test_frames_on_several_streams_wait_for_each_other(gpu):
             for k, out in got.items():
                 for n, v in want[k].items():
                     assert torch.equal(out[n], v), (persistent, list(order), k, n)
+
+
+def _two_sheets(n=20):
+    """Two triangulations of one flat square, each with normals of its own: a ray meets both at next to the same distance,
+    so which it keeps shows in the picture."""
+    def sheet(shift, normal):
+        x = np.linspace(-1.0, 1.0, n + 1, dtype=np.float32)
+        x[1:-1] += shift / n
+        g = np.stack(np.meshgrid(x, x, indexing="ij"), axis=-1).reshape(-1, 2)
+        v = np.concatenate([g, np.zeros((len(g), 1), np.float32)], axis=1)
+        i = np.arange((n + 1) * (n + 1)).reshape(n + 1, n + 1)
+        a, b, c, d = i[:-1, :-1].ravel(), i[1:, :-1].ravel(), i[1:, 1:].ravel(), i[:-1, 1:].ravel()
+        t = np.concatenate([np.stack([a, b, c], 1), np.stack([a, c, d], 1)])
+        return v, t, np.tile(np.float32(normal) / np.linalg.norm(normal), (len(v), 1))
+    v0, t0, n0 = sheet(0.0, [0.6, 0.0, 0.8])
+    v1, t1, n1 = sheet(0.9, [0.0, -0.6, 0.8])
+    return Mesh(np.concatenate([v0, v1]).astype(np.float32), np.concatenate([t0, t1 + len(v0)]).astype(np.uint32),
+                np.concatenate([n0, n1]).astype(np.float32))
+
+
+def test_small_pictures_do_not_depend_on_the_kernel_variant_or_the_launch(gpu):
+    """A picture of few rays draws its paths with a walk of its own. Where a ray meets two surfaces at once the walk decides
+    which it keeps, so the variant that is asked for and the kind of launch must not change the walk: the same bytes."""
+    _say("small pictures of mirrors with every RGB variant, persistent and not")
+    r = BatchRenderer(48, 40, 2, meshes=[_two_sheets()], lights=[Light((5.0, 12.0, 6.0), intensity=1.0, radius=0.5)],
+                      instances=[Instance(0, material=Material((0.8, 0.4, 0.3), 0.9, 0.2, 0.3, 40.0))] * 5)
+    rng = np.random.default_rng(8)
+    q = np.linalg.qr(rng.normal(size=(2, 5, 3, 3)))[0]
+    m = np.concatenate([q * 1.5, rng.uniform(-1.5, 1.5, size=(2, 5, 3, 1)) - np.float32([[0], [0], [5]])], axis=-1)
+    r.set_instance_transforms(m.astype(np.float32))
+    pictures = {}
+    for blocks in (0, 4, 5, 6, 7):
+        for persistent in (True, False):
+            r.set_trace_config(rgb_blocks=blocks, persistent=persistent)
+            pictures[blocks, persistent] = np.array(r.render(_eyes(2), 1.0, 2, rgb=True)["rgb"])
+    base = pictures[0, True]
+    assert len(np.unique(base.reshape(-1, 3), axis=0)) > 100
+    for k, v in pictures.items():
+        assert np.array_equal(v, base), k
