@@ -377,6 +377,20 @@ struct ngx_ctx {
         next = captured ? nullptr : counters(turns.set ^= 1);
     }
 
+    // The backwards' partial sums: one set of 7 floats a body for each of `parts` workgroups. Work of few workgroups is split
+    // over up to this many of them, so fewer rays may need more parts than more rays did: what is made for one call holds
+    // every call of less work, which may then be captured into a graph.
+    int split_workgroups() const { return 8 * compute_units; }
+    void hold_partial_sums(const size_t parts, hipStream_t s) {
+        const size_t floats = 7 * (size_t)bodies;
+        if (parts * floats <= partial_cap) return;
+        HIP_CHECK(hipStreamSynchronize(s));
+        partial_cap = 0;
+        const size_t held = std::max(parts, (size_t)split_workgroups()) * floats;
+        device_alloc(d_partial, held);
+        partial_cap = held;
+    }
+
     // The tiles of a picture: `shape` pixels wide and 64 in all, the longer side halved until a tile has `lanes` pixels.
     void set_tiles(ngx::RenderArgs &a, const int lanes, const int shape) const {
         a.tile_w = shape;
@@ -1247,7 +1261,7 @@ void pose_backward_depth(ngx_ctx *ctx, const float *body_poses, const float *cam
     ngx::RenderArgs grid = ctx->render_args(cams12, fov);
     ctx->set_tiles(grid, ctx->wave_lanes((long long)ctx->views * ctx->width * ctx->height, true), 8);
     const int few = std::max(1, std::min(16, ((ctx->width + 7) / 8) * ((ctx->height + 7) / 8) / 8));
-    int parts = std::max(few, std::min((grid.tiles_per_view + 3) / 4, 8 * ctx->compute_units / ctx->views));
+    int parts = std::max(few, std::min((grid.tiles_per_view + 3) / 4, ctx->split_workgroups() / ctx->views));
     if (no_alloc && (size_t)ctx->views * parts * ctx->bodies * 7 > ngx::NOALLOC_SCRATCH_FLOATS) parts = few;
     const size_t need = (size_t)ctx->views * parts * ctx->bodies * 7;
     if (no_alloc)
@@ -1259,11 +1273,7 @@ void pose_backward_depth(ngx_ctx *ctx, const float *body_poses, const float *cam
     const hipStream_t s = static_cast<hipStream_t>(stream);
     float *partial = ctx->d_noalloc_scratch;
     if (!no_alloc) {
-        if (need > ctx->partial_cap) {
-            HIP_CHECK(hipStreamSynchronize(s));
-            device_alloc(ctx->d_partial, need);
-            ctx->partial_cap = need;
-        }
+        ctx->hold_partial_sums((size_t)ctx->views * parts, s);
         partial = ctx->d_partial;
     }
     ctx->build_from_bodies(body_poses, s);
@@ -1332,13 +1342,8 @@ ngx_status ngx_pose_backward_range(ngx_ctx *ctx, const float *body_poses, const 
         // a chunk's rays are taken in groups of `lanes` from its first on; few chunks are split over more workgroups
         const int lanes = ctx->wave_lanes((long long)rays_per_world * ctx->worlds, true);
         const int groups = ((rays_per_world + chunks - 1) / chunks + lanes - 1) / lanes;
-        const int split = std::max(1, std::min((groups + 3) / 4, (int)(8ll * ctx->compute_units / ((long long)ctx->worlds * chunks))));
-        const size_t need = (size_t)ctx->worlds * chunks * split * ctx->bodies * 7;
-        if (need > ctx->partial_cap) {
-            HIP_CHECK(hipStreamSynchronize(s));
-            device_alloc(ctx->d_partial, need);
-            ctx->partial_cap = need;
-        }
+        const int split = std::max(1, std::min((groups + 3) / 4, (int)(ctx->split_workgroups() / ((long long)ctx->worlds * chunks))));
+        ctx->hold_partial_sums((size_t)ctx->worlds * chunks * split, s);
         ctx->build_from_bodies(body_poses, s);
         ngx::RangeBackwardArgs a{};
         a.s = ctx->trace_scene();

@@ -3,7 +3,7 @@ beside it."""
 import numpy as np
 import pytest
 
-from neraulgraphics_amd import _lib
+from neraulgraphics_amd import _lib, workloads
 from neraulgraphics_amd.batch import BatchRenderer
 from neraulgraphics_amd.geometry import Instance, Light, Material, Mesh, make_grid, make_icosphere
 
@@ -120,3 +120,31 @@ def test_small_pictures_do_not_depend_on_the_kernel_variant_or_the_launch(gpu):
     assert len(np.unique(base.reshape(-1, 3), axis=0)) > 100
     for k, v in pictures.items():
         assert np.array_equal(v, base), k
+
+
+def test_range_gradients_of_fewer_rays_under_capture(gpu):
+    """A scan's gradient splits few rays over more workgroups than many, each with its own partial sums: their memory, once
+    made for a call, holds every smaller one, so that it can be captured into a graph."""
+    import torch
+    _say("range gradient of 131,072 rays eagerly, then of fewer under capture")
+    cfg = workloads.make("posed_bodies", worlds=1)
+    r = workloads.make_renderer(cfg)
+    poses = torch.from_numpy(np.ascontiguousarray(cfg["body_poses"])).cuda()
+    rng = np.random.default_rng(4)
+    rays = 131072
+    d = torch.from_numpy((rng.normal(size=(1, rays, 3)) * [0.3, 0.3, 1.0] - [0, 0, 3]).astype(np.float32)).cuda()
+    o = torch.from_numpy(np.broadcast_to(cfg["cameras"].reshape(1, 1, 3, 4)[..., 3], (1, rays, 3)).astype(np.float32)).cuda()
+    dist = r.cast_rays(o, d, 50.0)["distance"].clone()
+    g = torch.from_numpy(rng.normal(size=(1, rays)).astype(np.float32)).cuda()
+    assert torch.isfinite(dist).float().mean() > 0.01
+    r.pose_backward_range(poses, o, d, 50.0, dist, g)
+    torch.cuda.synchronize()
+    few = {n: [a[:, :n].contiguous() for a in (o, d, dist, g)] for n in (65536, 20000, 4096)}
+    for n, (fo, fd, fdist, fg) in few.items():
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = r.pose_backward_range(poses, fo, fd, 50.0, fdist, fg)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = r.pose_backward_range(poses, fo, fd, 50.0, fdist, fg)
+        assert torch.equal(got, want) and want.abs().sum() > 0, n
