@@ -342,6 +342,11 @@ ngx_status ngx_debug_ray_order(int32_t device_id, const float *directions, int32
  * 0 before any), for checking which kernels ran. */
 ngx_status ngx_debug_rgb_passes(const ngx_ctx *ctx, int32_t *passes);
 
+/* No counterpart in the reference: how the last launch was laid out, for checking which of them ran: the rays a wavefront
+ * took in the last depth / normal / ID, RGB, ray-query or backward launch of this context (64, or fewer where the launch
+ * has few; 0 before any), and whether its last render laid out its views' tables first. */
+ngx_status ngx_debug_last_launch(const ngx_ctx *ctx, int32_t *wave_rays, int32_t *view_tables);
+
 /* No counterpart in the reference: how many entries (1 to 128, the default) of the LDS stack on which the shared
  * per-lane bottom-level walk gives far subtrees to idle lanes this context's later calls use; the lanes keep what does
  * not fit on their own stacks. Results do not depend on it (a ray's ties aside); a test lowers it to run that path. */

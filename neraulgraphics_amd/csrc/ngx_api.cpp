@@ -185,6 +185,7 @@ struct ngx_ctx {
     float4 *d_inst_mat = nullptr, *d_sphere_mat = nullptr, *d_lights = nullptr;
     uint8_t *d_rgb = nullptr;
     bool shade_no_bounce = false;       // every surface's reflectivity below the path's cut-off: paths end at their first hit
+    int last_wave_rays = 0, last_view_tables = 0;  // see ngx_debug_last_launch
     int last_rgb_passes = 0;            // how the last RGB picture was drawn: 1 or 2 passes (0 before any)
     int4 *d_rgb_hits = nullptr;         // the two-pass picture's hits, pixels
     float2 *d_rgb_uv = nullptr;         // and their barycentrics (meshes with vertex normals)
@@ -1127,6 +1128,7 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
         ngx::CounterTurns::Frame launches(in_turn ? &ctx->turns : nullptr);
         ngx_ctx::FrameEnd end(in_turn ? ctx : nullptr, s);
         ctx->prepare_views(a.tables, cams, fov, a.total_tiles, ctx->persistent && !timed ? ngx_ctx::CAPTURED_COUNTER_SETS : 0, s);
+        ctx->last_wave_rays = a.tile_w * a.tile_h;
         if (a.depth || a.normal || a.object_id) {
             ctx->take_counters(a.tile_counters, a.next_counters, 0, !timed);
             HIP_CHECK(ngx::launch_render(a, s, ctx->persistent ? ctx->compute_units : 0));
@@ -1157,6 +1159,7 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
                 HIP_CHECK(ngx::launch_rgb_two_pass(g, ctx->render_blocks, s, ctx->compute_units, shade_counters, shade_next));
             } else {
                 ctx->set_tiles(g.r, ctx->wave_lanes((long long)pixels, true, (ctx->shade_no_bounce ? 1ll : 2ll) * spp), ctx->tile_w);
+                ctx->last_wave_rays = g.r.tile_w * g.r.tile_h;
                 HIP_CHECK(ngx::launch_rgb(g, s, ctx->persistent ? ctx->compute_units : 0));
             }
             ctx->last_rgb_passes = two_pass ? 2 : 1;
@@ -1166,6 +1169,7 @@ ngx_status ngx_render_batch(ngx_ctx *ctx, const float *cams12, ngx_memory memory
         else if (timed) HIP_CHECK(hipEventRecord(ctx->ev1, s));
         ctx->timed = timed;
         ctx->timed_until = in_turn ? ctx->frame_done : ctx->ev1;
+        ctx->last_view_tables = a.tables.cams != nullptr ? 1 : 0;
         ctx->last_stream = s;
         *out = ngx_batch_frame{NGX_MEM_DEVICE, ctx->device, ctx->views, ctx->width, ctx->height, rgb, a.depth, a.normal, a.object_id};
     });
@@ -1222,6 +1226,7 @@ ngx_status ngx_cast_rays_batch(ngx_ctx *ctx, const float *origins, const float *
         a.object_id = ctx->d_hit_id;
         a.walk = ctx->walk_rays();
         a.lanes = ctx->wave_lanes(count, true);
+        ctx->last_wave_rays = a.lanes;
         a.blocks = ctx->ray_blocks;
         const bool timed = !ctx->capturing(s);
         if (timed) HIP_CHECK(hipEventRecord(ctx->ev0, s));
@@ -1297,6 +1302,7 @@ void pose_backward_depth(ngx_ctx *ctx, const float *body_poses, const float *cam
     a.tiles_x = grid.tiles_x;
     a.tiles = grid.tiles_per_view;
     a.parts = parts;
+    ctx->last_wave_rays = grid.tile_w * grid.tile_h;
     a.partial = partial;
     a.walk = ctx->walk();
     a.blocks = ctx->backward_blocks;
@@ -1353,6 +1359,7 @@ ngx_status ngx_pose_backward_range(ngx_ctx *ctx, const float *body_poses, const 
         a.chunks = chunks;
         a.split = split;
         a.lanes = lanes;
+        ctx->last_wave_rays = lanes;
         a.walk = ctx->walk_rays();
         a.max_distance = max_distance;
         a.distance = distance;
@@ -1773,6 +1780,14 @@ ngx_status ngx_debug_rgb_passes(const ngx_ctx *ctx, int32_t *passes) {
     return guarded([&] {
         require(ctx != nullptr && passes != nullptr, "context and passes must not be null");
         *passes = ctx->last_rgb_passes;
+    });
+}
+
+ngx_status ngx_debug_last_launch(const ngx_ctx *ctx, int32_t *wave_rays, int32_t *view_tables) {
+    return guarded([&] {
+        require(ctx != nullptr && wave_rays != nullptr && view_tables != nullptr, "context and results must not be null");
+        *wave_rays = ctx->last_wave_rays;
+        *view_tables = ctx->last_view_tables;
     });
 }
 

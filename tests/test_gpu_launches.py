@@ -148,3 +148,127 @@ def test_range_gradients_of_fewer_rays_under_capture(gpu):
         torch.cuda.synchronize()
         want = r.pose_backward_range(poses, fo, fd, 50.0, fdist, fg)
         assert torch.equal(got, want) and want.abs().sum() > 0, n
+
+
+def _last_launch(r):
+    """(rays a wavefront took in the last launch, whether the last render had view tables)"""
+    import ctypes
+    rays, tables = ctypes.c_int32(-1), ctypes.c_int32(-1)
+    _lib.check(r._lib.ngx_debug_last_launch(r._h, ctypes.byref(rays), ctypes.byref(tables)))
+    return rays.value, bool(tables.value)
+
+
+def _wave_rays(rays, shown=False, paths=1):
+    """The rays a wavefront takes, by the limits the launches choose by: up to 131,072 rays, or 65,536 where the triangle
+    shows, over the segments and samples of a path; few enough for two wavefronts of 64 a compute unit or not."""
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    if rays > (65536 if shown else 131072) // paths:
+        return 64
+    few = (rays + 63) // 64 <= 2 * cus
+    return (4 if few else 8) if paths > 1 else (8 if few else 16)
+
+
+MIRRORS = dict(lights=[Light((5.0, 12.0, 6.0), intensity=1.0, radius=0.5)])
+
+
+def _mirror_worlds(full, n, reflectivity):
+    instances = [Instance(i.mesh, i.transform, Material((0.8, 0.5, 0.3), 0.9, 0.2, reflectivity, 40.0)) for i in full["instances"]]
+    r = BatchRenderer(64, 64, n, meshes=full["meshes"], instances=instances, **MIRRORS)
+    r.bind_bodies(full["body_of_instance"], full["local_pose"], full["scale"], full["bodies"])
+    r.set_body_poses(full["body_poses"][:n])
+    return r
+
+
+@pytest.fixture(scope="module")
+def posed_1600(gpu):
+    """1,600 worlds of posed bodies, every launch over them of full wavefronts, and what they look like."""
+    import torch
+    full = workloads.make("posed_bodies", worlds=1600)
+    rng = np.random.default_rng(5)
+    rays = 2000
+    dirs = (rng.normal(size=(1600, rays, 3)) * [0.4, 0.4, 1.0] - [0, 0, 2]).astype(np.float32)
+    origins = np.repeat(full["cameras"].reshape(-1, 3, 4)[:, None, :, 3], rays, axis=1).astype(np.float32)
+    seeds = rng.normal(size=(1600, 64, 64)).astype(np.float32), rng.normal(size=(1600, rays)).astype(np.float32)
+
+    def run(n, kind):
+        up = lambda a: torch.from_numpy(np.ascontiguousarray(a[:n])).cuda()  # noqa: E731
+        cams, poses = up(full["cameras"]), up(full["body_poses"])
+        if kind in ("mirrors", "samples"):
+            r = _mirror_worlds(full, n, 0.3 if kind == "mirrors" else 0.0)
+            rgb = r.render(cams, full["fov"], 1 if kind == "mirrors" else 4, rgb=True, zero_copy=True)["rgb"]
+            return {"rgb": rgb.cpu().numpy()}, _last_launch(r)[0]
+        r = workloads.make_renderer(dict(full, worlds=n, cameras=full["cameras"][:n], body_poses=full["body_poses"][:n]))
+        if kind in ("depth", "normals"):
+            out = r.render(cams, full["fov"], depth=True, object_ids=True, normals=kind == "normals", zero_copy=True)
+        elif kind == "depth gradient":
+            depth = r.render(cams, full["fov"], depth=True, zero_copy=True)["depth"].clone()
+            out = {"gradient": r.pose_backward_depth(poses, cams, full["fov"], depth, up(seeds[0]))}
+        else:
+            o, d = up(origins), up(dirs)
+            out = r.cast_rays(o, d, 50.0)
+            if kind == "range gradient":
+                out = {"gradient": r.pose_backward_range(poses, o, d, 50.0, out["distance"].clone(), up(seeds[1]))}
+        return {k: v.cpu().numpy() for k, v in out.items()}, _last_launch(r)[0]
+
+    large = {}
+
+    def both(n, kind):
+        if kind not in large:
+            large[kind], lanes = run(1600, kind)
+            assert lanes == 64
+        small, lanes = run(n, kind)
+        return small, {k: v[:n] for k, v in large[kind].items()}, lanes
+
+    return both
+
+
+@pytest.mark.parametrize("kind,worlds", [("depth", (1, 8, 9, 31, 32, 33)), ("normals", (8, 9, 16, 17)), ("rays", (1, 16, 17, 32, 33)),
+                                         ("mirrors", (1, 8, 9)), ("samples", (1, 4, 5)), ("depth gradient", (1, 8, 9, 16, 17)),
+                                         ("range gradient", (1, 16, 17, 32, 33))])
+def test_part_wavefronts_either_side_of_their_limits(posed_1600, kind, worlds):
+    """Worlds drawn by launches of 4, 8, 16 and 64 rays a wavefront, on both sides of every limit between them, look as they
+    do in a batch of full wavefronts: the same triangle tests in another order, equal but for ties, of which these meshes
+    show next to none; gradients to the rounding of their sums of up to 4,096 terms in another grouping."""
+    seen = set()
+    for n in worlds:
+        small, large, lanes = posed_1600(n, kind)
+        _say(f"{kind}, {n} worlds: {lanes} rays a wavefront")
+        rays = n * (2000 if kind in ("rays", "range gradient") else 4096)
+        if kind != "depth gradient":
+            assert lanes == _wave_rays(rays, kind != "depth", {"mirrors": 2, "samples": 4}.get(kind, 1)), (kind, n)
+        seen.add(lanes)
+        for k, v in small.items():
+            assert v.shape == large[k].shape and np.abs(large[k]).sum() > 0, k
+            if k == "gradient":
+                assert np.abs(v - large[k]).max() <= 1e-4 * np.abs(large[k]).max(), (kind, n)
+            else:
+                assert np.mean(v != large[k]) < 1e-5, (kind, n, k)
+    assert 64 in seen and len(seen) > 1, seen
+
+
+def test_view_tables_are_made_where_they_should_be(gpu):
+    """Launches of 4,096 tiles or more, of at most four instances and camera a tile, have their views laid out first, others
+    do not, and the worlds both draw are the same: 64 rays a wavefront in both, so bit for bit."""
+    _say("view tables or none")
+    rng = np.random.default_rng(9)
+    n = 5
+    m = np.concatenate([np.linalg.qr(rng.normal(size=(4100, n, 3, 3)))[0] * rng.uniform(0.3, 1.2, size=(4100, n, 1, 1)),
+                        rng.uniform(-3, 3, size=(4100, n, 3, 1)) - [[0], [0], [5]]], axis=-1).astype(np.float32)
+
+    def run(worlds, instances=4, **config):
+        r = BatchRenderer(8, 8, worlds, meshes=[make_icosphere(1.0, 2)], instances=[Instance(0)] * instances)
+        r.set_trace_config(**config)
+        r.set_instance_transforms(m[:worlds, :instances])
+        out = r.render(_eyes(worlds), 1.0, depth=True, object_ids=True)
+        return out, *_last_launch(r)
+
+    many, lanes, tables = run(4100)
+    assert tables and lanes == 64 and np.isfinite(many["depth"]).sum() > 1000
+    few, lanes, tables = run(4090)
+    assert not tables and lanes == 64
+    loose, _, tables = run(4100, persistent=False)
+    assert not tables
+    assert not run(4100, 5)[2]
+    for k, v in many.items():
+        assert np.array_equal(few[k], v[:4090]) and np.array_equal(loose[k], v), k
