@@ -324,7 +324,8 @@ struct ngx_ctx {
     // which triangle it was (`shown`: normals, colours, gradients), in 3 x 10^7 where it shows the object alone, in 10^6 on a
     // mesh of very many small triangles. So part wavefronts are for launches of so few rays (`paths` times `rays`) that
     // hardly one of a hundred launches holds such a ray; shadow rays do not count, since whether one is blocked does not
-    // depend on the order.
+    // depend on the order. A gradient's re-trace is grouped as its forward was, a depth image or a ray query, so that it
+    // meets the triangles that the forward met.
     int wave_lanes(const long long rays, const bool shown, const long long paths = 1) const {
         if (walk() == 0 || (shown && max_mesh_tris > FINE_MESH_TRIANGLES)) return 64;
         if (rays > (shown ? PART_WAVE_MAX_SHOWN : PART_WAVE_MAX_RAYS) / paths) return 64;
@@ -1264,7 +1265,8 @@ void pose_backward_depth(ngx_ctx *ctx, const float *body_poses, const float *cam
     // enough workgroups to fill the GPU: each view's tiles are split over `parts` workgroups of 4 waves; where there are
     // few views, over as many as there are tiles for, if their partial sums fit
     ngx::RenderArgs grid = ctx->render_args(cams12, fov);
-    ctx->set_tiles(grid, ctx->wave_lanes((long long)ctx->views * ctx->width * ctx->height, true), 8);
+    // the rays a wavefront takes are those of a depth image, whose pixels' triangles are then met in the same grouping
+    ctx->set_tiles(grid, ctx->wave_lanes((long long)ctx->views * ctx->width * ctx->height, false), 8);
     const int few = std::max(1, std::min(16, ((ctx->width + 7) / 8) * ((ctx->height + 7) / 8) / 8));
     int parts = std::max(few, std::min((grid.tiles_per_view + 3) / 4, ctx->split_workgroups() / ctx->views));
     if (no_alloc && (size_t)ctx->views * parts * ctx->bodies * 7 > ngx::NOALLOC_SCRATCH_FLOATS) parts = few;

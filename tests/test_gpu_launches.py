@@ -224,7 +224,7 @@ def posed_1600(gpu):
 
 
 @pytest.mark.parametrize("kind,worlds", [("depth", (1, 8, 9, 31, 32, 33)), ("normals", (8, 9, 16, 17)), ("rays", (1, 16, 17, 32, 33)),
-                                         ("mirrors", (1, 8, 9)), ("samples", (1, 4, 5)), ("depth gradient", (1, 8, 9, 16, 17)),
+                                         ("mirrors", (1, 8, 9)), ("samples", (1, 4, 5)), ("depth gradient", (1, 8, 9, 32, 33)),
                                          ("range gradient", (1, 16, 17, 32, 33))])
 def test_part_wavefronts_either_side_of_their_limits(posed_1600, kind, worlds):
     """Worlds drawn by launches of 4, 8, 16 and 64 rays a wavefront, on both sides of every limit between them, look as they
@@ -235,8 +235,7 @@ def test_part_wavefronts_either_side_of_their_limits(posed_1600, kind, worlds):
         small, large, lanes = posed_1600(n, kind)
         _say(f"{kind}, {n} worlds: {lanes} rays a wavefront")
         rays = n * (2000 if kind in ("rays", "range gradient") else 4096)
-        if kind != "depth gradient":
-            assert lanes == _wave_rays(rays, kind != "depth", {"mirrors": 2, "samples": 4}.get(kind, 1)), (kind, n)
+        assert lanes == _wave_rays(rays, not kind.startswith("depth"), {"mirrors": 2, "samples": 4}.get(kind, 1)), (kind, n)
         seen.add(lanes)
         for k, v in small.items():
             assert v.shape == large[k].shape and np.abs(large[k]).sum() > 0, k
@@ -272,3 +271,25 @@ def test_view_tables_are_made_where_they_should_be(gpu):
     assert not run(4100, 5)[2]
     for k, v in many.items():
         assert np.array_equal(few[k], v[:4090]) and np.array_equal(loose[k], v), k
+
+
+@pytest.mark.parametrize("worlds", [1, 9, 16, 17, 32, 33])
+def test_a_gradient_takes_its_rays_as_its_forward_did(gpu, worlds):
+    """Which of two surfaces at one distance a ray keeps depends on the rays it is walked with: a depth image and its
+    gradient's re-trace, a range query and its gradient's, take as many a wavefront, on either side of the limits."""
+    import torch
+    from neraulgraphics_amd.autograd import cast_range, render_depth
+    cfg = workloads.make("posed_bodies", worlds=worlds)
+    r = workloads.make_renderer(cfg)
+    poses = torch.from_numpy(cfg["body_poses"]).cuda().requires_grad_()
+    depth = render_depth(r, poses, torch.from_numpy(cfg["cameras"]).cuda(), cfg["fov"])
+    forward = _last_launch(r)[0]
+    torch.where(torch.isfinite(depth), depth, 0.0).sum().backward()
+    _say(f"{worlds} worlds: {forward} rays a wavefront forward, {_last_launch(r)[0]} backward")
+    assert _last_launch(r)[0] == forward
+    d = torch.randn(worlds, 4096, 3, device="cuda", generator=torch.Generator("cuda").manual_seed(1)) * 0.3 - torch.tensor([0.0, 0.0, 1.0], device="cuda")
+    o = torch.from_numpy(np.repeat(cfg["cameras"].reshape(worlds, 1, 3, 4)[..., 3], 4096, axis=1)).cuda()
+    distance = cast_range(r, poses, o, d, 50.0)
+    forward = _last_launch(r)[0]
+    torch.where(torch.isfinite(distance), distance, 0.0).sum().backward()
+    assert _last_launch(r)[0] == forward
