@@ -2074,30 +2074,36 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void range_backward_kernel(const Ra
 // Sums the parts of each body, then projects the unit-quaternion gradient onto the raw quaternion: d unit / d q =
 // (I - u u^T) / |q|. Eight lanes a body, each taking every eighth part in order, their sums added pairwise: a fixed order.
 constexpr int FINISH_LANES = 8;
+constexpr int FINISH_BODIES = 256 / FINISH_LANES;  // a workgroup's, of as many runs of them as the grid leaves it
+constexpr long long FINISH_MOST_GROUPS = 1 << 22;
 __global__ __launch_bounds__(256) void pose_grad_finish_kernel(const PoseGradFinishArgs A) {
-    const int bodies = A.worlds * A.bodies_per_world;
-    const int i = (blockIdx.x * blockDim.x + threadIdx.x) / FINISH_LANES, part = threadIdx.x % FINISH_LANES;
-    float g[7] = {0, 0, 0, 0, 0, 0, 0};
-    if (i < bodies) {
-        const int w = i / A.bodies_per_world, b = i % A.bodies_per_world;
-        for (int p = part; p < A.parts; p += FINISH_LANES) {
-            const float *src = A.partial + (((size_t)w * A.parts + p) * A.bodies_per_world + b) * 7;
-            for (int k = 0; k < 7; ++k) g[k] += src[k];
+    const long long bodies = (long long)A.worlds * A.bodies_per_world;
+    const int part = threadIdx.x % FINISH_LANES;
+    for (long long first = (long long)blockIdx.x * FINISH_BODIES; first < bodies; first += (long long)gridDim.x * FINISH_BODIES) {
+        const long long i = first + threadIdx.x / FINISH_LANES;
+        float g[7] = {0, 0, 0, 0, 0, 0, 0};
+        if (i < bodies) {
+            const long long w = i / A.bodies_per_world;
+            const int b = (int)(i - w * A.bodies_per_world);
+            for (int p = part; p < A.parts; p += FINISH_LANES) {
+                const float *src = A.partial + (((size_t)w * A.parts + p) * A.bodies_per_world + b) * 7;
+                for (int k = 0; k < 7; ++k) g[k] += src[k];
+            }
         }
+        for (int o = 1; o < FINISH_LANES; o <<= 1)
+            for (int k = 0; k < 7; ++k) g[k] += __shfl_xor(g[k], o, 64);
+        if (i >= bodies || part != 0) continue;
+        const float *bp = A.body_poses + 7 * (size_t)i;
+        const float q[4] = {bp[3], bp[4], bp[5], bp[6]};
+        const float qn = sqrtf(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
+        const float u[4] = {q[0] / qn, q[1] / qn, q[2] / qn, q[3] / qn};
+        const float ug = u[0] * g[3] + u[1] * g[4] + u[2] * g[5] + u[3] * g[6];
+        float *out = A.grad + 7 * (size_t)i;
+        out[0] = g[0];
+        out[1] = g[1];
+        out[2] = g[2];
+        for (int k = 0; k < 4; ++k) out[3 + k] = (g[3 + k] - u[k] * ug) / qn;
     }
-    for (int o = 1; o < FINISH_LANES; o <<= 1)
-        for (int k = 0; k < 7; ++k) g[k] += __shfl_xor(g[k], o, 64);
-    if (i >= bodies || part != 0) return;
-    const float *bp = A.body_poses + 7 * (size_t)i;
-    const float q[4] = {bp[3], bp[4], bp[5], bp[6]};
-    const float qn = sqrtf(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
-    const float u[4] = {q[0] / qn, q[1] / qn, q[2] / qn, q[3] / qn};
-    const float ug = u[0] * g[3] + u[1] * g[4] + u[2] * g[5] + u[3] * g[6];
-    float *out = A.grad + 7 * (size_t)i;
-    out[0] = g[0];
-    out[1] = g[1];
-    out[2] = g[2];
-    for (int k = 0; k < 4; ++k) out[3 + k] = (g[3 + k] - u[k] * ug) / qn;
 }
 
 }  // namespace
@@ -2335,10 +2341,10 @@ hipError_t launch_range_backward(const RangeBackwardArgs &a, hipStream_t stream)
 }
 
 hipError_t launch_pose_grad_finish(const PoseGradFinishArgs &a, hipStream_t stream) {
-    const int n = a.worlds * a.bodies_per_world;
+    const long long n = (long long)a.worlds * a.bodies_per_world;
     if (n <= 0) return hipSuccess;
-    if (n > INT32_MAX / FINISH_LANES - 256) return hipErrorInvalidValue;
-    pose_grad_finish_kernel<<<(n * FINISH_LANES + 255) / 256, 256, 0, stream>>>(a);
+    const long long groups = std::min((n + FINISH_BODIES - 1) / FINISH_BODIES, FINISH_MOST_GROUPS);
+    pose_grad_finish_kernel<<<(unsigned)groups, 256, 0, stream>>>(a);
     return hipGetLastError();
 }
 

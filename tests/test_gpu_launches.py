@@ -293,3 +293,35 @@ def test_a_gradient_takes_its_rays_as_its_forward_did(gpu, worlds):
     forward = _last_launch(r)[0]
     torch.where(torch.isfinite(distance), distance, 0.0).sum().backward()
     assert _last_launch(r)[0] == forward
+
+
+def test_gradients_of_more_than_2_to_28_bodies(gpu):
+    """1,048,577 worlds of 256 bodies, of which each world shows one: the gradient is taken, the shown bodies' is that of a
+    batch of the first 154 worlds, and the others' is zero, the last world's among them."""
+    import torch
+    worlds, bodies, shown = (1 << 20) + 1, 256, 255
+    _say(f"gradient of {worlds} worlds x {bodies} bodies")
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 40 GB of device memory")
+
+    def run(n):
+        r = BatchRenderer(1, 1, n, meshes=[make_icosphere(1.0, 0)], instances=[Instance(0)])
+        r.bind_bodies([shown], [[0, 0, 0, 0, 0, 0, 1]], [[1, 1, 1]], bodies)
+        poses = torch.zeros(n, bodies, 7, device="cuda")
+        poses[..., 6] = 1.0
+        at = torch.arange(n, device="cuda")
+        poses[:, shown, 0] = 0.1 + 0.01 * (at % 7)
+        poses[:, shown, 1] = 0.2
+        poses[:, shown, 2] = -4.0 - 0.01 * (at % 11)
+        r.set_body_poses(poses)
+        cams = torch.from_numpy(_eyes(1)).cuda().repeat(n, 1)
+        depth = r.render(cams, 1.0, depth=True, zero_copy=True)["depth"].clone()
+        assert bool(torch.isfinite(depth).all())
+        return r.pose_backward_depth(poses, cams, 1.0, depth, torch.ones_like(depth))
+
+    few, many = run(154), run(worlds)
+    assert float(few[:, shown].abs().amin(dim=0).max()) > 0 and torch.equal(many[:154], few)
+    assert torch.equal(many[-1, shown], few[(worlds - 1) % 77, shown])
+    assert int(torch.count_nonzero(many[:, :shown])) == 0
+    del few, many
+    torch.cuda.empty_cache()
