@@ -831,6 +831,8 @@ template <class Stats>
 __device__ void trace_world_lanes(const Scene S, const int world, const float3 o, const float3 d, const bool live,
                                   float &tmax, LaneHit &h, Stats &stats) {
     constexpr int NODE = 0, LEAF = 1, BACK = 2, DONE = 3;
+    const WideNode *const top_nodes = S.tlas_wide(), *const bottom_nodes = S.blas_wide();
+    const int *const top_parents = S.tlas_parent(), *const bottom_parents = S.blas_parent();
     const float3 inv_d = safe_inverse(d);
     int state = DONE, level = 0;
     int cur_t = -1, cur_b = -1;
@@ -867,7 +869,7 @@ __device__ void trace_world_lanes(const Scene S, const int world, const float3 o
                 int depth = bottom ? depth_b : depth_t;
                 const bool pending = on_back && (bits & 1ull);
                 if (on_node || pending) {
-                    const float4 *np = reinterpret_cast<const float4 *>((bottom ? S.blas_wide() : S.tlas_wide()) + cur);
+                    const float4 *np = reinterpret_cast<const float4 *>((bottom ? bottom_nodes : top_nodes) + cur);
                     const float4 f0 = np[0], f1 = np[1], f2 = np[2];
                     const int4 f3 = *reinterpret_cast<const int4 *>(np + 3);
                     const float3 ro = bottom ? lo : o, ri = bottom ? inv_ld : inv_d;
@@ -916,7 +918,7 @@ __device__ void trace_world_lanes(const Scene S, const int world, const float3 o
                     }
                 } else {
                     // climb one level; a level whose root is finished hands back to the level above
-                    const int parent = cur < 0 ? -1 : (bottom ? S.blas_parent() : S.tlas_parent())[cur];
+                    const int parent = cur < 0 ? -1 : (bottom ? bottom_parents : top_parents)[cur];
                     if (parent < 0) {
                         if (bottom) level = 0;  // the instance is done: resume the top level where it left off
                         else state = DONE;
