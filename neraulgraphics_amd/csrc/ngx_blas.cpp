@@ -155,6 +155,8 @@ static void plan_refits(const std::vector<int> &wide_index, BuiltMeshes &out) {
     const std::vector<BlasNode> &nodes = out.nodes;
     std::vector<int> size(nodes.size()), slot(nodes.size(), -1), height(nodes.size());
     std::vector<uint8_t> done(nodes.size(), 0);
+    out.refit_entries.reserve(nodes.size());
+    std::vector<int> members, sorted, starts;
     for (size_t m = 0; m < out.roots.size(); ++m) {
         const int base = out.roots[m], end = m + 1 < out.roots.size() ? out.roots[m + 1] : static_cast<int>(nodes.size());
         std::vector<RefitLayer> layers;
@@ -167,7 +169,7 @@ static void plan_refits(const std::vector<int> &wide_index, BuiltMeshes &out) {
             RefitLayer layer{static_cast<int>(out.refit_treelets.size()), 0};
             for (int root = base; root < end; ++root) {
                 if (done[root] || size[root] > most || (root != base && size[out.node_parent[root]] <= most)) continue;
-                std::vector<int> members{root};
+                members.assign(1, root);
                 for (size_t k = 0; k < members.size(); ++k) {
                     const BlasNode &n = nodes[members[k]];
                     for (int c = 0; n.count == 0 && c < 2; ++c)
@@ -181,7 +183,13 @@ static void plan_refits(const std::vector<int> &wide_index, BuiltMeshes &out) {
                         if (!done[nodes[i].a + c]) height[i] = std::max(height[i], 1 + height[nodes[i].a + c]);
                     levels = std::max(levels, height[i] + 1);
                 }
-                std::stable_sort(members.begin(), members.end(), [&](const int x, const int y) { return height[x] < height[y]; });
+                // by height, stable: counted
+                starts.assign(static_cast<size_t>(levels) + 1, 0);
+                for (const int i : members) ++starts[height[i] + 1];
+                for (int l = 0; l < levels; ++l) starts[l + 1] += starts[l];
+                sorted.resize(members.size());
+                for (const int i : members) sorted[starts[height[i]]++] = i;
+                members.swap(sorted);
                 out.refit_treelets.push_back(RefitTreelet{static_cast<int>(out.refit_entries.size()),
                                                           static_cast<int>(out.refit_levels.size()), levels, root == base ? 1 : 0});
                 for (size_t k = 0; k < members.size(); ++k) {
