@@ -92,8 +92,11 @@ struct TraceScene {
 
 // The bottom level is copied once per ray octant, near planes first, while the copies take at most this many bytes: a
 // two-child step then needs no minimum and maximum per pair of planes, 12 of its 58 vector instructions (4096 worlds
-// 128x128: 7.01 -> 6.73 ms, 64x64: 1.081 -> 1.044 ms, three meshes of 2,332 triangles). Larger trees would lose more to
-// the caches than that saves: an XCD's L2 is 4 MB, and rays of all octants are under way at once.
+// 128x128: 7.01 -> 6.73 ms, 64x64: 1.081 -> 1.044 ms, three meshes of 2,332 triangles, 0.6 MB of copies). Larger trees lose
+// more to the caches than that saves: an XCD's L2 is 4 MB, and rays of all octants are under way at once. With copies over
+// without, 1,024 images of 64x64 take 0.95 of the time for grids of 480 triangles (0.1 MB), 0.97 to 0.99 for 1,500 to 4,950 (0.4
+// to 1.2 MB), as long at 6,000 (1.5 MB), 1.07 of it at 9,000 (2.2 MB) and 1.14 at 19,800; rays in all directions, 4.2 M of them,
+// as long up to 0.3 MB, 1.01 to 1.05 of it up to 1.5 MB and 1.06 beyond.
 constexpr size_t OCTANT_COPIES_MAX_BYTES = (size_t)2 << 20;
 
 // The walks' depth limits: a wave-uniform stack of WALK_STACK entries per level for the packet walk, a 64-bit trail per
@@ -253,8 +256,8 @@ struct PoseGradFinishArgs {
 // The variants each kernel is built in, by workgroups of 256 threads per compute unit (its register budget
 // follows: 512 / (blocks x 4 / 4 SIMDs) registers a lane). 0 in a trace configuration picks the default.
 constexpr int RENDER_BLOCKS[] = {5, 6, 7}, RENDER_BLOCKS_DEFAULT = 7;
-constexpr int RGB_BLOCKS[] = {4, 5, 6, 7}, RGB_BLOCKS_DEFAULT_PACKET = 4, RGB_BLOCKS_DEFAULT_HYBRID = 7, RGB_TWO_CHILD_BLOCKS = 4, RGB_FEW_INSTANCES = 96;
-// The two-pass picture's shading pass by default: 4 workgroups per compute unit, the build without spills (the reference's
+constexpr int RGB_BLOCKS[] = {4, 5, 6, 7}, RGB_BLOCKS_DEFAULT_PACKET = 4, RGB_BLOCKS_DEFAULT_HYBRID = 7, RGB_TWO_CHILD_BLOCKS = 4, RGB_FEW_INSTANCES = 72;
+// The two-pass picture's shading pass by default: 4 workgroups per compute unit, the build without vector spills (the reference's
 // falling-bodies scene, hybrid walk: 4.97 ms a frame for 32 bodies at 128x128 against 5.84 at 5). The build for one light,
 // which holds less across its shadow walk: 6 where worlds have SHADE_MANY_INSTANCES or more on average, whose shadow walks
 // are long and wait for each other's, and 5 below, where the shading around them weighs more and a build of 6 spills in it

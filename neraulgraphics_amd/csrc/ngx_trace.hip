@@ -1559,7 +1559,6 @@ __device__ __forceinline__ void write_rgb(const RgbArgs &G, const size_t index, 
 // the floor's checker tint, or the sphere's material.
 __device__ __forceinline__ void hit_material(const RgbArgs &G, const int kind, const float3 o, const float3 d, const float best,
                                              const LaneHit &h, float3 &point, float3 &normal, float4 &m0, float4 &m1) {
-    const RenderArgs &A = G.r;
     const ShadeScene &E = G.shade;
     point = add3(o, mul3(d, best));
     int object;
@@ -1629,7 +1628,6 @@ template <int WALK, class Shadow>
 __device__ __forceinline__ void shade_hit(const RgbArgs &G, PairLds *L, const int world, const int kind, const float best,
                                           const LaneHit &h, bool &active, float3 &o, float3 &d, uint32_t &rng,
                                           float3 &radiance, float &throughput) {
-    const RenderArgs &A = G.r;
     const ShadeScene &E = G.shade;
     const bool hit = active && kind != OBJECT_NONE;
     if (active && !hit) {
@@ -2207,9 +2205,11 @@ static int resident_grid(const int compute_units, const long long tiles) {
 }
 
 // The RGB kernels' variants: 4, 5, 6 or 7 workgroups per compute unit for the packet and hybrid walks, 4 for the per-lane
-// walk; by default 4 for the packet walk, and for the hybrid walk 4, which spills nothing, or 7 in worlds of many instances,
-// whose walks are long and wait for each other's (two or four samples: 64 worlds of 64 mirrors 6.73 ms at 4, 6.75 at 5, 7.29
-// at 7; 256 worlds of 40 instances 2.84, 2.97, 3.07; 1,024 worlds of 256 mirrors 219.7, 201.5, 192.2).
+// walk; by default 4 for the packet walk, and for the hybrid walk 4, which spills least (69 of 128 vector registers, 167 of 72
+// at 7), or 7 in worlds of many instances, whose walks are long and wait for each other's (two or four samples: 64 worlds of
+// 64 mirrors 128x128 6.73 ms at 4, 6.75 at 5, 7.29 at 7; 256 worlds of 40 instances 2.84, 2.97, 3.07; 1,024 worlds of 256
+// mirrors 219.7, 201.5, 192.2). The line lies between the sizes where one overtakes the other: 256 worlds of mirrors 96x96 of
+// 64 instances 7.75 and 7.82 ms at 4 and 7, of 80 9.98 and 9.63, of 96 11.69 and 11.36, of 128 15.01 and 14.23.
 static int rgb_hybrid_blocks(const RenderArgs &a) {
     return (long long)a.s.total * a.cameras_per_world > (long long)RGB_FEW_INSTANCES * a.views ? RGB_BLOCKS_DEFAULT_HYBRID : 4;
 }
