@@ -19,8 +19,10 @@ timed on this host on a bounded sample.
 python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--no-graph] [--no-tune] [--no-lidar] [--no-rgb] [--no-bwd]
                 [--only LEG] [--trace-config JSON]"""
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -544,9 +546,9 @@ _TRAFFIC_FIELDS = {
 }
 
 
-def _traffic(summary, kind, chosen):
-    """HBM bytes per launch from the summary (or one of its `variants`) profiled under the configuration this run
-    chose, compared on the fields the kernel depends on; else the summary's own figure. Returns (bytes, matched)."""
+def _profile_entry(summary, kind, chosen):
+    """The summary, or the one of its `variants`, that was profiled under the configuration this run chose, compared on the
+    fields the kernel depends on; else the summary itself. Returns (entry, matched)."""
     fields, variants = _TRAFFIC_FIELDS[kind]
 
     def key(c):
@@ -554,8 +556,53 @@ def _traffic(summary, kind, chosen):
 
     for entry in [summary] + list(summary.get("variants", [])):
         if entry.get("trace_config") is not None and key(entry["trace_config"]) == key(chosen):
-            return entry.get("hbm_bytes_per_launch"), True
-    return summary.get("hbm_bytes_per_launch"), False
+            return entry, True
+    return summary, False
+
+
+def _traffic(summary, kind, chosen):
+    """HBM bytes per launch of the entry profiled under the configuration this run chose, else of the summary itself.
+    Returns (bytes, matched)."""
+    entry, matched = _profile_entry(summary, kind, chosen)
+    return entry.get("hbm_bytes_per_launch"), matched
+
+
+_KERNEL_SOURCES = ("ngx_device.h", "ngx_kernels.h", "ngx_trace.hip", "ngx_tlas.hip")
+
+
+def _code_digest(*texts):
+    """A digest of C++ sources that does not change with their comments and white space."""
+    code = "".join(re.sub(r"//[^\n]*|/\*.*?\*/", " ", t, flags=re.S) for t in texts)
+    return hashlib.sha256("".join(code.split()).encode()).hexdigest()[:16]
+
+
+def kernel_digest():
+    """The digest of the kernels' sources; a profile holds the one of the kernels it was taken on."""
+    texts = []
+    for name in _KERNEL_SOURCES:
+        with open(os.path.join(ROOT, "neraulgraphics_amd", "csrc", name)) as f:
+            texts.append(f.read())
+    return _code_digest(*texts)
+
+
+def _built(config, instances_per_world, largest_mesh, bodies):
+    """The configuration with the variants that 0 stands for named, by the library's rules: the depth and hit passes' hybrid
+    walk is built for 8 workgroups per compute unit where the launch is persistent (and the bottom levels small, as every
+    scene's here is) and for 7 otherwise, a picture's shading pass under one light for 6 in worlds of 16 instances or more
+    and for 5 in smaller ones, and the depth backward for 6 up to 79 bodies a world and 5 beyond."""
+    c = dict(config)
+    hybrid = c.get("packet") and c.get("persistent") and largest_mesh >= c.get("lane_min_triangles", 0)
+    c["render_blocks"] = c.get("render_blocks") or (8 if hybrid else 7)
+    c["rgb_blocks"] = c.get("rgb_blocks") or (6 if instances_per_world >= 16 else 5)
+    c["backward_blocks"] = c.get("backward_blocks") or (6 if bodies <= 79 else 5)
+    return c
+
+
+def _profiled(summary, kind, built):
+    """(HBM bytes per launch, whether they were counted on the kernels this run's sources hold and under the configuration
+    it ran, the profile's entry)."""
+    entry, matched = _profile_entry(summary, kind, built)
+    return entry.get("hbm_bytes_per_launch"), matched and summary.get("kernel_digest") == kernel_digest(), entry
 
 
 def main():
@@ -651,7 +698,8 @@ def main():
         achieved = rb / (c2["render_ms"] * 1e-3) / 1e9
         kernel = "render_persistent_kernel" if c2["trace_config"].get("persistent") else "render_kernel"
         summary = _profile_summary(f"{kernel}_body_worlds_traffic.json")
-        traffic, same = _traffic(summary, "render", c2["trace_config"])
+        built = _built(c2["trace_config"], c2["instances"] / 4096, max(m.triangle_count for m in c2["cfg"]["meshes"]), 64)
+        traffic, same, entry = _profiled(summary, "render", built)
         bb = build_bytes(4096, 64, c2["instances"])
         line.update({
             "value": c2["views"] / sec,
@@ -667,13 +715,13 @@ def main():
             "hit_fraction": c2["hit_frac"],
             "roofline": {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                         # whether the traffic was counted under the configuration this run's autotuner chose (spills,
-                         # and so traffic, differ between builds)
+                         # whether the traffic was counted on these kernels and under the configuration this run's
+                         # autotuner chose (spills, and so traffic, differ between builds)
                          "traffic_same_config": same,
                          "algorithmic_bytes_per_launch": rb,
                          # the bound that holds: the fraction of cycles every SIMD issues a vector instruction
-                         # (rocprof, same kernel)
-                         "valu_busy": summary.get("kernels", {}).get("render_kernel_sq", {}).get("valu_busy")},
+                         # (rocprof, same kernel and configuration; null where there is no such profile)
+                         "valu_busy": entry.get("kernels", {}).get("render_kernel_sq", {}).get("valu_busy") if same else None},
             "step_hbm_frac": (rb + build_bytes(4096, 64, c2["instances"])) / sec / 1e9 / HBM_PEAK_GBS,
             # the top-level build alone, the step's one bandwidth-shaped phase: its algorithmic bytes over its event time
             "build_roofline": {"bound": "hbm", "kernel": "tlas_build_kernel",
@@ -693,8 +741,8 @@ def main():
         line.update(fwd_bwd_images_per_s=c4["fwd_bwd_images_per_s"], fwd_images_per_s=c4["fwd_images_per_s"],
                     fwd_bwd_over_fwd=c4["ratio"])
         bw = c4["backward_bytes"] / (c4["backward_kernel_ms"] * 1e-3) / 1e9
-        traffic, same = _traffic(_profile_summary("depth_backward_kernel_posed_bodies_traffic.json"), "backward",
-                                 c4["trace_config"])
+        traffic, same, _ = _profiled(_profile_summary("depth_backward_kernel_posed_bodies_traffic.json"), "backward",
+                                     _built(c4["trace_config"], 32, 320, 32))
         line["fwd_bwd_roofline"] = {
             "bound": "hbm", "kernel": "depth_backward_kernel", "achieved": bw, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": bw / HBM_PEAK_GBS, "traffic": traffic, "traffic_same_config": same,
@@ -706,9 +754,9 @@ def main():
                     rgb_depth_id_trace_config=crgb["trace_config"])
         rgbb = render_bytes(crgb["views"], 128, 128, crgb["instances"]) + picture_bytes(crgb["views"], 128, 128, crgb["instances"])
         summary = _profile_summary("rgb_two_pass_body_worlds_traffic.json")
-        traffic, same = _traffic(summary, "rgb", crgb["trace_config"])
+        traffic, same, entry = _profiled(summary, "rgb", _built(crgb["trace_config"], crgb["instances"] / crgb["views"], 2000, 64))
         if traffic is not None:
-            traffic += summary["kernels"]["render_persistent_kernel"]["hbm_bytes_per_launch"]
+            traffic += entry["kernels"]["render_persistent_kernel"]["hbm_bytes_per_launch"]
         achieved = rgbb / (crgb["kernel_ms"] * 1e-3) / 1e9
         line["rgb_depth_id_roofline"] = {
             "bound": "hbm", "kernel": "render_persistent_kernel + rgb_hit_kernel + rgb_shade_kernel (one render call)",
