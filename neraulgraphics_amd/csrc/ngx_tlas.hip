@@ -996,7 +996,7 @@ __global__ __launch_bounds__(1024) void ray_order_segment_kernel(const int R, co
                                                                  const uint32_t *before, const uint32_t *totals, int *order) {
     constexpr int NW = 16, STEPS = RAY_ORDER_SEGMENT / (64 * NW);
     __shared__ RayOrderShared<NW> sh;
-    __shared__ uint32_t start[RAY_ORDER_CELLS];  // the first place of the segment's rays of each cell
+    alignas(16) __shared__ uint32_t start[RAY_ORDER_CELLS];  // the first place of the segment's rays of each cell, written four at a time
     const int world = blockIdx.x / segments, s = blockIdx.x % segments;
     const size_t base = (size_t)world * R;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
