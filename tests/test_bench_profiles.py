@@ -47,3 +47,9 @@ def test_the_variants_that_zero_stands_for(bench):
     assert bench._built(dict(CONFIG, lane_min_triangles=1 << 30), 130, 2000, 64)["render_blocks"] == 7
     asked = dict(CONFIG, render_blocks=5, rgb_blocks=7, backward_blocks=4)
     assert bench._built(asked, 130, 2000, 64) == asked
+
+
+def test_committed_profiles_say_which_kernels_they_are_of(bench):
+    for name in os.listdir(os.path.join(ROOT, "profiles")):
+        if name.endswith("_traffic.json"):
+            assert len(bench._profile_summary(name).get("kernel_digest", "")) == 16, name
