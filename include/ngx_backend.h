@@ -147,7 +147,9 @@ typedef struct {
 } ngx_shading;
 
 /* make_cuda_backend (src/backend.h:88) with BatchRenderer's constructor checks (src/batch.cpp:47-75). More than
- * NGX_MAX_TRIANGLES triangles over all meshes are refused with NGX_UNSUPPORTED. */
+ * NGX_MAX_TRIANGLES triangles over all meshes are refused with NGX_UNSUPPORTED. A context whose pictures may gain by them
+ * (4,096 tiles or more) holds tables of its views from its creation on, 336 bytes an instance and camera, where they take
+ * at most 1 GiB and the device has room. */
 #define NGX_MAX_TRIANGLES 16777216
 ngx_status ngx_create(const ngx_scene_desc *scene, ngx_ctx **out);
 void ngx_destroy(ngx_ctx *ctx);
@@ -217,8 +219,8 @@ ngx_status ngx_pose_backward_depth(ngx_ctx *ctx, const float *body_poses, const 
  * its per-workgroup partial sums in a fixed device array of NGX_NOALLOC_SCRATCH_FLOATS floats (32 MiB) that each GPU
  * holds from ngx_create until the process ends, instead of memory the context allocates; it calls no allocator
  * and does not wait on the stream. It needs views x parts x bodies_per_world x 7 floats, parts = min(16,
- * max(1, tiles / 8)) for a frame of `tiles` 8x8 tiles; a larger call is refused with NGX_INVALID_ARGUMENT
- * before anything changes. Every call on one GPU shares that GPU's array (it keeps the last call's contents;
+ * max(1, tiles / 8)) for a frame of `tiles` 8x8 tiles (more where there are few views and the array holds them); a call
+ * that needs more than the array is refused with NGX_INVALID_ARGUMENT before anything changes. Every call on one GPU shares that GPU's array (it keeps the last call's contents;
  * each call overwrites what it reads): calls that overlap on one GPU, from other streams, threads or
  * contexts, race and give wrong gradients. */
 #define NGX_NOALLOC_SCRATCH_FLOATS (8 * 1024 * 1024)
@@ -258,9 +260,10 @@ const char *ngx_last_error(void);
  *  tile_w      a wavefront's pixels are a tile_w x (64 / tile_w) tile: 8, 16, 32 or 64;
  *  xcd_remap   1: consecutive workgroups, which the dispatcher deals round-robin over the eight XCDs, are
  *              renumbered so each XCD works through one contiguous range of tiles (one L2 per XCD);
- *  packet      1: the wavefront walks its 64 rays as a packet (the default); 0: each lane walks its own ray;
+ *  packet      1: the wavefront walks its rays as a packet (the default): 64, or 4 to 16 in launches of few rays (up to
+ *              131,072, or 65,536 where normals, colours or range gradients show the triangle); 0: each lane its own ray;
  *  pair_limit  packet walk: (ray, triangle) pairs queued before they are tested together, 1..64;
- *  persistent  1 (the default): a fixed grid of 8 workgroups per compute unit takes tiles from per-XCD
+ *  persistent  1 (the default): a fixed grid of as many workgroups as the device holds takes tiles from per-XCD
  *              counters; 0: one wavefront per tile, dealt by the dispatcher;
  *  lane_min_triangles  packet walk: the bottom level of meshes with at least this many triangles is walked
  *              lane by lane (each ray its own path) instead of as a packet (default 300);
@@ -274,11 +277,12 @@ const char *ngx_last_error(void);
 typedef struct {
     int32_t tile_w, xcd_remap, packet, pair_limit, persistent, lane_min_triangles, sort_rays;
     /* Kernel variants, by the workgroups of 256 threads per compute unit each is built for (the registers a lane
-     * may hold follow from it; 0 picks the walk's default): the depth / normal / ID kernel 5, 6 or 7 (default 7),
-     * the RGB kernel 4, 5, 6 or 7 (default 4 for the packet walk, 7 for the hybrid one; the two-pass picture's hit pass
-     * takes render_blocks and its shading pass rgb_blocks, default 5 for a scene of one light and 4 otherwise), the
-     * ray-query kernel 5, 6 or 7 (default 6), the depth backward 4, 5 or 6 (default 5). The per-lane walk has one
-     * variant of each, and so has the RGB kernel for pictures of few rays, whose wavefronts take 4 to 16 of them. */
+     * may hold follow from it; 0 picks the default): the depth / normal / ID kernel 5, 6 or 7 (default 7, and 8 for
+     * persistent launches of the hybrid walk where the bottom levels are small enough to be copied per ray octant), the
+     * RGB kernel 4, 5, 6 or 7 (default 4 for the packet walk; for the hybrid one 4, or 7 in worlds of more than 72 instances
+     * on average; the two-pass picture's hit pass takes render_blocks and its shading pass rgb_blocks, default 4, and for a
+     * scene of one light 5, or 6 in worlds of 16 instances or more), the ray-query kernel 5, 6 or 7 (default 6), the depth
+     * backward 4, 5 or 6 (default 6, or 5 for more than 79 bodies a world). The per-lane walk has one variant of each, and so has the RGB kernel for pictures of few rays, whose wavefronts take 4 to 16 of them. */
     int32_t render_blocks, rgb_blocks, ray_blocks, backward_blocks;
     int32_t rgb_two_pass;
 } ngx_trace_config;
